@@ -240,6 +240,12 @@ __device__ __forceinline__ TileCoord TileOf(int tiles_x, int tiles_y) {
   return t;
 }
 
+// Launch form of a run kernel: its points per lane VX, plus kRagged when a
+// grid's x extent is not a multiple of VX.
+constexpr int kRagged = 256;
+constexpr int FormVX(int form) { return form & (kRagged - 1); }
+constexpr bool FormRagged(int form) { return (form & kRagged) != 0; }
+
 // ------------------------------------------------------------- staged grid
 // One staged grid of element type T.  A block is BX = 64 lanes (one wave)
 // per row and BY waves; wave r owns tile row y0 - HY + r, so the first and
@@ -251,8 +257,16 @@ __device__ __forceinline__ TileCoord TileOf(int tiles_x, int tiles_y) {
 //   NSLOT   planes in the LDS ring (ZR - ZL + 2)
 //   M       element type in global memory; values are converted to T as
 //           they enter LDS (T = M for Physis grids)
+//   RAGGED  the grid's x extent need not be a multiple of VX.  A lane's
+//           vector may then hang over the end of its row, where it holds the
+//           linear neighbours (the next row's first points; the range check
+//           works dword by dword) and not the wrapped points of a periodic
+//           row, and is dropped whole when it starts before the window.  The
+//           right halo columns therefore follow the row's last point instead
+//           of the tile's: they are loaded one by one and stored after (over)
+//           the overhang.
 template <typename T, int VX, int BY, int HX, int HY, int NSLOT,
-          bool PERIODIC, typename M = T>
+          bool PERIODIC, typename M = T, bool RAGGED = false>
 struct Stage {
   static constexpr int BX = kWave;
   static constexpr int kTX = BX * VX;
@@ -287,12 +301,15 @@ struct Stage {
   // a plane step only adds the plane offset.
   struct Addr {
     int xo, ho, yo;
+    int hc;  // RAGGED: LDS column of the lane's halo point
   };
   __device__ __forceinline__ static Addr Prepare(const int *dim, int x0, int y,
                                                  int lane) {
     const int hl = lane < 2 * HX ? lane : 0;
-    const int hx = hl < HX ? x0 - HX + hl : x0 + kTX + (hl - HX);
+    const int rc = RAGGED && dim[0] - x0 < kTX ? dim[0] - x0 : kTX;
+    const int hx = hl < HX ? x0 - HX + hl : x0 + rc + (hl - HX);
     Addr a;
+    a.hc = hl < HX ? kPad - HX + hl : kPad + rc + (hl - HX);
     if (PERIODIC) {
       a.xo = WrapIndex(x0 + lane * VX, dim[0]);
       a.ho = WrapIndex(hx, dim[0]);
@@ -334,7 +351,19 @@ struct Stage {
   }
 
   // Writes the wave's row of the plane into one LDS slot.
+  __device__ __forceinline__ void Store(T *slot, int wave, int lane,
+                                        const Addr &a) const {
+    StoreAt(slot, wave, lane, RAGGED ? a.hc : HaloColumn(lane));
+  }
   __device__ __forceinline__ void Store(T *slot, int wave, int lane) const {
+    static_assert(!RAGGED, "a ragged row's halo columns come from its Addr");
+    StoreAt(slot, wave, lane, HaloColumn(lane));
+  }
+  __device__ __forceinline__ static int HaloColumn(int lane) {
+    return lane < HX ? kPad - HX + lane : kPad + kTX + (lane - HX);
+  }
+  __device__ __forceinline__ void StoreAt(T *slot, int wave, int lane,
+                                          int hc) const {
     T *row = slot + wave * kRow;
     if constexpr (__is_same(T, M)) {
       StoreVec(row + kPad + lane * VX, own);
@@ -344,9 +373,7 @@ struct Stage {
       for (int i = 0; i < VX; ++i) cv[i] = Convert<T, M>(own[i]);
       StoreVec(row + kPad + lane * VX, cv);
     }
-    if (lane < 2 * HX)
-      row[lane < HX ? kPad - HX + lane : kPad + kTX + (lane - HX)] =
-          Convert<T, M>(halo);
+    if (lane < 2 * HX) row[hc] = Convert<T, M>(halo);
   }
 
   // Row segment of `slot` at row `row` covering x offsets XL .. VX-1+XR

@@ -63,7 +63,8 @@ PROGRAM_SOURCES = [os.path.join(PROGRAMS, "diffusion7.c"),
                    os.path.join(PROGRAMS, "udt7.c"),
                    os.path.join(PROGRAMS, "stencil2d.c"),
                    os.path.join(PROGRAMS, "mixed7.c"),
-                   os.path.join(ROOT, "tests", "programs", "systests.c")]
+                   os.path.join(ROOT, "tests", "programs", "systests.c"),
+                   os.path.join(ROOT, "tests", "programs", "ragged.c")]
 
 
 def _run(cmd: list[str]) -> None:

@@ -151,15 +151,16 @@ __global__ __launch_bounds__(kWave *kBY) void SweepKernel(
   const int dim[3] = {nx, ny, nz};
   const BufWin<M> pw =
       BufWin<M>::Make(pin, n, (long)(zb - 2) * nxy, (long)(ze + 2) * nxy);
-  S st[kPD];
+  // (every load of the prologue is issued before the first one is stored)
+  S st[kPD], pro[3];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    st[0].Load(pw, pin, dim, x0, yrow, zb - 1 + k, lane);
-    st[0].Store(lds + k * S::kPlane, wave, lane);
-  }
+  for (int k = 0; k < 3; ++k)
+    pro[k].Load(pw, pin, dim, x0, yrow, zb - 1 + k, lane);
 #pragma unroll
   for (int k = 0; k < kPD; ++k)
     st[k].Load(pw, pin, dim, x0, yrow, zb + 2 + k, lane);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) pro[k].Store(lds + k * S::kPlane, wave, lane);
   int base = 0;
   const BufWin<M> ow =
       BufWin<M>::Make(pout, n, (long)zb * nxy, (long)ze * nxy);
@@ -282,13 +283,10 @@ __global__ __launch_bounds__(kWave *BY) void TwoSweepKernel(
   for (int g = 0; g < kNumF; ++g)
     fw[g] = BufWin<M>::Make(f.g[g], n, (long)(zb - 1) * nxy,
                             (long)(ze + 1) * nxy);
-  SA st[kPD];
+  SA st[kPD], pro[3];
   const typename SA::Addr ra = SA::Prepare(dim, x0, yrow, lane);
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    st[0].Load(aw, pin, dim, ra, zb - 2 + k);
-    st[0].Store(a_lds + k * SA::kPlane, wave, lane);
-  }
+  for (int k = 0; k < 3; ++k) pro[k].Load(aw, pin, dim, ra, zb - 2 + k);
 #pragma unroll
   for (int k = 0; k < kPD; ++k) st[k].Load(aw, pin, dim, ra, zb + 1 + k);
   constexpr bool kRing = sizeof(M) == 2 && VX == 2;
@@ -310,6 +308,8 @@ __global__ __launch_bounds__(kWave *BY) void TwoSweepKernel(
     }
   };
   load1(zb - 1, 0);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) pro[k].Store(a_lds + k * SA::kPlane, wave, lane);
   __syncthreads();
   for (int sc = zb - 1; sc <= ze + 1; sc += 4) {
 #pragma unroll
@@ -413,30 +413,26 @@ __global__ __launch_bounds__(kWave *kBY) void ResidualKernel(
     BufWin<ME> ew;
     if constexpr (UPDATE)
       ew = BufWin<ME>::Make(e, n, (long)(zb - 2) * nxy, (long)(ze + 2) * nxy);
-    S st[kPD];
-    SE se[kPD];
-    auto load = [&](int slot, int z) {
-      st[slot].Load(pw, pin, dim, x0, yrow, z, lane);
-      if constexpr (UPDATE) se[slot].Load(ew, e, dim, x0, yrow, z, lane);
+    S st[kPD], pro[3];
+    SE se[kPD], proe[3];
+    auto load = [&](S &p, SE &pe, int z) {
+      p.Load(pw, pin, dim, x0, yrow, z, lane);
+      if constexpr (UPDATE) pe.Load(ew, e, dim, x0, yrow, z, lane);
     };
-    auto store = [&](int slot, double *dst) {
+    auto store = [&](S &p, const SE &pe, double *dst) {
       if constexpr (UPDATE) {
 #pragma unroll
         for (int i = 0; i < VX; ++i)
-          st[slot].own[i] =
-              st[slot].own[i] + Convert<double, ME>(se[slot].own[i]) * inv_sigma;
-        st[slot].halo =
-            st[slot].halo + Convert<double, ME>(se[slot].halo) * inv_sigma;
+          p.own[i] = p.own[i] + Convert<double, ME>(pe.own[i]) * inv_sigma;
+        p.halo = p.halo + Convert<double, ME>(pe.halo) * inv_sigma;
       }
-      st[slot].Store(dst, wave, lane);
+      p.Store(dst, wave, lane);
     };
+    // (every load of the prologue is issued before the first one is stored)
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      load(0, zb - 1 + k);
-      store(0, lds + k * S::kPlane);
-    }
+    for (int k = 0; k < 3; ++k) load(pro[k], proe[k], zb - 1 + k);
 #pragma unroll
-    for (int k = 0; k < kPD; ++k) load(k, zb + 2 + k);
+    for (int k = 0; k < kPD; ++k) load(st[k], se[k], zb + 2 + k);
     int base = 0;
     BufWin<double> ow;
     if constexpr (UPDATE)
@@ -452,6 +448,8 @@ __global__ __launch_bounds__(kWave *kBY) void ResidualKernel(
       fw[g] = BufWin<float>::Make(f.g[g], n, (long)zb * nxy, (long)ze * nxy);
       fw[g].template Load<VX>(doff + zb * nxy, fv[g][0]);
     }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) store(pro[k], proe[k], lds + k * S::kPlane);
     __syncthreads();
     for (int zc = zb; zc < ze; zc += kPD) {
 #pragma unroll
@@ -490,9 +488,9 @@ __global__ __launch_bounds__(kWave *kBY) void ResidualKernel(
           if constexpr (WRHS)
             physis_hip::StoreMasked<ME, VX>(rw, off, rv, mask);
         }
-        store(k, lds + RingSlot<4>(base, 3) * S::kPlane);
+        store(st[k], se[k], lds + RingSlot<4>(base, 3) * S::kPlane);
         __syncthreads();
-        load(k, z + 2 + kPD);
+        load(st[k], se[k], z + 2 + kPD);
         base = RingSlot<4>(base, 1);
       }
     }

@@ -1794,8 +1794,11 @@ std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
        "// last " << k.hy << " load halo rows), staged planes PD steps ahead,\n"
        "// centre-only grids one step ahead.  RED: reduction operator of a\n"
        "// PSStencilMapReduce execution, or -1.\n";
-  o << "template <int VX, int BY, int RED>\n__global__ __launch_bounds__(64 * BY) "
-       "void __PSStencilRun_" << n << "(\n    " << Join(params, ", ") << ") {\n";
+  o << "// FORM: VX, plus kRagged for x extents that are not multiples of VX.\n"
+       "template <int FORM, int BY, int RED>\n__global__ __launch_bounds__(64 * BY) "
+       "void __PSStencilRun_" << n << "(\n    " << Join(params, ", ") << ") {\n"
+       "  constexpr int VX = physis_hip::FormVX(FORM);\n"
+       "  constexpr bool RAGGED = physis_hip::FormRagged(FORM);\n";
   o << "  constexpr int PD = " << PrefetchFor(k) << ";\n";
   o << "  constexpr int HY = " << k.hy << ";\n";
   o << "  constexpr int TX = 64 * VX, TY = BY - 2 * HY;\n";
@@ -1803,8 +1806,8 @@ std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
     if (g.mode != GridParam::kStaged) continue;
     int nslot = g.zr - g.zl + 2;
     o << "  typedef physis_hip::Stage<" << g.elem << ", VX, BY, " << g.hx
-      << ", HY, " << nslot << ", " << (g.periodic ? "true" : "false") << "> S_"
-      << g.name << ";\n";
+      << ", HY, " << nslot << ", " << (g.periodic ? "true" : "false") << ", "
+      << g.elem << ", RAGGED> S_" << g.name << ";\n";
     o << "  __shared__ __attribute__((aligned(16))) " << g.elem << " "
       << g.name << "_lds[S_" << g.name << "::kLdsElems];\n";
   }
@@ -1841,11 +1844,12 @@ std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
       o << "    S_" << G << " " << G << "_st[PD];\n";
       o << "    const typename S_" << G << "::Addr " << G << "_ra = S_" << G
         << "::Prepare(" << G << ".dim, x0, yrow, lane);\n";
-      o << "#pragma unroll\n    for (int k = 0; k < " << nslot - 1 << "; ++k) {\n"
-        << "      " << G << "_st[0].Load(" << G << "_w, " << G << ".p, " << G
-        << ".dim, " << G << "_ra, zb + " << g.zl << " + k);\n"
-        << "      " << G << "_st[0].Store(" << G << "_lds + k * S_" << G
-        << "::kPlane, wave, lane);\n    }\n";
+      // every load of the prologue is issued before the first one is
+      // stored: a short z chunk then waits for memory once
+      o << "    S_" << G << " " << G << "_pro[" << nslot - 1 << "];\n"
+        << "#pragma unroll\n    for (int k = 0; k < " << nslot - 1 << "; ++k)\n"
+        << "      " << G << "_pro[k].Load(" << G << "_w, " << G << ".p, " << G
+        << ".dim, " << G << "_ra, zb + " << g.zl << " + k);\n";
       o << "#pragma unroll\n    for (int k = 0; k < PD; ++k)\n      " << G
         << "_st[k].Load(" << G << "_w, " << G << ".p, " << G << ".dim, " << G
         << "_ra, zb + " << g.zr + 1 << " + k);\n";
@@ -1871,6 +1875,12 @@ std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
         << "_enxy, (long)ze * " << G << "_enxy);\n";
     }
   }
+  for (auto &g : k.grids)
+    if (g.mode == GridParam::kStaged)
+      o << "#pragma unroll\n    for (int k = 0; k < " << g.zr - g.zl + 1
+        << "; ++k)\n      " << g.name << "_pro[k].Store(" << g.name
+        << "_lds + k * S_" << g.name << "::kPlane, wave, lane, " << g.name
+        << "_ra);\n";
   o << "    __syncthreads();\n";
   o << "    __PSCtx_" << n << " ctx;\n";
   for (auto &g : k.grids)
@@ -1891,10 +1901,10 @@ std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
     o << "    ctx." << g.name << "_p = " << g.name << ".p;\n"
       << "    for (int d = 0; d < 3; ++d) ctx." << g.name << "_dim[d] = "
       << g.name << ".dim[d];\n";
-  // VX > 1 runs only when every grid's x extent is a multiple of 4 and
-  // tiles start at multiples of TX: the compiler may use the low bits
-  o << "    if constexpr (VX > 1) {\n"
-       "      __builtin_assume((xs & (VX - 1)) == 0);\n";
+  // tiles start at multiples of TX, and every grid's x extent is a multiple
+  // of 4 unless RAGGED: the compiler may use the low bits
+  o << "    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);\n"
+       "    if constexpr (VX > 1 && !RAGGED) {\n";
   for (auto &g : k.grids)
     if (!g.user && (g.read || g.emitted) && g.dims == (k.rows2d ? 2 : 3))
       o << "      __builtin_assume((ctx." << g.name << "_dim[0] & 3) == 0);\n";
@@ -2006,7 +2016,8 @@ std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
     int nslot = g.zr - g.zl + 2;
     o << "        " << g.name << "_st[k % PD].Store(" << g.name
       << "_lds + physis_hip::RingSlot<" << nslot << ">(" << g.name << "_base, "
-      << nslot - 1 << ") * S_" << g.name << "::kPlane, wave, lane);\n";
+      << nslot - 1 << ") * S_" << g.name << "::kPlane, wave, lane, " << g.name
+      << "_ra);\n";
   }
   o << "        __syncthreads();\n";
   for (auto &g : k.grids) {
@@ -2259,14 +2270,15 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
   if (rb)
     o << "// Red-black: one pass is one iteration (red sweep u', black sweep\n"
          "// u''); dom is the map's domain, gd the whole grid the pass tiles.\n";
-  o << "template <int VX, int BY>\n__global__ __launch_bounds__(64 * BY) void __PSStencilRun2_"
+  o << "// RAGGED: x extents that are not multiples of VX.\n"
+       "template <int VX, int BY, bool RAGGED>\n__global__ __launch_bounds__(64 * BY) void __PSStencilRun2_"
     << n << "(\n    __PSDomain dom, " << (rb ? "__PSDomain gd, " : "") << V
     << " src, " << V << " dst, " << T
     << " *__restrict__ mid" << (sp.empty() ? "" : ", " + Join(sp, ", "))
     << ", physis_hip::RunShape sh) {\n";
   o << "  constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;\n"
     << "  typedef physis_hip::Stage<" << T << ", VX, BY, 2, 2, 6, " << per
-    << "> SA;\n"
+    << ", " << T << ", RAGGED> SA;\n"
     << "  typedef physis_hip::Stage<" << T << ", VX, BY, 1, 1, 6, false> SB;\n"
     << "  __shared__ __attribute__((aligned(16))) " << T << " a_lds[SA::kLdsElems];\n"
     << "  __shared__ __attribute__((aligned(16))) " << T << " b_lds[SB::kLdsElems];\n"
@@ -2285,23 +2297,32 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
        "  const int xs = x0 + lane * VX;\n"
        "  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];\n"
        "  const int n = nxy * src.dim[2];\n"
-       "  // tiles start at multiples of TX and two-sweep runs need nx % 4 == 0\n"
+       "  // tiles start at multiples of TX\n"
        "  __builtin_assume((xs & (VX - 1)) == 0);\n"
-       "  __builtin_assume((nx & (VX - 1)) == 0);\n"
+       "  if constexpr (!RAGGED) __builtin_assume((nx & (VX - 1)) == 0);\n"
     << "  const physis_hip::BufWin<" << T << "> aw = physis_hip::BufWin<" << T
     << ">::Make(src.p, n, (long)(zb - 3) * nxy, (long)(ze + 3) * nxy);\n"
     << "  const physis_hip::BufWin<" << T << "> dw = physis_hip::BufWin<" << T
     << ">::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);\n"
     << "  const physis_hip::BufWin<" << T << "> mw = physis_hip::BufWin<" << T
     << ">::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);\n"
-    << "  SA st[PD];\n"
+    // A red-black pass issues every load of the prologue before the first
+    // one is stored (512^3 iterations 4% faster); a map pair stores each
+    // plane before the next is loaded: with all of them in flight the
+    // compiler schedules the loop worse (512^3 passes 8% slower).
+    << "  SA st[PD]" << (rb ? ", pro[4]" : "") << ";\n"
        "  const typename SA::Addr ra = SA::Prepare(src.dim, x0, yrow, lane);\n"
-       "#pragma unroll\n  for (int k = 0; k < 4; ++k) {\n"
-       "    st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);\n"
-       "    st[0].Store(a_lds + k * SA::kPlane, wave, lane);\n  }\n"
-       "#pragma unroll\n  for (int k = 0; k < PD; ++k)\n"
+    << (rb ? "#pragma unroll\n  for (int k = 0; k < 4; ++k)\n"
+             "    pro[k].Load(aw, src.p, src.dim, ra, zb - 2 + k);\n"
+           : "#pragma unroll\n  for (int k = 0; k < 4; ++k) {\n"
+             "    st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);\n"
+             "    st[0].Store(a_lds + k * SA::kPlane, wave, lane, ra);\n  }\n")
+    << "#pragma unroll\n  for (int k = 0; k < PD; ++k)\n"
        "    st[k].Load(aw, src.p, src.dim, ra, zb + 2 + k);\n"
-       "  __syncthreads();\n"
+    << (rb ? "#pragma unroll\n  for (int k = 0; k < 4; ++k)\n"
+             "    pro[k].Store(a_lds + k * SA::kPlane, wave, lane, ra);\n"
+           : "")
+    << "  __syncthreads();\n"
     << "  __PSCtx_" << n << " ctx;\n"
     << "  ctx." << I << "_p = src.p;\n  ctx." << O << "_p = dst.p;\n"
     // (a fusable pair's grids have equal extents: one set of extents lets
@@ -2390,8 +2411,8 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
        "(2 * j + 1) % 6);\n"
        "      __udouble(s0 - 3, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 4) % 6);\n"
        "      __udouble(s0 - 2, (2 * j + 3) % 6, (2 * j + 4) % 6, (2 * j + 5) % 6);\n"
-       "      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane);\n"
-       "      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane);\n"
+       "      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane, ra);\n"
+       "      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane, ra);\n"
        "      __syncthreads();\n"
        "      st[0].Load(aw, src.p, src.dim, ra, s0 + 5);\n"
        "      st[1].Load(aw, src.p, src.dim, ra, s0 + 6);\n"
@@ -2414,12 +2435,16 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
     << "  constexpr int VX = __PS2VX_" << n << ", BY = __PS2BY_" << n << ";\n"
     << (rb ? "  const __PSDomain gd = physis_hip::WholeDomain(s." + I + ");\n" : "")
     << "  static int per_cu = physis_hip::BlocksPerCU(\n"
-       "      (const void *)__PSStencilRun2_" << n << "<VX, BY>, 64 * BY);\n"
+       "      (const void *)__PSStencilRun2_" << n << "<VX, BY, false>, 64 * BY);\n"
     << "  const physis_hip::RunShape sh = physis_hip::PlanRun("
     << (rb ? "gd" : "s.dom") << ", 64 * VX, BY - 4, per_cu,\n"
        "      physis_hip::WindowChunkLimit({s." << I << "}, 3));\n"
     << "  if (sh.blocks == 0) return;\n"
-    << "  hipLaunchKernelGGL((__PSStencilRun2_" << n << "<VX, BY>), "
+    << "  if (s." << I << "->dim[0] % VX == 0)\n"
+    << "    hipLaunchKernelGGL((__PSStencilRun2_" << n << "<VX, BY, false>), "
+       "dim3(sh.blocks), dim3(64 * BY), 0, stream, "
+    << Join(largs, ", ") << ");\n  else\n"
+    << "    hipLaunchKernelGGL((__PSStencilRun2_" << n << "<VX, BY, true>), "
        "dim3(sh.blocks), dim3(64 * BY), 0, stream, "
     << Join(largs, ", ") << ");\n}\n\n";
   // run-time check
@@ -2428,13 +2453,12 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
     // grid (so no point of the domain reads past a face, and the halo
     // points the pass computes outside the grid are never updated)
     o << "// The red-black map s0 may run as one pass per iteration: both "
-         "colours, a domain\n// strictly inside a grid whose x extent is a "
-         "multiple of 4.\n";
+         "colours, a domain\n// strictly inside the grid.\n";
     o << "static bool __PSFusableRB_" << n << "(const struct __PSStencil_" << n
       << " &s0) {\n"
       << "  static const bool off = getenv(\"PHYSIS_HIP_NO_FUSE\") != NULL;\n"
       << "  const __PSGrid *a = s0." << I << ";\n"
-      << "  if (off || !a || s0.__rb != 2 || a->num_dims != 3 || a->dim[0] % 4) "
+      << "  if (off || !a || s0.__rb != 2 || a->num_dims != 3) "
          "return false;\n"
       << "  for (int d = 0; d < 3; ++d)\n"
          "    if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||\n"
@@ -2451,7 +2475,7 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
     << "  const __PSGrid *a = s0." << I << ", *b = s0." << O << ";\n"
     << "  if (off || !a || !b || a == b || s1." << I << " != b || s1." << O
     << " != a) return false;\n"
-    << "  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;\n"
+    << "  if (a->num_dims != 3 || b->num_dims != 3) return false;\n"
     << "  for (int d = 0; d < 3; ++d) {\n"
        "    if (a->dim[d] != b->dim[d]) return false;\n"
        "    if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;\n"
@@ -2541,7 +2565,7 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
       << "  static int per_cu = physis_hip::BlocksPerCU(\n"
       << "      (const void *)__PSStencilRun_" << n << "<VX, " << by
       << ", -1>, 64 * " << by << ");\n"
-      << "  return physis_hip::PlanRun(" << D << ", 64 * VX, " << by << " - 2 * "
+      << "  return physis_hip::PlanRun(" << D << ", 64 * physis_hip::FormVX(VX), " << by << " - 2 * "
       << k.hy << ", per_cu, physis_hip::WindowChunkLimit"
       << (k.rows2d ? "Rows" : "") << "({" << Join(wgrids, ", ") << "}, "
       << margin << "));\n}\n\n";
@@ -2570,9 +2594,12 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
     o << "      hipLaunchKernelGGL((__PSStencilRun_" << n << "<VX, " << by
       << ", -1>), grid, block, 0, stream, " << A << ", sh, (" << RT
       << " *)NULL" << RBA << ");\n  }\n  }\n  return sh.blocks;\n}\n\n";
-    // vector width: every 3-D grid's x extent a multiple of 4
+    // vector width: 4 points per lane, in the ragged form unless every
+    // grid's x extent is a multiple of 4.  The ragged form has the points
+    // past the end of a row of a staged grid only as halo columns, so a
+    // domain that reaches beyond such a row takes one point per lane.
     // (the member grids of one grid of user-defined points share its checks)
-    std::vector<std::string> conds, checks, emit_checks;
+    std::vector<std::string> conds, rconds, checks, emit_checks;
     auto add = [](std::vector<std::string> &v, const std::string &x) {
       if (std::find(v.begin(), v.end(), x) == v.end()) v.push_back(x);
     };
@@ -2581,6 +2608,8 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
         // (lower-dimensional grids are read through bounds-checked gets)
         if (g.member_of >= 0 || g.dims == (k.rows2d ? 2 : 3))
           add(conds, HostGrid(k, g) + "->dim[0] % 4 == 0");
+        if (g.mode == GridParam::kStaged)
+          add(rconds, "s.dom.local_max[0] <= " + HostGrid(k, g) + "->dim[0]");
         add(checks, g.member_of >= 0
                         ? "physis_hip::CheckUserGrid3D(" + HostGrid(k, g) + ")"
                         : "physis_hip::CheckGrid3D(s." + g.name + ", " +
@@ -2591,9 +2620,14 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
             "physis_hip::CheckEmitDomain(s.dom, " + HostGrid(k, g) + ")");
     }
     std::string vec = conds.empty() ? "true" : Join(conds, " && ");
+    std::string rag = rconds.empty() ? "true" : Join(rconds, " && ");
+    auto pick = [&](const std::string &f, const std::string &tail) {
+      return "  return (" + vec + ") ? " + f + "<4>" + tail + "\n         : (" +
+             rag + ") ? " + f + "<4 + physis_hip::kRagged>" + tail +
+             "\n         : " + f + "<1>" + tail + ";\n";
+    };
     o << "static int __PSBlocks_" << n << "(const struct __PSStencil_" << n
-      << " &s) {\n  return (" << vec << ") ? __PSShape_" << n
-      << "<4>(s).blocks : __PSShape_" << n << "<1>(s).blocks;\n}\n\n";
+      << " &s) {\n" << pick("__PSShape_" + n, "(s).blocks") << "}\n\n";
     o << "static int __PSRun_" << n << "(const struct __PSStencil_" << n
       << " &s, hipStream_t stream, void *red) {\n";
     for (auto &c : checks) o << "  " << c << ";\n";
@@ -2619,8 +2653,7 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
           << "    __warned = true;\n  }\n";
     }
     for (auto &c : emit_checks) o << "  " << c << ";\n";
-    o << "  return (" << vec << ") ? __PSLaunch_" << n
-      << "<4>(s, stream, red) : __PSLaunch_" << n << "<1>(s, stream, red);\n}\n\n";
+    o << pick("__PSLaunch_" + n, "(s, stream, red)") << "}\n\n";
   } else {
     o << "static dim3 __PSGridDim_" << n << "(const struct __PSStencil_" << n
       << " &s) {\n  const int nx = s.dom.local_max[0] - s.dom.local_min[0];\n"
@@ -2803,10 +2836,12 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
        "// tile and a one-point halo (bg's own values outside the domain) and\n"
        "// u'' = " << n << "(u') two planes behind; dst <- u'', and bg <- u'\n"
        "// when store_mid.  red1 / red2: per-block partials of the two sweeps.\n";
-  o << "template <int VX, int BY, int RED>\n__global__ __launch_bounds__(64 * BY) "
+  o << "// RAGGED: x extents that are not multiples of VX.\n"
+       "template <int VX, int BY, int RED, bool RAGGED>\n__global__ __launch_bounds__(64 * BY) "
        "void __PSStencilRun2_" << n << "(\n    " << Join(args, ", ") << ") {\n";
   o << "  constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;\n"
-    << "  typedef physis_hip::Stage<" << T << ", VX, BY, 2, 2, 4, false> SA;\n"
+    << "  typedef physis_hip::Stage<" << T << ", VX, BY, 2, 2, 4, false, " << T
+    << ", RAGGED> SA;\n"
     << "  typedef physis_hip::Stage<" << T << ", VX, BY, 1, 1, 4, false> SB;\n"
     << "  __shared__ __attribute__((aligned(16))) " << T << " a_lds[SA::kLdsElems];\n"
     << "  __shared__ __attribute__((aligned(16))) " << T << " b_lds[SB::kLdsElems];\n"
@@ -2826,9 +2861,8 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
        "    const int xs = x0 + lane * VX;\n"
        "    const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];\n"
        "    const int n = nxy * src.dim[2];\n"
-       "    if constexpr (VX > 1) {\n"
-       "      __builtin_assume((xs & (VX - 1)) == 0);\n"
-       "      __builtin_assume((nx & 3) == 0);\n    }\n"
+       "    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);\n"
+       "    if constexpr (VX > 1 && !RAGGED) __builtin_assume((nx & 3) == 0);\n"
        "    // u' halo columns x0 - 1 and x0 + TX of rows y0 - 1 .. y0 + TY: one\n"
        "    // point per lane of wave 0 (which otherwise only loads)\n"
        "    const bool hlane = wave == 0 && lane < 2 * (BY - 2);\n"
@@ -2854,11 +2888,10 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
     o << "    const physis_hip::BufWin<" << g->elem << "> " << g->name
       << "_w = physis_hip::BufWin<" << g->elem << ">::Make(" << g->name
       << ".p, n, (long)(zb - 1) * nxy, (long)(ze + 1) * nxy);\n";
-  o << "    SA st[PD];\n"
+  o << "    SA st[PD], pro[3];\n"
        "    const typename SA::Addr ra = SA::Prepare(src.dim, x0, yrow, lane);\n"
-       "#pragma unroll\n    for (int k = 0; k < 3; ++k) {\n"
-       "      st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);\n"
-       "      st[0].Store(a_lds + k * SA::kPlane, wave, lane);\n    }\n"
+       "#pragma unroll\n    for (int k = 0; k < 3; ++k)\n"
+       "      pro[k].Load(aw, src.p, src.dim, ra, zb - 2 + k);\n"
        "#pragma unroll\n    for (int k = 0; k < PD; ++k)\n"
        "      st[k].Load(aw, src.p, src.dim, ra, zb + 1 + k);\n";
   // centre values of the direct grids: plane s is loaded one step ahead of
@@ -2887,6 +2920,8 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
       << "_c1[slot]);\n";
   o << "        bw.template Load<VX>(ob, bg_c1[slot]);\n      }\n    };\n"
        "    load1(zb - 1, 0);\n"
+       "#pragma unroll\n    for (int k = 0; k < 3; ++k)\n"
+       "      pro[k].Store(a_lds + k * SA::kPlane, wave, lane, ra);\n"
        "    __syncthreads();\n";
   o << "    __PSCtx_" << n << " ctx;\n";
   for (auto &g : k.grids) {
@@ -2966,7 +3001,7 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
        "          physis_hip::StoreMasked<" << T
     << ", VX>(dw, xs + yrow * nx + (s - 2) * nxy, uu, m);\n        }\n"
        "        st[k % PD].Store(a_lds + physis_hip::RingSlot<4>(abase, 3) * SA::kPlane, "
-       "wave, lane);\n"
+       "wave, lane, ra);\n"
        "        __syncthreads();\n"
        "        st[k % PD].Load(aw, src.p, src.dim, ra, s + 2 + PD);\n"
        "      }\n    }\n  }\n";
@@ -2996,7 +3031,7 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
   o << "template <int VX, int BY>\nstatic physis_hip::RunShape __PSShape2_" << n
     << "(const struct __PSStencil_" << n << " &s) {\n"
     << "  static int per_cu = physis_hip::BlocksPerCU(\n"
-    << "      (const void *)__PSStencilRun2_" << n << "<VX, BY, -1>, 64 * BY);\n"
+    << "      (const void *)__PSStencilRun2_" << n << "<VX, BY, -1, false>, 64 * BY);\n"
     << "  return physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,\n"
     << "      physis_hip::WindowChunkLimit({" << Join(wgrids, ", ") << "}, 3));\n}\n\n";
   o << "static int __PSBlocks2_" << n << "(const struct __PSStencil_" << n
@@ -3012,7 +3047,8 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
   largs.push_back("(" + RT + " *)red1");
   largs.push_back("(" + RT + " *)red2");
   const std::string LA = Join(largs, ", ");
-  o << "static void __PSLaunch2_" << n << "(const struct __PSStencil_" << n
+  o << "template <bool RAGGED>\nstatic void __PSLaunch2R_" << n
+    << "(const struct __PSStencil_" << n
     << " &s, const " << V << " &src, const " << V
     << " &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {\n"
     << "  constexpr int VX = __PS2VX_" << n << ", BY = __PS2BY_" << n << ";\n"
@@ -3023,14 +3059,22 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
     o << "  switch (red1 || red2 ? s.__reduce_op : -1) {\n";
     for (const char *op : {"PS_MAX", "PS_MIN", "PS_SUM", "PS_PROD"})
       o << "    case " << op << ":\n      hipLaunchKernelGGL((__PSStencilRun2_" << n
-        << "<VX, BY, " << op << ">), grid, block, 0, stream, " << LA
+        << "<VX, BY, " << op << ", RAGGED>), grid, block, 0, stream, " << LA
         << ");\n      break;\n";
     o << "    default:\n";
   } else {
     o << "  {\n";
   }
   o << "      hipLaunchKernelGGL((__PSStencilRun2_" << n
-    << "<VX, BY, -1>), grid, block, 0, stream, " << LA << ");\n  }\n}\n\n";
+    << "<VX, BY, -1, RAGGED>), grid, block, 0, stream, " << LA << ");\n  }\n}\n\n";
+  o << "static void __PSLaunch2_" << n << "(const struct __PSStencil_" << n
+    << " &s, const " << V << " &src, const " << V
+    << " &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {\n"
+    << "  if (s." << I << "->dim[0] % __PS2VX_" << n << " == 0)\n"
+    << "    __PSLaunch2R_" << n << "<false>(s, src, dst, store_mid, stream, red1, red2);\n"
+    << "  else\n"
+    << "    __PSLaunch2R_" << n << "<__PS2VX_" << n
+    << " != 1>(s, src, dst, store_mid, stream, red1, red2);\n}\n\n";
   o << "// The pair (s0, s1) is " << n << "(a -> b), " << n
     << "(b -> a) over one domain strictly\n// inside the grids, with the same "
        "centre-only grids (neither a nor b) and\n// scalars: it may run as "
@@ -3041,7 +3085,7 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
     << "  const __PSGrid *a = s0." << I << ", *b = s0." << O << ";\n"
     << "  if (off || !a || !b || a == b || s1." << I << " != b || s1." << O
     << " != a) return false;\n"
-    << "  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;\n"
+    << "  if (a->num_dims != 3 || b->num_dims != 3) return false;\n"
     << "  for (int d = 0; d < 3; ++d) {\n"
        "    if (a->dim[d] != b->dim[d]) return false;\n"
        "    if (s0.dom.local_min[d] != s1.dom.local_min[d] ||\n"

@@ -83,13 +83,16 @@ __device__ __forceinline__ void diffusion7_kernel(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_diffusion7_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev g1, __PSGrid3DFloat_dev g2, float ce, float cw, float cn, float cs, float ct, float cb, float cc, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g1;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g1;
   __shared__ __attribute__((aligned(16))) float g1_lds[S_g1::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -106,25 +109,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_diffusion7_kernel(
     const physis_hip::BufWin<float> g1_w = physis_hip::BufWin<float>::Make(g1.p, g1_nxy * g1.dim[2], (long)(zb + -2) * g1_nxy, (long)(ze + 2) * g1_nxy);
     S_g1 g1_st[PD];
     const typename S_g1::Addr g1_ra = S_g1::Prepare(g1.dim, x0, yrow, lane);
+    S_g1 g1_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g1_st[0].Load(g1_w, g1.p, g1.dim, g1_ra, zb + -1 + k);
-      g1_st[0].Store(g1_lds + k * S_g1::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g1_pro[k].Load(g1_w, g1.p, g1.dim, g1_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g1_st[k].Load(g1_w, g1.p, g1.dim, g1_ra, zb + 2 + k);
     int g1_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g1_pro[k].Store(g1_lds + k * S_g1::kPlane, wave, lane, g1_ra);
     __syncthreads();
     __PSCtx_diffusion7_kernel ctx;
     ctx.g1_p = g1.p;
     for (int d = 0; d < 3; ++d) ctx.g1_dim[d] = g1.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g1_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -179,7 +184,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_diffusion7_kernel(
             __pts(physis_hip::Flag<false>{});
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g1_st[k % PD].Store(g1_lds + physis_hip::RingSlot<4>(g1_base, 3) * S_g1::kPlane, wave, lane);
+        g1_st[k % PD].Store(g1_lds + physis_hip::RingSlot<4>(g1_base, 3) * S_g1::kPlane, wave, lane, g1_ra);
         __syncthreads();
         g1_st[k % PD].Load(g1_w, g1.p, g1.dim, g1_ra, z + 2 + PD);
       }
@@ -192,7 +197,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_diffusion7_kernel<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
 }
 
 template <int VX>
@@ -210,14 +215,18 @@ static int __PSLaunch_diffusion7_kernel(const struct __PSStencil_diffusion7_kern
 }
 
 static int __PSBlocks_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s) {
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_diffusion7_kernel<4>(s).blocks : __PSShape_diffusion7_kernel<1>(s).blocks;
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_diffusion7_kernel<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_diffusion7_kernel<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_diffusion7_kernel<1>(s).blocks;
 }
 
 static int __PSRun_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g1, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_diffusion7_kernel<4>(s, stream, red) : __PSLaunch_diffusion7_kernel<1>(s, stream, red);
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_diffusion7_kernel<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_diffusion7_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_diffusion7_kernel<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of diffusion7_kernel (temporal blocking): one pass over src
@@ -227,11 +236,12 @@ static int __PSRun_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel 
 // planes s0 and s0 + 1 and u'' of s0 - 3 and s0 - 2 from rings of six
 // slots (source plane p in slot (p - zb + 2) % 6, u'(p) in slot
 // (p - zb + 1) % 6), then stores source planes s0 + 3 and s0 + 4.
-template <int VX, int BY>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ mid, float ce, float cw, float cn, float cs, float ct, float cb, float cc, physis_hip::RunShape sh) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, false> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, false, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 6, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -249,9 +259,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_kernel(
   const int xs = x0 + lane * VX;
   const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
   const int n = nxy * src.dim[2];
-  // tiles start at multiples of TX and two-sweep runs need nx % 4 == 0
+  // tiles start at multiples of TX
   __builtin_assume((xs & (VX - 1)) == 0);
-  __builtin_assume((nx & (VX - 1)) == 0);
+  if constexpr (!RAGGED) __builtin_assume((nx & (VX - 1)) == 0);
   const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, (long)(zb - 3) * nxy, (long)(ze + 3) * nxy);
   const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
   const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);
@@ -260,7 +270,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_kernel(
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-    st[0].Store(a_lds + k * SA::kPlane, wave, lane);
+    st[0].Store(a_lds + k * SA::kPlane, wave, lane, ra);
   }
 #pragma unroll
   for (int k = 0; k < PD; ++k)
@@ -381,8 +391,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_kernel(
       __uprime(s0 + 1, (2 * j + 1) % 6, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 1) % 6);
       __udouble(s0 - 3, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 4) % 6);
       __udouble(s0 - 2, (2 * j + 3) % 6, (2 * j + 4) % 6, (2 * j + 5) % 6);
-      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane);
-      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane);
+      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane, ra);
+      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane, ra);
       __syncthreads();
       st[0].Load(aw, src.p, src.dim, ra, s0 + 5);
       st[1].Load(aw, src.p, src.dim, ra, s0 + 6);
@@ -394,11 +404,14 @@ static constexpr int __PS2VX_diffusion7_kernel = 4, __PS2BY_diffusion7_kernel = 
 static void __PSLaunch2_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
   constexpr int VX = __PS2VX_diffusion7_kernel, BY = __PS2BY_diffusion7_kernel;
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_diffusion7_kernel<VX, BY>, 64 * BY);
+      (const void *)__PSStencilRun2_diffusion7_kernel<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g1}, 3));
   if (sh.blocks == 0) return;
-  hipLaunchKernelGGL((__PSStencilRun2_diffusion7_kernel<VX, BY>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+  if (s.g1->dim[0] % VX == 0)
+    hipLaunchKernelGGL((__PSStencilRun2_diffusion7_kernel<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+  else
+    hipLaunchKernelGGL((__PSStencilRun2_diffusion7_kernel<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
 }
 
 // The pair (s0, s1) is diffusion7_kernel(a -> b), diffusion7_kernel(b -> a) over the whole grid with the
@@ -407,7 +420,7 @@ static bool __PSFusable2_diffusion7_kernel(const struct __PSStencil_diffusion7_k
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g1, *b = s0.g2;
   if (off || !a || !b || a == b || s1.g1 != b || s1.g2 != a) return false;
-  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;
+  if (a->num_dims != 3 || b->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d) {
     if (a->dim[d] != b->dim[d]) return false;
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
@@ -477,13 +490,16 @@ __device__ __forceinline__ void diffusion7_periodic_kernel(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_diffusion7_periodic_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev g1, __PSGrid3DFloat_dev g2, float ce, float cw, float cn, float cs, float ct, float cb, float cc, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true> S_g1;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true, float, RAGGED> S_g1;
   __shared__ __attribute__((aligned(16))) float g1_lds[S_g1::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -500,25 +516,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_diffusion7_periodic_ke
     const physis_hip::BufWin<float> g1_w = physis_hip::BufWin<float>::Make(g1.p, g1_nxy * g1.dim[2], (long)(zb + -2) * g1_nxy, (long)(ze + 2) * g1_nxy);
     S_g1 g1_st[PD];
     const typename S_g1::Addr g1_ra = S_g1::Prepare(g1.dim, x0, yrow, lane);
+    S_g1 g1_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g1_st[0].Load(g1_w, g1.p, g1.dim, g1_ra, zb + -1 + k);
-      g1_st[0].Store(g1_lds + k * S_g1::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g1_pro[k].Load(g1_w, g1.p, g1.dim, g1_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g1_st[k].Load(g1_w, g1.p, g1.dim, g1_ra, zb + 2 + k);
     int g1_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g1_pro[k].Store(g1_lds + k * S_g1::kPlane, wave, lane, g1_ra);
     __syncthreads();
     __PSCtx_diffusion7_periodic_kernel ctx;
     ctx.g1_p = g1.p;
     for (int d = 0; d < 3; ++d) ctx.g1_dim[d] = g1.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g1_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -564,7 +582,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_diffusion7_periodic_ke
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g1_st[k % PD].Store(g1_lds + physis_hip::RingSlot<4>(g1_base, 3) * S_g1::kPlane, wave, lane);
+        g1_st[k % PD].Store(g1_lds + physis_hip::RingSlot<4>(g1_base, 3) * S_g1::kPlane, wave, lane, g1_ra);
         __syncthreads();
         g1_st[k % PD].Load(g1_w, g1.p, g1.dim, g1_ra, z + 2 + PD);
       }
@@ -577,7 +595,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_diffusion7_periodic_kernel<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
 }
 
 template <int VX>
@@ -595,14 +613,18 @@ static int __PSLaunch_diffusion7_periodic_kernel(const struct __PSStencil_diffus
 }
 
 static int __PSBlocks_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s) {
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_diffusion7_periodic_kernel<4>(s).blocks : __PSShape_diffusion7_periodic_kernel<1>(s).blocks;
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_diffusion7_periodic_kernel<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_diffusion7_periodic_kernel<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_diffusion7_periodic_kernel<1>(s).blocks;
 }
 
 static int __PSRun_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g1, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_diffusion7_periodic_kernel<4>(s, stream, red) : __PSLaunch_diffusion7_periodic_kernel<1>(s, stream, red);
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_diffusion7_periodic_kernel<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_diffusion7_periodic_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_diffusion7_periodic_kernel<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of diffusion7_periodic_kernel (temporal blocking): one pass over src
@@ -612,11 +634,12 @@ static int __PSRun_diffusion7_periodic_kernel(const struct __PSStencil_diffusion
 // planes s0 and s0 + 1 and u'' of s0 - 3 and s0 - 2 from rings of six
 // slots (source plane p in slot (p - zb + 2) % 6, u'(p) in slot
 // (p - zb + 1) % 6), then stores source planes s0 + 3 and s0 + 4.
-template <int VX, int BY>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_periodic_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ mid, float ce, float cw, float cn, float cs, float ct, float cb, float cc, physis_hip::RunShape sh) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, true> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, true, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 6, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -634,9 +657,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_periodic_k
   const int xs = x0 + lane * VX;
   const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
   const int n = nxy * src.dim[2];
-  // tiles start at multiples of TX and two-sweep runs need nx % 4 == 0
+  // tiles start at multiples of TX
   __builtin_assume((xs & (VX - 1)) == 0);
-  __builtin_assume((nx & (VX - 1)) == 0);
+  if constexpr (!RAGGED) __builtin_assume((nx & (VX - 1)) == 0);
   const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, (long)(zb - 3) * nxy, (long)(ze + 3) * nxy);
   const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
   const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);
@@ -645,7 +668,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_periodic_k
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-    st[0].Store(a_lds + k * SA::kPlane, wave, lane);
+    st[0].Store(a_lds + k * SA::kPlane, wave, lane, ra);
   }
 #pragma unroll
   for (int k = 0; k < PD; ++k)
@@ -748,8 +771,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_periodic_k
       __uprime(s0 + 1, (2 * j + 1) % 6, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 1) % 6);
       __udouble(s0 - 3, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 4) % 6);
       __udouble(s0 - 2, (2 * j + 3) % 6, (2 * j + 4) % 6, (2 * j + 5) % 6);
-      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane);
-      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane);
+      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane, ra);
+      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane, ra);
       __syncthreads();
       st[0].Load(aw, src.p, src.dim, ra, s0 + 5);
       st[1].Load(aw, src.p, src.dim, ra, s0 + 6);
@@ -761,11 +784,14 @@ static constexpr int __PS2VX_diffusion7_periodic_kernel = 4, __PS2BY_diffusion7_
 static void __PSLaunch2_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
   constexpr int VX = __PS2VX_diffusion7_periodic_kernel, BY = __PS2BY_diffusion7_periodic_kernel;
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_diffusion7_periodic_kernel<VX, BY>, 64 * BY);
+      (const void *)__PSStencilRun2_diffusion7_periodic_kernel<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g1}, 3));
   if (sh.blocks == 0) return;
-  hipLaunchKernelGGL((__PSStencilRun2_diffusion7_periodic_kernel<VX, BY>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+  if (s.g1->dim[0] % VX == 0)
+    hipLaunchKernelGGL((__PSStencilRun2_diffusion7_periodic_kernel<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+  else
+    hipLaunchKernelGGL((__PSStencilRun2_diffusion7_periodic_kernel<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
 }
 
 // The pair (s0, s1) is diffusion7_periodic_kernel(a -> b), diffusion7_periodic_kernel(b -> a) over the whole grid with the
@@ -774,7 +800,7 @@ static bool __PSFusable2_diffusion7_periodic_kernel(const struct __PSStencil_dif
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g1, *b = s0.g2;
   if (off || !a || !b || a == b || s1.g1 != b || s1.g2 != a) return false;
-  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;
+  if (a->num_dims != 3 || b->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d) {
     if (a->dim[d] != b->dim[d]) return false;
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;

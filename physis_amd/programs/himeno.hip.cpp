@@ -134,13 +134,16 @@ __device__ __forceinline__ float jacobi_kernel(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_jacobi_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev p0, __PSGrid3DFloat_dev p1, __PSGrid3DFloat_dev a0, __PSGrid3DFloat_dev a1, __PSGrid3DFloat_dev a2, __PSGrid3DFloat_dev a3, __PSGrid3DFloat_dev b0, __PSGrid3DFloat_dev b1, __PSGrid3DFloat_dev b2, __PSGrid3DFloat_dev c0, __PSGrid3DFloat_dev c1, __PSGrid3DFloat_dev c2, __PSGrid3DFloat_dev bnd, __PSGrid3DFloat_dev wrk1, float omega, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 2;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_p0;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_p0;
   __shared__ __attribute__((aligned(16))) float p0_lds[S_p0::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -163,11 +166,10 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_jacobi_kernel(
     const physis_hip::BufWin<float> p0_w = physis_hip::BufWin<float>::Make(p0.p, p0_nxy * p0.dim[2], (long)(zb + -2) * p0_nxy, (long)(ze + 2) * p0_nxy);
     S_p0 p0_st[PD];
     const typename S_p0::Addr p0_ra = S_p0::Prepare(p0.dim, x0, yrow, lane);
+    S_p0 p0_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      p0_st[0].Load(p0_w, p0.p, p0.dim, p0_ra, zb + -1 + k);
-      p0_st[0].Store(p0_lds + k * S_p0::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      p0_pro[k].Load(p0_w, p0.p, p0.dim, p0_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       p0_st[k].Load(p0_w, p0.p, p0.dim, p0_ra, zb + 2 + k);
@@ -222,6 +224,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_jacobi_kernel(
     const physis_hip::BufWin<float> wrk1_w = physis_hip::BufWin<float>::Make(wrk1.p, wrk1_nxy * wrk1.dim[2], (long)zb * wrk1_nxy, (long)ze * wrk1_nxy);
     float wrk1_dv[2][VX];
     wrk1_w.template Load<VX, physis_hip::kStreamLoad>(xs + drow * wrk1_nx + zb * wrk1_nxy, wrk1_dv[0]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      p0_pro[k].Store(p0_lds + k * S_p0::kPlane, wave, lane, p0_ra);
     __syncthreads();
     __PSCtx_jacobi_kernel ctx;
     ctx.p0_p = p0.p;
@@ -252,8 +257,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_jacobi_kernel(
     for (int d = 0; d < 3; ++d) ctx.bnd_dim[d] = bnd.dim[d];
     ctx.wrk1_p = wrk1.p;
     for (int d = 0; d < 3; ++d) ctx.wrk1_dim[d] = wrk1.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.p0_dim[0] & 3) == 0);
       __builtin_assume((ctx.p1_dim[0] & 3) == 0);
       __builtin_assume((ctx.a0_dim[0] & 3) == 0);
@@ -354,7 +359,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_jacobi_kernel(
           }
           physis_hip::StoreMasked<float, VX>(p1_ew, xs + yrow * p1_enx + z * p1_enxy, p1_out, p1_mask);
         }
-        p0_st[k % PD].Store(p0_lds + physis_hip::RingSlot<4>(p0_base, 3) * S_p0::kPlane, wave, lane);
+        p0_st[k % PD].Store(p0_lds + physis_hip::RingSlot<4>(p0_base, 3) * S_p0::kPlane, wave, lane, p0_ra);
         __syncthreads();
         p0_st[k % PD].Load(p0_w, p0.p, p0.dim, p0_ra, z + 2 + PD);
         p0_base = physis_hip::RingSlot<4>(p0_base, 1);
@@ -372,7 +377,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_jacobi_kernel<VX, 8, -1>, 64 * 8);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 8 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.p0, s.p1, s.a0, s.a1, s.a2, s.a3, s.b0, s.b1, s.b2, s.c0, s.c1, s.c2, s.bnd, s.wrk1}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 8 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.p0, s.p1, s.a0, s.a1, s.a2, s.a3, s.b0, s.b1, s.b2, s.c0, s.c1, s.c2, s.bnd, s.wrk1}, 2));
 }
 
 template <int VX>
@@ -402,7 +407,9 @@ static int __PSLaunch_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, h
 }
 
 static int __PSBlocks_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s) {
-  return (s.p0->dim[0] % 4 == 0 && s.p1->dim[0] % 4 == 0 && s.a0->dim[0] % 4 == 0 && s.a1->dim[0] % 4 == 0 && s.a2->dim[0] % 4 == 0 && s.a3->dim[0] % 4 == 0 && s.b0->dim[0] % 4 == 0 && s.b1->dim[0] % 4 == 0 && s.b2->dim[0] % 4 == 0 && s.c0->dim[0] % 4 == 0 && s.c1->dim[0] % 4 == 0 && s.c2->dim[0] % 4 == 0 && s.bnd->dim[0] % 4 == 0 && s.wrk1->dim[0] % 4 == 0) ? __PSShape_jacobi_kernel<4>(s).blocks : __PSShape_jacobi_kernel<1>(s).blocks;
+  return (s.p0->dim[0] % 4 == 0 && s.p1->dim[0] % 4 == 0 && s.a0->dim[0] % 4 == 0 && s.a1->dim[0] % 4 == 0 && s.a2->dim[0] % 4 == 0 && s.a3->dim[0] % 4 == 0 && s.b0->dim[0] % 4 == 0 && s.b1->dim[0] % 4 == 0 && s.b2->dim[0] % 4 == 0 && s.c0->dim[0] % 4 == 0 && s.c1->dim[0] % 4 == 0 && s.c2->dim[0] % 4 == 0 && s.bnd->dim[0] % 4 == 0 && s.wrk1->dim[0] % 4 == 0) ? __PSShape_jacobi_kernel<4>(s).blocks
+         : (s.dom.local_max[0] <= s.p0->dim[0]) ? __PSShape_jacobi_kernel<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_jacobi_kernel<1>(s).blocks;
 }
 
 static int __PSRun_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, hipStream_t stream, void *red) {
@@ -421,7 +428,9 @@ static int __PSRun_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, hipS
   physis_hip::CheckGrid3D(s.bnd, PS_FLOAT);
   physis_hip::CheckGrid3D(s.wrk1, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.p1);
-  return (s.p0->dim[0] % 4 == 0 && s.p1->dim[0] % 4 == 0 && s.a0->dim[0] % 4 == 0 && s.a1->dim[0] % 4 == 0 && s.a2->dim[0] % 4 == 0 && s.a3->dim[0] % 4 == 0 && s.b0->dim[0] % 4 == 0 && s.b1->dim[0] % 4 == 0 && s.b2->dim[0] % 4 == 0 && s.c0->dim[0] % 4 == 0 && s.c1->dim[0] % 4 == 0 && s.c2->dim[0] % 4 == 0 && s.bnd->dim[0] % 4 == 0 && s.wrk1->dim[0] % 4 == 0) ? __PSLaunch_jacobi_kernel<4>(s, stream, red) : __PSLaunch_jacobi_kernel<1>(s, stream, red);
+  return (s.p0->dim[0] % 4 == 0 && s.p1->dim[0] % 4 == 0 && s.a0->dim[0] % 4 == 0 && s.a1->dim[0] % 4 == 0 && s.a2->dim[0] % 4 == 0 && s.a3->dim[0] % 4 == 0 && s.b0->dim[0] % 4 == 0 && s.b1->dim[0] % 4 == 0 && s.b2->dim[0] % 4 == 0 && s.c0->dim[0] % 4 == 0 && s.c1->dim[0] % 4 == 0 && s.c2->dim[0] % 4 == 0 && s.bnd->dim[0] % 4 == 0 && s.wrk1->dim[0] % 4 == 0) ? __PSLaunch_jacobi_kernel<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.p0->dim[0]) ? __PSLaunch_jacobi_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_jacobi_kernel<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of jacobi_kernel over a domain strictly inside
@@ -429,11 +438,12 @@ static int __PSRun_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, hipS
 // tile and a one-point halo (bg's own values outside the domain) and
 // u'' = jacobi_kernel(u') two planes behind; dst <- u'', and bg <- u'
 // when store_mid.  red1 / red2: per-block partials of the two sweeps.
-template <int VX, int BY, int RED>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, int RED, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_jacobi_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, __PSGrid3DFloat_dev bg, int store_mid, __PSGrid3DFloat_dev a0, __PSGrid3DFloat_dev a1, __PSGrid3DFloat_dev a2, __PSGrid3DFloat_dev a3, __PSGrid3DFloat_dev b0, __PSGrid3DFloat_dev b1, __PSGrid3DFloat_dev b2, __PSGrid3DFloat_dev c0, __PSGrid3DFloat_dev c1, __PSGrid3DFloat_dev c2, __PSGrid3DFloat_dev bnd, __PSGrid3DFloat_dev wrk1, float omega, physis_hip::RunShape sh, float *__restrict__ red1, float *__restrict__ red2) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 4, false> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 4, false, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 4, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -453,10 +463,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_jacobi_kernel(
     const int xs = x0 + lane * VX;
     const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
     const int n = nxy * src.dim[2];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
-      __builtin_assume((nx & 3) == 0);
-    }
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) __builtin_assume((nx & 3) == 0);
     // u' halo columns x0 - 1 and x0 + TX of rows y0 - 1 .. y0 + TY: one
     // point per lane of wave 0 (which otherwise only loads)
     const bool hlane = wave == 0 && lane < 2 * (BY - 2);
@@ -487,13 +495,11 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_jacobi_kernel(
     const physis_hip::BufWin<float> c2_w = physis_hip::BufWin<float>::Make(c2.p, n, (long)(zb - 1) * nxy, (long)(ze + 1) * nxy);
     const physis_hip::BufWin<float> bnd_w = physis_hip::BufWin<float>::Make(bnd.p, n, (long)(zb - 1) * nxy, (long)(ze + 1) * nxy);
     const physis_hip::BufWin<float> wrk1_w = physis_hip::BufWin<float>::Make(wrk1.p, n, (long)(zb - 1) * nxy, (long)(ze + 1) * nxy);
-    SA st[PD];
+    SA st[PD], pro[3];
     const typename SA::Addr ra = SA::Prepare(src.dim, x0, yrow, lane);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-      st[0].Store(a_lds + k * SA::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      pro[k].Load(aw, src.p, src.dim, ra, zb - 2 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       st[k].Load(aw, src.p, src.dim, ra, zb + 1 + k);
@@ -549,6 +555,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_jacobi_kernel(
       }
     };
     load1(zb - 1, 0);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      pro[k].Store(a_lds + k * SA::kPlane, wave, lane, ra);
     __syncthreads();
     __PSCtx_jacobi_kernel ctx;
     ctx.p0_p = src.p;
@@ -755,7 +764,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_jacobi_kernel(
           }
           physis_hip::StoreMasked<float, VX>(dw, xs + yrow * nx + (s - 2) * nxy, uu, m);
         }
-        st[k % PD].Store(a_lds + physis_hip::RingSlot<4>(abase, 3) * SA::kPlane, wave, lane);
+        st[k % PD].Store(a_lds + physis_hip::RingSlot<4>(abase, 3) * SA::kPlane, wave, lane, ra);
         __syncthreads();
         st[k % PD].Load(aw, src.p, src.dim, ra, s + 2 + PD);
       }
@@ -778,7 +787,7 @@ static constexpr int __PS2VX_jacobi_kernel = 1, __PS2BY_jacobi_kernel = 12;
 template <int VX, int BY>
 static physis_hip::RunShape __PSShape2_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s) {
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_jacobi_kernel<VX, BY, -1>, 64 * BY);
+      (const void *)__PSStencilRun2_jacobi_kernel<VX, BY, -1, false>, 64 * BY);
   return physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.p0, s.p1, s.a0, s.a1, s.a2, s.a3, s.b0, s.b1, s.b2, s.c0, s.c1, s.c2, s.bnd, s.wrk1}, 3));
 }
@@ -787,27 +796,35 @@ static int __PSBlocks2_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s) 
   return __PSShape2_jacobi_kernel<__PS2VX_jacobi_kernel, __PS2BY_jacobi_kernel>(s).blocks;
 }
 
-static void __PSLaunch2_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
+template <bool RAGGED>
+static void __PSLaunch2R_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
   constexpr int VX = __PS2VX_jacobi_kernel, BY = __PS2BY_jacobi_kernel;
   const physis_hip::RunShape sh = __PSShape2_jacobi_kernel<VX, BY>(s);
   if (sh.blocks == 0) return;
   const dim3 grid(sh.blocks), block(64 * BY);
   switch (red1 || red2 ? s.__reduce_op : -1) {
     case PS_MAX:
-      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, PS_MAX>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
+      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, PS_MAX, RAGGED>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
       break;
     case PS_MIN:
-      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, PS_MIN>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
+      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, PS_MIN, RAGGED>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
       break;
     case PS_SUM:
-      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, PS_SUM>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
+      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, PS_SUM, RAGGED>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
       break;
     case PS_PROD:
-      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, PS_PROD>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
+      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, PS_PROD, RAGGED>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
       break;
     default:
-      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, -1>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
+      hipLaunchKernelGGL((__PSStencilRun2_jacobi_kernel<VX, BY, -1, RAGGED>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.p1), store_mid, physis_hip::DevView<__PSGrid3DFloat_dev>(s.a0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.a3), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.b2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c0), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c1), physis_hip::DevView<__PSGrid3DFloat_dev>(s.c2), physis_hip::DevView<__PSGrid3DFloat_dev>(s.bnd), physis_hip::DevView<__PSGrid3DFloat_dev>(s.wrk1), s.omega, sh, (float *)red1, (float *)red2);
   }
+}
+
+static void __PSLaunch2_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
+  if (s.p0->dim[0] % __PS2VX_jacobi_kernel == 0)
+    __PSLaunch2R_jacobi_kernel<false>(s, src, dst, store_mid, stream, red1, red2);
+  else
+    __PSLaunch2R_jacobi_kernel<__PS2VX_jacobi_kernel != 1>(s, src, dst, store_mid, stream, red1, red2);
 }
 
 // The pair (s0, s1) is jacobi_kernel(a -> b), jacobi_kernel(b -> a) over one domain strictly
@@ -817,7 +834,7 @@ static bool __PSFusable2_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.p0, *b = s0.p1;
   if (off || !a || !b || a == b || s1.p0 != b || s1.p1 != a) return false;
-  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;
+  if (a->num_dims != 3 || b->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d) {
     if (a->dim[d] != b->dim[d]) return false;
     if (s0.dom.local_min[d] != s1.dom.local_min[d] ||

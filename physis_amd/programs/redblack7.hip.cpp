@@ -79,13 +79,16 @@ __device__ __forceinline__ void redblack7_kernel(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_redblack7_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev g, float ce, float cw, float cn, float cs, float ct, float cb, float cc, physis_hip::RunShape sh, float *__restrict__ __red, int __rb) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -102,23 +105,25 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_redblack7_kernel(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g_enx = g.dim[0], g_enxy = g.dim[0] * g.dim[1];
     const physis_hip::BufWin<float> g_ew = physis_hip::BufWin<float>::Make(g.p, g_enxy * g.dim[2], (long)zb * g_enxy, (long)ze * g_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_redblack7_kernel ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
     }
     constexpr int U = 4;
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_redblack7_kernel(
           }
           physis_hip::StoreMasked<float, VX>(g_ew, xs + yrow * g_enx + z * g_enxy, g_out, g_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -177,7 +182,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_redblack7_kernel<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
 }
 
 template <int VX>
@@ -195,13 +200,17 @@ static int __PSLaunch_redblack7_kernel(const struct __PSStencil_redblack7_kernel
 }
 
 static int __PSBlocks_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s) {
-  return (s.g->dim[0] % 4 == 0) ? __PSShape_redblack7_kernel<4>(s).blocks : __PSShape_redblack7_kernel<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0) ? __PSShape_redblack7_kernel<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_redblack7_kernel<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_redblack7_kernel<1>(s).blocks;
 }
 
 static int __PSRun_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g);
-  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_redblack7_kernel<4>(s, stream, red) : __PSLaunch_redblack7_kernel<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_redblack7_kernel<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_redblack7_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_redblack7_kernel<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of redblack7_kernel (temporal blocking): one pass over src
@@ -213,11 +222,12 @@ static int __PSRun_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s
 // (p - zb + 1) % 6), then stores source planes s0 + 3 and s0 + 4.
 // Red-black: one pass is one iteration (red sweep u', black sweep
 // u''); dom is the map's domain, gd the whole grid the pass tiles.
-template <int VX, int BY>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_redblack7_kernel(
     __PSDomain dom, __PSDomain gd, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ mid, float ce, float cw, float cn, float cs, float ct, float cb, float cc, physis_hip::RunShape sh) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, false> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, false, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 6, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -235,22 +245,23 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_redblack7_kernel(
   const int xs = x0 + lane * VX;
   const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
   const int n = nxy * src.dim[2];
-  // tiles start at multiples of TX and two-sweep runs need nx % 4 == 0
+  // tiles start at multiples of TX
   __builtin_assume((xs & (VX - 1)) == 0);
-  __builtin_assume((nx & (VX - 1)) == 0);
+  if constexpr (!RAGGED) __builtin_assume((nx & (VX - 1)) == 0);
   const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, (long)(zb - 3) * nxy, (long)(ze + 3) * nxy);
   const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
   const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);
-  SA st[PD];
+  SA st[PD], pro[4];
   const typename SA::Addr ra = SA::Prepare(src.dim, x0, yrow, lane);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-    st[0].Store(a_lds + k * SA::kPlane, wave, lane);
-  }
+  for (int k = 0; k < 4; ++k)
+    pro[k].Load(aw, src.p, src.dim, ra, zb - 2 + k);
 #pragma unroll
   for (int k = 0; k < PD; ++k)
     st[k].Load(aw, src.p, src.dim, ra, zb + 2 + k);
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    pro[k].Store(a_lds + k * SA::kPlane, wave, lane, ra);
   __syncthreads();
   __PSCtx_redblack7_kernel ctx;
   ctx.g_p = src.p;
@@ -349,8 +360,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_redblack7_kernel(
       __uprime(s0 + 1, (2 * j + 1) % 6, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 1) % 6);
       __udouble(s0 - 3, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 4) % 6);
       __udouble(s0 - 2, (2 * j + 3) % 6, (2 * j + 4) % 6, (2 * j + 5) % 6);
-      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane);
-      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane);
+      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane, ra);
+      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane, ra);
       __syncthreads();
       st[0].Load(aw, src.p, src.dim, ra, s0 + 5);
       st[1].Load(aw, src.p, src.dim, ra, s0 + 6);
@@ -363,19 +374,22 @@ static void __PSLaunch2_redblack7_kernel(const struct __PSStencil_redblack7_kern
   constexpr int VX = __PS2VX_redblack7_kernel, BY = __PS2BY_redblack7_kernel;
   const __PSDomain gd = physis_hip::WholeDomain(s.g);
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_redblack7_kernel<VX, BY>, 64 * BY);
+      (const void *)__PSStencilRun2_redblack7_kernel<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(gd, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g}, 3));
   if (sh.blocks == 0) return;
-  hipLaunchKernelGGL((__PSStencilRun2_redblack7_kernel<VX, BY>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+  if (s.g->dim[0] % VX == 0)
+    hipLaunchKernelGGL((__PSStencilRun2_redblack7_kernel<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+  else
+    hipLaunchKernelGGL((__PSStencilRun2_redblack7_kernel<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
 }
 
 // The red-black map s0 may run as one pass per iteration: both colours, a domain
-// strictly inside a grid whose x extent is a multiple of 4.
+// strictly inside the grid.
 static bool __PSFusableRB_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s0) {
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g;
-  if (off || !a || s0.__rb != 2 || a->num_dims != 3 || a->dim[0] % 4) return false;
+  if (off || !a || s0.__rb != 2 || a->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;

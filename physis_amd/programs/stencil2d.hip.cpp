@@ -48,13 +48,16 @@ __device__ __forceinline__ void s2d5(
 // last 0 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_s2d5(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, float w, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 0;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -71,17 +74,19 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_s2d5(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_s2d5 ctx;
     ctx.g_p = g.p;
@@ -92,8 +97,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_s2d5(
     ctx.g2_dim[0] = g2.dim[0];
     ctx.g2_dim[1] = g2.dim[2];
     ctx.g2_dim[2] = 1;
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -133,7 +138,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_s2d5(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -146,7 +151,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_s2d5(const struct __PSStencil_s2d5 &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_s2d5<VX, 1, -1>, 64 * 1);
-  return physis_hip::PlanRun(physis_hip::RowDomain(s.dom), 64 * VX, 1 - 2 * 0, per_cu, physis_hip::WindowChunkLimitRows({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(physis_hip::RowDomain(s.dom), 64 * physis_hip::FormVX(VX), 1 - 2 * 0, per_cu, physis_hip::WindowChunkLimitRows({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -164,14 +169,18 @@ static int __PSLaunch_s2d5(const struct __PSStencil_s2d5 &s, hipStream_t stream,
 }
 
 static int __PSBlocks_s2d5(const struct __PSStencil_s2d5 &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_s2d5<4>(s).blocks : __PSShape_s2d5<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_s2d5<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_s2d5<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_s2d5<1>(s).blocks;
 }
 
 static int __PSRun_s2d5(const struct __PSStencil_s2d5 &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_s2d5<4>(s, stream, red) : __PSLaunch_s2d5<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_s2d5<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_s2d5<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_s2d5<1>(s, stream, red);
 }
 
 // ---------------------------------------------- stencil s2d9
@@ -215,13 +224,16 @@ __device__ __forceinline__ void s2d9(
 // last 0 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_s2d9(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, float w, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 0;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -238,17 +250,19 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_s2d9(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_s2d9 ctx;
     ctx.g_p = g.p;
@@ -259,8 +273,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_s2d9(
     ctx.g2_dim[0] = g2.dim[0];
     ctx.g2_dim[1] = g2.dim[2];
     ctx.g2_dim[2] = 1;
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -304,7 +318,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_s2d9(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -317,7 +331,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_s2d9(const struct __PSStencil_s2d9 &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_s2d9<VX, 1, -1>, 64 * 1);
-  return physis_hip::PlanRun(physis_hip::RowDomain(s.dom), 64 * VX, 1 - 2 * 0, per_cu, physis_hip::WindowChunkLimitRows({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(physis_hip::RowDomain(s.dom), 64 * physis_hip::FormVX(VX), 1 - 2 * 0, per_cu, physis_hip::WindowChunkLimitRows({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -335,14 +349,18 @@ static int __PSLaunch_s2d9(const struct __PSStencil_s2d9 &s, hipStream_t stream,
 }
 
 static int __PSBlocks_s2d9(const struct __PSStencil_s2d9 &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_s2d9<4>(s).blocks : __PSShape_s2d9<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_s2d9<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_s2d9<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_s2d9<1>(s).blocks;
 }
 
 static int __PSRun_s2d9(const struct __PSStencil_s2d9 &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_s2d9<4>(s, stream, red) : __PSLaunch_s2d9<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_s2d9<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_s2d9<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_s2d9<1>(s, stream, red);
 }
 
 static void __PSStencilRun_0(int iter, struct __PSStencil_s2d5 s0, struct __PSStencil_s2d5 s1) {

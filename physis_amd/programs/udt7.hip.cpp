@@ -108,13 +108,16 @@ __device__ __forceinline__ void udt7_kernel(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_udt7_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev g__p, __PSGrid3DFloat_dev g__q, float ce, float cw, float cn, float cs, float ct, float cb, float cc, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g__p;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g__p;
   __shared__ __attribute__((aligned(16))) float g__p_lds[S_g__p::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -131,25 +134,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_udt7_kernel(
     const physis_hip::BufWin<float> g__p_w = physis_hip::BufWin<float>::Make(g__p.p, g__p_nxy * g__p.dim[2], (long)(zb + -2) * g__p_nxy, (long)(ze + 2) * g__p_nxy);
     S_g__p g__p_st[PD];
     const typename S_g__p::Addr g__p_ra = S_g__p::Prepare(g__p.dim, x0, yrow, lane);
+    S_g__p g__p_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g__p_st[0].Load(g__p_w, g__p.p, g__p.dim, g__p_ra, zb + -1 + k);
-      g__p_st[0].Store(g__p_lds + k * S_g__p::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g__p_pro[k].Load(g__p_w, g__p.p, g__p.dim, g__p_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g__p_st[k].Load(g__p_w, g__p.p, g__p.dim, g__p_ra, zb + 2 + k);
     int g__p_base = 0;
     const int g__q_enx = g__q.dim[0], g__q_enxy = g__q.dim[0] * g__q.dim[1];
     const physis_hip::BufWin<float> g__q_ew = physis_hip::BufWin<float>::Make(g__q.p, g__q_enxy * g__q.dim[2], (long)zb * g__q_enxy, (long)ze * g__q_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g__p_pro[k].Store(g__p_lds + k * S_g__p::kPlane, wave, lane, g__p_ra);
     __syncthreads();
     __PSCtx_udt7_kernel ctx;
     ctx.g__p_p = g__p.p;
     for (int d = 0; d < 3; ++d) ctx.g__p_dim[d] = g__p.dim[d];
     ctx.g__q_p = g__q.p;
     for (int d = 0; d < 3; ++d) ctx.g__q_dim[d] = g__q.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g__p_dim[0] & 3) == 0);
       __builtin_assume((ctx.g__q_dim[0] & 3) == 0);
     }
@@ -195,7 +200,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_udt7_kernel(
           }
           physis_hip::StoreMasked<float, VX>(g__q_ew, xs + yrow * g__q_enx + z * g__q_enxy, g__q_out, g__q_mask);
         }
-        g__p_st[k % PD].Store(g__p_lds + physis_hip::RingSlot<4>(g__p_base, 3) * S_g__p::kPlane, wave, lane);
+        g__p_st[k % PD].Store(g__p_lds + physis_hip::RingSlot<4>(g__p_base, 3) * S_g__p::kPlane, wave, lane, g__p_ra);
         __syncthreads();
         g__p_st[k % PD].Load(g__p_w, g__p.p, g__p.dim, g__p_ra, z + 2 + PD);
       }
@@ -208,7 +213,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_udt7_kernel(const struct __PSStencil_udt7_kernel &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_udt7_kernel<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
 }
 
 template <int VX>
@@ -226,13 +231,17 @@ static int __PSLaunch_udt7_kernel(const struct __PSStencil_udt7_kernel &s, hipSt
 }
 
 static int __PSBlocks_udt7_kernel(const struct __PSStencil_udt7_kernel &s) {
-  return (s.g->dim[0] % 4 == 0) ? __PSShape_udt7_kernel<4>(s).blocks : __PSShape_udt7_kernel<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0) ? __PSShape_udt7_kernel<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_udt7_kernel<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_udt7_kernel<1>(s).blocks;
 }
 
 static int __PSRun_udt7_kernel(const struct __PSStencil_udt7_kernel &s, hipStream_t stream, void *red) {
   physis_hip::CheckUserGrid3D(s.g);
   physis_hip::CheckEmitDomain(s.dom, s.g);
-  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_udt7_kernel<4>(s, stream, red) : __PSLaunch_udt7_kernel<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_udt7_kernel<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_udt7_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_udt7_kernel<1>(s, stream, red);
 }
 
 // ---------------------------------------------- stencil udt7_whole_kernel
@@ -298,13 +307,16 @@ __device__ __forceinline__ void udt7_whole_kernel(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_udt7_whole_kernel(
     __PSDomain dom, __PSGrid3DFloat_dev g__p, __PSGrid3DFloat_dev g2__p, __PSGrid3DFloat_dev g2__q, float ce, float cw, float cn, float cs, float ct, float cb, float cc, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g__p;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g__p;
   __shared__ __attribute__((aligned(16))) float g__p_lds[S_g__p::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -321,11 +333,10 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_udt7_whole_kernel(
     const physis_hip::BufWin<float> g__p_w = physis_hip::BufWin<float>::Make(g__p.p, g__p_nxy * g__p.dim[2], (long)(zb + -2) * g__p_nxy, (long)(ze + 2) * g__p_nxy);
     S_g__p g__p_st[PD];
     const typename S_g__p::Addr g__p_ra = S_g__p::Prepare(g__p.dim, x0, yrow, lane);
+    S_g__p g__p_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g__p_st[0].Load(g__p_w, g__p.p, g__p.dim, g__p_ra, zb + -1 + k);
-      g__p_st[0].Store(g__p_lds + k * S_g__p::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g__p_pro[k].Load(g__p_w, g__p.p, g__p.dim, g__p_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g__p_st[k].Load(g__p_w, g__p.p, g__p.dim, g__p_ra, zb + 2 + k);
@@ -334,6 +345,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_udt7_whole_kernel(
     const physis_hip::BufWin<float> g2__p_ew = physis_hip::BufWin<float>::Make(g2__p.p, g2__p_enxy * g2__p.dim[2], (long)zb * g2__p_enxy, (long)ze * g2__p_enxy);
     const int g2__q_enx = g2__q.dim[0], g2__q_enxy = g2__q.dim[0] * g2__q.dim[1];
     const physis_hip::BufWin<float> g2__q_ew = physis_hip::BufWin<float>::Make(g2__q.p, g2__q_enxy * g2__q.dim[2], (long)zb * g2__q_enxy, (long)ze * g2__q_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g__p_pro[k].Store(g__p_lds + k * S_g__p::kPlane, wave, lane, g__p_ra);
     __syncthreads();
     __PSCtx_udt7_whole_kernel ctx;
     ctx.g__p_p = g__p.p;
@@ -342,8 +356,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_udt7_whole_kernel(
     for (int d = 0; d < 3; ++d) ctx.g2__p_dim[d] = g2__p.dim[d];
     ctx.g2__q_p = g2__q.p;
     for (int d = 0; d < 3; ++d) ctx.g2__q_dim[d] = g2__q.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g__p_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2__p_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2__q_dim[0] & 3) == 0);
@@ -396,7 +410,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_udt7_whole_kernel(
           physis_hip::StoreMasked<float, VX>(g2__p_ew, xs + yrow * g2__p_enx + z * g2__p_enxy, g2__p_out, g2__p_mask);
           physis_hip::StoreMasked<float, VX>(g2__q_ew, xs + yrow * g2__q_enx + z * g2__q_enxy, g2__q_out, g2__q_mask);
         }
-        g__p_st[k % PD].Store(g__p_lds + physis_hip::RingSlot<4>(g__p_base, 3) * S_g__p::kPlane, wave, lane);
+        g__p_st[k % PD].Store(g__p_lds + physis_hip::RingSlot<4>(g__p_base, 3) * S_g__p::kPlane, wave, lane, g__p_ra);
         __syncthreads();
         g__p_st[k % PD].Load(g__p_w, g__p.p, g__p.dim, g__p_ra, z + 2 + PD);
       }
@@ -409,7 +423,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_udt7_whole_kernel(const struct __PSStencil_udt7_whole_kernel &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_udt7_whole_kernel<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -427,14 +441,18 @@ static int __PSLaunch_udt7_whole_kernel(const struct __PSStencil_udt7_whole_kern
 }
 
 static int __PSBlocks_udt7_whole_kernel(const struct __PSStencil_udt7_whole_kernel &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_udt7_whole_kernel<4>(s).blocks : __PSShape_udt7_whole_kernel<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_udt7_whole_kernel<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_udt7_whole_kernel<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_udt7_whole_kernel<1>(s).blocks;
 }
 
 static int __PSRun_udt7_whole_kernel(const struct __PSStencil_udt7_whole_kernel &s, hipStream_t stream, void *red) {
   physis_hip::CheckUserGrid3D(s.g);
   physis_hip::CheckUserGrid3D(s.g2);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_udt7_whole_kernel<4>(s, stream, red) : __PSLaunch_udt7_whole_kernel<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_udt7_whole_kernel<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_udt7_whole_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_udt7_whole_kernel<1>(s, stream, red);
 }
 
 extern "C" {

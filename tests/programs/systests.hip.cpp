@@ -48,13 +48,16 @@ __device__ __forceinline__ void k7(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -71,25 +74,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_k7 ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -135,7 +140,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -148,7 +153,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_k7(const struct __PSStencil_k7 &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_k7<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -166,14 +171,18 @@ static int __PSLaunch_k7(const struct __PSStencil_k7 &s, hipStream_t stream, voi
 }
 
 static int __PSBlocks_k7(const struct __PSStencil_k7 &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7<4>(s).blocks : __PSShape_k7<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k7<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_k7<1>(s).blocks;
 }
 
 static int __PSRun_k7(const struct __PSStencil_k7 &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7<4>(s, stream, red) : __PSLaunch_k7<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k7<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_k7<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of k7 over a domain strictly inside
@@ -181,11 +190,12 @@ static int __PSRun_k7(const struct __PSStencil_k7 &s, hipStream_t stream, void *
 // tile and a one-point halo (bg's own values outside the domain) and
 // u'' = k7(u') two planes behind; dst <- u'', and bg <- u'
 // when store_mid.  red1 / red2: per-block partials of the two sweeps.
-template <int VX, int BY, int RED>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, int RED, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7(
     __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, __PSGrid3DFloat_dev bg, int store_mid, physis_hip::RunShape sh, float *__restrict__ red1, float *__restrict__ red2) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 4, false> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 4, false, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 4, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -205,10 +215,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7(
     const int xs = x0 + lane * VX;
     const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
     const int n = nxy * src.dim[2];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
-      __builtin_assume((nx & 3) == 0);
-    }
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) __builtin_assume((nx & 3) == 0);
     // u' halo columns x0 - 1 and x0 + TX of rows y0 - 1 .. y0 + TY: one
     // point per lane of wave 0 (which otherwise only loads)
     const bool hlane = wave == 0 && lane < 2 * (BY - 2);
@@ -227,13 +235,11 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7(
     const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
     const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg.p, n, (long)(zb - 1) * nxy, (long)(ze + 1) * nxy);
     const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(bg.p, n, (long)zb * nxy, (long)ze * nxy);
-    SA st[PD];
+    SA st[PD], pro[3];
     const typename SA::Addr ra = SA::Prepare(src.dim, x0, yrow, lane);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-      st[0].Store(a_lds + k * SA::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      pro[k].Load(aw, src.p, src.dim, ra, zb - 2 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       st[k].Load(aw, src.p, src.dim, ra, zb + 1 + k);
@@ -253,6 +259,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7(
       }
     };
     load1(zb - 1, 0);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      pro[k].Store(a_lds + k * SA::kPlane, wave, lane, ra);
     __syncthreads();
     __PSCtx_k7 ctx;
     ctx.g_p = src.p;
@@ -344,7 +353,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7(
           }
           physis_hip::StoreMasked<float, VX>(dw, xs + yrow * nx + (s - 2) * nxy, uu, m);
         }
-        st[k % PD].Store(a_lds + physis_hip::RingSlot<4>(abase, 3) * SA::kPlane, wave, lane);
+        st[k % PD].Store(a_lds + physis_hip::RingSlot<4>(abase, 3) * SA::kPlane, wave, lane, ra);
         __syncthreads();
         st[k % PD].Load(aw, src.p, src.dim, ra, s + 2 + PD);
       }
@@ -367,7 +376,7 @@ static constexpr int __PS2VX_k7 = 4, __PS2BY_k7 = 16;
 template <int VX, int BY>
 static physis_hip::RunShape __PSShape2_k7(const struct __PSStencil_k7 &s) {
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_k7<VX, BY, -1>, 64 * BY);
+      (const void *)__PSStencilRun2_k7<VX, BY, -1, false>, 64 * BY);
   return physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g, s.g2}, 3));
 }
@@ -376,14 +385,22 @@ static int __PSBlocks2_k7(const struct __PSStencil_k7 &s) {
   return __PSShape2_k7<__PS2VX_k7, __PS2BY_k7>(s).blocks;
 }
 
-static void __PSLaunch2_k7(const struct __PSStencil_k7 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
+template <bool RAGGED>
+static void __PSLaunch2R_k7(const struct __PSStencil_k7 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
   constexpr int VX = __PS2VX_k7, BY = __PS2BY_k7;
   const physis_hip::RunShape sh = __PSShape2_k7<VX, BY>(s);
   if (sh.blocks == 0) return;
   const dim3 grid(sh.blocks), block(64 * BY);
   {
-      hipLaunchKernelGGL((__PSStencilRun2_k7<VX, BY, -1>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.g2), store_mid, sh, (float *)red1, (float *)red2);
+      hipLaunchKernelGGL((__PSStencilRun2_k7<VX, BY, -1, RAGGED>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.g2), store_mid, sh, (float *)red1, (float *)red2);
   }
+}
+
+static void __PSLaunch2_k7(const struct __PSStencil_k7 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
+  if (s.g->dim[0] % __PS2VX_k7 == 0)
+    __PSLaunch2R_k7<false>(s, src, dst, store_mid, stream, red1, red2);
+  else
+    __PSLaunch2R_k7<__PS2VX_k7 != 1>(s, src, dst, store_mid, stream, red1, red2);
 }
 
 // The pair (s0, s1) is k7(a -> b), k7(b -> a) over one domain strictly
@@ -393,7 +410,7 @@ static bool __PSFusable2_k7(const struct __PSStencil_k7 &s0, const struct __PSSt
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g, *b = s0.g2;
   if (off || !a || !b || a == b || s1.g != b || s1.g2 != a) return false;
-  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;
+  if (a->num_dims != 3 || b->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d) {
     if (a->dim[d] != b->dim[d]) return false;
     if (s0.dom.local_min[d] != s1.dom.local_min[d] ||
@@ -445,13 +462,16 @@ __device__ __forceinline__ void k7p(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7p(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -468,25 +488,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7p(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_k7p ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -532,7 +554,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7p(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -545,7 +567,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_k7p(const struct __PSStencil_k7p &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_k7p<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -563,14 +585,18 @@ static int __PSLaunch_k7p(const struct __PSStencil_k7p &s, hipStream_t stream, v
 }
 
 static int __PSBlocks_k7p(const struct __PSStencil_k7p &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7p<4>(s).blocks : __PSShape_k7p<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7p<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k7p<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_k7p<1>(s).blocks;
 }
 
 static int __PSRun_k7p(const struct __PSStencil_k7p &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7p<4>(s, stream, red) : __PSLaunch_k7p<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7p<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k7p<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_k7p<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of k7p (temporal blocking): one pass over src
@@ -580,11 +606,12 @@ static int __PSRun_k7p(const struct __PSStencil_k7p &s, hipStream_t stream, void
 // planes s0 and s0 + 1 and u'' of s0 - 3 and s0 - 2 from rings of six
 // slots (source plane p in slot (p - zb + 2) % 6, u'(p) in slot
 // (p - zb + 1) % 6), then stores source planes s0 + 3 and s0 + 4.
-template <int VX, int BY>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7p(
     __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ mid, physis_hip::RunShape sh) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, true> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, true, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 6, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -602,9 +629,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7p(
   const int xs = x0 + lane * VX;
   const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
   const int n = nxy * src.dim[2];
-  // tiles start at multiples of TX and two-sweep runs need nx % 4 == 0
+  // tiles start at multiples of TX
   __builtin_assume((xs & (VX - 1)) == 0);
-  __builtin_assume((nx & (VX - 1)) == 0);
+  if constexpr (!RAGGED) __builtin_assume((nx & (VX - 1)) == 0);
   const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, (long)(zb - 3) * nxy, (long)(ze + 3) * nxy);
   const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
   const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);
@@ -613,7 +640,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7p(
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-    st[0].Store(a_lds + k * SA::kPlane, wave, lane);
+    st[0].Store(a_lds + k * SA::kPlane, wave, lane, ra);
   }
 #pragma unroll
   for (int k = 0; k < PD; ++k)
@@ -716,8 +743,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7p(
       __uprime(s0 + 1, (2 * j + 1) % 6, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 1) % 6);
       __udouble(s0 - 3, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 4) % 6);
       __udouble(s0 - 2, (2 * j + 3) % 6, (2 * j + 4) % 6, (2 * j + 5) % 6);
-      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane);
-      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane);
+      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane, ra);
+      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane, ra);
       __syncthreads();
       st[0].Load(aw, src.p, src.dim, ra, s0 + 5);
       st[1].Load(aw, src.p, src.dim, ra, s0 + 6);
@@ -729,11 +756,14 @@ static constexpr int __PS2VX_k7p = 4, __PS2BY_k7p = 12;
 static void __PSLaunch2_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
   constexpr int VX = __PS2VX_k7p, BY = __PS2BY_k7p;
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_k7p<VX, BY>, 64 * BY);
+      (const void *)__PSStencilRun2_k7p<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g}, 3));
   if (sh.blocks == 0) return;
-  hipLaunchKernelGGL((__PSStencilRun2_k7p<VX, BY>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+  if (s.g->dim[0] % VX == 0)
+    hipLaunchKernelGGL((__PSStencilRun2_k7p<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+  else
+    hipLaunchKernelGGL((__PSStencilRun2_k7p<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
 }
 
 // The pair (s0, s1) is k7p(a -> b), k7p(b -> a) over the whole grid with the
@@ -742,7 +772,7 @@ static bool __PSFusable2_k7p(const struct __PSStencil_k7p &s0, const struct __PS
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g, *b = s0.g2;
   if (off || !a || !b || a == b || s1.g != b || s1.g2 != a) return false;
-  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;
+  if (a->num_dims != 3 || b->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d) {
     if (a->dim[d] != b->dim[d]) return false;
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
@@ -821,13 +851,16 @@ __device__ __forceinline__ void k7n(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7n(
     __PSDomain dom, __PSGrid3DFloat_dev g1, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g1;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g1;
   __shared__ __attribute__((aligned(16))) float g1_lds[S_g1::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -844,25 +877,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7n(
     const physis_hip::BufWin<float> g1_w = physis_hip::BufWin<float>::Make(g1.p, g1_nxy * g1.dim[2], (long)(zb + -2) * g1_nxy, (long)(ze + 2) * g1_nxy);
     S_g1 g1_st[PD];
     const typename S_g1::Addr g1_ra = S_g1::Prepare(g1.dim, x0, yrow, lane);
+    S_g1 g1_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g1_st[0].Load(g1_w, g1.p, g1.dim, g1_ra, zb + -1 + k);
-      g1_st[0].Store(g1_lds + k * S_g1::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g1_pro[k].Load(g1_w, g1.p, g1.dim, g1_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g1_st[k].Load(g1_w, g1.p, g1.dim, g1_ra, zb + 2 + k);
     int g1_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g1_pro[k].Store(g1_lds + k * S_g1::kPlane, wave, lane, g1_ra);
     __syncthreads();
     __PSCtx_k7n ctx;
     ctx.g1_p = g1.p;
     for (int d = 0; d < 3; ++d) ctx.g1_dim[d] = g1.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g1_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -917,7 +952,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k7n(
             __pts(physis_hip::Flag<false>{});
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g1_st[k % PD].Store(g1_lds + physis_hip::RingSlot<4>(g1_base, 3) * S_g1::kPlane, wave, lane);
+        g1_st[k % PD].Store(g1_lds + physis_hip::RingSlot<4>(g1_base, 3) * S_g1::kPlane, wave, lane, g1_ra);
         __syncthreads();
         g1_st[k % PD].Load(g1_w, g1.p, g1.dim, g1_ra, z + 2 + PD);
       }
@@ -930,7 +965,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_k7n(const struct __PSStencil_k7n &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_k7n<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
 }
 
 template <int VX>
@@ -948,14 +983,18 @@ static int __PSLaunch_k7n(const struct __PSStencil_k7n &s, hipStream_t stream, v
 }
 
 static int __PSBlocks_k7n(const struct __PSStencil_k7n &s) {
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7n<4>(s).blocks : __PSShape_k7n<1>(s).blocks;
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7n<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_k7n<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_k7n<1>(s).blocks;
 }
 
 static int __PSRun_k7n(const struct __PSStencil_k7n &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g1, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7n<4>(s, stream, red) : __PSLaunch_k7n<1>(s, stream, red);
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7n<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_k7n<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_k7n<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of k7n (temporal blocking): one pass over src
@@ -965,11 +1004,12 @@ static int __PSRun_k7n(const struct __PSStencil_k7n &s, hipStream_t stream, void
 // planes s0 and s0 + 1 and u'' of s0 - 3 and s0 - 2 from rings of six
 // slots (source plane p in slot (p - zb + 2) % 6, u'(p) in slot
 // (p - zb + 1) % 6), then stores source planes s0 + 3 and s0 + 4.
-template <int VX, int BY>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7n(
     __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ mid, physis_hip::RunShape sh) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, false> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, false, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 6, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -987,9 +1027,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7n(
   const int xs = x0 + lane * VX;
   const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
   const int n = nxy * src.dim[2];
-  // tiles start at multiples of TX and two-sweep runs need nx % 4 == 0
+  // tiles start at multiples of TX
   __builtin_assume((xs & (VX - 1)) == 0);
-  __builtin_assume((nx & (VX - 1)) == 0);
+  if constexpr (!RAGGED) __builtin_assume((nx & (VX - 1)) == 0);
   const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, (long)(zb - 3) * nxy, (long)(ze + 3) * nxy);
   const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
   const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);
@@ -998,7 +1038,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7n(
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-    st[0].Store(a_lds + k * SA::kPlane, wave, lane);
+    st[0].Store(a_lds + k * SA::kPlane, wave, lane, ra);
   }
 #pragma unroll
   for (int k = 0; k < PD; ++k)
@@ -1119,8 +1159,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7n(
       __uprime(s0 + 1, (2 * j + 1) % 6, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 1) % 6);
       __udouble(s0 - 3, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 4) % 6);
       __udouble(s0 - 2, (2 * j + 3) % 6, (2 * j + 4) % 6, (2 * j + 5) % 6);
-      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane);
-      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane);
+      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane, ra);
+      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane, ra);
       __syncthreads();
       st[0].Load(aw, src.p, src.dim, ra, s0 + 5);
       st[1].Load(aw, src.p, src.dim, ra, s0 + 6);
@@ -1132,11 +1172,14 @@ static constexpr int __PS2VX_k7n = 4, __PS2BY_k7n = 12;
 static void __PSLaunch2_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
   constexpr int VX = __PS2VX_k7n, BY = __PS2BY_k7n;
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_k7n<VX, BY>, 64 * BY);
+      (const void *)__PSStencilRun2_k7n<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g1}, 3));
   if (sh.blocks == 0) return;
-  hipLaunchKernelGGL((__PSStencilRun2_k7n<VX, BY>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+  if (s.g1->dim[0] % VX == 0)
+    hipLaunchKernelGGL((__PSStencilRun2_k7n<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+  else
+    hipLaunchKernelGGL((__PSStencilRun2_k7n<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
 }
 
 // The pair (s0, s1) is k7n(a -> b), k7n(b -> a) over the whole grid with the
@@ -1145,7 +1188,7 @@ static bool __PSFusable2_k7n(const struct __PSStencil_k7n &s0, const struct __PS
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g1, *b = s0.g2;
   if (off || !a || !b || a == b || s1.g1 != b || s1.g2 != a) return false;
-  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;
+  if (a->num_dims != 3 || b->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d) {
     if (a->dim[d] != b->dim[d]) return false;
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
@@ -1195,13 +1238,16 @@ __device__ __forceinline__ void kasym(
 // last 2 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kasym(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 2;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 2, HY, 5, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 2, HY, 5, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -1218,25 +1264,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kasym(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -3) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -2 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 4; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -2 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_kasym ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -1272,7 +1320,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kasym(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<5>(g_base, 4) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<5>(g_base, 4) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
         g_base = physis_hip::RingSlot<5>(g_base, 1);
@@ -1286,7 +1334,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_kasym(const struct __PSStencil_kasym &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_kasym<VX, 8, -1>, 64 * 8);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 8 - 2 * 2, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 3));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 8 - 2 * 2, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 3));
 }
 
 template <int VX>
@@ -1304,14 +1352,18 @@ static int __PSLaunch_kasym(const struct __PSStencil_kasym &s, hipStream_t strea
 }
 
 static int __PSBlocks_kasym(const struct __PSStencil_kasym &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kasym<4>(s).blocks : __PSShape_kasym<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kasym<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_kasym<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_kasym<1>(s).blocks;
 }
 
 static int __PSRun_kasym(const struct __PSStencil_kasym &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kasym<4>(s, stream, red) : __PSLaunch_kasym<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kasym<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_kasym<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_kasym<1>(s, stream, red);
 }
 
 // ---------------------------------------------- stencil kasymp
@@ -1355,13 +1407,16 @@ __device__ __forceinline__ void kasymp(
 // last 0 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kasymp(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 0;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 2, HY, 2, true> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 2, HY, 2, true, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -1378,25 +1433,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kasymp(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -1) * g_nxy, (long)(ze + 1) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[1];
 #pragma unroll
-    for (int k = 0; k < 1; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + 0 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 1; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + 0 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 1 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 1; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_kasymp ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -1429,7 +1486,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kasymp(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<2>(g_base, 1) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<2>(g_base, 1) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 1 + PD);
       }
@@ -1442,7 +1499,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_kasymp(const struct __PSStencil_kasymp &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_kasymp<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 1));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 1));
 }
 
 template <int VX>
@@ -1460,14 +1517,18 @@ static int __PSLaunch_kasymp(const struct __PSStencil_kasymp &s, hipStream_t str
 }
 
 static int __PSBlocks_kasymp(const struct __PSStencil_kasymp &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kasymp<4>(s).blocks : __PSShape_kasymp<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kasymp<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_kasymp<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_kasymp<1>(s).blocks;
 }
 
 static int __PSRun_kasymp(const struct __PSStencil_kasymp &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kasymp<4>(s, stream, red) : __PSLaunch_kasymp<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kasymp<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_kasymp<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_kasymp<1>(s, stream, red);
 }
 
 // ---------------------------------------------- stencil k27
@@ -1511,13 +1572,16 @@ __device__ __forceinline__ void k27(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 2;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -1534,25 +1598,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_k27 ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -1624,7 +1690,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
         g_base = physis_hip::RingSlot<4>(g_base, 1);
@@ -1638,7 +1704,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_k27(const struct __PSStencil_k27 &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_k27<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -1656,14 +1722,18 @@ static int __PSLaunch_k27(const struct __PSStencil_k27 &s, hipStream_t stream, v
 }
 
 static int __PSBlocks_k27(const struct __PSStencil_k27 &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27<4>(s).blocks : __PSShape_k27<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k27<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_k27<1>(s).blocks;
 }
 
 static int __PSRun_k27(const struct __PSStencil_k27 &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27<4>(s, stream, red) : __PSLaunch_k27<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k27<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_k27<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of k27 over a domain strictly inside
@@ -1671,11 +1741,12 @@ static int __PSRun_k27(const struct __PSStencil_k27 &s, hipStream_t stream, void
 // tile and a one-point halo (bg's own values outside the domain) and
 // u'' = k27(u') two planes behind; dst <- u'', and bg <- u'
 // when store_mid.  red1 / red2: per-block partials of the two sweeps.
-template <int VX, int BY, int RED>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, int RED, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27(
     __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, __PSGrid3DFloat_dev bg, int store_mid, physis_hip::RunShape sh, float *__restrict__ red1, float *__restrict__ red2) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 4, false> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 4, false, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 4, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -1695,10 +1766,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27(
     const int xs = x0 + lane * VX;
     const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
     const int n = nxy * src.dim[2];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
-      __builtin_assume((nx & 3) == 0);
-    }
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) __builtin_assume((nx & 3) == 0);
     // u' halo columns x0 - 1 and x0 + TX of rows y0 - 1 .. y0 + TY: one
     // point per lane of wave 0 (which otherwise only loads)
     const bool hlane = wave == 0 && lane < 2 * (BY - 2);
@@ -1717,13 +1786,11 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27(
     const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
     const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg.p, n, (long)(zb - 1) * nxy, (long)(ze + 1) * nxy);
     const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(bg.p, n, (long)zb * nxy, (long)ze * nxy);
-    SA st[PD];
+    SA st[PD], pro[3];
     const typename SA::Addr ra = SA::Prepare(src.dim, x0, yrow, lane);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-      st[0].Store(a_lds + k * SA::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      pro[k].Load(aw, src.p, src.dim, ra, zb - 2 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       st[k].Load(aw, src.p, src.dim, ra, zb + 1 + k);
@@ -1743,6 +1810,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27(
       }
     };
     load1(zb - 1, 0);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      pro[k].Store(a_lds + k * SA::kPlane, wave, lane, ra);
     __syncthreads();
     __PSCtx_k27 ctx;
     ctx.g_p = src.p;
@@ -1910,7 +1980,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27(
           }
           physis_hip::StoreMasked<float, VX>(dw, xs + yrow * nx + (s - 2) * nxy, uu, m);
         }
-        st[k % PD].Store(a_lds + physis_hip::RingSlot<4>(abase, 3) * SA::kPlane, wave, lane);
+        st[k % PD].Store(a_lds + physis_hip::RingSlot<4>(abase, 3) * SA::kPlane, wave, lane, ra);
         __syncthreads();
         st[k % PD].Load(aw, src.p, src.dim, ra, s + 2 + PD);
       }
@@ -1933,7 +2003,7 @@ static constexpr int __PS2VX_k27 = 4, __PS2BY_k27 = 16;
 template <int VX, int BY>
 static physis_hip::RunShape __PSShape2_k27(const struct __PSStencil_k27 &s) {
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_k27<VX, BY, -1>, 64 * BY);
+      (const void *)__PSStencilRun2_k27<VX, BY, -1, false>, 64 * BY);
   return physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g, s.g2}, 3));
 }
@@ -1942,14 +2012,22 @@ static int __PSBlocks2_k27(const struct __PSStencil_k27 &s) {
   return __PSShape2_k27<__PS2VX_k27, __PS2BY_k27>(s).blocks;
 }
 
-static void __PSLaunch2_k27(const struct __PSStencil_k27 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
+template <bool RAGGED>
+static void __PSLaunch2R_k27(const struct __PSStencil_k27 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
   constexpr int VX = __PS2VX_k27, BY = __PS2BY_k27;
   const physis_hip::RunShape sh = __PSShape2_k27<VX, BY>(s);
   if (sh.blocks == 0) return;
   const dim3 grid(sh.blocks), block(64 * BY);
   {
-      hipLaunchKernelGGL((__PSStencilRun2_k27<VX, BY, -1>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.g2), store_mid, sh, (float *)red1, (float *)red2);
+      hipLaunchKernelGGL((__PSStencilRun2_k27<VX, BY, -1, RAGGED>), grid, block, 0, stream, s.dom, src, dst, physis_hip::DevView<__PSGrid3DFloat_dev>(s.g2), store_mid, sh, (float *)red1, (float *)red2);
   }
+}
+
+static void __PSLaunch2_k27(const struct __PSStencil_k27 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, int store_mid, hipStream_t stream, void *red1, void *red2) {
+  if (s.g->dim[0] % __PS2VX_k27 == 0)
+    __PSLaunch2R_k27<false>(s, src, dst, store_mid, stream, red1, red2);
+  else
+    __PSLaunch2R_k27<__PS2VX_k27 != 1>(s, src, dst, store_mid, stream, red1, red2);
 }
 
 // The pair (s0, s1) is k27(a -> b), k27(b -> a) over one domain strictly
@@ -1959,7 +2037,7 @@ static bool __PSFusable2_k27(const struct __PSStencil_k27 &s0, const struct __PS
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g, *b = s0.g2;
   if (off || !a || !b || a == b || s1.g != b || s1.g2 != a) return false;
-  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;
+  if (a->num_dims != 3 || b->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d) {
     if (a->dim[d] != b->dim[d]) return false;
     if (s0.dom.local_min[d] != s1.dom.local_min[d] ||
@@ -2011,13 +2089,16 @@ __device__ __forceinline__ void k27p(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27p(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 2;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -2034,25 +2115,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27p(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_k27p ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -2124,7 +2207,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27p(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
         g_base = physis_hip::RingSlot<4>(g_base, 1);
@@ -2138,7 +2221,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_k27p(const struct __PSStencil_k27p &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_k27p<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -2156,14 +2239,18 @@ static int __PSLaunch_k27p(const struct __PSStencil_k27p &s, hipStream_t stream,
 }
 
 static int __PSBlocks_k27p(const struct __PSStencil_k27p &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27p<4>(s).blocks : __PSShape_k27p<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27p<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k27p<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_k27p<1>(s).blocks;
 }
 
 static int __PSRun_k27p(const struct __PSStencil_k27p &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27p<4>(s, stream, red) : __PSLaunch_k27p<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27p<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k27p<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_k27p<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of k27p (temporal blocking): one pass over src
@@ -2173,11 +2260,12 @@ static int __PSRun_k27p(const struct __PSStencil_k27p &s, hipStream_t stream, vo
 // planes s0 and s0 + 1 and u'' of s0 - 3 and s0 - 2 from rings of six
 // slots (source plane p in slot (p - zb + 2) % 6, u'(p) in slot
 // (p - zb + 1) % 6), then stores source planes s0 + 3 and s0 + 4.
-template <int VX, int BY>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27p(
     __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ mid, physis_hip::RunShape sh) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, true> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, true, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 6, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -2195,9 +2283,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27p(
   const int xs = x0 + lane * VX;
   const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
   const int n = nxy * src.dim[2];
-  // tiles start at multiples of TX and two-sweep runs need nx % 4 == 0
+  // tiles start at multiples of TX
   __builtin_assume((xs & (VX - 1)) == 0);
-  __builtin_assume((nx & (VX - 1)) == 0);
+  if constexpr (!RAGGED) __builtin_assume((nx & (VX - 1)) == 0);
   const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, (long)(zb - 3) * nxy, (long)(ze + 3) * nxy);
   const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
   const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);
@@ -2206,7 +2294,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27p(
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-    st[0].Store(a_lds + k * SA::kPlane, wave, lane);
+    st[0].Store(a_lds + k * SA::kPlane, wave, lane, ra);
   }
 #pragma unroll
   for (int k = 0; k < PD; ++k)
@@ -2385,8 +2473,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27p(
       __uprime(s0 + 1, (2 * j + 1) % 6, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 1) % 6);
       __udouble(s0 - 3, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 4) % 6);
       __udouble(s0 - 2, (2 * j + 3) % 6, (2 * j + 4) % 6, (2 * j + 5) % 6);
-      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane);
-      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane);
+      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane, ra);
+      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane, ra);
       __syncthreads();
       st[0].Load(aw, src.p, src.dim, ra, s0 + 5);
       st[1].Load(aw, src.p, src.dim, ra, s0 + 6);
@@ -2398,11 +2486,14 @@ static constexpr int __PS2VX_k27p = 4, __PS2BY_k27p = 12;
 static void __PSLaunch2_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
   constexpr int VX = __PS2VX_k27p, BY = __PS2BY_k27p;
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_k27p<VX, BY>, 64 * BY);
+      (const void *)__PSStencilRun2_k27p<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g}, 3));
   if (sh.blocks == 0) return;
-  hipLaunchKernelGGL((__PSStencilRun2_k27p<VX, BY>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+  if (s.g->dim[0] % VX == 0)
+    hipLaunchKernelGGL((__PSStencilRun2_k27p<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+  else
+    hipLaunchKernelGGL((__PSStencilRun2_k27p<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
 }
 
 // The pair (s0, s1) is k27p(a -> b), k27p(b -> a) over the whole grid with the
@@ -2411,7 +2502,7 @@ static bool __PSFusable2_k27p(const struct __PSStencil_k27p &s0, const struct __
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g, *b = s0.g2;
   if (off || !a || !b || a == b || s1.g != b || s1.g2 != a) return false;
-  if (a->num_dims != 3 || b->num_dims != 3 || a->dim[0] % 4) return false;
+  if (a->num_dims != 3 || b->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d) {
     if (a->dim[d] != b->dim[d]) return false;
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
@@ -2461,13 +2552,16 @@ __device__ __forceinline__ void k27i(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27i(
     __PSDomain dom, __PSGrid3DInt_dev g, __PSGrid3DInt_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 2;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<int, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<int, VX, BY, 1, HY, 4, false, int, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) int g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -2484,25 +2578,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27i(
     const physis_hip::BufWin<int> g_w = physis_hip::BufWin<int>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<int> g2_ew = physis_hip::BufWin<int>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_k27i ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -2574,7 +2670,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k27i(
           }
           physis_hip::StoreMasked<int, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
         g_base = physis_hip::RingSlot<4>(g_base, 1);
@@ -2588,7 +2684,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_k27i(const struct __PSStencil_k27i &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_k27i<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -2606,14 +2702,18 @@ static int __PSLaunch_k27i(const struct __PSStencil_k27i &s, hipStream_t stream,
 }
 
 static int __PSBlocks_k27i(const struct __PSStencil_k27i &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27i<4>(s).blocks : __PSShape_k27i<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27i<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k27i<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_k27i<1>(s).blocks;
 }
 
 static int __PSRun_k27i(const struct __PSStencil_k27i &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_INT);
   physis_hip::CheckGrid3D(s.g2, PS_INT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27i<4>(s, stream, red) : __PSLaunch_k27i<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27i<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k27i<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_k27i<1>(s, stream, red);
 }
 
 static void __PSStencilRun_0(int iter, struct __PSStencil_k7 s0) {
@@ -2937,13 +3037,16 @@ __device__ __forceinline__ void krb(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_krb(
     __PSDomain dom, __PSGrid3DFloat_dev g, physis_hip::RunShape sh, float *__restrict__ __red, int __rb) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -2960,23 +3063,25 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_krb(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g_enx = g.dim[0], g_enxy = g.dim[0] * g.dim[1];
     const physis_hip::BufWin<float> g_ew = physis_hip::BufWin<float>::Make(g.p, g_enxy * g.dim[2], (long)zb * g_enxy, (long)ze * g_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_krb ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
     }
     constexpr int U = 4;
@@ -3022,7 +3127,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_krb(
           }
           physis_hip::StoreMasked<float, VX>(g_ew, xs + yrow * g_enx + z * g_enxy, g_out, g_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -3035,7 +3140,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_krb(const struct __PSStencil_krb &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_krb<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
 }
 
 template <int VX>
@@ -3053,13 +3158,17 @@ static int __PSLaunch_krb(const struct __PSStencil_krb &s, hipStream_t stream, v
 }
 
 static int __PSBlocks_krb(const struct __PSStencil_krb &s) {
-  return (s.g->dim[0] % 4 == 0) ? __PSShape_krb<4>(s).blocks : __PSShape_krb<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0) ? __PSShape_krb<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_krb<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_krb<1>(s).blocks;
 }
 
 static int __PSRun_krb(const struct __PSStencil_krb &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g);
-  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_krb<4>(s, stream, red) : __PSLaunch_krb<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_krb<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_krb<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_krb<1>(s, stream, red);
 }
 
 // Two-sweep run kernel of krb (temporal blocking): one pass over src
@@ -3071,11 +3180,12 @@ static int __PSRun_krb(const struct __PSStencil_krb &s, hipStream_t stream, void
 // (p - zb + 1) % 6), then stores source planes s0 + 3 and s0 + 4.
 // Red-black: one pass is one iteration (red sweep u', black sweep
 // u''); dom is the map's domain, gd the whole grid the pass tiles.
-template <int VX, int BY>
+// RAGGED: x extents that are not multiples of VX.
+template <int VX, int BY, bool RAGGED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
     __PSDomain dom, __PSDomain gd, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ mid, physis_hip::RunShape sh) {
   constexpr int PD = 2, TX = 64 * VX, TY = BY - 4;
-  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, false> SA;
+  typedef physis_hip::Stage<float, VX, BY, 2, 2, 6, false, float, RAGGED> SA;
   typedef physis_hip::Stage<float, VX, BY, 1, 1, 6, false> SB;
   __shared__ __attribute__((aligned(16))) float a_lds[SA::kLdsElems];
   __shared__ __attribute__((aligned(16))) float b_lds[SB::kLdsElems];
@@ -3093,22 +3203,23 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
   const int xs = x0 + lane * VX;
   const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
   const int n = nxy * src.dim[2];
-  // tiles start at multiples of TX and two-sweep runs need nx % 4 == 0
+  // tiles start at multiples of TX
   __builtin_assume((xs & (VX - 1)) == 0);
-  __builtin_assume((nx & (VX - 1)) == 0);
+  if constexpr (!RAGGED) __builtin_assume((nx & (VX - 1)) == 0);
   const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, (long)(zb - 3) * nxy, (long)(ze + 3) * nxy);
   const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nxy, (long)ze * nxy);
   const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);
-  SA st[PD];
+  SA st[PD], pro[4];
   const typename SA::Addr ra = SA::Prepare(src.dim, x0, yrow, lane);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    st[0].Load(aw, src.p, src.dim, ra, zb - 2 + k);
-    st[0].Store(a_lds + k * SA::kPlane, wave, lane);
-  }
+  for (int k = 0; k < 4; ++k)
+    pro[k].Load(aw, src.p, src.dim, ra, zb - 2 + k);
 #pragma unroll
   for (int k = 0; k < PD; ++k)
     st[k].Load(aw, src.p, src.dim, ra, zb + 2 + k);
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    pro[k].Store(a_lds + k * SA::kPlane, wave, lane, ra);
   __syncthreads();
   __PSCtx_krb ctx;
   ctx.g_p = src.p;
@@ -3207,8 +3318,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
       __uprime(s0 + 1, (2 * j + 1) % 6, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 1) % 6);
       __udouble(s0 - 3, (2 * j + 2) % 6, (2 * j + 3) % 6, (2 * j + 4) % 6);
       __udouble(s0 - 2, (2 * j + 3) % 6, (2 * j + 4) % 6, (2 * j + 5) % 6);
-      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane);
-      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane);
+      st[0].Store(a_lds + ((2 * j + 4) % 6) * SA::kPlane, wave, lane, ra);
+      st[1].Store(a_lds + ((2 * j + 5) % 6) * SA::kPlane, wave, lane, ra);
       __syncthreads();
       st[0].Load(aw, src.p, src.dim, ra, s0 + 5);
       st[1].Load(aw, src.p, src.dim, ra, s0 + 6);
@@ -3221,19 +3332,22 @@ static void __PSLaunch2_krb(const struct __PSStencil_krb &s, const __PSGrid3DFlo
   constexpr int VX = __PS2VX_krb, BY = __PS2BY_krb;
   const __PSDomain gd = physis_hip::WholeDomain(s.g);
   static int per_cu = physis_hip::BlocksPerCU(
-      (const void *)__PSStencilRun2_krb<VX, BY>, 64 * BY);
+      (const void *)__PSStencilRun2_krb<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(gd, 64 * VX, BY - 4, per_cu,
       physis_hip::WindowChunkLimit({s.g}, 3));
   if (sh.blocks == 0) return;
-  hipLaunchKernelGGL((__PSStencilRun2_krb<VX, BY>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, sh);
+  if (s.g->dim[0] % VX == 0)
+    hipLaunchKernelGGL((__PSStencilRun2_krb<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, sh);
+  else
+    hipLaunchKernelGGL((__PSStencilRun2_krb<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, sh);
 }
 
 // The red-black map s0 may run as one pass per iteration: both colours, a domain
-// strictly inside a grid whose x extent is a multiple of 4.
+// strictly inside the grid.
 static bool __PSFusableRB_krb(const struct __PSStencil_krb &s0) {
   static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
   const __PSGrid *a = s0.g;
-  if (off || !a || s0.__rb != 2 || a->num_dims != 3 || a->dim[0] % 4) return false;
+  if (off || !a || s0.__rb != 2 || a->num_dims != 3) return false;
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
@@ -3299,13 +3413,16 @@ __device__ __forceinline__ void krbp(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_krbp(
     __PSDomain dom, __PSGrid3DFloat_dev g, physis_hip::RunShape sh, float *__restrict__ __red, int __rb) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -3322,23 +3439,25 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_krbp(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g_enx = g.dim[0], g_enxy = g.dim[0] * g.dim[1];
     const physis_hip::BufWin<float> g_ew = physis_hip::BufWin<float>::Make(g.p, g_enxy * g.dim[2], (long)zb * g_enxy, (long)ze * g_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_krbp ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
     }
     constexpr int U = 4;
@@ -3384,7 +3503,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_krbp(
           }
           physis_hip::StoreMasked<float, VX>(g_ew, xs + yrow * g_enx + z * g_enxy, g_out, g_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -3397,7 +3516,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_krbp(const struct __PSStencil_krbp &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_krbp<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
 }
 
 template <int VX>
@@ -3415,7 +3534,9 @@ static int __PSLaunch_krbp(const struct __PSStencil_krbp &s, hipStream_t stream,
 }
 
 static int __PSBlocks_krbp(const struct __PSStencil_krbp &s) {
-  return (s.g->dim[0] % 4 == 0) ? __PSShape_krbp<4>(s).blocks : __PSShape_krbp<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0) ? __PSShape_krbp<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_krbp<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_krbp<1>(s).blocks;
 }
 
 static int __PSRun_krbp(const struct __PSStencil_krbp &s, hipStream_t stream, void *red) {
@@ -3426,7 +3547,9 @@ static int __PSRun_krbp(const struct __PSStencil_krbp &s, hipStream_t stream, vo
     __warned = true;
   }
   physis_hip::CheckEmitDomain(s.dom, s.g);
-  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_krbp<4>(s, stream, red) : __PSLaunch_krbp<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_krbp<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_krbp<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_krbp<1>(s, stream, red);
 }
 
 static void __PSStencilRun_10(int iter, struct __PSStencil_krb s0) {
@@ -3633,13 +3756,16 @@ __device__ __forceinline__ void k5(
 // last 0 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k5(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 0;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -3656,17 +3782,19 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k5(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_k5 ctx;
     ctx.g_p = g.p;
@@ -3677,8 +3805,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k5(
     ctx.g2_dim[0] = g2.dim[0];
     ctx.g2_dim[1] = g2.dim[2];
     ctx.g2_dim[2] = 1;
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -3718,7 +3846,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_k5(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -3731,7 +3859,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_k5(const struct __PSStencil_k5 &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_k5<VX, 1, -1>, 64 * 1);
-  return physis_hip::PlanRun(physis_hip::RowDomain(s.dom), 64 * VX, 1 - 2 * 0, per_cu, physis_hip::WindowChunkLimitRows({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(physis_hip::RowDomain(s.dom), 64 * physis_hip::FormVX(VX), 1 - 2 * 0, per_cu, physis_hip::WindowChunkLimitRows({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -3749,14 +3877,18 @@ static int __PSLaunch_k5(const struct __PSStencil_k5 &s, hipStream_t stream, voi
 }
 
 static int __PSBlocks_k5(const struct __PSStencil_k5 &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k5<4>(s).blocks : __PSShape_k5<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k5<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k5<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_k5<1>(s).blocks;
 }
 
 static int __PSRun_k5(const struct __PSStencil_k5 &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k5<4>(s, stream, red) : __PSLaunch_k5<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k5<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k5<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_k5<1>(s, stream, red);
 }
 
 static void __PSStencilRun_13(int iter, struct __PSStencil_k3 s0) {
@@ -3872,13 +4004,16 @@ __device__ __forceinline__ void kmix(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kmix(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, __PSGrid1DFloat_dev i, __PSGrid2DFloat_dev j, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -3895,17 +4030,19 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kmix(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_kmix ctx;
     ctx.g_p = g.p;
@@ -3916,8 +4053,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kmix(
     for (int d = 0; d < 3; ++d) ctx.i_dim[d] = d < 1 ? i.dim[d] : 1;
     ctx.j_p = j.p;
     for (int d = 0; d < 3; ++d) ctx.j_dim[d] = d < 2 ? j.dim[d] : 1;
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -3963,7 +4100,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kmix(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
       }
@@ -3976,7 +4113,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_kmix(const struct __PSStencil_kmix &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_kmix<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 2));
 }
 
 template <int VX>
@@ -3994,7 +4131,9 @@ static int __PSLaunch_kmix(const struct __PSStencil_kmix &s, hipStream_t stream,
 }
 
 static int __PSBlocks_kmix(const struct __PSStencil_kmix &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kmix<4>(s).blocks : __PSShape_kmix<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kmix<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_kmix<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_kmix<1>(s).blocks;
 }
 
 static int __PSRun_kmix(const struct __PSStencil_kmix &s, hipStream_t stream, void *red) {
@@ -4003,7 +4142,9 @@ static int __PSRun_kmix(const struct __PSStencil_kmix &s, hipStream_t stream, vo
   physis_hip::CheckGrid3D(s.i, PS_FLOAT);
   physis_hip::CheckGrid3D(s.j, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kmix<4>(s, stream, red) : __PSLaunch_kmix<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kmix<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_kmix<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_kmix<1>(s, stream, red);
 }
 
 static void __PSStencilRun_15(int iter, struct __PSStencil_kmix s0) {
@@ -4089,13 +4230,16 @@ __device__ __forceinline__ void khole(
 // last 0 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_khole(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 0;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 2, HY, 2, false> S_g;
+  typedef physis_hip::Stage<float, VX, BY, 2, HY, 2, false, float, RAGGED> S_g;
   __shared__ __attribute__((aligned(16))) float g_lds[S_g::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -4112,25 +4256,27 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_khole(
     const physis_hip::BufWin<float> g_w = physis_hip::BufWin<float>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -1) * g_nxy, (long)(ze + 1) * g_nxy);
     S_g g_st[PD];
     const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[1];
 #pragma unroll
-    for (int k = 0; k < 1; ++k) {
-      g_st[0].Load(g_w, g.p, g.dim, g_ra, zb + 0 + k);
-      g_st[0].Store(g_lds + k * S_g::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 1; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + 0 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 1 + k);
     int g_base = 0;
     const int g2_enx = g2.dim[0], g2_enxy = g2.dim[0] * g2.dim[1];
     const physis_hip::BufWin<float> g2_ew = physis_hip::BufWin<float>::Make(g2.p, g2_enxy * g2.dim[2], (long)zb * g2_enxy, (long)ze * g2_enxy);
+#pragma unroll
+    for (int k = 0; k < 1; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
     __syncthreads();
     __PSCtx_khole ctx;
     ctx.g_p = g.p;
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -4164,7 +4310,7 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_khole(
           }
           physis_hip::StoreMasked<float, VX>(g2_ew, xs + yrow * g2_enx + z * g2_enxy, g2_out, g2_mask);
         }
-        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<2>(g_base, 1) * S_g::kPlane, wave, lane);
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<2>(g_base, 1) * S_g::kPlane, wave, lane, g_ra);
         __syncthreads();
         g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 1 + PD);
       }
@@ -4177,7 +4323,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_khole(const struct __PSStencil_khole &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_khole<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 1));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 1));
 }
 
 template <int VX>
@@ -4195,14 +4341,18 @@ static int __PSLaunch_khole(const struct __PSStencil_khole &s, hipStream_t strea
 }
 
 static int __PSBlocks_khole(const struct __PSStencil_khole &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_khole<4>(s).blocks : __PSShape_khole<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_khole<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_khole<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_khole<1>(s).blocks;
 }
 
 static int __PSRun_khole(const struct __PSStencil_khole &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_khole<4>(s, stream, red) : __PSLaunch_khole<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_khole<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_khole<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_khole<1>(s, stream, red);
 }
 
 static void __PSStencilRun_16(int iter, struct __PSStencil_khole s0) {
@@ -4359,17 +4509,20 @@ __device__ __forceinline__ void kvec3(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kvec3(
     __PSDomain dom, __PSGrid3DFloat_dev g1__x, __PSGrid3DFloat_dev g1__y, __PSGrid3DFloat_dev g1__z, __PSGrid3DFloat_dev g2__x, __PSGrid3DFloat_dev g2__y, __PSGrid3DFloat_dev g2__z, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 2;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 2, false> S_g1__x;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 2, false, float, RAGGED> S_g1__x;
   __shared__ __attribute__((aligned(16))) float g1__x_lds[S_g1__x::kLdsElems];
-  typedef physis_hip::Stage<float, VX, BY, 0, HY, 4, false> S_g1__y;
+  typedef physis_hip::Stage<float, VX, BY, 0, HY, 4, false, float, RAGGED> S_g1__y;
   __shared__ __attribute__((aligned(16))) float g1__y_lds[S_g1__y::kLdsElems];
-  typedef physis_hip::Stage<float, VX, BY, 0, HY, 4, false> S_g1__z;
+  typedef physis_hip::Stage<float, VX, BY, 0, HY, 4, false, float, RAGGED> S_g1__z;
   __shared__ __attribute__((aligned(16))) float g1__z_lds[S_g1__z::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -4386,11 +4539,10 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kvec3(
     const physis_hip::BufWin<float> g1__x_w = physis_hip::BufWin<float>::Make(g1__x.p, g1__x_nxy * g1__x.dim[2], (long)(zb + -1) * g1__x_nxy, (long)(ze + 1) * g1__x_nxy);
     S_g1__x g1__x_st[PD];
     const typename S_g1__x::Addr g1__x_ra = S_g1__x::Prepare(g1__x.dim, x0, yrow, lane);
+    S_g1__x g1__x_pro[1];
 #pragma unroll
-    for (int k = 0; k < 1; ++k) {
-      g1__x_st[0].Load(g1__x_w, g1__x.p, g1__x.dim, g1__x_ra, zb + 0 + k);
-      g1__x_st[0].Store(g1__x_lds + k * S_g1__x::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 1; ++k)
+      g1__x_pro[k].Load(g1__x_w, g1__x.p, g1__x.dim, g1__x_ra, zb + 0 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g1__x_st[k].Load(g1__x_w, g1__x.p, g1__x.dim, g1__x_ra, zb + 1 + k);
@@ -4399,11 +4551,10 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kvec3(
     const physis_hip::BufWin<float> g1__y_w = physis_hip::BufWin<float>::Make(g1__y.p, g1__y_nxy * g1__y.dim[2], (long)(zb + -2) * g1__y_nxy, (long)(ze + 2) * g1__y_nxy);
     S_g1__y g1__y_st[PD];
     const typename S_g1__y::Addr g1__y_ra = S_g1__y::Prepare(g1__y.dim, x0, yrow, lane);
+    S_g1__y g1__y_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g1__y_st[0].Load(g1__y_w, g1__y.p, g1__y.dim, g1__y_ra, zb + -1 + k);
-      g1__y_st[0].Store(g1__y_lds + k * S_g1__y::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g1__y_pro[k].Load(g1__y_w, g1__y.p, g1__y.dim, g1__y_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g1__y_st[k].Load(g1__y_w, g1__y.p, g1__y.dim, g1__y_ra, zb + 2 + k);
@@ -4412,11 +4563,10 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kvec3(
     const physis_hip::BufWin<float> g1__z_w = physis_hip::BufWin<float>::Make(g1__z.p, g1__z_nxy * g1__z.dim[2], (long)(zb + -2) * g1__z_nxy, (long)(ze + 2) * g1__z_nxy);
     S_g1__z g1__z_st[PD];
     const typename S_g1__z::Addr g1__z_ra = S_g1__z::Prepare(g1__z.dim, x0, yrow, lane);
+    S_g1__z g1__z_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g1__z_st[0].Load(g1__z_w, g1__z.p, g1__z.dim, g1__z_ra, zb + -1 + k);
-      g1__z_st[0].Store(g1__z_lds + k * S_g1__z::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g1__z_pro[k].Load(g1__z_w, g1__z.p, g1__z.dim, g1__z_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g1__z_st[k].Load(g1__z_w, g1__z.p, g1__z.dim, g1__z_ra, zb + 2 + k);
@@ -4427,6 +4577,15 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kvec3(
     const physis_hip::BufWin<float> g2__y_ew = physis_hip::BufWin<float>::Make(g2__y.p, g2__y_enxy * g2__y.dim[2], (long)zb * g2__y_enxy, (long)ze * g2__y_enxy);
     const int g2__z_enx = g2__z.dim[0], g2__z_enxy = g2__z.dim[0] * g2__z.dim[1];
     const physis_hip::BufWin<float> g2__z_ew = physis_hip::BufWin<float>::Make(g2__z.p, g2__z_enxy * g2__z.dim[2], (long)zb * g2__z_enxy, (long)ze * g2__z_enxy);
+#pragma unroll
+    for (int k = 0; k < 1; ++k)
+      g1__x_pro[k].Store(g1__x_lds + k * S_g1__x::kPlane, wave, lane, g1__x_ra);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g1__y_pro[k].Store(g1__y_lds + k * S_g1__y::kPlane, wave, lane, g1__y_ra);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g1__z_pro[k].Store(g1__z_lds + k * S_g1__z::kPlane, wave, lane, g1__z_ra);
     __syncthreads();
     __PSCtx_kvec3 ctx;
     ctx.g1__x_p = g1__x.p;
@@ -4441,8 +4600,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kvec3(
     for (int d = 0; d < 3; ++d) ctx.g2__y_dim[d] = g2__y.dim[d];
     ctx.g2__z_p = g2__z.p;
     for (int d = 0; d < 3; ++d) ctx.g2__z_dim[d] = g2__z.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g1__x_dim[0] & 3) == 0);
       __builtin_assume((ctx.g1__y_dim[0] & 3) == 0);
       __builtin_assume((ctx.g1__z_dim[0] & 3) == 0);
@@ -4514,9 +4673,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kvec3(
           physis_hip::StoreMasked<float, VX>(g2__y_ew, xs + yrow * g2__y_enx + z * g2__y_enxy, g2__y_out, g2__y_mask);
           physis_hip::StoreMasked<float, VX>(g2__z_ew, xs + yrow * g2__z_enx + z * g2__z_enxy, g2__z_out, g2__z_mask);
         }
-        g1__x_st[k % PD].Store(g1__x_lds + physis_hip::RingSlot<2>(g1__x_base, 1) * S_g1__x::kPlane, wave, lane);
-        g1__y_st[k % PD].Store(g1__y_lds + physis_hip::RingSlot<4>(g1__y_base, 3) * S_g1__y::kPlane, wave, lane);
-        g1__z_st[k % PD].Store(g1__z_lds + physis_hip::RingSlot<4>(g1__z_base, 3) * S_g1__z::kPlane, wave, lane);
+        g1__x_st[k % PD].Store(g1__x_lds + physis_hip::RingSlot<2>(g1__x_base, 1) * S_g1__x::kPlane, wave, lane, g1__x_ra);
+        g1__y_st[k % PD].Store(g1__y_lds + physis_hip::RingSlot<4>(g1__y_base, 3) * S_g1__y::kPlane, wave, lane, g1__y_ra);
+        g1__z_st[k % PD].Store(g1__z_lds + physis_hip::RingSlot<4>(g1__z_base, 3) * S_g1__z::kPlane, wave, lane, g1__z_ra);
         __syncthreads();
         g1__x_st[k % PD].Load(g1__x_w, g1__x.p, g1__x.dim, g1__x_ra, z + 1 + PD);
         g1__x_base = physis_hip::RingSlot<2>(g1__x_base, 1);
@@ -4534,7 +4693,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_kvec3(const struct __PSStencil_kvec3 &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_kvec3<VX, 4, -1>, 64 * 4);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 4 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 4 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
 }
 
 template <int VX>
@@ -4552,14 +4711,18 @@ static int __PSLaunch_kvec3(const struct __PSStencil_kvec3 &s, hipStream_t strea
 }
 
 static int __PSBlocks_kvec3(const struct __PSStencil_kvec3 &s) {
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kvec3<4>(s).blocks : __PSShape_kvec3<1>(s).blocks;
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kvec3<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_kvec3<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_kvec3<1>(s).blocks;
 }
 
 static int __PSRun_kvec3(const struct __PSStencil_kvec3 &s, hipStream_t stream, void *red) {
   physis_hip::CheckUserGrid3D(s.g1);
   physis_hip::CheckUserGrid3D(s.g2);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kvec3<4>(s, stream, red) : __PSLaunch_kvec3<1>(s, stream, red);
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kvec3<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_kvec3<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_kvec3<1>(s, stream, red);
 }
 
 static void __PSStencilRun_17(int iter, struct __PSStencil_kvec3 s0, struct __PSStencil_kvec3 s1) {
@@ -4682,15 +4845,18 @@ __device__ __forceinline__ void ktensor(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_ktensor(
     __PSDomain dom, __PSGrid3DFloat_dev g__p_0_0, __PSGrid3DFloat_dev g__p_2_1, __PSGrid3DFloat_dev g__p_1_0, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 2;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g__p_0_0;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g__p_0_0;
   __shared__ __attribute__((aligned(16))) float g__p_0_0_lds[S_g__p_0_0::kLdsElems];
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false> S_g__p_2_1;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, false, float, RAGGED> S_g__p_2_1;
   __shared__ __attribute__((aligned(16))) float g__p_2_1_lds[S_g__p_2_1::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -4707,11 +4873,10 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_ktensor(
     const physis_hip::BufWin<float> g__p_0_0_w = physis_hip::BufWin<float>::Make(g__p_0_0.p, g__p_0_0_nxy * g__p_0_0.dim[2], (long)(zb + -2) * g__p_0_0_nxy, (long)(ze + 2) * g__p_0_0_nxy);
     S_g__p_0_0 g__p_0_0_st[PD];
     const typename S_g__p_0_0::Addr g__p_0_0_ra = S_g__p_0_0::Prepare(g__p_0_0.dim, x0, yrow, lane);
+    S_g__p_0_0 g__p_0_0_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g__p_0_0_st[0].Load(g__p_0_0_w, g__p_0_0.p, g__p_0_0.dim, g__p_0_0_ra, zb + -1 + k);
-      g__p_0_0_st[0].Store(g__p_0_0_lds + k * S_g__p_0_0::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g__p_0_0_pro[k].Load(g__p_0_0_w, g__p_0_0.p, g__p_0_0.dim, g__p_0_0_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g__p_0_0_st[k].Load(g__p_0_0_w, g__p_0_0.p, g__p_0_0.dim, g__p_0_0_ra, zb + 2 + k);
@@ -4720,17 +4885,22 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_ktensor(
     const physis_hip::BufWin<float> g__p_2_1_w = physis_hip::BufWin<float>::Make(g__p_2_1.p, g__p_2_1_nxy * g__p_2_1.dim[2], (long)(zb + -2) * g__p_2_1_nxy, (long)(ze + 2) * g__p_2_1_nxy);
     S_g__p_2_1 g__p_2_1_st[PD];
     const typename S_g__p_2_1::Addr g__p_2_1_ra = S_g__p_2_1::Prepare(g__p_2_1.dim, x0, yrow, lane);
+    S_g__p_2_1 g__p_2_1_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g__p_2_1_st[0].Load(g__p_2_1_w, g__p_2_1.p, g__p_2_1.dim, g__p_2_1_ra, zb + -1 + k);
-      g__p_2_1_st[0].Store(g__p_2_1_lds + k * S_g__p_2_1::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g__p_2_1_pro[k].Load(g__p_2_1_w, g__p_2_1.p, g__p_2_1.dim, g__p_2_1_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g__p_2_1_st[k].Load(g__p_2_1_w, g__p_2_1.p, g__p_2_1.dim, g__p_2_1_ra, zb + 2 + k);
     int g__p_2_1_base = 0;
     const int g__p_1_0_enx = g__p_1_0.dim[0], g__p_1_0_enxy = g__p_1_0.dim[0] * g__p_1_0.dim[1];
     const physis_hip::BufWin<float> g__p_1_0_ew = physis_hip::BufWin<float>::Make(g__p_1_0.p, g__p_1_0_enxy * g__p_1_0.dim[2], (long)zb * g__p_1_0_enxy, (long)ze * g__p_1_0_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g__p_0_0_pro[k].Store(g__p_0_0_lds + k * S_g__p_0_0::kPlane, wave, lane, g__p_0_0_ra);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g__p_2_1_pro[k].Store(g__p_2_1_lds + k * S_g__p_2_1::kPlane, wave, lane, g__p_2_1_ra);
     __syncthreads();
     __PSCtx_ktensor ctx;
     ctx.g__p_0_0_p = g__p_0_0.p;
@@ -4739,8 +4909,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_ktensor(
     for (int d = 0; d < 3; ++d) ctx.g__p_2_1_dim[d] = g__p_2_1.dim[d];
     ctx.g__p_1_0_p = g__p_1_0.p;
     for (int d = 0; d < 3; ++d) ctx.g__p_1_0_dim[d] = g__p_1_0.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g__p_0_0_dim[0] & 3) == 0);
       __builtin_assume((ctx.g__p_2_1_dim[0] & 3) == 0);
       __builtin_assume((ctx.g__p_1_0_dim[0] & 3) == 0);
@@ -4802,8 +4972,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_ktensor(
           }
           physis_hip::StoreMasked<float, VX>(g__p_1_0_ew, xs + yrow * g__p_1_0_enx + z * g__p_1_0_enxy, g__p_1_0_out, g__p_1_0_mask);
         }
-        g__p_0_0_st[k % PD].Store(g__p_0_0_lds + physis_hip::RingSlot<4>(g__p_0_0_base, 3) * S_g__p_0_0::kPlane, wave, lane);
-        g__p_2_1_st[k % PD].Store(g__p_2_1_lds + physis_hip::RingSlot<4>(g__p_2_1_base, 3) * S_g__p_2_1::kPlane, wave, lane);
+        g__p_0_0_st[k % PD].Store(g__p_0_0_lds + physis_hip::RingSlot<4>(g__p_0_0_base, 3) * S_g__p_0_0::kPlane, wave, lane, g__p_0_0_ra);
+        g__p_2_1_st[k % PD].Store(g__p_2_1_lds + physis_hip::RingSlot<4>(g__p_2_1_base, 3) * S_g__p_2_1::kPlane, wave, lane, g__p_2_1_ra);
         __syncthreads();
         g__p_0_0_st[k % PD].Load(g__p_0_0_w, g__p_0_0.p, g__p_0_0.dim, g__p_0_0_ra, z + 2 + PD);
         g__p_0_0_base = physis_hip::RingSlot<4>(g__p_0_0_base, 1);
@@ -4819,7 +4989,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_ktensor(const struct __PSStencil_ktensor &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_ktensor<VX, 8, -1>, 64 * 8);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 8 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 8 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
 }
 
 template <int VX>
@@ -4837,13 +5007,17 @@ static int __PSLaunch_ktensor(const struct __PSStencil_ktensor &s, hipStream_t s
 }
 
 static int __PSBlocks_ktensor(const struct __PSStencil_ktensor &s) {
-  return (s.g->dim[0] % 4 == 0) ? __PSShape_ktensor<4>(s).blocks : __PSShape_ktensor<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0) ? __PSShape_ktensor<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_ktensor<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_ktensor<1>(s).blocks;
 }
 
 static int __PSRun_ktensor(const struct __PSStencil_ktensor &s, hipStream_t stream, void *red) {
   physis_hip::CheckUserGrid3D(s.g);
   physis_hip::CheckEmitDomain(s.dom, s.g);
-  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_ktensor<4>(s, stream, red) : __PSLaunch_ktensor<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_ktensor<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_ktensor<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_ktensor<1>(s, stream, red);
 }
 
 static void __PSStencilRun_18(int iter, struct __PSStencil_ktensor s0) {
@@ -4989,15 +5163,18 @@ __device__ __forceinline__ void kcplx(
 // last 1 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kcplx(
     __PSDomain dom, __PSGrid3DFloat_dev g1__r, __PSGrid3DFloat_dev g1__i, __PSGrid3DFloat_dev g2__r, __PSGrid3DFloat_dev g2__i, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 2;
   constexpr int HY = 1;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true> S_g1__r;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true, float, RAGGED> S_g1__r;
   __shared__ __attribute__((aligned(16))) float g1__r_lds[S_g1__r::kLdsElems];
-  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true> S_g1__i;
+  typedef physis_hip::Stage<float, VX, BY, 1, HY, 4, true, float, RAGGED> S_g1__i;
   __shared__ __attribute__((aligned(16))) float g1__i_lds[S_g1__i::kLdsElems];
   const int lane = threadIdx.x % 64;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -5014,11 +5191,10 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kcplx(
     const physis_hip::BufWin<float> g1__r_w = physis_hip::BufWin<float>::Make(g1__r.p, g1__r_nxy * g1__r.dim[2], (long)(zb + -2) * g1__r_nxy, (long)(ze + 2) * g1__r_nxy);
     S_g1__r g1__r_st[PD];
     const typename S_g1__r::Addr g1__r_ra = S_g1__r::Prepare(g1__r.dim, x0, yrow, lane);
+    S_g1__r g1__r_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g1__r_st[0].Load(g1__r_w, g1__r.p, g1__r.dim, g1__r_ra, zb + -1 + k);
-      g1__r_st[0].Store(g1__r_lds + k * S_g1__r::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g1__r_pro[k].Load(g1__r_w, g1__r.p, g1__r.dim, g1__r_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g1__r_st[k].Load(g1__r_w, g1__r.p, g1__r.dim, g1__r_ra, zb + 2 + k);
@@ -5027,11 +5203,10 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kcplx(
     const physis_hip::BufWin<float> g1__i_w = physis_hip::BufWin<float>::Make(g1__i.p, g1__i_nxy * g1__i.dim[2], (long)(zb + -2) * g1__i_nxy, (long)(ze + 2) * g1__i_nxy);
     S_g1__i g1__i_st[PD];
     const typename S_g1__i::Addr g1__i_ra = S_g1__i::Prepare(g1__i.dim, x0, yrow, lane);
+    S_g1__i g1__i_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g1__i_st[0].Load(g1__i_w, g1__i.p, g1__i.dim, g1__i_ra, zb + -1 + k);
-      g1__i_st[0].Store(g1__i_lds + k * S_g1__i::kPlane, wave, lane);
-    }
+    for (int k = 0; k < 3; ++k)
+      g1__i_pro[k].Load(g1__i_w, g1__i.p, g1__i.dim, g1__i_ra, zb + -1 + k);
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       g1__i_st[k].Load(g1__i_w, g1__i.p, g1__i.dim, g1__i_ra, zb + 2 + k);
@@ -5040,6 +5215,12 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kcplx(
     const physis_hip::BufWin<float> g2__r_ew = physis_hip::BufWin<float>::Make(g2__r.p, g2__r_enxy * g2__r.dim[2], (long)zb * g2__r_enxy, (long)ze * g2__r_enxy);
     const int g2__i_enx = g2__i.dim[0], g2__i_enxy = g2__i.dim[0] * g2__i.dim[1];
     const physis_hip::BufWin<float> g2__i_ew = physis_hip::BufWin<float>::Make(g2__i.p, g2__i_enxy * g2__i.dim[2], (long)zb * g2__i_enxy, (long)ze * g2__i_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g1__r_pro[k].Store(g1__r_lds + k * S_g1__r::kPlane, wave, lane, g1__r_ra);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g1__i_pro[k].Store(g1__i_lds + k * S_g1__i::kPlane, wave, lane, g1__i_ra);
     __syncthreads();
     __PSCtx_kcplx ctx;
     ctx.g1__r_p = g1__r.p;
@@ -5050,8 +5231,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kcplx(
     for (int d = 0; d < 3; ++d) ctx.g2__r_dim[d] = g2__r.dim[d];
     ctx.g2__i_p = g2__i.p;
     for (int d = 0; d < 3; ++d) ctx.g2__i_dim[d] = g2__i.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g1__r_dim[0] & 3) == 0);
       __builtin_assume((ctx.g1__i_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2__r_dim[0] & 3) == 0);
@@ -5120,8 +5301,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kcplx(
           physis_hip::StoreMasked<float, VX>(g2__r_ew, xs + yrow * g2__r_enx + z * g2__r_enxy, g2__r_out, g2__r_mask);
           physis_hip::StoreMasked<float, VX>(g2__i_ew, xs + yrow * g2__i_enx + z * g2__i_enxy, g2__i_out, g2__i_mask);
         }
-        g1__r_st[k % PD].Store(g1__r_lds + physis_hip::RingSlot<4>(g1__r_base, 3) * S_g1__r::kPlane, wave, lane);
-        g1__i_st[k % PD].Store(g1__i_lds + physis_hip::RingSlot<4>(g1__i_base, 3) * S_g1__i::kPlane, wave, lane);
+        g1__r_st[k % PD].Store(g1__r_lds + physis_hip::RingSlot<4>(g1__r_base, 3) * S_g1__r::kPlane, wave, lane, g1__r_ra);
+        g1__i_st[k % PD].Store(g1__i_lds + physis_hip::RingSlot<4>(g1__i_base, 3) * S_g1__i::kPlane, wave, lane, g1__i_ra);
         __syncthreads();
         g1__r_st[k % PD].Load(g1__r_w, g1__r.p, g1__r.dim, g1__r_ra, z + 2 + PD);
         g1__r_base = physis_hip::RingSlot<4>(g1__r_base, 1);
@@ -5137,7 +5318,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_kcplx(const struct __PSStencil_kcplx &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_kcplx<VX, 8, -1>, 64 * 8);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 8 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 8 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g1, s.g2}, 2));
 }
 
 template <int VX>
@@ -5155,14 +5336,18 @@ static int __PSLaunch_kcplx(const struct __PSStencil_kcplx &s, hipStream_t strea
 }
 
 static int __PSBlocks_kcplx(const struct __PSStencil_kcplx &s) {
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kcplx<4>(s).blocks : __PSShape_kcplx<1>(s).blocks;
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kcplx<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_kcplx<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_kcplx<1>(s).blocks;
 }
 
 static int __PSRun_kcplx(const struct __PSStencil_kcplx &s, hipStream_t stream, void *red) {
   physis_hip::CheckUserGrid3D(s.g1);
   physis_hip::CheckUserGrid3D(s.g2);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kcplx<4>(s, stream, red) : __PSLaunch_kcplx<1>(s, stream, red);
+  return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kcplx<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_kcplx<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_kcplx<1>(s, stream, red);
 }
 
 static void __PSStencilRun_19(int iter, struct __PSStencil_kcplx s0) {
@@ -5235,9 +5420,12 @@ __device__ __forceinline__ void kdouble(
 // last 0 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kdouble(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 0;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
@@ -5268,8 +5456,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kdouble(
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -5309,7 +5497,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_kdouble(const struct __PSStencil_kdouble &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_kdouble<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 0));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 0));
 }
 
 template <int VX>
@@ -5327,14 +5515,18 @@ static int __PSLaunch_kdouble(const struct __PSStencil_kdouble &s, hipStream_t s
 }
 
 static int __PSBlocks_kdouble(const struct __PSStencil_kdouble &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kdouble<4>(s).blocks : __PSShape_kdouble<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kdouble<4>(s).blocks
+         : (true) ? __PSShape_kdouble<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_kdouble<1>(s).blocks;
 }
 
 static int __PSRun_kdouble(const struct __PSStencil_kdouble &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kdouble<4>(s, stream, red) : __PSLaunch_kdouble<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kdouble<4>(s, stream, red)
+         : (true) ? __PSLaunch_kdouble<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_kdouble<1>(s, stream, red);
 }
 
 static void __PSStencilRun_20(int iter, struct __PSStencil_kdouble s0) {
@@ -5413,9 +5605,12 @@ __device__ __forceinline__ void kshadow(
 // last 0 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kshadow(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 0;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
@@ -5438,8 +5633,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kshadow(
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -5477,7 +5672,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_kshadow(const struct __PSStencil_kshadow &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_kshadow<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 0));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 0));
 }
 
 template <int VX>
@@ -5495,14 +5690,18 @@ static int __PSLaunch_kshadow(const struct __PSStencil_kshadow &s, hipStream_t s
 }
 
 static int __PSBlocks_kshadow(const struct __PSStencil_kshadow &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kshadow<4>(s).blocks : __PSShape_kshadow<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kshadow<4>(s).blocks
+         : (true) ? __PSShape_kshadow<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_kshadow<1>(s).blocks;
 }
 
 static int __PSRun_kshadow(const struct __PSStencil_kshadow &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kshadow<4>(s, stream, red) : __PSLaunch_kshadow<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kshadow<4>(s, stream, red)
+         : (true) ? __PSLaunch_kshadow<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_kshadow<1>(s, stream, red);
 }
 
 static void __PSStencilRun_21(int iter, struct __PSStencil_kshadow s0) {
@@ -5581,9 +5780,12 @@ __device__ __forceinline__ float kscaled(
 // last 0 load halo rows), staged planes PD steps ahead,
 // centre-only grids one step ahead.  RED: reduction operator of a
 // PSStencilMapReduce execution, or -1.
-template <int VX, int BY, int RED>
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
 __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kscaled(
     __PSDomain dom, __PSGrid3DFloat_dev g, __PSGrid3DFloat_dev g2, float s, physis_hip::RunShape sh, float *__restrict__ __red) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
   constexpr int PD = 4;
   constexpr int HY = 0;
   constexpr int TX = 64 * VX, TY = BY - 2 * HY;
@@ -5616,8 +5818,8 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_kscaled(
     for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
     ctx.g2_p = g2.p;
     for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = g2.dim[d];
-    if constexpr (VX > 1) {
-      __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
       __builtin_assume((ctx.g_dim[0] & 3) == 0);
       __builtin_assume((ctx.g2_dim[0] & 3) == 0);
     }
@@ -5662,7 +5864,7 @@ template <int VX>
 static physis_hip::RunShape __PSShape_kscaled(const struct __PSStencil_kscaled &s) {
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun_kscaled<VX, 16, -1>, 64 * 16);
-  return physis_hip::PlanRun(s.dom, 64 * VX, 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 0));
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 16 - 2 * 0, per_cu, physis_hip::WindowChunkLimit({s.g, s.g2}, 0));
 }
 
 template <int VX>
@@ -5692,14 +5894,18 @@ static int __PSLaunch_kscaled(const struct __PSStencil_kscaled &s, hipStream_t s
 }
 
 static int __PSBlocks_kscaled(const struct __PSStencil_kscaled &s) {
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kscaled<4>(s).blocks : __PSShape_kscaled<1>(s).blocks;
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kscaled<4>(s).blocks
+         : (true) ? __PSShape_kscaled<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_kscaled<1>(s).blocks;
 }
 
 static int __PSRun_kscaled(const struct __PSStencil_kscaled &s, hipStream_t stream, void *red) {
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
-  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kscaled<4>(s, stream, red) : __PSLaunch_kscaled<1>(s, stream, red);
+  return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kscaled<4>(s, stream, red)
+         : (true) ? __PSLaunch_kscaled<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_kscaled<1>(s, stream, red);
 }
 
 static void __PSStencilRun_22(int iter, struct __PSStencil_kscaled s0, struct __PSStencil_kscaled s1, struct __PSStencil_kscaled s2, struct __PSStencil_kscaled s3, struct __PSStencil_kscaled s4, struct __PSStencil_kscaled s5, struct __PSStencil_kscaled s6) {

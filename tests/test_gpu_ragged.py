@@ -1,0 +1,140 @@
+"""Run kernels on rows whose extents are not multiples of the vector width
+(tests/programs/ragged.c), bit for bit against numpy: the points past the
+end of a row (the next row's, 0 outside the grid, the wrapped ones of a
+periodic get) at the sizes where a lane's vector hangs over a row's end, a
+tile's end or the grid's end."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 3, 4), (3, 5, 4), (5, 1, 3), (6, 7, 2), (63, 4, 5), (65, 17, 3),
+          (255, 3, 4), (257, 16, 9), (258, 5, 3), (511, 4, 3), (64, 9, 4)]
+
+
+@pytest.fixture(scope="module")
+def prog(ps):
+    L = ps.load_program("ragged")
+    G = ps.PSGridPtr
+    for f in ("corners", "corners_double", "corners2d", "wrap2"):
+        getattr(L, "ragged_" + f).argtypes = [G, G]
+    L.ragged_inner.argtypes = [G, G, C.c_int, C.c_float]
+    return L
+
+
+def _run(ps, fn, a, shape2=None, b=None):
+    """Grids with a and b (zeros) in, fn(g, g2), both grids out."""
+    dims = a.shape[::-1]
+    g = ps.PSGridNew(dims, a.dtype)
+    g2 = ps.PSGridNew((shape2 or dims), a.dtype)
+    ps.PSGridCopyin(g, a)
+    if b is not None:
+        ps.PSGridCopyin(g2, b)
+    fn(g.handle, g2.handle)
+    out = [ps.PSGridCopyout(x) for x in (g, g2)]
+    ps.PSGridFree(g)
+    ps.PSGridFree(g2)
+    return out
+
+
+def _linear(a, x, y, z, d):
+    """Element at the linear offset of (x, y, z) + d, 0 outside the grid."""
+    nz, ny, nx = a.shape
+    off = x + d[0] + (y + d[1]) * nx + (z + d[2]) * nx * ny
+    ok = (off >= 0) & (off < a.size)
+    return np.where(ok, a.reshape(-1)[np.clip(off, 0, a.size - 1)],
+                    a.dtype.type(0))
+
+
+def _sum(get, terms, t):
+    v = None
+    for w, d in terms:
+        p = get(d) if w is None else t(w) * get(d)
+        v = p if v is None else v + p
+    return v
+
+
+CORNERS = [(0.5, (0, 0, 0)), (None, (1, 0, 0)), (2.0, (1, -1, 0)),
+           (3.0, (-1, 1, 0)), (4.0, (1, 1, 1)), (5.0, (-1, -1, -1)),
+           (6.0, (1, 0, -1))]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_rows_past_their_ends(ps, prog, shape, dtype):
+    print(f"corners {shape} {dtype.__name__}", flush=True)
+    nx, ny, nz = shape
+    a = np.random.default_rng(nx).standard_normal((nz, ny, nx)).astype(dtype)
+    fn = prog.ragged_corners if dtype == np.float32 else \
+        prog.ragged_corners_double
+    got = _run(ps, fn, a)[1]
+    z, y, x = np.meshgrid(*map(np.arange, (nz, ny, nx)), indexing="ij")
+    want = _sum(lambda d: _linear(a, x, y, z, d), CORNERS, dtype)
+    assert np.array_equal(got, want.reshape(-1))
+
+
+@pytest.mark.parametrize("shape,shape2", [((5, 4, 3), (9, 3, 3)),
+                                          ((61, 5, 4), (67, 5, 3))])
+def test_domain_wider_than_the_grid_read(ps, prog, shape, shape2):
+    """The map covers g2, whose rows are longer than those it reads."""
+    print(f"corners {shape} -> {shape2}", flush=True)
+    nx, ny, nz = shape
+    a = np.random.default_rng(nx).standard_normal((nz, ny, nx)) \
+        .astype(np.float32)
+    got = _run(ps, prog.ragged_corners, a, shape2)[1]
+    z, y, x = np.meshgrid(*map(np.arange, shape2[::-1]), indexing="ij")
+    want = _sum(lambda d: _linear(a, x, y, z, d), CORNERS, np.float32)
+    assert np.array_equal(got, want.reshape(-1))
+
+
+@pytest.mark.parametrize("shape", [(3, 4), (5, 1), (63, 7), (257, 9),
+                                   (1023, 5)])
+def test_two_dimensional_rows(ps, prog, shape):
+    print(f"corners2d {shape}", flush=True)
+    nx, ny = shape
+    a = np.random.default_rng(nx).standard_normal((ny, nx)).astype(np.float32)
+    got = _run(ps, prog.ragged_corners2d, a)[1]
+    y, x = np.meshgrid(np.arange(ny), np.arange(nx), indexing="ij")
+    want = _sum(lambda d: _linear(a[None], x, y, 0 * x, d),
+                [(0.5, (0, 0, 0)), (2.0, (1, -1, 0)), (3.0, (-1, 1, 0)),
+                 (4.0, (1, 0, 0))], np.float32)
+    assert np.array_equal(got, want.reshape(-1))
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_periodic_rows(ps, prog, shape):
+    print(f"wrap2 {shape}", flush=True)
+    nx, ny, nz = shape
+    a = np.random.default_rng(nx).standard_normal((nz, ny, nx)) \
+        .astype(np.float32)
+    got = _run(ps, prog.ragged_wrap2, a)[1]
+    want = _sum(lambda d: np.roll(a, (-d[2], -d[1], -d[0]), (0, 1, 2)),
+                [(0.5, (0, 0, 0)), (2.0, (2, -1, 0)), (3.0, (-2, 1, 0)),
+                 (4.0, (1, 0, 1)), (5.0, (-1, 0, -1))], np.float32)
+    assert np.array_equal(got, want.reshape(-1))
+
+
+@pytest.mark.parametrize("count", [1, 2, 3])
+@pytest.mark.parametrize("shape", [(3, 3, 3), (7, 5, 4), (65, 18, 6),
+                                   (257, 14, 5), (259, 30, 4), (64, 9, 5)])
+def test_interior_pairs(ps, prog, shape, count):
+    """Pairs over the interior: both grids as single sweeps leave them."""
+    print(f"inner {shape} x {count}", flush=True)
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nx)
+    a, b = rng.standard_normal((2, nz, ny, nx)).astype(np.float32)
+    w = np.float32(0.2)
+    got = _run(ps, lambda g, g2: prog.ragged_inner(g, g2, count, w), a, None,
+               b)
+    z, y, x = np.meshgrid(*(np.arange(1, n - 1) for n in (nz, ny, nx)),
+                          indexing="ij")
+    u = [a.copy(), b.copy()]
+    for k in range(2 * count):
+        v = _sum(lambda d: u[k % 2][z + d[2], y + d[1], x + d[0]],
+                 [(None, (0, 0, 0)), (None, (1, -1, 0)), (None, (-1, 1, 0)),
+                  (None, (0, 0, 1)), (None, (0, 0, -1))], np.float32)
+        u[1 - k % 2][1:-1, 1:-1, 1:-1] = v * w
+    for k in range(2):
+        assert np.array_equal(got[k], u[k].reshape(-1)), k
