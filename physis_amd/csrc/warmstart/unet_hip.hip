@@ -62,116 +62,29 @@ __device__ __forceinline__ bf16x8 Zero8() {
   return __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
 }
 
+// Two floats rounded to BF16 (nearest even) in one word.
+__device__ __forceinline__ unsigned Pack2(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(
+      unsigned, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
+// The halves of v whose activation (the halves of a) is positive.
+__device__ __forceinline__ unsigned GateWord(unsigned v, unsigned a) {
+  return (__uint_as_float(a << 16) > 0.0f ? v & 0xffffu : 0u) |
+         (__uint_as_float(a & 0xffff0000u) > 0.0f ? v & 0xffff0000u : 0u);
+}
+
 constexpr int KPad(int cin) { return ((27 * cin + 31) / 32) * 32; }
 
 // ------------------------------------------------------------ convolution
-// Block (x tile, 4-row group, n*D + z) copies planes z-1..z+1, rows
-// y0-1..y0+4, x0-1 .. x0+XT of the input (channels-last, zero outside the
-// grid) into LDS with 16-byte loads; wave w then computes row y0+w over the
-// tile in segments of 16 x: D[16 x][16 cout] accumulated over K steps of
-// 32, every A operand (8 channels of one tap at one position) one aligned
-// 16-byte LDS read.  The weight fragments of all K steps stay in registers
-// when there are at most 14 of them (more cost occupancy: 21 for 24 -> 8
-// held 200 VGPRs), else they are read per step (L1-resident).
-template <int CIN, int COUT, bool RELU, int XT>
-__global__ __launch_bounds__(256) void ConvKernel(
-    const u16 *__restrict__ x, const u16 *__restrict__ wt,
-    const float *__restrict__ bias, u16 *__restrict__ y, int D, int H,
-    int W) {
-  constexpr int K = 27 * CIN, KB = (K + 31) / 32, KP = KB * 32;
-  constexpr int NT = (COUT + 15) / 16;
-  constexpr bool kPre = KB * NT <= 14;
-  constexpr int XS = XT + 2, NV = CIN / 8;
-  __shared__ __attribute__((aligned(16))) u16 tile[18 * XS * CIN];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int g = lane >> 4, r = lane & 15;
-  const int tiles_x = (W + XT - 1) / XT;
-  const int x0 = (blockIdx.x % tiles_x) * XT, y0 = (blockIdx.x / tiles_x) * 4;
-  const int nz = blockIdx.y;
-  const int n = nz / D, z = nz - n * D;
-  for (int v = threadIdx.x; v < 18 * XS * NV; v += 256) {
-    const int c8 = v % NV, t = v / NV;
-    const int xp = t % XS, pr = t / XS;
-    const int zz = z + pr / 6 - 1, yy = y0 + pr % 6 - 1, xx = x0 - 1 + xp;
-    uint4 u = make_uint4(0, 0, 0, 0);
-    if (zz >= 0 && zz < D && yy >= 0 && yy < H && xx >= 0 && xx < W)
-      u = *reinterpret_cast<const uint4 *>(
-          x + ((((long)n * D + zz) * H + yy) * W + xx) * CIN + c8 * 8);
-    *reinterpret_cast<uint4 *>(tile + t * CIN + c8 * 8) = u;
-  }
-  bf16x8 bw[kPre ? KB : 1][NT];
-  if constexpr (kPre) {
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int co = t * 16 + r;
-        bw[kb][t] = co < COUT ? Load8(wt + (long)co * KP + kb * 32 + 8 * g)
-                              : Zero8();
-      }
-  }
-  float bb[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int co = t * 16 + r;
-    bb[t] = (bias && co < COUT) ? bias[co] : 0.0f;
-  }
-  __syncthreads();
-  const int yy = y0 + wv;
-  if (yy >= H) return;  // whole wave; no barrier follows
-  const long row = (((long)n * D + z) * H + yy) * W;
-  for (int xs0 = 0; xs0 < XT && x0 + xs0 < W; xs0 += 16) {
-    f32x4 acc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int xa = xs0 + r;
-#pragma unroll 4
-    for (int kb = 0; kb < KB; ++kb) {
-      const int k0 = kb * 32 + 8 * g;
-      bf16x8 a = Zero8();
-      if (k0 < K) {
-        const int tap = k0 / CIN, ci0 = k0 - tap * CIN;
-        // staged plane dz+1 = tap/9, row wv + dy+1, x xa + dx+1
-        a = *reinterpret_cast<const bf16x8 *>(
-            tile + (((tap / 9) * 6 + wv + (tap / 3) % 3) * XS + xa + tap % 3) *
-                       CIN + ci0);
-      }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        bf16x8 b;
-        if constexpr (kPre) {
-          b = bw[kb][t];
-        } else {
-          const int co = t * 16 + r;
-          b = co < COUT ? Load8(wt + (long)co * KP + kb * 32 + 8 * g)
-                        : Zero8();
-        }
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int co = t * 16 + r;
-      if (co >= COUT) continue;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int xo = x0 + xs0 + 4 * g + v;
-        if (xo >= W) continue;
-        float val = acc[t][v] + bb[t];
-        if (RELU) val = val > 0.0f ? val : 0.0f;
-        y[(row + xo) * COUT + co] = F2Bf(val);
-      }
-    }
-  }
-}
-
 // 3x3x3 convolution marching z (the 2.5D scheme of the stencil run
 // kernels).  Block (x tile, y tile, problem n, z chunk) owns XT x TY output
 // positions of every plane of its chunk.  An LDS ring holds the input planes
 // z-1 .. z+1 over rows y0-1 .. y0+TY and x0-1 .. x0+XT (zero outside the
 // grid) and the plane z+2 being staged; the plane after that is loaded into
-// registers a step ahead.  Each input plane is thus staged once per tile
-// (the per-plane kernel above stages three), with one barrier per step.
+// registers a step ahead.  Each input plane is thus staged once per tile,
+// with one barrier per step.
 // The GEMM is D[cout][16 x] = W[cout][32 k] X[32 k][16 x]: the weights are
 // the A operand (registers, or LDS when they are many), the staged input the
 // B operand (one aligned 16-byte LDS read per lane), and a lane's result is
@@ -179,8 +92,8 @@ __global__ __launch_bounds__(256) void ConvKernel(
 template <int CIN, int COUT, bool RELU, int XT, int TY>
 __global__ __launch_bounds__(64 * TY) void ConvZKernel(
     const u16 *__restrict__ x, const u16 *__restrict__ wt,
-    const float *__restrict__ bias, u16 *__restrict__ y, int D, int H, int W,
-    int tz, int zchunk) {
+    const float *__restrict__ bias, const u16 *__restrict__ act,
+    u16 *__restrict__ y, int D, int H, int W, int tz, int zchunk) {
   constexpr int K = 27 * CIN, KB = (K + 31) / 32, KP = KB * 32;
   constexpr int MT = (COUT + 15) / 16;
   constexpr bool kRegW = KB * MT <= kRegWeightSteps;
@@ -351,6 +264,12 @@ __global__ __launch_bounds__(64 * TY) void ConvZKernel(
               }
               w2[h] = (unsigned)F2Bf(v0) | ((unsigned)F2Bf(v1) << 16);
             }
+            if (act) {  // gated by the ReLU whose input gradient this is
+              const uint2 a = *reinterpret_cast<const uint2 *>(
+                  act + (row + xo) * COUT + co);
+              w2[0] = GateWord(w2[0], a.x);
+              w2[1] = GateWord(w2[1], a.y);
+            }
             *reinterpret_cast<uint2 *>(y + (row + xo) * COUT + co) =
                 make_uint2(w2[0], w2[1]);
           }
@@ -363,139 +282,430 @@ __global__ __launch_bounds__(64 * TY) void ConvZKernel(
   }
 }
 
-// The z-marching convolution for 8 output channels, two output rows per
-// wave.  With COUT = 8 half of the 16 A rows of the tap-major kernel are
-// zero; here row q = 8 h + co of the A operand is output channel co of
-// output row y + h (h = 0, 1), and K runs over the input rows y - 1 .. y + 2
-// of both: k = ((dz 4 + ry) 3 + dx) CIN + ci, A[q][k] = W[co][9 dz + 3 (ry -
-// h) + dx][ci] when 0 <= ry - h <= 2, else 0.  One B operand (8 channels of
-// one staged input position) then serves both rows: 36 CIN / 32 K steps per
-// 16 x positions of two rows instead of 2 x 27 CIN / 32 (CIN = 24: 27
-// instead of 42 MFMAs and B reads).  Block (x tile, 2 TY rows, problem, z
-// chunk); the ring and the staging are those of ConvZKernel.
-template <int CIN, bool RELU, int XT, int TY>
-__global__ __launch_bounds__(64 * TY) void ConvZPairKernel(
-    const u16 *__restrict__ x, const u16 *__restrict__ wt,
-    const float *__restrict__ bias, u16 *__restrict__ y, int D, int H, int W,
-    int tz, int zchunk) {
-  constexpr int COUT = 8;
-  constexpr int KW = 27 * CIN, KPW = ((KW + 31) / 32) * 32;  // wt layout
-  constexpr int K = 36 * CIN, KB = (K + 31) / 32;
-  constexpr int ROWS = 2 * TY;
-  constexpr int XS = XT + 2, RS = ROWS + 2, NV = CIN / 8;
-  constexpr int PLANE = RS * XS * CIN;  // u16 elements of a staged plane
-  constexpr int SV = RS * XS * NV;      // 16-byte vectors of a staged plane
-  constexpr int NTH = 64 * TY;
-  constexpr int VPT = (SV + NTH - 1) / NTH;
-  __shared__ __attribute__((aligned(16))) u16 ring[4 * PLANE];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int g = lane >> 4, r = lane & 15;
-  const int tiles_x = (W + XT - 1) / XT;
-  const int x0 = (blockIdx.x % tiles_x) * XT;
-  const int y0 = (blockIdx.x / tiles_x) * ROWS;
-  const int n = blockIdx.y / tz;
-  const int zb = (blockIdx.y - n * tz) * zchunk;
-  const int ze = min(zb + zchunk, D);
-  if (zb >= ze) return;  // uniform over the block
-  auto fetch = [&](int zz, uint4 (&buf)[VPT]) {
+// ------------------------------------------------- staging of input planes
+// A block's view of one input plane: rows y0-1 .. y0+RS-2 and x0-1 ..
+// x0+XS-2 of problem n, CIN channels per position in LDS.  A stream moves
+// NCH of them (from channel COFF) between a channels-last tensor and LDS,
+// 16 bytes per thread and load; the tensor has the staged resolution, or
+// (UP) a quarter of it per axis, read once per fine position: an upsampled
+// tensor is never written out.  Positions outside the grid are zero: the
+// loads are range-checked buffer loads over one plane (none of it for a
+// plane outside the problem), whose offsets are computed once.
+constexpr int kOutside = (int)0x80000000u;
+
+template <int CIN, int NCH, int COFF, bool UP, int RS, int XS, int NTH>
+struct PlaneStream {
+  static constexpr int NV = NCH / 8, SV = RS * XS * NV;
+  static constexpr int VPT = (SV + NTH - 1) / NTH;
+  int off[VPT];  // byte offset within a plane, kOutside outside the grid
+  uint4 buf[VPT];
+
+  __device__ __forceinline__ void Init(int y0, int x0, int H, int W) {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int v = threadIdx.x + i * NTH;
       const int c8 = v % NV, t = v / NV;
-      const int xp = t % XS, pr = t / XS;
-      const int yy = y0 - 1 + pr, xx = x0 - 1 + xp;
-      uint4 u = make_uint4(0, 0, 0, 0);
-      if (v < SV && zz >= 0 && zz < D && yy >= 0 && yy < H && xx >= 0 &&
-          xx < W)
-        u = *reinterpret_cast<const uint4 *>(
-            x + ((((long)n * D + zz) * H + yy) * W + xx) * CIN + c8 * 8);
-      buf[i] = u;
+      const int yy = y0 - 1 + t / XS, xx = x0 - 1 + t % XS;
+      const bool in = v < SV && yy >= 0 && yy < H && xx >= 0 && xx < W;
+      const int pos = UP ? (yy / kPool) * (W / kPool) + xx / kPool
+                         : yy * W + xx;
+      off[i] = in ? (pos * NCH + c8 * 8) * 2 : kOutside;
     }
-  };
-  auto put = [&](int slot, const uint4 (&buf)[VPT]) {
+  }
+  __device__ __forceinline__ void Fetch(const u16 *p, int n, int z, int D,
+                                        int H, int W) {
+    const bool in = z >= 0 && z < D;
+    const int q = UP ? kPool : 1;
+    const int plane = (H / q) * (W / q) * NCH;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<u16 *>(p) + (in ? ((long)n * (D / q) + z / q) * plane : 0),
+        0, in ? plane * 2 : 0, physis_hip::kBufDword3);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+      buf[i] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off[i], 0, 0));
+  }
+  __device__ __forceinline__ void Put(u16 *plane) const {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int v = threadIdx.x + i * NTH;
       if (v < SV)
-        *reinterpret_cast<uint4 *>(ring + slot * PLANE + v * 8) = buf[i];
+        *reinterpret_cast<uint4 *>(plane + (v / NV) * CIN + COFF +
+                                   (v % NV) * 8) = buf[i];
     }
-  };
-  uint4 buf[VPT];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    fetch(zb - 1 + k, buf);
-    put(k, buf);
   }
-  fetch(zb + 2, buf);
-  // A fragments (registers) and the B operand's offsets of every K step:
-  // u16 elements within a staged plane relative to the wave's first row and
-  // the lane's x, with the input plane (0..2) in bits 24 and up; -1 past K
-  const int co = r & 7, h = r >> 3;
-  bf16x8 aw[KB];
-  int boff[KB];
+};
+
+// Sources of a convolution's input.
+struct SrcArgs {
+  const void *a, *b;  // tensor; or coarse tensor and skip; or rhs and bnd
+  long off;           // first element of rhs and bnd
+};
+template <int CIN, int RS, int XS, int NTH>
+struct PlainSrc {
+  PlaneStream<CIN, CIN, 0, false, RS, XS, NTH> s;
+  __device__ __forceinline__ void Init(int y0, int x0, int H, int W) {
+    s.Init(y0, x0, H, W);
+  }
+  __device__ __forceinline__ void Fetch(const SrcArgs &p, int n, int z, int D,
+                                        int H, int W) {
+    s.Fetch((const u16 *)p.a, n, z, D, H, W);
+  }
+  __device__ __forceinline__ void Put(u16 *plane) const { s.Put(plane); }
+};
+// Concatenation of an upsampled coarse tensor (two thirds of the channels)
+// and a skip tensor.
+template <int CIN, int RS, int XS, int NTH>
+struct ConcatSrc {
+  static constexpr int CA = CIN / 3 * 2, CB = CIN - CA;
+  PlaneStream<CIN, CA, 0, true, RS, XS, NTH> up;
+  PlaneStream<CIN, CB, CA, false, RS, XS, NTH> skip;
+  __device__ __forceinline__ void Init(int y0, int x0, int H, int W) {
+    up.Init(y0, x0, H, W);
+    skip.Init(y0, x0, H, W);
+  }
+  __device__ __forceinline__ void Fetch(const SrcArgs &p, int n, int z, int D,
+                                        int H, int W) {
+    up.Fetch((const u16 *)p.a, n, z, D, H, W);
+    skip.Fetch((const u16 *)p.b, n, z, D, H, W);
+  }
+  __device__ __forceinline__ void Put(u16 *plane) const {
+    up.Put(plane);
+    skip.Put(plane);
+  }
+};
+// The network input: channels (rhs, bnd) rounded to BF16 from the float
+// grids, two channels (CIN = 2) per position.
+template <int CIN, int RS, int XS, int NTH>
+struct InputSrc {
+  static_assert(CIN == 2, "rhs and bnd");
+  static constexpr int SV = RS * XS, VPT = (SV + NTH - 1) / NTH;
+  int off[VPT];
+  float r[VPT], m[VPT];
+  __device__ __forceinline__ void Init(int y0, int x0, int H, int W) {
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
+    for (int i = 0; i < VPT; ++i) {
+      const int v = threadIdx.x + i * NTH;
+      const int yy = y0 - 1 + v / XS, xx = x0 - 1 + v % XS;
+      const bool in = v < SV && yy >= 0 && yy < H && xx >= 0 && xx < W;
+      off[i] = in ? (yy * W + xx) * 4 : kOutside;
+    }
+  }
+  __device__ __forceinline__ void Fetch(const SrcArgs &p, int n, int z, int D,
+                                        int H, int W) {
+    const bool in = z >= 0 && z < D;
+    const long first = in ? p.off + ((long)n * D + z) * H * W : 0;
+    const int bytes = in ? H * W * 4 : 0;
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        (float *)const_cast<void *>(p.a) + first, 0, bytes,
+        physis_hip::kBufDword3);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        (float *)const_cast<void *>(p.b) + first, 0, bytes,
+        physis_hip::kBufDword3);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      r[i] = __uint_as_float(
+          __builtin_amdgcn_raw_buffer_load_b32(ra, off[i], 0, 0));
+      m[i] = __uint_as_float(
+          __builtin_amdgcn_raw_buffer_load_b32(rb, off[i], 0, 0));
+    }
+  }
+  __device__ __forceinline__ void Put(u16 *plane) const {
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const int v = threadIdx.x + i * NTH;
+      if (v < SV)
+        *reinterpret_cast<unsigned *>(plane + v * 2) =
+            (unsigned)F2Bf(r[i]) | ((unsigned)F2Bf(m[i]) << 16);
+    }
+  }
+};
+
+// What becomes of a convolution's results (COUT 8 or 24 channels).
+enum Epi {
+  kEpiStore,    // + bias, ReLU when RELU, rounded and stored
+  kEpiGate,     // gated by act > 0 (the ReLU whose input gradient this is)
+  kEpiPredict,  // + bias, ReLU, rounded, 1x1 head, p = scale out bnd
+  kEpiUpSkip    // 24 channels: 16 summed over the 4x4x4 cells of the coarse
+                // grid, gated by act and stored there, 8 stored
+};
+struct EpiArgs {
+  const float *bias = nullptr;
+  u16 *y = nullptr;            // stored channels (kEpiUpSkip: the last 8)
+  const u16 *act = nullptr;    // kEpiGate, kEpiUpSkip
+  u16 *coarse = nullptr;       // kEpiUpSkip
+  const float *head = nullptr; // kEpiPredict: 8 weights and the bias
+  const float *bnd = nullptr;  // kEpiPredict, from element off, as p
+  void *p = nullptr;
+  long off = 0;
+  float scale = 0.0f;
+};
+
+// 3x3x3 convolution marching the input planes: wave w of a block owns output
+// rows y0 + 2w and y0 + 2w + 1 over XT positions of every plane of a z chunk
+// of one problem.  Step z' stages input plane z' + 1 while the MFMAs
+// (D[16 rows][16 x] += A[16][32 k] B[32 k][16 x]) apply plane z' to the three
+// output planes it reaches: the B operand of a K step (8 channels of one
+// staged position per lane: k = (3 ry + dx) CIN + ci over the four input rows
+// ry of the two output rows) is read from LDS once and feeds the three z
+// taps, whose sums live in registers and rotate.  A rows: with 8 output
+// channels, 8 h + co of output row y + h (zero where ry - h is no tap); with
+// 24, sets 0 and 1 hold channels 0 .. 15 of the two rows and set 2 channels
+// 16 .. 23 of both.  With 2 input channels k = (4 ry + dx) 2 + ci, one K step.
+// The kernel it replaces held a ring of planes and read every B operand
+// three times: LDS reads bounded it (24 -> 8 at 8 x 128^3: 184 us of LDS
+// time in 396 us).
+template <int CIN, int COUT, bool RELU, int XT, int TY,
+          template <int, int, int, int> class SRC, int EPI,
+          typename PT = double>
+__global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
+    SrcArgs src, const u16 *__restrict__ wt, EpiArgs ep, int D, int H, int W,
+    int tz, int zchunk) {
+  static_assert(COUT == 8 || COUT == 24, "output channels");
+  static_assert(EPI == kEpiStore || (EPI == kEpiUpSkip) == (COUT == 24), "");
+  constexpr int S = COUT == 8 ? 1 : 3;  // A operands per B operand
+  constexpr int WC = CIN == 2 ? 8 : CIN;  // channels of the stored weights
+  constexpr int KPW = KPad(WC);
+  constexpr int KS = CIN == 2 ? 1 : 12 * CIN / 32;  // K steps per plane
+  constexpr int NTH = 64 * TY, ROWS = 2 * TY;
+  constexpr int XS = XT + 2, RS = ROWS + 2;
+  constexpr int PLANE = RS * XS * CIN;  // u16 elements of a staged plane
+  constexpr int SEG = XT / 16;
+  constexpr bool kCells = EPI == kEpiUpSkip;  // sums over 4x4x4 cells
+  __shared__ __attribute__((aligned(16))) u16 ring[2 * PLANE];
+  __shared__ __attribute__((aligned(16))) float cells[kCells ? TY / 2 : 1]
+      [kCells ? SEG : 1][kCells ? 64 : 1];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r = lane & 15;
+  const int tiles_x = (W + XT - 1) / XT, tiles_y = (H + ROWS - 1) / ROWS;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = (b % tiles_x) * XT;
+  b /= tiles_x;
+  const int y0 = (b % tiles_y) * ROWS;
+  b /= tiles_y;
+  const int n = b / tz, zb = (b - n * tz) * zchunk;
+  const int ze = min(zb + zchunk, D);
+  if (zb >= ze) return;  // uniform over the block
+  SRC<CIN, RS, XS, NTH> in;
+  in.Init(y0, x0, H, W);
+  in.Fetch(src, n, zb - 1, D, H, W);
+  in.Put(ring);
+  in.Fetch(src, n, zb, D, H, W);
+  // A operands of (set, z tap, K step), and the LDS offset of each K step's
+  // B operand relative to the wave's first row and the lane's x
+  bf16x8 aw[S][3][KS];
+  int boff[KS];
+#pragma unroll
+  for (int kb = 0; kb < KS; ++kb) {
     const int k0 = kb * 32 + 8 * g;
-    aw[kb] = Zero8();
-    boff[kb] = -1;
-    if (k0 < K) {
-      const int cell = k0 / CIN, ci0 = k0 - cell * CIN;
-      const int dz = cell / 12, ry = (cell / 3) % 4, dx = cell % 3;
+    const int cell = CIN == 2 ? 0 : k0 / CIN, ci0 = k0 - cell * CIN;
+    const int ry = CIN == 2 ? g : cell / 3, dx = CIN == 2 ? 0 : cell % 3;
+    boff[kb] = (ry * XS + dx) * CIN + (CIN == 2 ? 0 : ci0);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int h = COUT == 8 || s == 2 ? r >> 3 : s;
+      const int co = COUT == 8 ? r & 7 : (s == 2 ? 16 + (r & 7) : r);
       const int dy = ry - h;
-      if (dy >= 0 && dy <= 2)
-        aw[kb] = Load8(wt + (long)co * KPW + (9 * dz + 3 * dy + dx) * CIN + ci0);
-      boff[kb] = ((ry * XS + dx) * CIN + ci0) | (dz << 24);
-    }
-  }
-  // bias of the four outputs (row y + (g >> 1), channels 4 (g & 1) + v)
-  float bb[4];
 #pragma unroll
-  for (int v = 0; v < 4; ++v) bb[v] = bias ? bias[4 * (g & 1) + v] : 0.0f;
-  __syncthreads();
-  const int yy0 = y0 + 2 * wv;  // the wave's first output row
-  const int yo = yy0 + (g >> 1);  // the row of this lane's outputs
-  for (int z = zb; z < ze; ++z) {
-    const int base = z - zb;  // ring slot of plane z - 1 (mod 4)
-    if (yy0 < H) {
-      const long row = (((long)n * D + z) * H + yo) * W;
-      const int so[3] = {(base & 3) * PLANE, ((base + 1) & 3) * PLANE,
-                         ((base + 2) & 3) * PLANE};
-      for (int xs0 = 0; xs0 < XT && x0 + xs0 < W; xs0 += 16) {
-        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-        const u16 *rb = ring + (2 * wv * XS + xs0 + r) * CIN;
+      for (int t = 0; t < 3; ++t) {
+        bf16x8 a = Zero8();
+        if (dy >= 0 && dy <= 2) {
+          const u16 *w = wt + (long)co * KPW + (9 * t + 3 * dy + dx) * WC;
+          if constexpr (CIN == 2) {
+            unsigned v[4];
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          bf16x8 b = Zero8();
-          if (boff[kb] >= 0) {
-            const int pz = boff[kb] >> 24;
-            const int sp = pz == 0 ? so[0] : (pz == 1 ? so[1] : so[2]);
-            b = *reinterpret_cast<const bf16x8 *>(rb + sp +
-                                                  (boff[kb] & 0xffffff));
+            for (int d = 0; d < 3; ++d)
+              v[d] = *reinterpret_cast<const unsigned *>(w + d * WC);
+            v[3] = 0;
+            a = __builtin_bit_cast(bf16x8, make_uint4(v[0], v[1], v[2], v[3]));
+          } else {
+            a = Load8(w + ci0);
           }
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aw[kb], b, acc, 0, 0,
-                                                        0);
         }
-        const int xo = x0 + xs0 + r;
-        if (xo < W && yo < H) {
-          unsigned w2[2];
-#pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            float v0 = acc[2 * q] + bb[2 * q];
-            float v1 = acc[2 * q + 1] + bb[2 * q + 1];
-            if (RELU) {
-              v0 = v0 > 0.0f ? v0 : 0.0f;
-              v1 = v1 > 0.0f ? v1 : 0.0f;
-            }
-            w2[q] = (unsigned)F2Bf(v0) | ((unsigned)F2Bf(v1) << 16);
-          }
-          *reinterpret_cast<uint2 *>(y + (row + xo) * COUT + 4 * (g & 1)) =
-              make_uint2(w2[0], w2[1]);
-        }
+        aw[s][t][kb] = a;
       }
     }
-    put((base + 3) & 3, buf);
-    __syncthreads();
-    fetch(z + 3, buf);
+  }
+  // bias of the lane's four channels of the paired results, and of sets 0, 1
+  float bb[4], ba[S == 1 ? 1 : 4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    bb[v] = ep.bias ? ep.bias[COUT - 8 + 4 * (g & 1) + v] : 0.0f;
+    if constexpr (S > 1) ba[v] = ep.bias ? ep.bias[4 * g + v] : 0.0f;
+  }
+  float hw[4], hb = 0.0f;  // head weights of the lane's four channels
+  if constexpr (EPI == kEpiPredict) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) hw[v] = ep.head[4 * (g & 1) + v];
+    hb = ep.head[8];
+  }
+  const int yw = y0 + 2 * wv;    // the wave's first output row
+  const int yo = yw + (g >> 1);  // row of the lane's paired results
+  f32x4 acc[SEG][S][3];
+  f32x4 csum[kCells ? SEG : 1];
+#pragma unroll
+  for (int i = 0; i < SEG; ++i) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int t = 0; t < 3; ++t) acc[i][s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (kCells) csum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  __syncthreads();
+  for (int m0 = 0;; m0 += 3) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int m = m0 + j, zp = zb - 1 + m;  // input plane of this step
+      if (zp > ze) return;  // uniform over the block
+      const int z = zp - 1;  // output plane this step completes
+      const bool done = z >= zb;
+      const long row = (((long)n * D + z) * H + yo) * W;
+      // what the epilogue reads, ahead of the MFMAs
+      uint2 av[EPI == kEpiGate ? SEG : 1];
+      // (a pair of segments shares its stores: lanes of odd g take the
+      // second, so that no lane is idle)
+      constexpr int PSEG = (SEG + 1) / 2;
+      float bv[EPI == kEpiPredict ? PSEG : 1], pv[EPI == kEpiPredict ? SEG : 1];
+      const int px = SEG > 1 ? 16 * (g & 1) : 0;
+#pragma unroll
+      for (int i = 0; i < SEG; ++i) {
+        const int xo = x0 + 16 * i + r;
+        const bool in_row = done && yo < H && xo < W;
+        if constexpr (EPI == kEpiGate)
+          av[i] = in_row ? *reinterpret_cast<const uint2 *>(
+                               ep.act + (row + xo) * 8 + 4 * (g & 1))
+                         : make_uint2(0, 0);
+        if constexpr (EPI == kEpiPredict) {
+          if (i % 2 == 0)
+            bv[i / 2] = done && yo < H && xo + px < W
+                            ? ep.bnd[ep.off + row + xo + px] : 0.0f;
+        }
+      }
+      const u16 *rb = ring + (m & 1) * PLANE + (2 * wv * XS + r) * CIN;
+#pragma unroll
+      for (int i = 0; i < SEG; ++i)
+#pragma unroll
+        for (int kb = 0; kb < KS; ++kb) {
+          bf16x8 bo;
+          if constexpr (CIN == 2) {
+            const unsigned *w = reinterpret_cast<const unsigned *>(
+                rb + 16 * i * CIN + boff[kb]);
+            // (the fourth position has no weight)
+            bo = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], 0u));
+          } else {
+            bo = *reinterpret_cast<const bf16x8 *>(rb + 16 * i * CIN + boff[kb]);
+          }
+          // plane zp is tap t of output plane zp + 1 - t (slot (j - t) mod 3)
+#pragma unroll
+          for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+              acc[i][s][(j + 3 - t) % 3] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                      aw[s][t][kb], bo, acc[i][s][(j + 3 - t) % 3], 0, 0, 0);
+        }
+#pragma unroll
+      for (int i = 0; i < SEG; ++i) {
+        const int xo = x0 + 16 * i + r;
+        const bool in_row = done && yo < H && xo < W;
+        if constexpr (EPI == kEpiUpSkip) {
+          if (done) csum[i] += acc[i][0][(j + 1) % 3] + acc[i][1][(j + 1) % 3];
+        }
+        if constexpr (COUT == 24 && EPI == kEpiStore) {
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            if (done && yw + s < H && xo < W) {
+              f32x4 v = acc[i][s][(j + 1) % 3];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                v[e] += ba[e];
+                if (RELU) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
+              }
+              *reinterpret_cast<uint2 *>(
+                  ep.y + ((((long)n * D + z) * H + yw + s) * W + xo) * 24 +
+                  4 * g) = make_uint2(Pack2(v[0], v[1]), Pack2(v[2], v[3]));
+            }
+          }
+        }
+        f32x4 v = acc[i][S - 1][(j + 1) % 3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] += bb[e];
+          if (RELU) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
+        }
+        uint2 w2 = make_uint2(Pack2(v[0], v[1]), Pack2(v[2], v[3]));
+        if constexpr (EPI == kEpiGate) {
+          w2.x = GateWord(w2.x, av[i].x);
+          w2.y = GateWord(w2.y, av[i].y);
+        }
+        if constexpr (EPI == kEpiPredict) {
+          float s = hw[0] * __uint_as_float(w2.x << 16);
+          s += hw[1] * __uint_as_float(w2.x & 0xffff0000u);
+          s += hw[2] * __uint_as_float(w2.y << 16);
+          s += hw[3] * __uint_as_float(w2.y & 0xffff0000u);
+          pv[i] = s + __shfl_xor(s, 16, 64);
+          if (i % 2 == 1 || i == SEG - 1) {  // the pair's stores
+            const int xp = x0 + 16 * (i & ~1) + r + px;
+            const float q = (g & 1) && i % 2 == 1 ? pv[i] : pv[i & ~1];
+            if (done && yo < H && xp < W && (SEG > 1 || !(g & 1)))
+              ((PT *)ep.p)[ep.off + row + xp] =
+                  (PT)(ep.scale * (q + hb)) * (PT)bv[i / 2];
+          }
+        } else if (in_row) {
+          if constexpr (COUT == 24 && EPI == kEpiStore)
+            *reinterpret_cast<uint2 *>(ep.y + (row + xo) * 24 + 16 +
+                                       4 * (g & 1)) = w2;
+          else
+            *reinterpret_cast<uint2 *>(ep.y + (row + xo) * 8 + 4 * (g & 1)) =
+                w2;
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          acc[i][s][(j + 1) % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      if constexpr (kCells) {
+        // the last plane of a row of cells: sums over 4 x (lanes) and over
+        // the rows of a pair of waves (LDS), in a fixed order
+        if (done && (z & (kPool - 1)) == kPool - 1) {  // uniform
+#pragma unroll
+          for (int i = 0; i < SEG; ++i) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              csum[i][e] += __shfl_xor(csum[i][e], 1, 64);
+              csum[i][e] += __shfl_xor(csum[i][e], 2, 64);
+            }
+            if ((wv & 1) && (r & 3) == 0)
+              *reinterpret_cast<f32x4 *>(&cells[wv >> 1][i][4 * (4 * g + (r >> 2))]) =
+                  csum[i];
+          }
+          __syncthreads();
+          if (!(wv & 1)) {
+            const int Wc = W / kPool;
+            const long crow = (((long)n * (D / kPool) + z / kPool) *
+                                   (H / kPool) + yw / kPool) * Wc;
+#pragma unroll
+            for (int i = 0; i < SEG; ++i) {
+              const int xo = x0 + 16 * i + r;
+              if ((r & 3) == 0 && xo < W && yw < H) {
+                const f32x4 v = csum[i] + *reinterpret_cast<const f32x4 *>(
+                    &cells[wv >> 1][i][4 * (4 * g + (r >> 2))]);
+                const long o = (crow + xo / kPool) * 16 + 4 * g;
+                const uint2 a = *reinterpret_cast<const uint2 *>(ep.act + o);
+                *reinterpret_cast<uint2 *>(ep.coarse + o) =
+                    make_uint2(GateWord(Pack2(v[0], v[1]), a.x),
+                               GateWord(Pack2(v[2], v[3]), a.y));
+              }
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < SEG; ++i) csum[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+      in.Put(ring + ((m + 1) & 1) * PLANE);
+      __syncthreads();
+      in.Fetch(src, n, zp + 2, D, H, W);
+    }
   }
 }
 
@@ -881,154 +1091,6 @@ __global__ __launch_bounds__(256) void WgradKernel(
   }
 }
 
-// Filter gradient partials through LDS, for rows whose width is a multiple
-// of 32.  Block b covers positions [b*chunk, (b+1)*chunk) (a multiple of 32)
-// and every column of k; each step takes 32 positions of one row:
-//   - dz of the 32 positions is staged transposed, dzT[co][p], so the A
-//     operand of a lane (channel co, positions 8g .. 8g+7) is one 16-byte
-//     LDS read;
-//   - x of the 3 x 3 neighbouring rows (z-1..z+1, y-1..y+1) at x0-1 ..
-//     x0+32 is staged transposed, xT[row][ci][x], zero outside the grid, so
-//     the B operand of column (tap, ci) is 8 consecutive LDS elements;
-//   - wave w accumulates column tiles w, w+4, w+8, ... against the shared
-//     A operands.
-// Both operand tiles come from 16-byte global loads of whole channel
-// vectors, in place of the 2-byte gathers of WgradKernel.  Partials and
-// bias partials have WgradKernel's layout; the bias is summed in position
-// order by threads 0 .. COUT-1.
-template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void WgradLdsKernel(
-    const u16 *__restrict__ x, const u16 *__restrict__ dz,
-    float *__restrict__ part, float *__restrict__ bpart, int P, int D, int H,
-    int W, int chunk) {
-  constexpr int K = 27 * CIN, NTN = (K + 15) / 16, MT = (COUT + 15) / 16;
-  constexpr int TPW = (NTN + 3) / 4;  // column tiles per wave
-  constexpr int XR = 34;              // staged x: x0-1 .. x0+32
-  // xT[row][ci][x] as 16-bit elements, written and read as 32-bit words
-  // (pairs of neighbouring x); 4 words of padding for the last row's
-  // 5-word reads
-  __shared__ unsigned xT[9 * CIN * XR / 2 + 4];
-  __shared__ __attribute__((aligned(16))) u16 dzT[COUT * 32];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int g = lane >> 4, r = lane & 15;
-  const int p0 = blockIdx.x * chunk;
-  const int p1 = p0 + chunk < P ? p0 + chunk : P;
-  // LDS offset of each tile's column for this lane (-1: padding column)
-  int lofs[TPW];
-#pragma unroll
-  for (int i = 0; i < TPW; ++i) {
-    const int col = (wv + 4 * i) * 16 + r;
-    if (col < K) {
-      const int tap = col / CIN, ci = col - tap * CIN;
-      lofs[i] = ((tap / 3) * CIN + ci) * XR + tap % 3;
-    } else {
-      lofs[i] = -1;
-    }
-  }
-  f32x4 acc[TPW][MT];
-#pragma unroll
-  for (int i = 0; i < TPW; ++i)
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[i][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float bsum = 0.0f;
-  for (int s = p0; s < p1; s += 32) {
-    int q = s;
-    const int x0 = q % W;
-    q /= W;
-    const int y = q % H;
-    q /= H;
-    const int z = q % D;
-    const int n = q / D;
-    // x pairs (xp, xp+1), xp even: one 32-bit word per channel
-    for (int v = threadIdx.x; v < 9 * (XR / 2) * (CIN / 8); v += 256) {
-      const int c8 = v % (CIN / 8), t = v / (CIN / 8);
-      const int xp = 2 * (t % (XR / 2)), row = t / (XR / 2);
-      const int zz = z + row / 3 - 1, yy = y + row % 3 - 1, xx = x0 - 1 + xp;
-      uint4 u0 = make_uint4(0, 0, 0, 0), u1 = u0;
-      if (zz >= 0 && zz < D && yy >= 0 && yy < H) {
-        const u16 *src =
-            x + ((((long)n * D + zz) * H + yy) * W + xx) * CIN + c8 * 8;
-        if (xx >= 0 && xx < W) u0 = *reinterpret_cast<const uint4 *>(src);
-        if (xx + 1 >= 0 && xx + 1 < W)
-          u1 = *reinterpret_cast<const uint4 *>(src + CIN);
-      }
-      const unsigned a4[4] = {u0.x, u0.y, u0.z, u0.w};
-      const unsigned b4[4] = {u1.x, u1.y, u1.z, u1.w};
-      unsigned *dst = xT + ((row * CIN + c8 * 8) * XR + xp) / 2;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {  // channels 2j, 2j+1 of the vector
-        dst[(2 * j) * (XR / 2)] = (a4[j] & 0xffffu) | (b4[j] << 16);
-        dst[(2 * j + 1) * (XR / 2)] = (a4[j] >> 16) | (b4[j] & 0xffff0000u);
-      }
-    }
-    for (int v = threadIdx.x; v < 32 * (COUT / 8); v += 256) {
-      const int c8 = v % (COUT / 8), pp = v / (COUT / 8);
-      const uint4 u = *reinterpret_cast<const uint4 *>(
-          dz + (long)(s + pp) * COUT + c8 * 8);
-      const unsigned w4[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        dzT[(c8 * 8 + 2 * j) * 32 + pp] = (u16)(w4[j] & 0xffffu);
-        dzT[(c8 * 8 + 2 * j + 1) * 32 + pp] = (u16)(w4[j] >> 16);
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x < COUT)
-      for (int pp = 0; pp < 32; ++pp) bsum += Bf2F(dzT[threadIdx.x * 32 + pp]);
-    bf16x8 a[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const int co = m * 16 + r;
-      a[m] = co < COUT
-                 ? *reinterpret_cast<const bf16x8 *>(dzT + co * 32 + 8 * g)
-                 : Zero8();
-    }
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      if (wv + 4 * i >= NTN) break;  // wave-uniform
-      bf16x8 b = Zero8();
-      if (lofs[i] >= 0) {
-        // elements e .. e+7 from the 5 words that cover them; an odd e
-        // shifts each output word by one element
-        const int e = lofs[i] + 8 * g;
-        const unsigned *wsrc = xT + (e >> 1);
-        unsigned w[5];
-#pragma unroll
-        for (int k = 0; k < 5; ++k) w[k] = wsrc[k];
-        uint4 o;
-        if (e & 1) {
-          o = make_uint4(__builtin_amdgcn_alignbit(w[1], w[0], 16),
-                         __builtin_amdgcn_alignbit(w[2], w[1], 16),
-                         __builtin_amdgcn_alignbit(w[3], w[2], 16),
-                         __builtin_amdgcn_alignbit(w[4], w[3], 16));
-        } else {
-          o = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-        b = __builtin_bit_cast(bf16x8, o);
-      }
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-        acc[i][m] =
-            __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b, acc[i][m], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < TPW; ++i) {
-    const int col = (wv + 4 * i) * 16 + r;
-    if (wv + 4 * i >= NTN || col >= K) continue;
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int co = m * 16 + 4 * g + v;
-        if (co < COUT)
-          part[((long)blockIdx.x * COUT + co) * K + col] = acc[i][m][v];
-      }
-  }
-  if (threadIdx.x < COUT) bpart[(long)blockIdx.x * COUT + threadIdx.x] = bsum;
-}
-
 // Deterministic sum over blocks of part[b][i]: stage 1 sums segment s of
 // the blocks in order into tmp[s][i], stage 2 sums the segments in order.
 __global__ void SumSegmentsKernel(const float *__restrict__ part, int nparts,
@@ -1140,10 +1202,12 @@ __global__ void UpConcatKernel(const u16 *__restrict__ coarse,
 }
 
 // Gradient of the upsampled part of a concatenation: gc[coarse][c] = FP32
-// sum over the 64 fine positions of g[fine][c], c < CA of C channels.
-__global__ void UpBackKernel(const u16 *__restrict__ g, u16 *__restrict__ gc,
-                             int CA, int C, int Dc, int Hc, int Wc,
-                             int total) {
+// sum over the 64 fine positions of g[fine][c], c < CA of C channels, gated
+// by the coarse activation.
+__global__ void UpBackKernel(const u16 *__restrict__ g,
+                             const u16 *__restrict__ act,
+                             u16 *__restrict__ gc, int CA, int C, int Dc,
+                             int Hc, int Wc, int total) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int GA = CA / 8;
   if (i >= total) return;
@@ -1162,6 +1226,10 @@ __global__ void UpBackKernel(const u16 *__restrict__ g, u16 *__restrict__ gc,
 #pragma unroll
         for (int k = 0; k < 8; ++k) s.v[k] += a.v[k];
       }
+  const V8 a = Load8F(act + (long)i * 8);
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    if (!(a.v[k] > 0.0f)) s.v[k] = 0.0f;
   Store8F(gc + (long)i * 8, s);
 }
 
@@ -1192,24 +1260,6 @@ __global__ void PoolBackSkipGateKernel(const u16 *__restrict__ gpool,
   Store8F(dz + (long)i * 8, o);
 }
 
-// g *= (act > 0): ReLU gradient, in place, 8 values per thread.
-__global__ void GateKernel(u16 *__restrict__ g, const u16 *__restrict__ act,
-                           long n8) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i >= n8) return;
-  uint4 gv = *reinterpret_cast<const uint4 *>(g + i * 8);
-  const uint4 av = *reinterpret_cast<const uint4 *>(act + i * 8);
-  unsigned *gw = reinterpret_cast<unsigned *>(&gv);
-  const unsigned aw[4] = {av.x, av.y, av.z, av.w};
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const bool lo = __uint_as_float(aw[k] << 16) > 0.0f;
-    const bool hi = __uint_as_float(aw[k] & 0xffff0000u) > 0.0f;
-    gw[k] = (lo ? gw[k] & 0xffffu : 0u) | (hi ? gw[k] & 0xffff0000u : 0u);
-  }
-  *reinterpret_cast<uint4 *>(g + i * 8) = gv;
-}
-
 // Network input: ch0 = rhs, ch1 = bnd, ch2..7 = 0 (problems [first, ...)).
 __global__ void InputKernel(const float *__restrict__ rhs,
                             const float *__restrict__ bnd,
@@ -1221,14 +1271,17 @@ __global__ void InputKernel(const float *__restrict__ rhs,
   *reinterpret_cast<uint4 *>(x + p * 8) = v;
 }
 
-// 1x1 convolution 8 -> 1: out[p] = sum_c w[c] in[p][c] + b (FP32).
+// 1x1 convolution 8 -> 1: out[p] = sum_c w[c] in[p][c] + b (FP32), for the
+// cell means of the smooth loss terms.
 __global__ void HeadKernel(const u16 *__restrict__ in,
                            const float *__restrict__ w,
                            float *__restrict__ out, long P) {
   const long p = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (p >= P) return;
+  const V8 a = Load8F(in + p * 8);
   float s = 0.0f;
-  for (int c = 0; c < 8; ++c) s += w[c] * Bf2F(in[p * 8 + c]);
+#pragma unroll
+  for (int c = 0; c < 8; ++c) s += w[c] * a.v[c];
   out[p] = s + w[8];
 }
 
@@ -1275,23 +1328,45 @@ __global__ void SmoothCoarseKernel(const float *__restrict__ e4,
   e16[c] = s * (1.0f / 64.0f);
 }
 
-// Loss partials and its gradient dout.  With d = out - target * inv_scale,
-// e4 / e16 the means of d over the point's 4^3 / 16^3 cell:
+// Head, loss, and the head's backward in one pass over the last layer's
+// activations `in`: out = w . in + b (1x1 convolution 8 -> 1, FP32),
+// d = out - target * inv_scale, and with e4 / e16 the means of d over the
+// point's 4^3 / 16^3 cell
 //   loss = (1/P) sum_p (d^2 + w4 e4^2 + w16 e16^2)
 //        = mean d^2 + w4 mean over 4^3 cells e4^2 + w16 mean e16^2,
-//   dout = 2 (d + w4 e4 + w16 e16) / P.
-// SMOOTH false: w4 = w16 = 0 (e4, e16 unused).
+//   dout = 2 (d + w4 e4 + w16 e16) / P,
+// din[p][c] = w[c] dout[p] gated by in (BF16), and per-block partials of the
+// loss, dw[c] = sum dout[p] in[p][c] and db = sum dout[p].  SMOOTH false:
+// w4 = w16 = 0 (e4, e16 unused).  Bound by its 36 bytes per point (in,
+// target, din); as three passes (head, loss, head backward with 2-byte
+// loads) it took 364 us at 8 x 128^3.
+constexpr int kHeadThreads = 512;
 template <bool SMOOTH>
-__global__ __launch_bounds__(256) void LossKernel(
-    const float *__restrict__ out, const float *__restrict__ target,
-    long toff, float inv_scale, const float *__restrict__ e4,
-    const float *__restrict__ e16, float w4, float w16, int D1, int H1,
-    int W1, float *__restrict__ dout, double *__restrict__ part, long P) {
-  __shared__ double red[4];
+__global__ __launch_bounds__(kHeadThreads) void HeadLossBackKernel(
+    const u16 *__restrict__ in, const float *__restrict__ w,
+    const float *__restrict__ target, long toff, float inv_scale,
+    const float *__restrict__ e4, const float *__restrict__ e16, float w4,
+    float w16, int D1, int H1, int W1, u16 *__restrict__ din,
+    double *__restrict__ lpart, float *__restrict__ part, long P) {
+  __shared__ double lred[kHeadThreads / 64];
+  __shared__ float red[9][kHeadThreads / 64];
+  float wc[9], acc[9];
+#pragma unroll
+  for (int c = 0; c < 9; ++c) {
+    wc[c] = w[c];
+    acc[c] = 0.0f;
+  }
   double s = 0.0;
-  for (long p = blockIdx.x * (long)blockDim.x + threadIdx.x; p < P;
-       p += (long)gridDim.x * blockDim.x) {
-    const float d = out[p] - target[toff + p] * inv_scale;
+#pragma unroll 2
+  for (long p = blockIdx.x * (long)kHeadThreads + threadIdx.x; p < P;
+       p += (long)gridDim.x * kHeadThreads) {
+    const V8 a = Load8F(in + p * 8);
+    float o = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) o += wc[c] * a.v[c];
+    o += wc[8];
+    const float d = o - target[toff + p] * inv_scale;
+    float g;
     if constexpr (SMOOTH) {
       const int x = (int)(p % W1), y = (int)((p / W1) % H1);
       const long nz = p / ((long)W1 * H1);
@@ -1302,50 +1377,32 @@ __global__ __launch_bounds__(256) void LossKernel(
       const int W3 = W2 / kPool, H3 = H2 / kPool, D3 = D2 / kPool;
       const long c3 = ((n * D3 + z / (kPool * kPool)) * H3 +
                        y / (kPool * kPool)) * W3 + x / (kPool * kPool);
-      const float a = e4[c2], b = e16[c3];
-      dout[p] = 2.0f * (d + w4 * a + w16 * b) / (float)P;
-      s += (double)d * d + (double)w4 * a * a + (double)w16 * b * b;
+      const float m4 = e4[c2], m16 = e16[c3];
+      g = 2.0f * (d + w4 * m4 + w16 * m16) / (float)P;
+      s += (double)d * d + (double)w4 * m4 * m4 + (double)w16 * m16 * m16;
     } else {
-      dout[p] = 2.0f * d / (float)P;
+      g = 2.0f * d / (float)P;
       s += (double)d * d;
     }
-  }
-  s = physis_hip::BlockReduce<double, PS_SUM, 256>(s, red);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-// Head backward: din[p][c] = w[c] dout[p] (BF16, gated by act), and
-// per-block partials of dw[c] = sum dout[p] in[p][c], db = sum dout[p].
-__global__ __launch_bounds__(256) void HeadBackKernel(
-    const u16 *__restrict__ in, const float *__restrict__ w,
-    const float *__restrict__ dout, u16 *__restrict__ din,
-    float *__restrict__ part, long P) {
-  __shared__ float red[9][4];
-  float acc[9];
-  for (int c = 0; c < 9; ++c) acc[c] = 0.0f;
-  for (long p = blockIdx.x * (long)blockDim.x + threadIdx.x; p < P;
-       p += (long)gridDim.x * blockDim.x) {
-    const float d = dout[p];
+    float v[8];
+#pragma unroll
     for (int c = 0; c < 8; ++c) {
-      const float a = Bf2F(in[p * 8 + c]);
-      acc[c] += d * a;
-      din[p * 8 + c] = a > 0.0f ? F2Bf(w[c] * d) : (u16)0;
+      acc[c] += g * a.v[c];
+      v[c] = a.v[c] > 0.0f ? wc[c] * g : 0.0f;
     }
-    acc[8] += d;
+    acc[8] += g;
+    *reinterpret_cast<uint4 *>(din + p * 8) =
+        make_uint4(Pack2(v[0], v[1]), Pack2(v[2], v[3]), Pack2(v[4], v[5]),
+                   Pack2(v[6], v[7]));
   }
+  s = physis_hip::BlockReduce<double, PS_SUM, kHeadThreads>(s, lred);
+  if (threadIdx.x == 0) lpart[blockIdx.x] = s;
+#pragma unroll
   for (int c = 0; c < 9; ++c) {
-    const float s = physis_hip::BlockReduce<float, PS_SUM, 256>(acc[c], red[c]);
-    if (threadIdx.x == 0) part[blockIdx.x * 9 + c] = s;
+    const float t =
+        physis_hip::BlockReduce<float, PS_SUM, kHeadThreads>(acc[c], red[c]);
+    if (threadIdx.x == 0) part[blockIdx.x * 9 + c] = t;
   }
-}
-
-// Prediction: p[off + i] = scale * out[i] * bnd[off + i] (FP32 or FP64 p).
-template <typename T>
-__global__ void PredictKernel(const float *__restrict__ out,
-                              const float *__restrict__ bnd, T *__restrict__ p,
-                              long off, float scale, long P) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i < P) p[off + i] = (T)(scale * out[i]) * (T)bnd[off + i];
 }
 
 // Weights: wt[co][k] = bf16(W[co][k]) (zero for k >= 27 cin) and the
@@ -1410,20 +1467,6 @@ hipStream_t Stream() { return (hipStream_t)__PSHipStream(); }
 void Check() { PS_HIP_CHECK(hipGetLastError()); }
 unsigned Blocks(long n, int t = 256) { return (unsigned)((n + t - 1) / t); }
 
-template <int CIN, int COUT, int XT>
-void ConvLaunch(const u16 *x, const u16 *wt, const float *b, bool relu,
-                u16 *y, int N, int D, int H, int W) {
-  const int tiles_x = (W + XT - 1) / XT;
-  const dim3 grid(tiles_x * ((H + 3) / 4), N * D), block(256);
-  if (relu)
-    hipLaunchKernelGGL((ConvKernel<CIN, COUT, true, XT>), grid, block, 0,
-                       Stream(), x, wt, b, y, D, H, W);
-  else
-    hipLaunchKernelGGL((ConvKernel<CIN, COUT, false, XT>), grid, block, 0,
-                       Stream(), x, wt, b, y, D, H, W);
-  Check();
-}
-
 // Blocks per compute unit that the z-marching launches aim for (measured
 // at level 1 of batch 8 x 128^3: the plane-marching filter gradient is
 // fastest with 2, e.g. 8 -> 8 213 us against 223 with 4 and 237 with 8,
@@ -1444,61 +1487,96 @@ void ZChunks(long tiles, int N, int D, int per_cu, int *tz, int *zchunk) {
 
 template <int CIN, int COUT, int XT, int TY>
 void ConvZLaunch(const u16 *x, const u16 *wt, const float *b, bool relu,
-                 u16 *y, int N, int D, int H, int W) {
+                 const u16 *act, u16 *y, int N, int D, int H, int W) {
   const int tiles = ((W + XT - 1) / XT) * ((H + TY - 1) / TY);
   int tz, zchunk;
   ZChunks(tiles, N, D, kConvZBlocksPerCU, &tz, &zchunk);
   const dim3 grid(tiles, N * tz), block(64 * TY);
   if (relu)
     hipLaunchKernelGGL((ConvZKernel<CIN, COUT, true, XT, TY>), grid, block, 0,
-                       Stream(), x, wt, b, y, D, H, W, tz, zchunk);
+                       Stream(), x, wt, b, act, y, D, H, W, tz, zchunk);
   else
     hipLaunchKernelGGL((ConvZKernel<CIN, COUT, false, XT, TY>), grid, block,
-                       0, Stream(), x, wt, b, y, D, H, W, tz, zchunk);
+                       0, Stream(), x, wt, b, act, y, D, H, W, tz, zchunk);
   Check();
 }
 
-template <int CIN, int XT, int TY>
-void ConvZPairLaunch(const u16 *x, const u16 *wt, const float *b, bool relu,
-                     u16 *y, int N, int D, int H, int W) {
-  const int tiles = ((W + XT - 1) / XT) * ((H + 2 * TY - 1) / (2 * TY));
+// The input-marching convolution (8 or 24 output channels).  Block shapes
+// (XT positions by 2 TY rows) measured at 8 x 128^3, us, of 64x8, 32x8, 64x16
+// and 32x16: plain 8 -> 8 115 / 102 / 131 / 109; gated 164 / 216 / 177 / 150;
+// prediction 202 / 228 / 201 / 143; network input 91 / 113 / 101 / 118;
+// 24 -> 8 (32x8, 32x16) 234 / 267; 8 -> 24 with cell sums 401 / 288.  Rows of
+// at most 16 positions take XT = 16.
+constexpr int kConvMWavesPerCU = 16;
+template <int CIN, int COUT, bool RELU, int XT, int TY,
+          template <int, int, int, int> class SRC, int EPI, typename PT>
+void ConvMLaunchXT(const SrcArgs &src, const u16 *wt, const EpiArgs &ep, int N,
+                   int D, int H, int W) {
+  static_assert(EPI != kEpiPredict || XT == 16 || XT % 32 == 0, "pairs");
+  const long tiles = (long)((W + XT - 1) / XT) * ((H + 2 * TY - 1) / (2 * TY));
   int tz, zchunk;
-  ZChunks(tiles, N, D, kConvZBlocksPerCU, &tz, &zchunk);
-  const dim3 grid(tiles, N * tz), block(64 * TY);
-  if (relu)
-    hipLaunchKernelGGL((ConvZPairKernel<CIN, true, XT, TY>), grid, block, 0,
-                       Stream(), x, wt, b, y, D, H, W, tz, zchunk);
-  else
-    hipLaunchKernelGGL((ConvZPairKernel<CIN, false, XT, TY>), grid, block, 0,
-                       Stream(), x, wt, b, y, D, H, W, tz, zchunk);
+  ZChunks(tiles, N, D, kConvMWavesPerCU / TY, &tz, &zchunk);
+  if (EPI == kEpiUpSkip) {  // whole cells
+    zchunk = (zchunk + kPool - 1) / kPool * kPool;
+    tz = (D + zchunk - 1) / zchunk;
+  }
+  hipLaunchKernelGGL((ConvMKernel<CIN, COUT, RELU, XT, TY, SRC, EPI, PT>),
+                     dim3((unsigned)(tiles * N * tz)), dim3(64 * TY), 0,
+                     Stream(), src, wt, ep, D, H, W, tz, zchunk);
   Check();
 }
+template <int CIN, int COUT, bool RELU,
+          template <int, int, int, int> class SRC, int EPI,
+          typename PT = double>
+void ConvMLaunch(const SrcArgs &src, const u16 *wt, const EpiArgs &ep, int N,
+                 int D, int H, int W) {
+  constexpr int XT = CIN == 2 ? 64 : 32;
+  constexpr int TY = COUT == 24 || EPI == kEpiGate || EPI == kEpiPredict ? 8 : 4;
+  if (W > 16)
+    ConvMLaunchXT<CIN, COUT, RELU, XT, TY, SRC, EPI, PT>(src, wt, ep, N, D, H,
+                                                         W);
+  else
+    ConvMLaunchXT<CIN, COUT, RELU, 16, 4, SRC, EPI, PT>(src, wt, ep, N, D, H,
+                                                        W);
+}
 
-// z-marching convolution: x tile of 64 positions below 24 input channels,
-// else 32, 16 for rows of at most 16; 8 rows per block below 24 input
-// channels, else 4 (the ring of 4 staged planes then stays within LDS).
+// A convolution of whole tensors; act: gate of the results, or NULL.  8 and
+// 24 output channels march the input planes (ConvMKernel); more keep the
+// ring of planes: x tile of 64 positions below 24 input channels, else 32,
+// 16 for rows of at most 16; 8 rows per block below 24 input channels, else
+// 4 (the ring of 4 staged planes then stays within LDS).
 template <int CIN, int COUT>
-void ConvT(const u16 *x, const u16 *wt, const float *b, bool relu, u16 *y,
-           int N, int D, int H, int W) {
-  if constexpr (COUT == 8) {
-    // two output rows per wave: 8 rows per block of 4 waves
+void ConvT(const u16 *x, const u16 *wt, const float *b, bool relu,
+           const u16 *act, u16 *y, int N, int D, int H, int W) {
+  if constexpr (COUT == 8 || COUT == 24) {
+    SrcArgs src{x, nullptr, 0};
+    EpiArgs ep;
+    ep.bias = b;
+    ep.act = act;
+    ep.y = y;
+    if constexpr (COUT == 8) {
+      if (act)
+        return ConvMLaunch<CIN, 8, false, PlainSrc, kEpiGate>(src, wt, ep, N,
+                                                              D, H, W);
+    }
+    if (relu)
+      ConvMLaunch<CIN, COUT, true, PlainSrc, kEpiStore>(src, wt, ep, N, D, H,
+                                                        W);
+    else
+      ConvMLaunch<CIN, COUT, false, PlainSrc, kEpiStore>(src, wt, ep, N, D, H,
+                                                         W);
+  } else {
+    constexpr int TY = CIN < 24 ? 8 : 4;
     if constexpr (CIN < 24) {
       if (W > 32)
-        return ConvZPairLaunch<CIN, 64, 4>(x, wt, b, relu, y, N, D, H, W);
+        return ConvZLaunch<CIN, COUT, 64, TY>(x, wt, b, relu, act, y, N, D, H,
+                                              W);
     }
     if (W > 16)
-      return ConvZPairLaunch<CIN, 32, 4>(x, wt, b, relu, y, N, D, H, W);
-    return ConvZPairLaunch<CIN, 16, 4>(x, wt, b, relu, y, N, D, H, W);
+      ConvZLaunch<CIN, COUT, 32, TY>(x, wt, b, relu, act, y, N, D, H, W);
+    else
+      ConvZLaunch<CIN, COUT, 16, TY>(x, wt, b, relu, act, y, N, D, H, W);
   }
-  constexpr int TY = CIN < 24 ? 8 : 4;
-  if constexpr (CIN < 24) {
-    if (W > 32)
-      return ConvZLaunch<CIN, COUT, 64, TY>(x, wt, b, relu, y, N, D, H, W);
-  }
-  if (W > 16)
-    ConvZLaunch<CIN, COUT, 32, TY>(x, wt, b, relu, y, N, D, H, W);
-  else
-    ConvZLaunch<CIN, COUT, 16, TY>(x, wt, b, relu, y, N, D, H, W);
 }
 
 // Positions per filter-gradient block: about P / 512 (a multiple of 32),
@@ -1606,9 +1684,10 @@ void SumParts(const float *part, int nparts, long n, float *tmp, float *out) {
   X(16, 8) X(32, 16) X(16, 48) X(8, 24)
 
 void Conv(int cin, int cout, const u16 *x, const u16 *wt, const float *b,
-          bool relu, u16 *y, int N, int D, int H, int W) {
+          bool relu, const u16 *act, u16 *y, int N, int D, int H, int W) {
 #define PS_CASE(I, O) \
-  if (cin == I && cout == O) return ConvT<I, O>(x, wt, b, relu, y, N, D, H, W);
+  if (cin == I && cout == O) \
+    return ConvT<I, O>(x, wt, b, relu, act, y, N, D, H, W);
   PS_UNET_PAIRS(PS_CASE)
 #undef PS_CASE
   PS_FATAL("no convolution kernel for %d -> %d channels", cin, cout);
@@ -1663,7 +1742,7 @@ struct __PSUNet {
   // activations (BF16) at batch max_batch
   u16 *x0 = nullptr, *a[10] = {}, *q1 = nullptr, *q2 = nullptr,
       *c2 = nullptr, *c1 = nullptr;
-  float *out = nullptr, *dout = nullptr;
+  float *out = nullptr;
   // gradient scratch
   u16 *g1a = nullptr, *g1b = nullptr, *gc1 = nullptr;  // level 1
   u16 *g2a = nullptr, *g2b = nullptr, *gc2 = nullptr;  // level 2
@@ -1680,8 +1759,7 @@ namespace {
 
 const int kLayerCh[10][2] = {{8, 8},  {8, 8},   {8, 16},  {16, 16}, {16, 32},
                              {32, 32}, {48, 16}, {16, 16}, {24, 8},  {8, 8}};
-constexpr int kLossBlocks = 1024;
-constexpr int kHeadBlocks = 1024;
+constexpr int kHeadBlocks = 1024;  // of HeadLossBackKernel: its partials
 
 void Upload(__PSUNet *net) {  // master weights -> BF16 copies
   for (auto &L : net->layers) {
@@ -1711,7 +1789,8 @@ Dims DimsOf(const __PSUNet *net, int count) {
 void ConvL(const __PSUNet *net, int l, const u16 *in, u16 *out, int N, int D,
            int H, int W) {
   const Layer &L = net->layers[l];
-  Conv(L.cin, L.cout, in, L.wt, net->params + L.b_off, true, out, N, D, H, W);
+  Conv(L.cin, L.cout, in, L.wt, net->params + L.b_off, true, nullptr, out, N,
+       D, H, W);
 }
 
 void CheckGrid(const __PSUNet *net, const __PSGrid *g, int first, int count,
@@ -1726,21 +1805,46 @@ void CheckGrid(const __PSUNet *net, const __PSGrid *g, int first, int count,
              first, first + count, nb, net->max_batch);
 }
 
-// Forward pass of problems [first, first+count): fills the activations and
-// net->out.
+// An 8-channel layer on a source of its own (the network input, or an
+// upsampled tensor next to a skip connection).
+template <int CIN, template <int, int, int, int> class SRC>
+void ConvSrc(const __PSUNet *net, int l, const SrcArgs &src, u16 *out, int N,
+             int D, int H, int W) {
+  const Layer &L = net->layers[l];
+  EpiArgs ep;
+  ep.bias = net->params + L.b_off;
+  ep.y = out;
+  ConvMLaunch<CIN, 8, true, SRC, kEpiStore>(src, L.wt, ep, N, D, H, W);
+}
+
+// The last layer, the head and the scaled, masked prediction into p.
+template <typename T>
+void ConvPredict(const __PSUNet *net, const __PSGrid *bnd, __PSGrid *p,
+                 long off, int N, int D, int H, int W) {
+  const Layer &L = net->layers[9];
+  EpiArgs ep;
+  ep.bias = net->params + L.b_off;
+  ep.head = net->params + net->head_off;
+  ep.bnd = (const float *)bnd->p;
+  ep.p = p->p;
+  ep.off = off;
+  ep.scale = net->out_scale;
+  ConvMLaunch<8, 8, true, PlainSrc, kEpiPredict, T>(
+      SrcArgs{net->a[8], nullptr, 0}, L.wt, ep, N, D, H, W);
+}
+
+// Forward pass of problems [first, first+count): fills the activations; with
+// p the last layer's are not kept, the prediction goes to p.
 void Forward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
-             int first, int count) {
+             int first, int count, __PSGrid *p) {
   CheckGrid(net, rhs, first, count, "rhs");
   CheckGrid(net, bnd, first, count, "bnd");
   if (rhs->type != PS_FLOAT || bnd->type != PS_FLOAT)
     PS_FATAL("U-Net: rhs and bnd must be float grids");
   const Dims d = DimsOf(net, count);
   const long off = (long)first * net->nx * net->ny * net->nzs;
-  hipLaunchKernelGGL(InputKernel, dim3(Blocks(d.P1)), dim3(256), 0, Stream(),
-                     (const float *)rhs->p, (const float *)bnd->p, net->x0,
-                     off, d.P1);
-  Check();
-  ConvL(net, 0, net->x0, net->a[0], d.N, d.D1, d.H1, d.W1);
+  ConvSrc<2, InputSrc>(net, 0, SrcArgs{rhs->p, bnd->p, off}, net->a[0], d.N,
+                       d.D1, d.H1, d.W1);
   ConvL(net, 1, net->a[0], net->a[1], d.N, d.D1, d.H1, d.W1);
   hipLaunchKernelGGL(PoolKernel, dim3(Blocks(d.P2)), dim3(256), 0, Stream(),
                      net->a[1], net->q1, 8, d.D2, d.H2, d.W2, (int)d.P2);
@@ -1759,15 +1863,14 @@ void Forward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
   Check();
   ConvL(net, 6, net->c2, net->a[6], d.N, d.D2, d.H2, d.W2);
   ConvL(net, 7, net->a[6], net->a[7], d.N, d.D2, d.H2, d.W2);
-  hipLaunchKernelGGL(UpConcatKernel, dim3(Blocks(d.P1 * 3)), dim3(256), 0,
-                     Stream(), net->a[7], net->a[1], net->c1, 16, 8, d.D1,
-                     d.H1, d.W1, (int)(d.P1 * 3));
-  Check();
-  ConvL(net, 8, net->c1, net->a[8], d.N, d.D1, d.H1, d.W1);
-  ConvL(net, 9, net->a[8], net->a[9], d.N, d.D1, d.H1, d.W1);
-  hipLaunchKernelGGL(HeadKernel, dim3(Blocks(d.P1)), dim3(256), 0, Stream(),
-                     net->a[9], net->params + net->head_off, net->out, d.P1);
-  Check();
+  ConvSrc<24, ConcatSrc>(net, 8, SrcArgs{net->a[7], net->a[1], 0}, net->a[8],
+                         d.N, d.D1, d.H1, d.W1);
+  if (!p)
+    ConvL(net, 9, net->a[8], net->a[9], d.N, d.D1, d.H1, d.W1);
+  else if (p->type == PS_DOUBLE)
+    ConvPredict<double>(net, bnd, p, off, d.N, d.D1, d.H1, d.W1);
+  else
+    ConvPredict<float>(net, bnd, p, off, d.N, d.D1, d.H1, d.W1);
 }
 
 // Filter gradient of layer l from input `in` and gated output gradient dz.
@@ -1783,28 +1886,39 @@ void LayerWgrad(__PSUNet *net, int l, const u16 *in, const u16 *dz, int N,
   SumParts(net->bpart, np, (long)L.cout, net->tmp, net->grad + L.b_off);
 }
 
-// Data gradient of layer l: dx = conv(dz, flipped W), no bias, no ReLU.
-void LayerDgrad(__PSUNet *net, int l, const u16 *dz, u16 *dx, int N, int D,
-                int H, int W) {
+// Data gradient of layer l: dx = conv(dz, flipped W), no bias, no ReLU,
+// gated by the activation act when not NULL (the ReLU of the layer before).
+void LayerDgrad(__PSUNet *net, int l, const u16 *dz, const u16 *act, u16 *dx,
+                int N, int D, int H, int W) {
   const Layer &L = net->layers[l];
-  Conv(L.cout, L.cin, dz, L.wf, nullptr, false, dx, N, D, H, W);
-}
-
-void Gate(u16 *g, const u16 *act, long n) {  // n: a multiple of 8
-  hipLaunchKernelGGL(GateKernel, dim3(Blocks(n / 8)), dim3(256), 0, Stream(),
-                     g, act, n / 8);
-  Check();
+  Conv(L.cout, L.cin, dz, L.wf, nullptr, false, act, dx, N, D, H, W);
 }
 
 // Loss of the current forward pass against target, and the full gradient
 // into net->grad.
-double Backward(__PSUNet *net, const __PSGrid *target, int first, int count) {
+double Backward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
+                const __PSGrid *target, int first, int count) {
   CheckGrid(net, target, first, count, "target");
   if (target->type != PS_FLOAT) PS_FATAL("U-Net: target must be a float grid");
   const Dims d = DimsOf(net, count);
   const long off = (long)first * net->nx * net->ny * net->nzs;
   const float inv_scale = 1.0f / net->out_scale;
-  if (net->w4 != 0.0f || net->w16 != 0.0f) {
+  // the filter gradients read the first layer's input and the level-1
+  // concatenation as tensors
+  hipLaunchKernelGGL(InputKernel, dim3(Blocks(d.P1)), dim3(256), 0, Stream(),
+                     (const float *)rhs->p, (const float *)bnd->p, net->x0,
+                     off, d.P1);
+  Check();
+  hipLaunchKernelGGL(UpConcatKernel, dim3(Blocks(d.P1 * 3)), dim3(256), 0,
+                     Stream(), net->a[7], net->a[1], net->c1, 16, 8, d.D1,
+                     d.H1, d.W1, (int)(d.P1 * 3));
+  Check();
+  // head and loss: g1a = gated dD1 (layer 9's dz), partials in part, lpart
+  const bool smooth = net->w4 != 0.0f || net->w16 != 0.0f;
+  if (smooth) {
+    hipLaunchKernelGGL(HeadKernel, dim3(Blocks(d.P1)), dim3(256), 0, Stream(),
+                       net->a[9], net->params + net->head_off, net->out, d.P1);
+    Check();
     hipLaunchKernelGGL(SmoothCellKernel, dim3(Blocks(d.P2 * 64)), dim3(256),
                        0, Stream(), net->out, (const float *)target->p, off,
                        inv_scale, net->e4, d.D1, d.H1, d.W1, d.P2);
@@ -1812,76 +1926,67 @@ double Backward(__PSUNet *net, const __PSGrid *target, int first, int count) {
     hipLaunchKernelGGL(SmoothCoarseKernel, dim3(Blocks(d.P3)), dim3(256), 0,
                        Stream(), net->e4, net->e16, d.D2, d.H2, d.W2, d.P3);
     Check();
-    hipLaunchKernelGGL(LossKernel<true>, dim3(kLossBlocks), dim3(256), 0,
-                       Stream(), net->out, (const float *)target->p, off,
-                       inv_scale, net->e4, net->e16, net->w4, net->w16, d.D1,
-                       d.H1, d.W1, net->dout, net->lpart, d.P1);
-  } else {
-    hipLaunchKernelGGL(LossKernel<false>, dim3(kLossBlocks), dim3(256), 0,
-                       Stream(), net->out, (const float *)target->p, off,
-                       inv_scale, nullptr, nullptr, 0.0f, 0.0f, d.D1, d.H1,
-                       d.W1, net->dout, net->lpart, d.P1);
   }
-  Check();
-  // head: g1a = gated dD1 (layer 9's dz), head partials in part
-  hipLaunchKernelGGL(HeadBackKernel, dim3(kHeadBlocks), dim3(256), 0,
-                     Stream(), net->a[9], net->params + net->head_off,
-                     net->dout, net->g1a, net->part, d.P1);
+  const auto head = smooth ? HeadLossBackKernel<true> : HeadLossBackKernel<false>;
+  hipLaunchKernelGGL(head, dim3(kHeadBlocks), dim3(kHeadThreads), 0, Stream(),
+                     net->a[9], net->params + net->head_off,
+                     (const float *)target->p, off, inv_scale, net->e4,
+                     net->e16, net->w4, net->w16, d.D1, d.H1, d.W1, net->g1a,
+                     net->lpart, net->part, d.P1);
   Check();
   SumParts(net->part, kHeadBlocks, 9L, net->tmp, net->grad + net->head_off);
   // level 1 decoder
   LayerWgrad(net, 9, net->a[8], net->g1a, d.N, d.D1, d.H1, d.W1);
-  LayerDgrad(net, 9, net->g1a, net->g1b, d.N, d.D1, d.H1, d.W1);
-  Gate(net->g1b, net->a[8], d.P1 * 8);
+  LayerDgrad(net, 9, net->g1a, net->a[8], net->g1b, d.N, d.D1, d.H1, d.W1);
   LayerWgrad(net, 8, net->c1, net->g1b, d.N, d.D1, d.H1, d.W1);
-  LayerDgrad(net, 8, net->g1b, net->gc1, d.N, d.D1, d.H1, d.W1);  // 24 ch
-  hipLaunchKernelGGL(UpBackKernel, dim3(Blocks(d.P2 * 2)), dim3(256), 0,
-                     Stream(), net->gc1, net->g2a, 16, 24, d.D2, d.H2, d.W2,
-                     (int)(d.P2 * 2));
-  Check();
+  // 24 channels: 16 to the level-2 decoder (summed over the upsampled cells
+  // and gated: g2a), 8 to the skip connection (gc1)
+  {
+    const Layer &L = net->layers[8];
+    EpiArgs ep;
+    ep.y = net->gc1;
+    ep.act = net->a[7];
+    ep.coarse = net->g2a;
+    ConvMLaunch<8, 24, false, PlainSrc, kEpiUpSkip>(
+        SrcArgs{net->g1b, nullptr, 0}, L.wf, ep, d.N, d.D1, d.H1, d.W1);
+  }
   // level 2 decoder
-  Gate(net->g2a, net->a[7], d.P2 * 16);
   LayerWgrad(net, 7, net->a[6], net->g2a, d.N, d.D2, d.H2, d.W2);
-  LayerDgrad(net, 7, net->g2a, net->g2b, d.N, d.D2, d.H2, d.W2);
-  Gate(net->g2b, net->a[6], d.P2 * 16);
+  LayerDgrad(net, 7, net->g2a, net->a[6], net->g2b, d.N, d.D2, d.H2, d.W2);
   LayerWgrad(net, 6, net->c2, net->g2b, d.N, d.D2, d.H2, d.W2);
-  LayerDgrad(net, 6, net->g2b, net->gc2, d.N, d.D2, d.H2, d.W2);  // 48 ch
+  LayerDgrad(net, 6, net->g2b, nullptr, net->gc2, d.N, d.D2, d.H2, d.W2);
   hipLaunchKernelGGL(UpBackKernel, dim3(Blocks(d.P3 * 4)), dim3(256), 0,
-                     Stream(), net->gc2, net->g3a, 32, 48, d.D3, d.H3, d.W3,
-                     (int)(d.P3 * 4));
+                     Stream(), net->gc2, net->a[5], net->g3a, 32, 48, d.D3,
+                     d.H3, d.W3, (int)(d.P3 * 4));
   Check();
   // level 3
-  Gate(net->g3a, net->a[5], d.P3 * 32);
   LayerWgrad(net, 5, net->a[4], net->g3a, d.N, d.D3, d.H3, d.W3);
-  LayerDgrad(net, 5, net->g3a, net->g3b, d.N, d.D3, d.H3, d.W3);
-  Gate(net->g3b, net->a[4], d.P3 * 32);
+  LayerDgrad(net, 5, net->g3a, net->a[4], net->g3b, d.N, d.D3, d.H3, d.W3);
   LayerWgrad(net, 4, net->q2, net->g3b, d.N, d.D3, d.H3, d.W3);
-  LayerDgrad(net, 4, net->g3b, net->g3a, d.N, d.D3, d.H3, d.W3);  // 16 ch
+  LayerDgrad(net, 4, net->g3b, nullptr, net->g3a, d.N, d.D3, d.H3, d.W3);
   // level 2 encoder: E2 receives the pool gradient and the skip gradient
   hipLaunchKernelGGL(PoolBackSkipGateKernel, dim3(Blocks(d.P2 * 2)),
                      dim3(256), 0, Stream(), net->g3a, net->gc2, net->a[3],
                      net->g2a, 16, 32, d.D2, d.H2, d.W2, (int)(d.P2 * 2));
   Check();
   LayerWgrad(net, 3, net->a[2], net->g2a, d.N, d.D2, d.H2, d.W2);
-  LayerDgrad(net, 3, net->g2a, net->g2b, d.N, d.D2, d.H2, d.W2);
-  Gate(net->g2b, net->a[2], d.P2 * 16);
+  LayerDgrad(net, 3, net->g2a, net->a[2], net->g2b, d.N, d.D2, d.H2, d.W2);
   LayerWgrad(net, 2, net->q1, net->g2b, d.N, d.D2, d.H2, d.W2);
-  LayerDgrad(net, 2, net->g2b, net->g2a, d.N, d.D2, d.H2, d.W2);  // 8 ch
+  LayerDgrad(net, 2, net->g2b, nullptr, net->g2a, d.N, d.D2, d.H2, d.W2);
   // level 1 encoder
   hipLaunchKernelGGL(PoolBackSkipGateKernel, dim3(Blocks(d.P1)), dim3(256),
                      0, Stream(), net->g2a, net->gc1, net->a[1], net->g1a, 8,
-                     16, d.D1, d.H1, d.W1, (int)d.P1);
+                     0, d.D1, d.H1, d.W1, (int)d.P1);
   Check();
   LayerWgrad(net, 1, net->a[0], net->g1a, d.N, d.D1, d.H1, d.W1);
-  LayerDgrad(net, 1, net->g1a, net->g1b, d.N, d.D1, d.H1, d.W1);
-  Gate(net->g1b, net->a[0], d.P1 * 8);
+  LayerDgrad(net, 1, net->g1a, net->a[0], net->g1b, d.N, d.D1, d.H1, d.W1);
   LayerWgrad(net, 0, net->x0, net->g1b, d.N, d.D1, d.H1, d.W1);
   PS_HIP_CHECK(hipMemcpyAsync(net->lhost, net->lpart,
-                              sizeof(double) * kLossBlocks,
+                              sizeof(double) * kHeadBlocks,
                               hipMemcpyDeviceToHost, Stream()));
   PS_HIP_CHECK(hipStreamSynchronize(Stream()));
   double loss = 0.0;
-  for (int b = 0; b < kLossBlocks; ++b) loss += net->lhost[b];
+  for (int b = 0; b < kHeadBlocks; ++b) loss += net->lhost[b];
   return loss / (double)d.P1;
 }
 
@@ -1889,7 +1994,7 @@ void FreeNet(__PSUNet *net) {
   (void)hipStreamSynchronize(Stream());
   std::vector<void *> ptrs = {net->params, net->grad, net->adam_m,
                               net->adam_v, net->x0, net->q1, net->q2,
-                              net->c2, net->c1, net->out, net->dout, net->g1a,
+                              net->c2, net->c1, net->out, net->g1a,
                               net->g1b, net->gc1, net->g2a, net->g2b,
                               net->gc2, net->g3a, net->g3b, net->part,
                               net->bpart, net->tmp, net->lpart, net->e4,
@@ -1997,10 +2102,9 @@ __PSUNet *PSUNetNew(int nx, int ny, int nzs, int max_batch, float out_scale,
   net->c2 = A16(d.P2 * 48);
   net->c1 = A16(d.P1 * 24);
   net->out = A32(d.P1);
-  net->dout = A32(d.P1);
   net->g1a = A16(d.P1 * 8);
   net->g1b = A16(d.P1 * 8);
-  net->gc1 = A16(d.P1 * 24);
+  net->gc1 = A16(d.P1 * 8);
   net->g2a = A16(d.P2 * 16);
   net->g2b = A16(d.P2 * 16);
   net->gc2 = A16(d.P2 * 48);
@@ -2032,9 +2136,9 @@ __PSUNet *PSUNetNew(int nx, int ny, int nzs, int max_batch, float out_scale,
   net->tmp = A32((long)(te * kSumSegments));
   net->e4 = A32(d.P2);
   net->e16 = A32(d.P3);
-  net->lpart = (double *)Alloc(sizeof(double) * kLossBlocks);
+  net->lpart = (double *)Alloc(sizeof(double) * kHeadBlocks);
   ok = ok && net->lpart;
-  if (ok && hipHostMalloc((void **)&net->lhost, sizeof(double) * kLossBlocks) !=
+  if (ok && hipHostMalloc((void **)&net->lhost, sizeof(double) * kHeadBlocks) !=
                 hipSuccess) {
     (void)hipGetLastError();
     ok = false;
@@ -2078,18 +2182,7 @@ void PSUNetPredict(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
   CheckGrid(net, p, first, count, "p");
   if (p->type != PS_FLOAT && p->type != PS_DOUBLE)
     PS_FATAL("U-Net: p must be a float or double grid");
-  Forward(net, rhs, bnd, first, count);
-  const Dims d = DimsOf(net, count);
-  const long off = (long)first * net->nx * net->ny * net->nzs;
-  if (p->type == PS_DOUBLE)
-    hipLaunchKernelGGL(PredictKernel<double>, dim3(Blocks(d.P1)), dim3(256), 0,
-                       Stream(), net->out, (const float *)bnd->p,
-                       (double *)p->p, off, net->out_scale, d.P1);
-  else
-    hipLaunchKernelGGL(PredictKernel<float>, dim3(Blocks(d.P1)), dim3(256), 0,
-                       Stream(), net->out, (const float *)bnd->p,
-                       (float *)p->p, off, net->out_scale, d.P1);
-  Check();
+  Forward(net, rhs, bnd, first, count, p);
   PS_HIP_CHECK(hipStreamSynchronize(Stream()));
 }
 
@@ -2117,8 +2210,8 @@ void PSUNetReflect(const __PSGrid *src, int first, int count, __PSGrid *dst,
 double PSUNetLossGrad(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
                       const __PSGrid *target, int first, int count,
                       float *grad_host) {
-  Forward(net, rhs, bnd, first, count);
-  const double loss = Backward(net, target, first, count);
+  Forward(net, rhs, bnd, first, count, nullptr);
+  const double loss = Backward(net, rhs, bnd, target, first, count);
   if (grad_host)
     PS_HIP_CHECK(hipMemcpy(grad_host, net->grad, sizeof(float) * net->nparams,
                            hipMemcpyDeviceToHost));
@@ -2135,8 +2228,8 @@ void PSUNetSetLossWeights(__PSUNet *net, float w4, float w16) {
 double PSUNetTrainStep(__PSUNet *net, const __PSGrid *rhs,
                        const __PSGrid *bnd, const __PSGrid *target, int first,
                        int count, float lr) {
-  Forward(net, rhs, bnd, first, count);
-  const double loss = Backward(net, target, first, count);
+  Forward(net, rhs, bnd, first, count, nullptr);
+  const double loss = Backward(net, rhs, bnd, target, first, count);
   net->step += 1;
   const float c1 = 1.0f - std::pow(0.9f, (float)net->step);
   const float c2 = 1.0f - std::pow(0.999f, (float)net->step);
@@ -2170,7 +2263,7 @@ void PSConv3dForwardHost(const uint16_t *x, const uint16_t *w,
                      cout);
   Check();
   Conv(cin, cout, (const u16 *)dx.p, (const u16 *)dwt.p, (const float *)db.p,
-       relu != 0, (u16 *)dy.p, n, d, h, wd);
+       relu != 0, nullptr, (u16 *)dy.p, n, d, h, wd);
   PS_HIP_CHECK(hipStreamSynchronize(Stream()));
   PS_HIP_CHECK(hipMemcpy(y, dy.p, P * cout * 2, hipMemcpyDeviceToHost));
 }
@@ -2196,7 +2289,7 @@ void PSConv3dBackwardDataHost(const uint16_t *dy, const uint16_t *w, int n,
                      cout);
   Check();
   Conv(cout, cin, (const u16 *)ddy.p, (const u16 *)dwf.p, nullptr, false,
-       (u16 *)ddx.p, n, d, h, wd);
+       nullptr, (u16 *)ddx.p, n, d, h, wd);
   PS_HIP_CHECK(hipStreamSynchronize(Stream()));
   PS_HIP_CHECK(hipMemcpy(dx, ddx.p, P * cin * 2, hipMemcpyDeviceToHost));
 }
