@@ -6,16 +6,15 @@
 // MFMA lane feeds are one 16-byte load.
 //
 // 3x3x3 convolution as an implicit GEMM on v_mfma_f32_16x16x32_bf16:
-//   forward   D[16 x-positions][16 cout] += A[16 pos][32 k] B[32 k][16 cout],
-//             k = tap * CIN + ci, A read from an LDS-staged input tile with
-//             zero padding, B the weights stored [cout][k] (K padded to 32);
+//   forward   D[16 cout][16 x] += W[16 cout][32 k] X[32 k][16 x], k = tap *
+//             CIN + ci, X read from LDS-staged input planes with zero
+//             padding, W the weights stored [cout][k] (K padded to 32);
 //   backward  dX = the forward kernel on dZ with the flipped, transposed
 //             weights Wf[ci][tap' * COUT + co] = W[co][26 - tap'][ci];
 //   filter    dW[co][k] = sum over positions of dZ[p][co] X[p + off(k)][ci]:
-//             GEMM with the positions as K, split over blocks of up to
-//             16384 positions into FP32 partials summed in block order
-//             (deterministic); both operands staged transposed in LDS for
-//             rows of a multiple of 32 positions.
+//             GEMM with the positions as K, FP32 partials per block summed in
+//             a fixed order (deterministic); both operands read transposed
+//             from LDS.
 // MFMA lane layout (checked on the device against a host product): lane l
 // feeds A row l%16 and B column l%16 with k = 8*(l/16) .. +7, and receives
 // D rows 4*(l/16) .. +3 of column l%16.
@@ -40,8 +39,9 @@ namespace physis_unet {
 typedef unsigned short u16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kWgradChunk = 16384;  // max positions per filter-gradient block
 constexpr int kPool = 4;           // pooling / upsampling factor per axis
 // Weight fragments (K steps x 16-channel tiles) that the z-marching
 // convolution keeps in registers; more are staged in LDS.  21 covers the
@@ -375,10 +375,10 @@ struct ConcatSrc {
   }
 };
 // The network input: channels (rhs, bnd) rounded to BF16 from the float
-// grids, two channels (CIN = 2) per position.
+// grids; with CIN = 4 two more per position, which are not written.
 template <int CIN, int RS, int XS, int NTH>
 struct InputSrc {
-  static_assert(CIN == 2, "rhs and bnd");
+  static_assert(CIN == 2 || CIN == 4, "rhs and bnd");
   static constexpr int SV = RS * XS, VPT = (SV + NTH - 1) / NTH;
   int off[VPT];
   float r[VPT], m[VPT];
@@ -415,8 +415,7 @@ struct InputSrc {
     for (int i = 0; i < VPT; ++i) {
       const int v = threadIdx.x + i * NTH;
       if (v < SV)
-        *reinterpret_cast<unsigned *>(plane + v * 2) =
-            (unsigned)F2Bf(r[i]) | ((unsigned)F2Bf(m[i]) << 16);
+        *reinterpret_cast<unsigned *>(plane + v * CIN) = Pack2(r[i], m[i]);
     }
   }
 };
@@ -454,7 +453,10 @@ struct EpiArgs {
 // 16 .. 23 of both.  With 2 input channels k = (4 ry + dx) 2 + ci, one K step.
 // The kernel it replaces held a ring of planes and read every B operand
 // three times: LDS reads bounded it (24 -> 8 at 8 x 128^3: 184 us of LDS
-// time in 396 us).
+// time in 396 us, now 245 with the concatenation read in place, which was
+// another 240; 8 -> 8 172 -> 105).  The 8-channel layers run near what their
+// bytes take (92 us at the rate of a copy, 140 gated), the 24-channel ones
+// are bound by latency at two waves per SIMD (92 us of MFMA).
 template <int CIN, int COUT, bool RELU, int XT, int TY,
           template <int, int, int, int> class SRC, int EPI,
           typename PT = double>
@@ -711,171 +713,141 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
 
 // Filter gradient partials marching the input planes: block (x tile, y
 // tile, problem, z chunk [zb, ze) of output-gradient planes) sums over its
-// XT x TY x zchunk positions
+// XT x ROWS x zchunk positions
 //   part[block][co][k] = sum_p dz[p][co] x[p + off(k)][ci],  k = tap CIN + ci
-// as a GEMM over positions (K) on v_mfma_f32_16x16x32_bf16.  Step z' stages
-// input plane z' (transposed, xT[row][ci][x], 3 slots) and uses it for the
-// three taps whose z offset t - 1 maps it to output-gradient plane
-// z' + 1 - t (t = 0, 1, 2; planes outside [zb, ze) stage as zeros, dzT
-// [co][y][x] in a ring of 4).  B = the shifted input (8 consecutive x of
-// one channel at one (dy, dx) offset: column (3 dy + dx) CIN + ci, read as
-// 32-bit words with a funnel shift for odd offsets) is read once per step
-// and feeds every t: the A operand's rows pack (t, co) pairs, row
-// q = t COUT + co, so COUT = 8 needs 2 MFMAs per B operand (the tap-major
-// order needed 3, each half empty, and read B three times).  Waves split
-// into WT groups over column tiles and TY / WT groups over the 32-position
-// steps of a plane; the step groups' sums are added in a fixed order at
-// the end (deterministic).  One barrier per step.
-template <int CIN, int COUT, int XT, int TY, int WT>
-__global__ __launch_bounds__(64 * TY) void WgradZKernel(
-    const u16 *__restrict__ x, const u16 *__restrict__ dz,
-    float *__restrict__ part, float *__restrict__ bpart, int D, int H, int W,
-    int tz, int zchunk) {
+// as a GEMM over positions (K) on v_mfma_f32_16x16x32_bf16.  Step z' uses
+// input plane z' (2 slots) for the three taps whose z offset t - 1 maps it
+// to output-gradient plane z' + 1 - t (t = 0, 1, 2; planes outside [zb, ze)
+// stage as zeros, ring of 4).  Both are staged channels-last, as they lie in
+// memory, and the transposing LDS read (ds_read_b64_tr_b16: four positions of
+// 16 channels per 16 lanes, each lane's address its own) makes the operands:
+// the shift of a tap is an address, and 16 columns may be any four runs of
+// four channels.  B columns (3 dy + dx) CIN + ci, then a column of ones (the
+// bias gradient); A rows (t, co), q = t COUT + co, so that one B operand
+// feeds every t.  CIN is the staged channel count: 4 for the network input
+// (2 of them real), whose other weights of WC = 8 get zero gradients.
+// Waves split into WT groups over column tiles and NW / WT over the steps of
+// 32 positions of a plane; the step groups' sums are added in a fixed order
+// at the end (deterministic).  One barrier per step.
+// The version it replaces stored both operands transposed, 2 bytes at a time,
+// and shifted B by register: at 8 x 128^3 24 -> 8 took 471 us, now 249, and
+// 8 -> 8 207, now 122 (92 us of bytes); rows that are not multiples of 32 ran
+// on a kernel that gathered its operands 2 bytes at a time.
+__device__ __forceinline__ bf16x8 ReadTr(const u16 *a, const u16 *b) {
+  typedef __attribute__((address_space(3))) s16x4 *P;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)a);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)b);
+  return __builtin_bit_cast(
+      bf16x8, s16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+}
+
+template <int CIN, int WC, int COUT, int XT, int ROWS, int NW, int WT,
+          template <int, int, int, int> class SRC>
+__global__ __launch_bounds__(64 * NW) void WgradZKernel(
+    SrcArgs src, const u16 *__restrict__ dz, float *__restrict__ part,
+    float *__restrict__ bpart, int D, int H, int W, int tz, int zchunk) {
   static_assert(XT % 32 == 0, "steps of 32 positions along x");
-  static_assert(TY % WT == 0, "wave groups");
-  constexpr int K = 27 * CIN, NC = 9 * CIN;
-  constexpr int NTN = (NC + 15) / 16;       // column tiles
+  static_assert(NW % WT == 0, "wave groups");
+  constexpr int K = 27 * WC, NC = 9 * CIN;
+  constexpr int NTN = (NC + 16) / 16;       // column tiles (with the ones)
   constexpr int MM = (3 * COUT + 15) / 16;  // MFMAs per B operand
-  constexpr int WS = TY / WT;               // step groups
+  constexpr int WS = NW / WT;               // step groups
   constexpr int TPW = (NTN + WT - 1) / WT;  // column tiles per wave
-  constexpr int NSTEP = TY * XT / 32;       // 32-position steps per plane
+  constexpr int NSTEP = ROWS * XT / 32;     // 32-position steps per plane
   static_assert(NSTEP % WS == 0, "steps split evenly");
-  constexpr int XR = XT + 2, RS = TY + 2;
-  constexpr int RW = CIN * XR / 2;          // 32-bit words per staged row
-  constexpr int PW = RS * RW;               // words per staged plane
-  constexpr int NTH = 64 * TY;
-  constexpr int XV = RS * XR * (CIN / 8);   // 16-byte input vectors per plane
-  constexpr int XVT = (XV + NTH - 1) / NTH;
-  constexpr int DROW = TY * XT + 8;         // dzT row (one channel), padded
-  constexpr int DPL = COUT * DROW;          // u16 per staged dz plane
-  constexpr int DV = TY * XT * (COUT / 8);  // 16-byte dz vectors per plane
-  constexpr int DVT = (DV + NTH - 1) / NTH;
-  constexpr int LOOP_WORDS = 3 * PW + 4 + 4 * DPL / 2;
-  constexpr int RED_WORDS = (WS - 1) * WT * (TPW * MM * 4 + MM) * 64;
+  constexpr int XR = XT + 2, RS = ROWS + 2, NTH = 64 * NW;
+  constexpr int XPL = RS * XR * CIN;        // u16 per staged x plane
+  constexpr int DPL = ROWS * XT * COUT;     // u16 per staged dz plane
+  constexpr int DV = DPL / 8, DVT = (DV + NTH - 1) / NTH;
+  constexpr int LOOP_WORDS = (2 * XPL + 4 * DPL) / 2;
+  constexpr int RED_WORDS = (WS - 1) * WT * TPW * MM * 4 * 64;
   constexpr int LDS_WORDS = LOOP_WORDS > RED_WORDS ? LOOP_WORDS : RED_WORDS;
-  static_assert(XR % 2 == 0 && DROW % 8 == 0, "alignment");
   __shared__ __attribute__((aligned(16))) unsigned lds[LDS_WORDS];
-  unsigned *const xT = lds;
-  u16 *const dzT = reinterpret_cast<u16 *>(lds + 3 * PW + 4);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  u16 *const xs = reinterpret_cast<u16 *>(lds);
+  u16 *const ds = xs + 2 * XPL;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wt = wv % WT, ws = wv / WT;
   const int g = lane >> 4, r = lane & 15;
-  const int tiles_x = (W + XT - 1) / XT;
-  const int x0 = (blockIdx.x % tiles_x) * XT, y0 = (blockIdx.x / tiles_x) * TY;
-  const int n = blockIdx.y / tz;
-  const int zb = (blockIdx.y - n * tz) * zchunk;
+  const int tiles_x = (W + XT - 1) / XT, tiles_y = (H + ROWS - 1) / ROWS;
+  const long bid = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  int b = (int)bid;
+  const int x0 = (b % tiles_x) * XT;
+  b /= tiles_x;
+  const int y0 = (b % tiles_y) * ROWS;
+  b /= tiles_y;
+  const int n = b / tz, zb = (b - n * tz) * zchunk;
   const int ze = min(zb + zchunk, D);
-  const long bid = (long)blockIdx.y * gridDim.x + blockIdx.x;
-  // element offset (within a staged plane) of each tile column's (dy, ci,
-  // dx) origin; -1 past the last column
-  int lofs[TPW];
+  // What this lane addresses in a transposing read: position 8g + (r >> 2)
+  // (+ 4 in the second half) of the step, and four columns from 4 (r & 3).
+  const int pos = 8 * g + (r >> 2), c4 = 4 * (r & 3);
+  int lofs[TPW];  // element offset of (step position 0, the lane's columns)
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
-    const int col = (wt + WT * i) * 16 + r;
-    if (col < NC) {
-      const int o = col / CIN, ci = col - o * CIN;
-      lofs[i] = ((o / 3) * CIN + ci) * XR + o % 3;
-    } else {
-      lofs[i] = -1;
-    }
+    int col = (wt + WT * i) * 16 + c4;
+    col = col < NC ? col : 0;  // (columns past the last are not used)
+    const int o = col / CIN, ci = col - o * CIN;
+    lofs[i] = ((o / 3) * XR + o % 3 + pos) * CIN + ci;
   }
-  // A rows of this lane: q = 16 m + r -> (t, co); t = 3 means none
-  int at[MM], aco[MM];
+  int at[MM], aofs[MM];  // z tap and offset of the lane's A rows
 #pragma unroll
   for (int m = 0; m < MM; ++m) {
-    const int q = 16 * m + r;
-    at[m] = q < 3 * COUT ? q / COUT : 3;
-    aco[m] = q < 3 * COUT ? q % COUT : 0;
+    const int q = 16 * m + c4;
+    at[m] = q < 3 * COUT ? q / COUT : 2;  // (rows past the last: not used)
+    aofs[m] = pos * COUT + q % COUT;
   }
   f32x4 acc[TPW][MM];
 #pragma unroll
   for (int i = 0; i < TPW; ++i)
 #pragma unroll
     for (int m = 0; m < MM; ++m) acc[i][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float bsum[MM];  // dz sums of the t = 1 rows (bias gradient)
-#pragma unroll
-  for (int m = 0; m < MM; ++m) bsum[m] = 0.0f;
-  // input plane zz, rows y0-1 .. y0+TY, x0-1 .. x0+XT
-  auto fetchx = [&](int zz, uint4 (&buf)[XVT]) {
-#pragma unroll
-    for (int i = 0; i < XVT; ++i) {
-      const int v = threadIdx.x + i * NTH;
-      const int c8 = v % (CIN / 8), t = v / (CIN / 8);
-      const int xp = t % XR, row = t / XR;
-      const int yy = y0 - 1 + row, xx = x0 - 1 + xp;
-      uint4 u = make_uint4(0, 0, 0, 0);
-      if (v < XV && zz >= 0 && zz < D && yy >= 0 && yy < H && xx >= 0 &&
-          xx < W)
-        u = *reinterpret_cast<const uint4 *>(
-            x + ((((long)n * D + zz) * H + yy) * W + xx) * CIN + c8 * 8);
-      buf[i] = u;
-    }
-  };
-  // transposed into slot `slot` of xT: [row][ci][x] (16-bit elements)
-  auto putx = [&](int slot, const uint4 (&buf)[XVT]) {
-    u16 *base = reinterpret_cast<u16 *>(xT + slot * PW);
-#pragma unroll
-    for (int i = 0; i < XVT; ++i) {
-      const int v = threadIdx.x + i * NTH;
-      if (v >= XV) continue;
-      const int c8 = v % (CIN / 8), t = v / (CIN / 8);
-      const int xp = t % XR, row = t / XR;
-      const unsigned w4[4] = {buf[i].x, buf[i].y, buf[i].z, buf[i].w};
-      u16 *dst = base + (row * CIN + c8 * 8) * XR + xp;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        dst[(2 * j) * XR] = (u16)(w4[j] & 0xffffu);
-        dst[(2 * j + 1) * XR] = (u16)(w4[j] >> 16);
-      }
-    }
-  };
-  // output-gradient plane zz (zeros outside [zb, ze))
-  auto fetchd = [&](int zz, uint4 (&buf)[DVT]) {
-#pragma unroll
-    for (int i = 0; i < DVT; ++i) {
-      const int v = threadIdx.x + i * NTH;
-      const int c8 = v % (COUT / 8), t = v / (COUT / 8);
-      const int xp = t % XT, row = t / XT;
-      const int yy = y0 + row, xx = x0 + xp;
-      uint4 u = make_uint4(0, 0, 0, 0);
-      if (v < DV && zz >= zb && zz < ze && yy < H && xx < W)
-        u = *reinterpret_cast<const uint4 *>(
-            dz + ((((long)n * D + zz) * H + yy) * W + xx) * COUT + c8 * 8);
-      buf[i] = u;
-    }
-  };
-  auto putd = [&](int slot, const uint4 (&buf)[DVT]) {
-    u16 *base = dzT + slot * DPL;
-#pragma unroll
-    for (int i = 0; i < DVT; ++i) {
-      const int v = threadIdx.x + i * NTH;
-      if (v >= DV) continue;
-      const int c8 = v % (COUT / 8), t = v / (COUT / 8);
-      const unsigned w4[4] = {buf[i].x, buf[i].y, buf[i].z, buf[i].w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        base[(c8 * 8 + 2 * j) * DROW + t] = (u16)(w4[j] & 0xffffu);
-        base[(c8 * 8 + 2 * j + 1) * DROW + t] = (u16)(w4[j] >> 16);
-      }
-    }
-  };
   if (zb < ze) {
-    // x plane zz in slot (zz - zb + 1) % 3, dz plane zz in (zz - zb + 2) & 3
-    uint4 bx[XVT], bd[DVT];
-    fetchx(zb - 1, bx);
-    putx(0, bx);
+    SRC<CIN, RS, XR, NTH> in;
+    in.Init(y0, x0, H, W);
+    // output-gradient plane zz (zeros outside [zb, ze))
+    uint4 bd[DVT];
+    int doff[DVT];
+#pragma unroll
+    for (int i = 0; i < DVT; ++i) {
+      const int v = threadIdx.x + i * NTH, t = v / (COUT / 8);
+      const int yy = y0 + t / XT, xx = x0 + t % XT;
+      doff[i] = v < DV && yy < H && xx < W
+                    ? ((yy * W + xx) * COUT + v % (COUT / 8) * 8) * 2
+                    : kOutside;
+    }
+    auto fetchd = [&](int zz) {
+      const bool ok = zz >= zb && zz < ze;
+      const int plane = H * W * COUT;
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<u16 *>(dz) + (ok ? ((long)n * D + zz) * plane : 0), 0,
+          ok ? plane * 2 : 0, physis_hip::kBufDword3);
+#pragma unroll
+      for (int i = 0; i < DVT; ++i)
+        bd[i] = __builtin_bit_cast(
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, doff[i], 0, 0));
+    };
+    auto putd = [&](int slot) {
+#pragma unroll
+      for (int i = 0; i < DVT; ++i) {
+        const int v = threadIdx.x + i * NTH;
+        if (v < DV)
+          *reinterpret_cast<uint4 *>(ds + slot * DPL + v * 8) = bd[i];
+      }
+    };
+    // x plane zz in slot (zz - zb + 1) & 1, dz plane zz in (zz - zb + 2) & 3
+    in.Fetch(src, n, zb - 1, D, H, W);
+    in.Put(xs);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      fetchd(zb - 2 + k, bd);
-      putd(k, bd);
+      fetchd(zb - 2 + k);
+      putd(k);
     }
-    fetchx(zb, bx);
-    fetchd(zb + 1, bd);
+    in.Fetch(src, n, zb, D, H, W);
+    fetchd(zb + 1);
     __syncthreads();
     for (int zp = zb - 1; zp <= ze; ++zp) {
-      const int xs = (zp - zb + 1) % 3;
-      const int dbase = zp - zb + 3;  // dz slot of t is (dbase - t) & 3
-      const unsigned *xplane = xT + xs * PW;
+      const int k = zp - zb + 1;  // dz plane zp + 1 - t in slot (k + 2 - t) & 3
+      const u16 *const xp = xs + (k & 1) * XPL;
 #pragma unroll
       for (int j = 0; j < NSTEP / WS; ++j) {
         const int st = (ws * (NSTEP / WS) + j) * 32;  // first position
@@ -883,57 +855,40 @@ __global__ __launch_bounds__(64 * TY) void WgradZKernel(
         bf16x8 a[MM];
 #pragma unroll
         for (int m = 0; m < MM; ++m) {
-          a[m] = at[m] < 3
-                     ? *reinterpret_cast<const bf16x8 *>(
-                           dzT + ((dbase - at[m]) & 3) * DPL + aco[m] * DROW +
-                           st + 8 * g)
-                     : Zero8();
-          if (wt == 0 && at[m] == 1) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) bsum[m] += (float)a[m][e];
-          }
+          const u16 *p =
+              ds + ((k + 2 - at[m]) & 3) * DPL + st * COUT + aofs[m];
+          a[m] = ReadTr(p, p + 4 * COUT);
         }
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
           if (wt + WT * i >= NTN) break;  // wave-uniform
-          bf16x8 b = Zero8();
-          if (lofs[i] >= 0) {
-            const int e = lofs[i] + ry * CIN * XR + rx + 8 * g;
-            const unsigned *wsrc = xplane + (e >> 1);
-            unsigned w[5];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) w[k] = wsrc[k];
-            uint4 o;
-            if (e & 1)
-              o = make_uint4(__builtin_amdgcn_alignbit(w[1], w[0], 16),
-                             __builtin_amdgcn_alignbit(w[2], w[1], 16),
-                             __builtin_amdgcn_alignbit(w[3], w[2], 16),
-                             __builtin_amdgcn_alignbit(w[4], w[3], 16));
-            else
-              o = make_uint4(w[0], w[1], w[2], w[3]);
-            b = __builtin_bit_cast(bf16x8, o);
-          }
+          const u16 *p = xp + (ry * XR + rx) * CIN + lofs[i];
+          bf16x8 o = ReadTr(p, p + 4 * CIN);
+          if (wt + WT * i == NC / 16 && r == NC % 16)  // the column of ones
+            o = __builtin_bit_cast(
+                bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u,
+                                   0x3f803f80u));
 #pragma unroll
           for (int m = 0; m < MM; ++m)
-            acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b,
+            acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], o,
                                                                 acc[i][m], 0,
                                                                 0, 0);
         }
       }
       // x plane zp + 1 and dz plane zp + 2 into the slots no wave reads in
-      // this step (x: plane zp - 2, dz: plane zp - 2)
-      putx((zp - zb + 2) % 3, bx);
-      putd((zp - zb + 4) & 3, bd);
+      // this step (x: plane zp - 1, dz: plane zp - 2)
+      in.Put(xs + ((k + 1) & 1) * XPL);
+      putd((k + 3) & 3);
       __syncthreads();
-      fetchx(zp + 2, bx);
-      fetchd(zp + 3, bd);
+      in.Fetch(src, n, zp + 2, D, H, W);
+      fetchd(zp + 3);
     }
   }
   // step groups 1 .. WS-1 hand their sums to group 0 through LDS
   if constexpr (WS > 1) {
     __syncthreads();  // the staged planes are no longer read
     float *red = reinterpret_cast<float *>(lds);
-    constexpr int PER = TPW * MM * 4 + MM;  // floats per lane and wave
+    constexpr int PER = TPW * MM * 4;  // floats per lane and wave
     if (ws > 0) {
       float *o = red + ((ws - 1) * WT + wt) * PER * 64;
 #pragma unroll
@@ -943,8 +898,6 @@ __global__ __launch_bounds__(64 * TY) void WgradZKernel(
 #pragma unroll
           for (int v = 0; v < 4; ++v)
             o[((i * MM + m) * 4 + v) * 64 + lane] = acc[i][m][v];
-#pragma unroll
-      for (int m = 0; m < MM; ++m) o[(TPW * MM * 4 + m) * 64 + lane] = bsum[m];
     }
     __syncthreads();
     if (ws == 0) {
@@ -957,9 +910,6 @@ __global__ __launch_bounds__(64 * TY) void WgradZKernel(
 #pragma unroll
             for (int v = 0; v < 4; ++v)
               acc[i][m][v] += o[((i * MM + m) * 4 + v) * 64 + lane];
-#pragma unroll
-        for (int m = 0; m < MM; ++m)
-          bsum[m] += o[(TPW * MM * 4 + m) * 64 + lane];
       }
     }
   }
@@ -967,7 +917,8 @@ __global__ __launch_bounds__(64 * TY) void WgradZKernel(
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
       const int col = (wt + WT * i) * 16 + r;
-      if (wt + WT * i >= NTN || col >= NC) continue;
+      if (wt + WT * i >= NTN || col > NC) continue;
+      const int o = col / CIN, ci = col - o * CIN;
 #pragma unroll
       for (int m = 0; m < MM; ++m)
 #pragma unroll
@@ -975,143 +926,49 @@ __global__ __launch_bounds__(64 * TY) void WgradZKernel(
           const int q = 16 * m + 4 * g + v;
           if (q >= 3 * COUT) continue;
           const int t = q / COUT, co = q - t * COUT;
-          part[(bid * COUT + co) * K + 9 * t * CIN + col] = acc[i][m][v];
+          if (col == NC) {
+            if (t == 1) bpart[bid * COUT + co] = acc[i][m][v];
+          } else if (CIN == WC) {
+            part[(bid * COUT + co) * K + 9 * t * CIN + col] = acc[i][m][v];
+          } else {  // 2 real channels of WC
+            float *w = part + (bid * COUT + co) * K + (9 * t + o) * WC;
+            w[ci < 2 ? ci : ci * 3 - 4] = ci < 2 ? acc[i][m][v] : 0.0f;
+            if (ci >= 2) w[ci * 3 - 3] = w[ci * 3 - 2] = 0.0f;
+          }
         }
-    }
-    if (wt == 0) {
-      // lanes r of the four groups g hold disjoint positions of row q = 16 m
-      // + r: fold the groups in order
-#pragma unroll
-      for (int m = 0; m < MM; ++m) {
-        float sm = bsum[m];
-        sm += __shfl_xor(sm, 16, 64);
-        sm += __shfl_xor(sm, 32, 64);
-        if (g == 0 && at[m] == 1) bpart[bid * COUT + aco[m]] = sm;
-      }
     }
   }
 }
 
-// Filter gradient partials: block (b, t) covers positions [b*chunk,
-// (b+1)*chunk) and column tiles 4t .. 4t+3 of k (one per wave) and writes
-// part[b][co][k]; blocks (b, 0) also write bpart[b][co].  A lane decodes its
-// first position of a 32-position step once and walks the next 7
-// incrementally.
-template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void WgradKernel(
-    const u16 *__restrict__ x, const u16 *__restrict__ dz,
-    float *__restrict__ part, float *__restrict__ bpart, int P, int D, int H,
-    int W, int chunk) {
-  constexpr int K = 27 * CIN, NTN = (K + 15) / 16, MT = (COUT + 15) / 16;
+// Deterministic sums over blocks: out[i] = sum_b part[b][i] for i < n, and
+// out2[i] = sum_b part2[b][i] for i < n2.  A block owns 64 columns; its 16
+// waves sum an equal run of the blocks each, in order, then the runs are
+// added in order.
+constexpr int kSumWaves = 16;
+__global__ __launch_bounds__(64 * kSumWaves) void SumPartsKernel(
+    const float *__restrict__ part, long n, float *__restrict__ out,
+    const float *__restrict__ part2, long n2, float *__restrict__ out2,
+    int nparts) {
+  __shared__ float red[kSumWaves][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int g = lane >> 4, r = lane & 15;
-  const int p0 = blockIdx.x * chunk;
-  const int p1 = p0 + chunk < P ? p0 + chunk : P;
-  const int nt = blockIdx.y * 4 + wv;
-  if (nt < NTN) {
-    f32x4 acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int col = nt * 16 + r;
-    const bool colv = col < K;
-    const int tap = colv ? col / CIN : 0, ci = colv ? col - tap * CIN : 0;
-    const int dzo = tap / 9 - 1, dyo = (tap / 3) % 3 - 1, dxo = tap % 3 - 1;
-    for (int kp = p0; kp < p1; kp += 32) {
-      bf16x8 b = Zero8();
-      bf16x8 a[MT];
-#pragma unroll
-      for (int m = 0; m < MT; ++m) a[m] = Zero8();
-      const int pb = kp + 8 * g;
-      int q = pb;
-      int xx = q % W;
-      q /= W;
-      int yy = q % H;
-      q /= H;
-      int zz = q % D;
-      int nn = q / D;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int pos = pb + j;
-        if (pos < p1) {
-          const int xs = xx + dxo, ys = yy + dyo, zs = zz + dzo;
-          if (colv && xs >= 0 && xs < W && ys >= 0 && ys < H && zs >= 0 &&
-              zs < D)
-            b[j] = __builtin_bit_cast(
-                __bf16, x[((long)((nn * D + zs) * H + ys) * W + xs) * CIN + ci]);
-#pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            const int co = m * 16 + r;
-            if (co < COUT)
-              a[m][j] = __builtin_bit_cast(__bf16, dz[(long)pos * COUT + co]);
-          }
-        }
-        if (++xx == W) {
-          xx = 0;
-          if (++yy == H) {
-            yy = 0;
-            if (++zz == D) {
-              zz = 0;
-              ++nn;
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b, acc[m], 0, 0, 0);
-    }
-    if (colv) {
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int co = m * 16 + 4 * g + v;
-          if (co < COUT)
-            part[((long)blockIdx.x * COUT + co) * K + col] = acc[m][v];
-        }
-    }
-  }
-  // bias (blocks of the first tile group): thread t sums channel t % COUT
-  // over every (256 / COUT)-th position, then the partial sums of each
-  // channel are added in order
-  if (blockIdx.y != 0) return;
-  constexpr int kLanes = 256 / COUT;
-  __shared__ float red[256];
+  const long nb = (n + 63) / 64;  // blocks of the first sum
+  const bool second = (long)blockIdx.x >= nb;
+  const float *p = second ? part2 : part;
+  const long m = second ? n2 : n;
+  const long i = ((long)blockIdx.x - (second ? nb : 0)) * 64 + lane;
+  const int run = (nparts + kSumWaves - 1) / kSumWaves;
+  const int b0 = wv * run, b1 = b0 + run < nparts ? b0 + run : nparts;
   float s = 0.0f;
-  const int c = threadIdx.x % COUT, lid = threadIdx.x / COUT;
-  if (lid < kLanes)
-    for (int p = p0 + lid; p < p1; p += kLanes)
-      s += Bf2F(dz[(long)p * COUT + c]);
-  red[threadIdx.x] = s;
+  if (i < m) {
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) s += p[b * m + i];
+  }
+  red[wv][lane] = s;
   __syncthreads();
-  if (threadIdx.x < COUT) {
-    float t = 0.0f;
-    for (int i = 0; i < kLanes; ++i) t += red[threadIdx.x + COUT * i];
-    bpart[(long)blockIdx.x * COUT + threadIdx.x] = t;
+  if (wv == 0 && i < m) {
+    for (int k = 1; k < kSumWaves; ++k) s += red[k][lane];
+    (second ? out2 : out)[i] = s;
   }
-}
-
-// Deterministic sum over blocks of part[b][i]: stage 1 sums segment s of
-// the blocks in order into tmp[s][i], stage 2 sums the segments in order.
-__global__ void SumSegmentsKernel(const float *__restrict__ part, int nparts,
-                                  long stride, int seglen,
-                                  float *__restrict__ tmp, long n) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int b0 = blockIdx.y * seglen;
-  const int b1 = b0 + seglen < nparts ? b0 + seglen : nparts;
-  float s = 0.0f;
-  for (int b = b0; b < b1; ++b) s += part[b * stride + i];
-  tmp[blockIdx.y * n + i] = s;
-}
-
-__global__ void SumPartsKernel(const float *__restrict__ part, int nparts,
-                               long stride, float *__restrict__ out, long n) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.0f;
-  for (int b = 0; b < nparts; ++b) s += part[b * stride + i];
-  out[i] = s;
 }
 
 // ------------------------------------------------------ elementwise layers
@@ -1258,17 +1115,6 @@ __global__ void PoolBackSkipGateKernel(const u16 *__restrict__ gpool,
   for (int k = 0; k < 8; ++k)
     o.v[k] = a.v[k] > 0.0f ? gp.v[k] * (1.0f / 64.0f) + gs.v[k] : 0.0f;
   Store8F(dz + (long)i * 8, o);
-}
-
-// Network input: ch0 = rhs, ch1 = bnd, ch2..7 = 0 (problems [first, ...)).
-__global__ void InputKernel(const float *__restrict__ rhs,
-                            const float *__restrict__ bnd,
-                            u16 *__restrict__ x, long off, long P) {
-  const long p = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (p >= P) return;
-  uint4 v = make_uint4(0, 0, 0, 0);
-  v.x = (unsigned)F2Bf(rhs[off + p]) | ((unsigned)F2Bf(bnd[off + p]) << 16);
-  *reinterpret_cast<uint4 *>(x + p * 8) = v;
 }
 
 // 1x1 convolution 8 -> 1: out[p] = sum_c w[c] in[p][c] + b (FP32), for the
@@ -1467,10 +1313,8 @@ hipStream_t Stream() { return (hipStream_t)__PSHipStream(); }
 void Check() { PS_HIP_CHECK(hipGetLastError()); }
 unsigned Blocks(long n, int t = 256) { return (unsigned)((n + t - 1) / t); }
 
-// Blocks per compute unit that the z-marching launches aim for (measured
-// at level 1 of batch 8 x 128^3: the plane-marching filter gradient is
-// fastest with 2, e.g. 8 -> 8 213 us against 223 with 4 and 237 with 8,
-// and so are the convolutions).
+// Blocks per compute unit that the ring convolutions and the filter gradient
+// aim for: what their registers and LDS let reside at level 1.
 constexpr int kConvZBlocksPerCU = 2;
 constexpr int kWgradZBlocksPerCU = 2;
 
@@ -1579,32 +1423,22 @@ void ConvT(const u16 *x, const u16 *wt, const float *b, bool relu,
   }
 }
 
-// Positions per filter-gradient block: about P / 512 (a multiple of 32),
-// between 256 and kWgradChunk, so that small levels still spread over many
-// blocks.
-int WgradChunk(long P) {
-  long c = ((P / 512 + 31) / 32) * 32;
-  if (c < 256) c = 256;
-  if (c > kWgradChunk) c = kWgradChunk;
-  return (int)c;
-}
-
-// Launch shape of the z-marching filter gradient (rows of a multiple of 32
-// positions): x tile 64 when the row allows it and the input has at most
-// 24 channels (24 -> 8 at level 1: 479 us against 526 with 32), else 32;
-// 4 rows per block; z chunks as the convolution.
+// Launch shape of the filter gradient: x tile 64 when the rows are multiples
+// of 64 and the input has at most 24 channels, else 32 (positions past a
+// row's end stage as zeros).
 // Returns the block count (= partials).
-constexpr int kWgradZRows = 4;
+constexpr int WgradZRows(int cin) { return cin <= 8 ? 8 : 4; }
+constexpr int kWgradZWaves = 4;
 // Wave groups over the column tiles (9 cin / 16 of them): one up to 5
-// tiles, two up to 14, else four (the rest of the 4 waves split the steps).
+// tiles, two up to 14, else four (the rest of the waves split the steps).
 constexpr int WgradZGroups(int cin) {
-  return (9 * cin + 15) / 16 <= 5 ? 1 : ((9 * cin + 15) / 16 <= 14 ? 2 : 4);
+  return (9 * cin + 16) / 16 <= 5 ? 1 : ((9 * cin + 16) / 16 <= 14 ? 2 : 4);
 }
 int WgradZXT(int cin, int W) { return (W % 64 == 0 && cin <= 24) ? 64 : 32; }
 long WgradZBlocks(int cin, int N, int D, int H, int W, int *tz, int *zchunk) {
   const int xt = WgradZXT(cin, W);
   const long tiles = (long)((W + xt - 1) / xt) *
-                     ((H + kWgradZRows - 1) / kWgradZRows);
+                     ((H + WgradZRows(cin) - 1) / WgradZRows(cin));
   ZChunks(tiles, N, D, kWgradZBlocksPerCU, tz, zchunk);
   return tiles * N * *tz;
 }
@@ -1613,69 +1447,51 @@ long WgradZBlocks(int cin, int N, int D, int H, int W, int *tz, int *zchunk) {
 // D x H x W positions with cin input channels: every buffer of partials is
 // sized by this.
 long WgradBlocks(int cin, int N, int D, int H, int W) {
-  if (W % 32 == 0) {
-    int tz, zchunk;
-    return WgradZBlocks(cin, N, D, H, W, &tz, &zchunk);
-  }
-  const long P = (long)N * D * H * W;
-  const long chunk = WgradChunk(P);
-  return (P + chunk - 1) / chunk;
+  int tz, zchunk;
+  return WgradZBlocks(cin, N, D, H, W, &tz, &zchunk);
 }
 
-// Launches the filter gradient into part / bpart, which hold `capacity`
-// blocks of partials; *nparts receives the blocks written.
-template <int CIN, int COUT>
-void WgradT(const u16 *x, const u16 *dz, float *part, float *bpart, int N,
-            int D, int H, int W, long capacity, int *nparts) {
-  constexpr int NTN = (27 * CIN + 15) / 16;
+// The filter gradient of a layer with CIN input channels (SC staged: 4 for the
+// network input) into part / bpart, which hold `capacity` blocks of partials;
+// *nparts receives the blocks written.
+template <int SC, int CIN, int COUT,
+          template <int, int, int, int> class SRC>
+void WgradZLaunch(const SrcArgs &src, const u16 *dz, float *part, float *bpart,
+                  int N, int D, int H, int W, long capacity, int *nparts) {
   const long P = (long)N * D * H * W;
-  if (P >= (1L << 31) - kWgradChunk)
+  if (P >= 1L << 31)
     PS_FATAL("filter gradient: %ld positions exceed 32-bit indexing", P);
-  if (WgradBlocks(CIN, N, D, H, W) > capacity)
+  int tz, zchunk;
+  const long nb = WgradZBlocks(CIN, N, D, H, W, &tz, &zchunk);
+  if (nb > capacity)
     PS_FATAL("filter gradient: %ld partial blocks exceed the %ld allocated",
-             WgradBlocks(CIN, N, D, H, W), capacity);
-  // rows of a multiple of 32 positions: the z-marching kernel
-  if (W % 32 == 0) {
-    int tz, zchunk;
-    const long nb = WgradZBlocks(CIN, N, D, H, W, &tz, &zchunk);
-    const int tiles = (int)(nb / ((long)N * tz));
-    const dim3 grid(tiles, N * tz), block(64 * kWgradZRows);
-    if (WgradZXT(CIN, W) == 64) {
-      if constexpr (CIN <= 24)
-        hipLaunchKernelGGL(
-            (WgradZKernel<CIN, COUT, 64, kWgradZRows, WgradZGroups(CIN)>),
-            grid, block, 0, Stream(), x, dz, part, bpart, D, H, W, tz,
-            zchunk);
-    } else {
-      hipLaunchKernelGGL(
-          (WgradZKernel<CIN, COUT, 32, kWgradZRows, WgradZGroups(CIN)>), grid,
-          block, 0, Stream(), x, dz, part, bpart, D, H, W, tz, zchunk);
-    }
-    Check();
-    *nparts = (int)nb;
-    return;
+             nb, capacity);
+  constexpr int R = WgradZRows(CIN), NW = kWgradZWaves;
+  const dim3 grid((unsigned)nb), block(64 * NW);
+  if (WgradZXT(CIN, W) == 64) {
+    if constexpr (CIN <= 24)
+      hipLaunchKernelGGL((WgradZKernel<SC, CIN, COUT, 64, R, NW,
+                                       WgradZGroups(SC), SRC>),
+                         grid, block, 0, Stream(), src, dz, part, bpart, D, H,
+                         W, tz, zchunk);
+  } else {
+    hipLaunchKernelGGL((WgradZKernel<SC, CIN, COUT, 32, R, NW,
+                                     WgradZGroups(SC), SRC>),
+                       grid, block, 0, Stream(), src, dz, part, bpart, D, H, W,
+                       tz, zchunk);
   }
-  const int chunk = WgradChunk(P);
-  const int nb = (int)((P + chunk - 1) / chunk);
-  hipLaunchKernelGGL((WgradKernel<CIN, COUT>), dim3(nb, (NTN + 3) / 4),
-                     dim3(256), 0, Stream(), x, dz, part, bpart, (int)P, D,
-                     H, W, chunk);
   Check();
-  *nparts = nb;
+  *nparts = (int)nb;
 }
 
-// out[0..n) = sum over nparts blocks of part[b * n + i], via tmp
-// (kSumSegments * n floats).
-constexpr int kSumSegments = 64;
-void SumParts(const float *part, int nparts, long n, float *tmp, float *out) {
-  const int seg = nparts < kSumSegments ? nparts : kSumSegments;
-  const int seglen = (nparts + seg - 1) / seg;
-  const int nseg = (nparts + seglen - 1) / seglen;
-  hipLaunchKernelGGL(SumSegmentsKernel, dim3(Blocks(n), nseg), dim3(256), 0,
-                     Stream(), part, nparts, n, seglen, tmp, n);
-  Check();
-  hipLaunchKernelGGL(SumPartsKernel, dim3(Blocks(n)), dim3(256), 0, Stream(),
-                     tmp, nseg, n, out, n);
+// out = sums of n columns over nparts blocks of part, out2 of n2 columns of
+// part2 (n2 = 0: none).
+void SumParts(const float *part, long n, float *out, const float *part2,
+              long n2, float *out2, int nparts) {
+  hipLaunchKernelGGL(SumPartsKernel,
+                     dim3((unsigned)((n + 63) / 64 + (n2 + 63) / 64)),
+                     dim3(64 * kSumWaves), 0, Stream(), part, n, out, part2,
+                     n2, out2, nparts);
   Check();
 }
 
@@ -1698,7 +1514,8 @@ void Wgrad(int cin, int cout, const u16 *x, const u16 *dz, float *part,
            int *nparts) {
 #define PS_CASE(I, O) \
   if (cin == I && cout == O) \
-    return WgradT<I, O>(x, dz, part, bpart, N, D, H, W, capacity, nparts);
+    return WgradZLaunch<I, I, O, PlainSrc>(SrcArgs{x, nullptr, 0}, dz, part, \
+                                           bpart, N, D, H, W, capacity, nparts);
   PS_UNET_PAIRS(PS_CASE)
 #undef PS_CASE
   PS_FATAL("no filter-gradient kernel for %d -> %d channels", cin, cout);
@@ -1740,14 +1557,13 @@ struct __PSUNet {
         *adam_v = nullptr;
   long step = 0;
   // activations (BF16) at batch max_batch
-  u16 *x0 = nullptr, *a[10] = {}, *q1 = nullptr, *q2 = nullptr,
-      *c2 = nullptr, *c1 = nullptr;
+  u16 *a[10] = {}, *q1 = nullptr, *q2 = nullptr, *c2 = nullptr;
   float *out = nullptr;
   // gradient scratch
   u16 *g1a = nullptr, *g1b = nullptr, *gc1 = nullptr;  // level 1
   u16 *g2a = nullptr, *g2b = nullptr, *gc2 = nullptr;  // level 2
   u16 *g3a = nullptr, *g3b = nullptr;                  // level 3
-  float *part = nullptr, *bpart = nullptr, *tmp = nullptr;
+  float *part = nullptr, *bpart = nullptr;
   double *lpart = nullptr, *lhost = nullptr;
   size_t part_elems = 0, bpart_elems = 0;
   // smooth-error loss weights and the cell means of the error
@@ -1873,17 +1689,35 @@ void Forward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
     ConvPredict<float>(net, bnd, p, off, d.N, d.D1, d.H1, d.W1);
 }
 
+// Blocks of partials that layer l may write.
+long WgradCapacity(const __PSUNet *net, const Layer &L) {
+  return std::min<long>((long)net->part_elems / ((long)L.cout * 27 * L.cin),
+                        (long)net->bpart_elems / L.cout);
+}
+void SumLayer(__PSUNet *net, const Layer &L, int np) {
+  SumParts(net->part, (long)L.cout * 27 * L.cin, net->grad + L.w_off,
+           net->bpart, L.cout, net->grad + L.b_off, np);
+}
+
 // Filter gradient of layer l from input `in` and gated output gradient dz.
 void LayerWgrad(__PSUNet *net, int l, const u16 *in, const u16 *dz, int N,
                 int D, int H, int W) {
   const Layer &L = net->layers[l];
   int np = 0;
-  const long nw = (long)L.cout * 27 * L.cin;
-  const long cap = std::min<long>((long)net->part_elems / nw,
-                                  (long)net->bpart_elems / L.cout);
-  Wgrad(L.cin, L.cout, in, dz, net->part, net->bpart, N, D, H, W, cap, &np);
-  SumParts(net->part, np, nw, net->tmp, net->grad + L.w_off);
-  SumParts(net->bpart, np, (long)L.cout, net->tmp, net->grad + L.b_off);
+  Wgrad(L.cin, L.cout, in, dz, net->part, net->bpart, N, D, H, W,
+        WgradCapacity(net, L), &np);
+  SumLayer(net, L, np);
+}
+
+// The same from a source of its own.
+template <int SC, int CIN, template <int, int, int, int> class SRC>
+void SrcWgrad(__PSUNet *net, int l, const SrcArgs &src, const u16 *dz, int N,
+              int D, int H, int W) {
+  const Layer &L = net->layers[l];
+  int np = 0;
+  WgradZLaunch<SC, CIN, 8, SRC>(src, dz, net->part, net->bpart, N, D, H, W,
+                                WgradCapacity(net, L), &np);
+  SumLayer(net, L, np);
 }
 
 // Data gradient of layer l: dx = conv(dz, flipped W), no bias, no ReLU,
@@ -1903,16 +1737,6 @@ double Backward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
   const Dims d = DimsOf(net, count);
   const long off = (long)first * net->nx * net->ny * net->nzs;
   const float inv_scale = 1.0f / net->out_scale;
-  // the filter gradients read the first layer's input and the level-1
-  // concatenation as tensors
-  hipLaunchKernelGGL(InputKernel, dim3(Blocks(d.P1)), dim3(256), 0, Stream(),
-                     (const float *)rhs->p, (const float *)bnd->p, net->x0,
-                     off, d.P1);
-  Check();
-  hipLaunchKernelGGL(UpConcatKernel, dim3(Blocks(d.P1 * 3)), dim3(256), 0,
-                     Stream(), net->a[7], net->a[1], net->c1, 16, 8, d.D1,
-                     d.H1, d.W1, (int)(d.P1 * 3));
-  Check();
   // head and loss: g1a = gated dD1 (layer 9's dz), partials in part, lpart
   const bool smooth = net->w4 != 0.0f || net->w16 != 0.0f;
   if (smooth) {
@@ -1934,11 +1758,13 @@ double Backward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
                      net->e16, net->w4, net->w16, d.D1, d.H1, d.W1, net->g1a,
                      net->lpart, net->part, d.P1);
   Check();
-  SumParts(net->part, kHeadBlocks, 9L, net->tmp, net->grad + net->head_off);
+  SumParts(net->part, 9, net->grad + net->head_off, nullptr, 0, nullptr,
+           kHeadBlocks);
   // level 1 decoder
   LayerWgrad(net, 9, net->a[8], net->g1a, d.N, d.D1, d.H1, d.W1);
   LayerDgrad(net, 9, net->g1a, net->a[8], net->g1b, d.N, d.D1, d.H1, d.W1);
-  LayerWgrad(net, 8, net->c1, net->g1b, d.N, d.D1, d.H1, d.W1);
+  SrcWgrad<24, 24, ConcatSrc>(net, 8, SrcArgs{net->a[7], net->a[1], 0},
+                              net->g1b, d.N, d.D1, d.H1, d.W1);
   // 24 channels: 16 to the level-2 decoder (summed over the upsampled cells
   // and gated: g2a), 8 to the skip connection (gc1)
   {
@@ -1980,7 +1806,8 @@ double Backward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
   Check();
   LayerWgrad(net, 1, net->a[0], net->g1a, d.N, d.D1, d.H1, d.W1);
   LayerDgrad(net, 1, net->g1a, net->a[0], net->g1b, d.N, d.D1, d.H1, d.W1);
-  LayerWgrad(net, 0, net->x0, net->g1b, d.N, d.D1, d.H1, d.W1);
+  SrcWgrad<4, 8, InputSrc>(net, 0, SrcArgs{rhs->p, bnd->p, off}, net->g1b,
+                           d.N, d.D1, d.H1, d.W1);
   PS_HIP_CHECK(hipMemcpyAsync(net->lhost, net->lpart,
                               sizeof(double) * kHeadBlocks,
                               hipMemcpyDeviceToHost, Stream()));
@@ -1993,11 +1820,11 @@ double Backward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
 void FreeNet(__PSUNet *net) {
   (void)hipStreamSynchronize(Stream());
   std::vector<void *> ptrs = {net->params, net->grad, net->adam_m,
-                              net->adam_v, net->x0, net->q1, net->q2,
-                              net->c2, net->c1, net->out, net->g1a,
+                              net->adam_v, net->q1, net->q2,
+                              net->c2, net->out, net->g1a,
                               net->g1b, net->gc1, net->g2a, net->g2b,
                               net->gc2, net->g3a, net->g3b, net->part,
-                              net->bpart, net->tmp, net->lpart, net->e4,
+                              net->bpart, net->lpart, net->e4,
                               net->e16};
   for (int i = 0; i < 10; ++i) ptrs.push_back(net->a[i]);
   for (auto &L : net->layers) {
@@ -2093,14 +1920,12 @@ __PSUNet *PSUNetNew(int nx, int ny, int nzs, int max_batch, float out_scale,
     L.wt = A16((long)L.cout * KPad(L.cin));
     L.wf = A16((long)L.cin * KPad(L.cout));
   }
-  net->x0 = A16(d.P1 * 8);
   const long act[10] = {d.P1 * 8,  d.P1 * 8,  d.P2 * 16, d.P2 * 16, d.P3 * 32,
                         d.P3 * 32, d.P2 * 16, d.P2 * 16, d.P1 * 8,  d.P1 * 8};
   for (int l = 0; l < 10; ++l) net->a[l] = A16(act[l]);
   net->q1 = A16(d.P2 * 8);
   net->q2 = A16(d.P3 * 16);
   net->c2 = A16(d.P2 * 48);
-  net->c1 = A16(d.P1 * 24);
   net->out = A32(d.P1);
   net->g1a = A16(d.P1 * 8);
   net->g1b = A16(d.P1 * 8);
@@ -2110,7 +1935,7 @@ __PSUNet *PSUNetNew(int nx, int ny, int nzs, int max_batch, float out_scale,
   net->gc2 = A16(d.P2 * 48);
   net->g3a = A16(d.P3 * 32);
   net->g3b = A16(d.P3 * 32);
-  size_t pe = (size_t)kHeadBlocks * 9, be = 0, te = 9;
+  size_t pe = (size_t)kHeadBlocks * 9, be = 0;
   for (int l = 0; l < 10; ++l) {
     const int lv = l < 2 || l > 7 ? 1 : (l < 4 || l > 5 ? 2 : 3);
     const long P = lv == 1 ? d.P1 : (lv == 2 ? d.P2 : d.P3);
@@ -2127,13 +1952,11 @@ __PSUNet *PSUNetNew(int nx, int ny, int nzs, int max_batch, float out_scale,
     const size_t nw = (size_t)net->layers[l].cout * 27 * net->layers[l].cin;
     pe = std::max(pe, nb * nw);
     be = std::max(be, nb * net->layers[l].cout);
-    te = std::max(te, nw);
   }
   net->part_elems = pe;
   net->bpart_elems = be;
   net->part = A32((long)pe);
   net->bpart = A32((long)be);
-  net->tmp = A32((long)(te * kSumSegments));
   net->e4 = A32(d.P2);
   net->e16 = A32(d.P3);
   net->lpart = (double *)Alloc(sizeof(double) * kHeadBlocks);
@@ -2302,17 +2125,14 @@ void PSConv3dBackwardFilterHost(const uint16_t *x, const uint16_t *dy, int n,
   const long nb = WgradBlocks(cin, n, d, h, wd);
   const size_t nw = (size_t)cout * 27 * cin;
   DevBuf ddx(P * cin * 2), ddy(P * cout * 2), part(nb * nw * 4),
-      bpart(nb * cout * 4), dw_d(nw * 4), db_d(cout * 4),
-      tmp(nw * kSumSegments * 4);
+      bpart(nb * cout * 4), dw_d(nw * 4), db_d(cout * 4);
   PS_HIP_CHECK(hipMemcpy(ddx.p, x, P * cin * 2, hipMemcpyHostToDevice));
   PS_HIP_CHECK(hipMemcpy(ddy.p, dy, P * cout * 2, hipMemcpyHostToDevice));
   int np = 0;
   Wgrad(cin, cout, (const u16 *)ddx.p, (const u16 *)ddy.p, (float *)part.p,
         (float *)bpart.p, n, d, h, wd, nb, &np);
-  SumParts((const float *)part.p, np, (long)nw, (float *)tmp.p,
-           (float *)dw_d.p);
-  SumParts((const float *)bpart.p, np, (long)cout, (float *)tmp.p,
-           (float *)db_d.p);
+  SumParts((const float *)part.p, (long)nw, (float *)dw_d.p,
+           (const float *)bpart.p, cout, (float *)db_d.p, np);
   PS_HIP_CHECK(hipStreamSynchronize(Stream()));
   PS_HIP_CHECK(hipMemcpy(dw, dw_d.p, nw * 4, hipMemcpyDeviceToHost));
   PS_HIP_CHECK(hipMemcpy(db, db_d.p, cout * 4, hipMemcpyDeviceToHost));

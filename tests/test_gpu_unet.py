@@ -78,9 +78,9 @@ def test_conv_backward(ps, dims):
     assert np.max(np.abs(db - rdb)) <= 1e-4 * np.max(np.abs(rdb))
 
 
-# Rows of a multiple of 32 positions take the LDS-staged filter-gradient
-# kernel (the widths above take the gathering one): both channel layouts of
-# every level, a batch of two, and several blocks.
+# Filter gradients on rows of whole 32-position steps (the widths above leave
+# part of the last step empty): both channel layouts of every level, a batch
+# of two, and several blocks.
 WGRAD_LDS_DIMS = [(1, 3, 4, 32, 8, 8), (2, 3, 4, 32, 8, 16),
                   (1, 2, 3, 64, 24, 8), (1, 3, 3, 32, 48, 16),
                   (1, 2, 3, 32, 16, 48), (1, 2, 2, 32, 32, 32),
@@ -103,9 +103,8 @@ def test_wgrad_lds_rows(ps, dims):
 
 
 def test_wgrad_spans_several_blocks(ps):
-    """More positions than one filter-gradient block (256 positions at this
-    size): partials of several blocks, the last one ragged, through the
-    gathering kernel (rows of 40)."""
+    """Partials of several filter-gradient blocks, the last x tile ragged
+    (rows of 40)."""
     from physis_amd.warmstart import conv_backward_filter_host
     dims = (1, 9, 16, 40, 8, 8)  # 5760 positions
     n, d, h, wd, cin, cout = dims
