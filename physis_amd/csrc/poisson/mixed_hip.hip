@@ -5,14 +5,12 @@
 //
 // Kernels (all 2.5D z-marching, one LDS ring of planes per staged grid,
 // built from the same Stage / BufWin blocks as the Physis run kernels):
-//   SweepKernel<M>     one Jacobi sweep; p and the 12 coefficient/rhs grids
+//   TwoSweepKernel<M>  two Jacobi sweeps; p and the 12 coefficient/rhs grids
 //                      stored as M (float, bfloat16 or binary16), FP32
 //                      arithmetic in the operand order of the Himeno
 //                      jacobi_kernel (reference examples/himeno/
-//                      himenobmtxpa_physis.c:340-359).  Bytes per point:
-//                      14 * sizeof(M).  The 12 centre-only fields are read
-//                      by the compute waves only, non-temporally when they
-//                      exceed the last-level cache.
+//                      himenobmtxpa_physis.c:340-359).  Bytes per point and
+//                      pass: 14 * sizeof(M).
 //   ResidualKernel     FP64 residual r = (s0 - p / a3) bnd from FP32
 //                      coefficients, optionally fused with the refinement
 //                      update p' = p + E / sigma (written to a second FP64
@@ -121,95 +119,6 @@ __device__ __forceinline__ ZRange BlockZ(const Plan &pl, int bz) {
   return r;
 }
 
-// ------------------------------------------------------------- Jacobi sweep
-// LAUX: cache policy of the coefficient loads (physis_hip::kStreamLoad when
-// the fields exceed the last-level cache, else 0: re-read every sweep, they
-// then stay cached).
-template <typename M, int VX, int LAUX>
-__global__ __launch_bounds__(kWave *kBY) void SweepKernel(
-    const M *__restrict__ pin, M *__restrict__ pout, Fields<M> f, int nx,
-    int ny, int nz, float omega, Plan pl) {
-  constexpr int TX = kWave * VX, TY = kBY - 2;
-  typedef Stage<float, VX, kBY, 1, 1, 4, false, M> S;
-  __shared__ __attribute__((aligned(16))) float lds[S::kLdsElems];
-  const int lane = threadIdx.x % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const TileCoord tc = TileOf(pl.tiles_x, pl.tiles_y);
-  const ZRange zr = BlockZ(pl, tc.bz);
-  const int zb = zr.zb, ze = zr.ze;
-  if (zb >= ze) return;  // uniform over the block
-  const int x0 = tc.bx * TX, y0 = tc.by * TY;
-  const int yrow = y0 - 1 + wave;
-  const bool computes = wave >= 1 && wave < kBY - 1 && yrow < ny;
-  const int xs = x0 + lane * VX;
-  // centre-only grids: halo waves issue the same loads at an out-of-range
-  // offset, which the buffer range check drops (no memory access), so
-  // every wave keeps the same count of loads in flight
-  const bool dl = wave >= 1 && wave < kBY - 1;
-  const int drow = dl ? yrow : y0;
-  const int nxy = nx * ny, n = nxy * nz;
-  const int dim[3] = {nx, ny, nz};
-  const BufWin<M> pw =
-      BufWin<M>::Make(pin, n, (long)(zb - 2) * nxy, (long)(ze + 2) * nxy);
-  // (every load of the prologue is issued before the first one is stored)
-  S st[kPD], pro[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-    pro[k].Load(pw, pin, dim, x0, yrow, zb - 1 + k, lane);
-#pragma unroll
-  for (int k = 0; k < kPD; ++k)
-    st[k].Load(pw, pin, dim, x0, yrow, zb + 2 + k, lane);
-#pragma unroll
-  for (int k = 0; k < 3; ++k) pro[k].Store(lds + k * S::kPlane, wave, lane);
-  int base = 0;
-  const BufWin<M> ow =
-      BufWin<M>::Make(pout, n, (long)zb * nxy, (long)ze * nxy);
-  BufWin<M> fw[kNumF];
-  M fv[kNumF][2][VX];
-  const int doff = xs + drow * nx;
-#pragma unroll
-  for (int g = 0; g < kNumF; ++g) {
-    fw[g] = BufWin<M>::Make(f.g[g], n, (long)zb * nxy, (long)ze * nxy);
-    fw[g].template Load<VX, LAUX>(
-        dl ? doff + zb * nxy : physis_hip::kDrop, fv[g][0]);
-  }
-  __syncthreads();
-  for (int zc = zb; zc < ze; zc += kPD) {
-#pragma unroll
-    for (int k = 0; k < kPD; ++k) {
-      const int z = zc + k, cur = k & 1, nxt = cur ^ 1;
-#pragma unroll
-      for (int g = 0; g < kNumF; ++g)
-        fw[g].template Load<VX, LAUX>(
-            dl ? doff + (z + 1) * nxy : physis_hip::kDrop, fv[g][nxt]);
-      if (computes && z < ze) {
-        Rows19<float, VX> r;
-        r.template Read<S>(lds, base, wave, lane);
-        M out[VX];
-        unsigned mask = 0;
-#pragma unroll
-        for (int i = 0; i < VX; ++i) {
-          float c[kNumF];
-#pragma unroll
-          for (int g = 0; g < kNumF; ++g) c[g] = Convert<float, M>(fv[g][cur][i]);
-          const float pc = r.Centre(i);
-          const float s0 = r.S0(c, i);
-          const float ss = (s0 * c[3] - pc) * c[10];
-          // bnd = 0 points keep their value whatever their neighbours hold
-          out[i] = Convert<M, float>(c[10] != 0.0f ? pc + omega * ss : pc);
-          if (xs + i < nx) mask |= 1u << i;
-        }
-        physis_hip::StoreMasked<M, VX>(ow, xs + yrow * nx + z * nxy, out,
-                                       mask);
-      }
-      st[k].Store(lds + RingSlot<4>(base, 3) * S::kPlane, wave, lane);
-      __syncthreads();
-      st[k].Load(pw, pin, dim, x0, yrow, z + 2 + kPD, lane);
-      base = RingSlot<4>(base, 1);
-    }
-  }
-}
-
 // s0 of the Himeno operator at one point whose neighbours come from p(dx,
 // dy, dz), in the operand order of Rows19::S0.
 template <typename P>
@@ -238,16 +147,18 @@ __device__ __forceinline__ M UpdateM(const float (&c)[kNumF], float pc,
 // per two sweeps.  Ring A holds the source planes s-1..s+1 with a
 // two-point halo, ring B the intermediate planes s-3..s-1 with a one-point
 // halo, as the floats of the storage-type values the first sweep would
-// store (so the pass is bit-identical to two SweepKernel launches).  Step s
+// store (so the pass is bit-identical to two sweeps of their own).  Step s
 // computes E'(s) on rows y0-1 .. y0+TY (the columns x0-1 and x0+TX by lanes
 // of wave 0) and E''(s-2) on the tile; one barrier per step.  Points with
 // bnd = 0 (every problem's faces, and points outside the grid, whose
 // fields load as 0) keep their value, so the E' values the pass computes
-// beyond the grid feed only points that ignore them.  With 16-bit storage
-// and two points per lane the fields of plane s are read once, one step
-// ahead of E'(s), and stay in a register ring of 4 planes until E''(s) two
-// steps later (the rows of E'' are rows of E'); otherwise (the ring would
-// not fit the register budget) they are read again for E''.
+// beyond the grid feed only points that ignore them.  The fields of plane s
+// are read once, one step ahead of E'(s), and stay in a register ring of 4
+// planes until E''(s) two steps later (the rows of E'' are rows of E').
+// Bound by latency across the barrier of each step and by the arithmetic
+// (about 71 VALU instructions per point update), not by bytes: FP32 at
+// 512x256x256 444 us per pass, 0.75 of the rate of 13 streams in and one out;
+// BF16 302 us, 0.53 of it.
 template <typename M, int VX, int BY>
 __global__ __launch_bounds__(kWave *BY) void TwoSweepKernel(
     const M *__restrict__ pin, M *__restrict__ pout, Fields<M> f, int nx,
@@ -289,9 +200,7 @@ __global__ __launch_bounds__(kWave *BY) void TwoSweepKernel(
   for (int k = 0; k < 3; ++k) pro[k].Load(aw, pin, dim, ra, zb - 2 + k);
 #pragma unroll
   for (int k = 0; k < kPD; ++k) st[k].Load(aw, pin, dim, ra, zb + 1 + k);
-  constexpr bool kRing = sizeof(M) == 2 && VX == 2;
-  // kRing: plane s in slot (s - zb + 1) & 3; else slots 0/1 alternate
-  M f1[kNumF][kRing ? 4 : 2][VX], f2[kNumF][kRing ? 1 : VX];
+  M f1[kNumF][4][VX];  // plane s in slot (s - zb + 1) & 3
   // fields of plane z for E': the lane's VX points on rows y0-1 .. y0+TY,
   // its halo point in wave 0
   auto load1 = [&](int z, int slot) {
@@ -315,18 +224,9 @@ __global__ __launch_bounds__(kWave *BY) void TwoSweepKernel(
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int s = sc + k;
-      const int cur = kRing ? k : k & 1;
-      const int nxt = kRing ? (k + 1) & 3 : cur ^ 1;
+      const int cur = k, nxt = (k + 1) & 3, old = (k + 2) & 3;
       if (s > ze + 1) break;  // uniform over the block
       load1(s + 1, nxt);
-      if constexpr (!kRing) {
-        const int o2 = out_row && s - 2 >= zb
-                           ? xs + yrow * nx + (s - 2) * nxy
-                           : physis_hip::kDrop;
-#pragma unroll
-        for (int g = 0; g < kNumF; ++g)
-          fw[g].template Load<VX, physis_hip::kStreamLoad>(o2, f2[g]);
-      }
       if (mid_row && s <= ze) {
         Rows19<float, VX> r;
         r.template Read<SA>(a_lds, k, wave, lane);
@@ -363,8 +263,7 @@ __global__ __launch_bounds__(kWave *BY) void TwoSweepKernel(
           float c[kNumF];
 #pragma unroll
           for (int g = 0; g < kNumF; ++g)
-            c[g] = Convert<float, M>(kRing ? f1[g][(k + 2) & 3][i]
-                                           : f2[g][kRing ? 0 : i]);
+            c[g] = Convert<float, M>(f1[g][old][i]);
           out[i] = UpdateM<M>(c, r.Centre(i), r.S0(c, i), omega);
           if (xs + i < nx) mask |= 1u << i;
         }
@@ -570,10 +469,10 @@ struct __PSPoisson {
   float *t32 = nullptr;  // FP32 partner grid of the plain solve
   double *partials = nullptr;
   double *host_partials = nullptr;
-  int sweep_vx;
-  Plan sweep_plan, res_plan;
-  int sweep2_vx;     // two-sweep passes
-  Plan sweep2_plan;
+  // two-sweep passes of the storage type and of FP32 (plain sweeps run on a
+  // solver of any storage)
+  int sweep2_vx;
+  Plan sweep2_plan, plain_plan, res_plan;
 };
 
 namespace {
@@ -596,95 +495,66 @@ Fields<float> MasterFields(const __PSPoisson *s) {
   return f;
 }
 
-// MI355X's last-level cache (AMD Infinity Cache): 256 MiB.
-constexpr size_t kLastLevelCacheBytes = size_t(256) << 20;
-
-template <typename M, int VX>
-void LaunchSweepVX(const __PSPoisson *s, const M *in, M *out, Fields<M> f,
-                   float omega) {
-  const dim3 grid(s->sweep_plan.blocks), block(kWave * kBY);
-  const size_t field_bytes =
-      (size_t)kNumF * s->nx * s->ny * s->nz * sizeof(M);
-  if (field_bytes > kLastLevelCacheBytes)
-    hipLaunchKernelGGL((SweepKernel<M, VX, physis_hip::kStreamLoad>), grid,
-                       block, 0, Stream(), in, out, f, s->nx, s->ny, s->nz,
-                       omega, s->sweep_plan);
-  else
-    hipLaunchKernelGGL((SweepKernel<M, VX, 0>), grid, block, 0, Stream(), in,
-                       out, f, s->nx, s->ny, s->nz, omega, s->sweep_plan);
+// Points per lane of the two-sweep kernel in 12-wave blocks (8 output rows):
+// the field ring takes 48 values per point.  FP32 runs at one (us per sweep
+// at 512x256x256, 162x150x140 and 64^3: 221, 26.1 and 4.5, against 366, 56.9
+// and 8.9 at two and 263, - and 9.8 at four points, whose fields were read
+// twice in 8-wave blocks).  16-bit fields run at two (BF16 151, 24.3, 5.3; at
+// one 175, 23.4, 4.4) unless one point per lane leaves fewer lanes past the
+// ends of the rows: 128-wide tiles cover 162 points with 256 lanes' points,
+// 64-wide ones with 192.
+constexpr int kTwoSweepBY = 12;
+template <typename M>
+int TwoSweepVX(int nx) {
+  if (sizeof(M) == 4) return 1;
+  return (nx + 63) / 64 * 64 < (nx + 127) / 128 * 128 ? 1 : 2;
 }
-
-template <typename M>
-void LaunchSweep(const __PSPoisson *s, const M *in, M *out, Fields<M> f,
-                 float omega) {
-  if (s->sweep_vx == 4)
-    LaunchSweepVX<M, 4>(s, in, out, f, omega);
-  else
-    LaunchSweepVX<M, 2>(s, in, out, f, omega);
-  CheckLaunch();
-}
-
-// Waves per block of the two-sweep kernel (TY = BY - 4 output rows) and its
-// points per lane.  The fields take 2 * VX values of E' in flight and VX of
-// E'' per lane.  Measured at 512^3 (ms per sweep; pairs of single sweeps:
-// 0.807 BF16, 1.448 FP32): 16-bit fields run best at VX = 2 in 12-wave
-// blocks (0.655; 130 VGPRs, three waves per SIMD; VX = 4 in 8-wave blocks
-// 0.827, in 12-wave blocks 0.732 with spills), FP32 fields at VX = 4 in
-// 8-wave blocks (0.984; VX = 2 in 12-wave blocks 1.104).
-template <typename M> struct TwoSweepBY { static constexpr int value = 12; };
-template <> struct TwoSweepBY<float> { static constexpr int value = 8; };
-template <typename M>
-int TwoSweepVX(int nx) { return 2; }
-template <>
-int TwoSweepVX<float>(int nx) { return (nx % 4 == 0 && nx > 128) ? 4 : 2; }
-
-template <typename M>
-const void *TwoSweepFn(int vx) {
-  constexpr int BY = TwoSweepBY<M>::value;
-  return vx == 4 ? (const void *)TwoSweepKernel<M, 4, BY>
-                 : (const void *)TwoSweepKernel<M, 2, BY>;
+// f(kernel) for the kernel of vx points per lane.
+template <typename M, typename F>
+void TwoSweepFor(int vx, F f) {
+  if constexpr (sizeof(M) == 2) {
+    if (vx == 2) return f(TwoSweepKernel<M, 2, kTwoSweepBY>);
+  }
+  f(TwoSweepKernel<M, 1, kTwoSweepBY>);
 }
 
 // Two sweeps in -> out in one launch.
 template <typename M>
 void LaunchTwoSweep(const __PSPoisson *s, const M *in, M *out, Fields<M> f,
                     float omega) {
-  constexpr int BY = TwoSweepBY<M>::value;
-  const dim3 grid(s->sweep2_plan.blocks), block(kWave * BY);
-  if (s->sweep2_vx == 4)
-    hipLaunchKernelGGL((TwoSweepKernel<M, 4, BY>), grid, block, 0, Stream(),
-                       in, out, f, s->nx, s->ny, s->nz, omega, s->sweep2_plan);
-  else
-    hipLaunchKernelGGL((TwoSweepKernel<M, 2, BY>), grid, block, 0, Stream(),
-                       in, out, f, s->nx, s->ny, s->nz, omega, s->sweep2_plan);
+  const Plan &pl = sizeof(M) == 4 ? s->plain_plan : s->sweep2_plan;
+  TwoSweepFor<M>(s->sweep2_vx, [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(pl.blocks), dim3(kWave * kTwoSweepBY), 0,
+                       Stream(), in, out, f, s->nx, s->ny, s->nz, omega, pl);
+  });
   CheckLaunch();
 }
 
-// n (even) sweeps a -> t -> a ... ending in a: pairs of sweeps run as
-// two-sweep passes a -> t, t -> a; an odd pair count starts with one pair
-// of single sweeps.
+// n (even) sweeps a -> t -> a ... in n / 2 passes; returns where they end: a
+// for an even number of passes, else t.
 template <typename M>
-void SweepPairs(__PSPoisson *s, M *a, M *t, Fields<M> f, int n,
-                float omega) {
-  int pairs = n / 2;
-  if (pairs % 2) {
-    LaunchSweep<M>(s, a, t, f, omega);
-    LaunchSweep<M>(s, t, a, f, omega);
-    --pairs;
-  }
-  for (int i = 0; i < pairs; i += 2) {
+M *SweepPairs(const __PSPoisson *s, M *a, M *t, Fields<M> f, int n,
+              float omega) {
+  for (int i = 0; i < n / 2; ++i) {
     LaunchTwoSweep<M>(s, a, t, f, omega);
-    LaunchTwoSweep<M>(s, t, a, f, omega);
+    std::swap(a, t);
   }
+  return a;
 }
 
 template <typename M>
 void InnerSweeps(__PSPoisson *s, int n, float omega) {
-  SweepPairs<M>(s, (M *)s->e[0], (M *)s->e[1], InnerFields<M>(s), n, omega);
+  if (SweepPairs<M>(s, (M *)s->e[0], (M *)s->e[1], InnerFields<M>(s), n,
+                    omega) != (M *)s->e[0])
+    std::swap(s->e[0], s->e[1]);  // E is e[0]
 }
 
 void PlainSweeps(__PSPoisson *s, float *p, int n, float omega) {
-  SweepPairs<float>(s, p, s->t32, MasterFields(s), n, omega);
+  const float *end =
+      SweepPairs<float>(s, p, s->t32, MasterFields(s), n, omega);
+  if (end != p)
+    PS_HIP_CHECK(hipMemcpyAsync(p, end, s->elems * sizeof(float),
+                                hipMemcpyDeviceToDevice, Stream()));
 }
 
 template <typename PT, typename ME, bool UPDATE, bool WRHS>
@@ -867,38 +737,22 @@ __PSPoisson *PSPoissonNew(__PSGrid *const coef[12], int nbatch, int storage) {
   s->e[0] = DevAlloc(s->elems * s->esize);
   s->e[1] = DevAlloc(s->elems * s->esize);
   ok = ok && s->rhs && s->e[0] && s->e[1];
-  s->sweep_vx = (nx % 4 == 0 && nx > 128) ? 4 : 2;
-  int per_cu_sweep = 1, per_cu_res = 1;
-  switch (storage) {
-    case PS_STORAGE_BF16:
-      per_cu_sweep = physis_hip::BlocksPerCU(
-          s->sweep_vx == 4 ? (const void *)SweepKernel<bf16_t, 4, 0>
-                           : (const void *)SweepKernel<bf16_t, 2, 0>, kWave * kBY);
-      break;
-    case PS_STORAGE_FP16:
-      per_cu_sweep = physis_hip::BlocksPerCU(
-          s->sweep_vx == 4 ? (const void *)SweepKernel<fp16_t, 4, 0>
-                           : (const void *)SweepKernel<fp16_t, 2, 0>, kWave * kBY);
-      break;
-    default:
-      per_cu_sweep = physis_hip::BlocksPerCU(
-          s->sweep_vx == 4 ? (const void *)SweepKernel<float, 4, 0>
-                           : (const void *)SweepKernel<float, 2, 0>, kWave * kBY);
-  }
-  per_cu_res = physis_hip::BlocksPerCU(
+  const int per_cu_res = physis_hip::BlocksPerCU(
       (const void *)ResidualKernel<double, bf16_t, 2, true, true>, kWave * kBY);
-  s->sweep_plan = MakePlan(nx, ny, s->nzs, nbatch, s->sweep_vx, per_cu_sweep);
-  {
-    s->sweep2_vx = storage == PS_STORAGE_FP32 ? TwoSweepVX<float>(nx)
-                                              : TwoSweepVX<bf16_t>(nx);
-    const void *fn = storage == PS_STORAGE_BF16   ? TwoSweepFn<bf16_t>(s->sweep2_vx)
-                     : storage == PS_STORAGE_FP16 ? TwoSweepFn<fp16_t>(s->sweep2_vx)
-                                                  : TwoSweepFn<float>(s->sweep2_vx);
-    const int by = storage == PS_STORAGE_FP32 ? TwoSweepBY<float>::value
-                                              : TwoSweepBY<bf16_t>::value;
-    s->sweep2_plan = MakePlan(nx, ny, s->nzs, nbatch, s->sweep2_vx,
-                              physis_hip::BlocksPerCU(fn, kWave * by), by - 4);
-  }
+  const auto plan = [&](auto m, int vx) {
+    Plan p;
+    TwoSweepFor<decltype(m)>(vx, [&](auto kernel) {
+      p = MakePlan(
+          nx, ny, s->nzs, nbatch, vx,
+          physis_hip::BlocksPerCU((const void *)kernel, kWave * kTwoSweepBY),
+          kTwoSweepBY - 4);
+    });
+    return p;
+  };
+  s->plain_plan = plan(float{}, TwoSweepVX<float>(nx));
+  s->sweep2_vx = TwoSweepVX<bf16_t>(nx);
+  s->sweep2_plan = storage == PS_STORAGE_BF16 ? plan(bf16_t{}, s->sweep2_vx)
+                                              : plan(fp16_t{}, s->sweep2_vx);
   s->res_plan = MakePlan(nx, ny, s->nzs, nbatch, 2, per_cu_res);
   s->partials = (double *)DevAlloc(sizeof(double) * 3 * s->res_plan.blocks);
   ok = ok && s->partials;
