@@ -177,6 +177,15 @@ extern void *__PSHipScratch(int slot, size_t bytes);
  * Synchronous. */
 extern void __PSHipReduceFold(int type, int op, const void *partials,
                               int nparts, int count, void *host_out);
+/* Pinned host area number `slot` (0 <= slot < 10) of at least `bytes`, kept
+ * and grown across calls: kernels write it, the host reads it after a wait
+ * on the runtime stream.  Generated run functions keep the results of fused
+ * reductions in slots 1..7; slot 0 is __PSHipReduceFold's own. */
+extern void *__PSHipPinned(int slot, size_t bytes);
+/* __PSHipReduceFold without the wait: the results are in `out` (pinned or
+ * device memory) once the runtime stream has drained. */
+extern void __PSHipReduceFoldAsync(int type, int op, const void *partials,
+                                   int nparts, int count, void *out);
 
 /* ---- offset helpers (physis_cuda.h:196-269): host and device versions. */
 #if defined(__HIPCC__)

@@ -63,6 +63,24 @@ void *HostResultSlot() {
   return r.host_result;
 }
 
+// Pinned host memory that kernels write and the host reads after a wait.
+void *Pinned(int slot, size_t bytes) {
+  Runtime &r = rt();
+  EnsureInit();
+  if (slot < 0 || slot >= Runtime::kScratchSlots)
+    PS_FATAL("pinned slot %d out of range", slot);
+  if (bytes > r.pinned_bytes[slot]) {
+    if (r.pinned[slot]) {
+      PS_HIP_CHECK(hipStreamSynchronize(r.stream));
+      PS_HIP_CHECK(hipHostFree(r.pinned[slot]));
+    }
+    size_t cap = bytes < 4096 ? 4096 : bytes;
+    PS_HIP_CHECK(hipHostMalloc(&r.pinned[slot], cap));
+    r.pinned_bytes[slot] = cap;
+  }
+  return r.pinned[slot];
+}
+
 namespace {
 
 // Removes "--physis-trace" from argv and turns tracing on, as the reference
@@ -163,6 +181,11 @@ void PSFinalize(void) {
     if (r.scratch[i]) PS_HIP_CHECK(hipFree(r.scratch[i]));
     r.scratch[i] = nullptr;
     r.scratch_bytes[i] = 0;
+  }
+  for (int i = 0; i < Runtime::kScratchSlots; ++i) {
+    if (r.pinned[i]) PS_HIP_CHECK(hipHostFree(r.pinned[i]));
+    r.pinned[i] = nullptr;
+    r.pinned_bytes[i] = 0;
   }
   if (r.host_result) PS_HIP_CHECK(hipHostFree(r.host_result));
   r.host_result = nullptr;
@@ -389,5 +412,7 @@ int __PSHipNumCUs(void) {
 }
 
 void *__PSHipScratch(int slot, size_t bytes) { return Scratch(slot, bytes); }
+
+void *__PSHipPinned(int slot, size_t bytes) { return Pinned(slot, bytes); }
 
 }  // extern "C"

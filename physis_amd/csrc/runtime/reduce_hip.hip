@@ -112,11 +112,11 @@ int StageBlocks(int64_t n) {
 }
 
 // Both stages on the runtime stream: nb partials into `parts`, the result
-// (one T) into `out`; then the result is copied to host_out and the stream
-// drained.
+// (one T) into `out`, which the host may read after a wait when it is pinned
+// memory.
 template <typename T, int OP>
 void LaunchStages(const T *p, int64_t n, int nb,
-                  typename Acc<T, OP>::A *parts, T *out, void *host_out) {
+                  typename Acc<T, OP>::A *parts, T *out) {
   Runtime &r = rt();
   hipLaunchKernelGGL((ReduceStage1<T, OP>), dim3(nb), dim3(kThreads), 0,
                      r.stream, p, n, parts);
@@ -124,17 +124,17 @@ void LaunchStages(const T *p, int64_t n, int nb,
   hipLaunchKernelGGL((ReduceStage2<T, OP>), dim3(1), dim3(1024), 0, r.stream,
                      parts, nb, out);
   PS_HIP_CHECK(hipGetLastError());
-  PS_HIP_CHECK(hipMemcpyAsync(host_out, out, sizeof(T), hipMemcpyDeviceToHost,
-                              r.stream));
-  PS_HIP_CHECK(hipStreamSynchronize(r.stream));
 }
 
 template <typename T, int OP>
 void Launch(const T *p, int64_t n, void *host_out) {
   const int nb = StageBlocks<T>(n);
   typedef typename Acc<T, OP>::A A;
-  A *parts = (A *)Scratch(0, sizeof(A) * (size_t)(nb + 1));
-  LaunchStages<T, OP>(p, n, nb, parts, (T *)(parts + nb), host_out);
+  A *parts = (A *)Scratch(0, sizeof(A) * (size_t)nb);
+  // the result goes straight to the pinned slot: a copy of its own took
+  // another 10 us
+  LaunchStages<T, OP>(p, n, nb, parts, (T *)host_out);
+  PS_HIP_CHECK(hipStreamSynchronize(rt().stream));
 }
 
 template <typename T>
@@ -191,7 +191,11 @@ void LaunchNoAlloc(const T *p, int64_t n, void *buf, unsigned char *area) {
     PS_FATAL("reduction needs %zu scratch bytes, more than the %zu of the "
              "no-allocation area", need, kNoAllocScratchBytes);
   A *parts = (A *)area;
-  LaunchStages<T, OP>(p, n, nb, parts, (T *)(parts + nb), buf);
+  T *out = (T *)(parts + nb);
+  LaunchStages<T, OP>(p, n, nb, parts, out);
+  PS_HIP_CHECK(hipMemcpyAsync(buf, out, sizeof(T), hipMemcpyDeviceToHost,
+                              rt().stream));
+  PS_HIP_CHECK(hipStreamSynchronize(rt().stream));
 }
 
 template <typename T>
@@ -283,17 +287,9 @@ __global__ __launch_bounds__(256) void FoldRows(const T *__restrict__ partials,
 
 template <typename T>
 void FoldTyped(int op, const void *partials, int nparts, int count,
-               void *host_out) {
+               void *out) {
   Runtime &r = rt();
-  // Results land after the partials in the scratch area of the caller, so
-  // they use a separate small device buffer.
-  static T *dev_out = nullptr;
-  static int dev_cap = 0;
-  if (count > dev_cap) {
-    if (dev_out) PS_HIP_CHECK(hipFree(dev_out));
-    PS_HIP_CHECK(hipMalloc(&dev_out, sizeof(T) * (size_t)count));
-    dev_cap = count;
-  }
+  T *dev_out = (T *)out;
   const T *p = (const T *)partials;
   switch (op) {
     case PS_MAX: hipLaunchKernelGGL((FoldRows<T, PS_MAX>), dim3(count), dim3(256), 0, r.stream, p, nparts, dev_out); break;
@@ -303,24 +299,33 @@ void FoldTyped(int op, const void *partials, int nparts, int count,
     default: PS_FATAL("unknown reduction operator %d", op);
   }
   PS_HIP_CHECK(hipGetLastError());
-  PS_HIP_CHECK(hipMemcpyAsync(host_out, dev_out, sizeof(T) * (size_t)count,
-                              hipMemcpyDeviceToHost, r.stream));
-  PS_HIP_CHECK(hipStreamSynchronize(r.stream));
 }
 
 }  // namespace physis_hip
 
-extern "C" void __PSHipReduceFold(int type, int op, const void *partials,
-                                  int nparts, int count, void *host_out) {
+extern "C" void __PSHipReduceFoldAsync(int type, int op, const void *partials,
+                                       int nparts, int count, void *out) {
   using namespace physis_hip;
   EnsureInit();
   if (count <= 0) return;
   if (nparts <= 0) PS_FATAL("reduction over an empty domain");
   switch (type) {
-    case PS_FLOAT: FoldTyped<float>(op, partials, nparts, count, host_out); break;
-    case PS_DOUBLE: FoldTyped<double>(op, partials, nparts, count, host_out); break;
-    case PS_INT: FoldTyped<int>(op, partials, nparts, count, host_out); break;
-    case PS_LONG: FoldTyped<long>(op, partials, nparts, count, host_out); break;
+    case PS_FLOAT: FoldTyped<float>(op, partials, nparts, count, out); break;
+    case PS_DOUBLE: FoldTyped<double>(op, partials, nparts, count, out); break;
+    case PS_INT: FoldTyped<int>(op, partials, nparts, count, out); break;
+    case PS_LONG: FoldTyped<long>(op, partials, nparts, count, out); break;
     default: PS_FATAL("unsupported reduction type %d", type);
   }
+}
+
+extern "C" void __PSHipReduceFold(int type, int op, const void *partials,
+                                  int nparts, int count, void *host_out) {
+  using namespace physis_hip;
+  if (count <= 0) return;
+  const size_t bytes =
+      (size_t)count * (type == PS_DOUBLE || type == PS_LONG ? 8 : 4);
+  void *out = Pinned(0, bytes);
+  __PSHipReduceFoldAsync(type, op, partials, nparts, count, out);
+  PS_HIP_CHECK(hipStreamSynchronize(rt().stream));
+  std::memcpy(host_out, out, bytes);
 }

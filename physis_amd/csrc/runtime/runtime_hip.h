@@ -42,6 +42,8 @@ struct Runtime {
   void *scratch[kScratchSlots] = {};  // partial results, grown on demand
   size_t scratch_bytes[kScratchSlots] = {};
   void *host_result = nullptr;   // pinned landing slot for scalar results
+  void *pinned[kScratchSlots] = {};  // pinned host areas, grown on demand
+  size_t pinned_bytes[kScratchSlots] = {};
 };
 
 Runtime &rt();
@@ -50,6 +52,7 @@ Runtime &rt();
 void EnsureInit();
 void *Scratch(int slot, size_t bytes);
 void *HostResultSlot();
+void *Pinned(int slot, size_t bytes);
 
 // reduce_hip.hip
 void ReduceGrid(void *buf, PSReduceOp op, const __PSGrid *g, PSType type);

@@ -3183,6 +3183,9 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
     if (kernels_.at(r.kernels[i]).ret_type != "void")
       o << "    red" << i << ".After(i);\n";
   o << "  }\n";
+  for (size_t i = 0; i < r.kernels.size(); ++i)
+    if (kernels_.at(r.kernels[i]).ret_type != "void")
+      o << "  red" << i << ".Finish(stream);\n";
   if (cfg_.kernel_error_check) o << "  __PSCheckHipError(\"Kernel Execution Failed!\");\n";
   o << "  __PSTraceStencilPost(timer.Stop());\n}\n\n";
   return o.str();

@@ -926,6 +926,8 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_jacobi_kernel s0, stru
     red0.After(i);
     red1.After(i);
   }
+  red0.Finish(stream);
+  red1.Finish(stream);
   __PSTraceStencilPost(timer.Stop());
 }
 
@@ -980,6 +982,8 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_jacobi_kernel s0, stru
     red0.After(i);
     red1.After(i);
   }
+  red0.Finish(stream);
+  red1.Finish(stream);
   __PSTraceStencilPost(timer.Stop());
 }
 

@@ -5943,6 +5943,13 @@ static void __PSStencilRun_22(int iter, struct __PSStencil_kscaled s0, struct __
     red5.After(i);
     red6.After(i);
   }
+  red0.Finish(stream);
+  red1.Finish(stream);
+  red2.Finish(stream);
+  red3.Finish(stream);
+  red4.Finish(stream);
+  red5.Finish(stream);
+  red6.Finish(stream);
   __PSTraceStencilPost(timer.Stop());
 }
 
