@@ -1,0 +1,178 @@
+// Building blocks of the resident-tile passes that physisc-hip emits for
+// fusable maps on small grids.
+//
+// A small grid's z-marching pass is a chain of latencies: a launch, then a
+// barrier and a load per few planes, on blocks that own a handful of points.
+// A resident-tile pass does T sweeps of a map pair per launch on tiles that
+// stay in LDS: a block loads its tile with a T-point halo once, then computes
+// sweep after sweep between two LDS buffers, each on a box one point smaller,
+// and stores the last (one barrier per sweep).  The price is the halo's
+// arithmetic (a tile of 16x8x8 computes 2.4 times its points over 4 sweeps),
+// which is cheap as long as the grid leaves most of the chip idle.
+#ifndef PHYSIS_HIP_TILE_H_
+#define PHYSIS_HIP_TILE_H_
+
+#include <cstdint>
+
+#include "physis/hip/stencil.h"
+#include "physis/physis_hip.h"
+
+namespace physis_hip {
+
+// Shape of a resident tile of TX x TY x TZ points for T sweeps by NT
+// threads.  The points are numbered by shells: shell s is the points s
+// points outside the tile (shell 0 the tile itself); sweep t (1 .. T)
+// computes shells 0 .. T - t.  Thread i owns points i, i + NT, ... of each
+// shell, so that a sweep's loop ends with its shells.
+template <int T_, int TX_, int TY_, int TZ_, int NT_>
+struct Tile {
+  static constexpr int T = T_, TX = TX_, TY = TY_, TZ = TZ_, NT = NT_;
+  // the staged box: halo T, row pitch RX
+  static constexpr int RX = TX + 2 * T, RY = TY + 2 * T, RZ = TZ + 2 * T;
+  static constexpr int kElems = RX * RY * RZ;
+  static constexpr int kLoads = (kElems + NT - 1) / NT;
+  static constexpr int Box(int s) {  // points of shells 0 .. s
+    return (TX + 2 * s) * (TY + 2 * s) * (TZ + 2 * s);
+  }
+  static constexpr int Shell(int s) { return s == 0 ? Box(0) : Box(s) - Box(s - 1); }
+  // owned points per thread in shells 0 .. s
+  static constexpr int Owned(int s) {
+    int k = 0;
+    for (int i = 0; i <= s; ++i) k += (Shell(i) + NT - 1) / NT;
+    return k;
+  }
+  static constexpr int K = Owned(T - 1);
+  // Points of the sweep t's loop: k < Count(t)
+  static constexpr int Count(int t) { return Owned(T - t); }
+
+  // LDS offsets (x + RX (y + RY z)) of the owned points: entry k * NT + i is
+  // thread i's k-th point, -1 where a shell has none left.
+  struct Table {
+    short at[K * NT];
+  };
+  static constexpr Table Make() {
+    Table t{};
+    int k0 = 0;
+    for (int s = 0; s < T; ++s) {
+      const int x0 = T - s, y0 = T - s, z0 = T - s;
+      const int x1 = T + TX + s, y1 = T + TY + s, z1 = T + TZ + s;
+      int n = k0 * NT;
+      for (int z = z0; z < z1; ++z)
+        for (int y = y0; y < y1; ++y) {
+          const bool rim = s == 0 || z == z0 || z == z1 - 1 || y == y0 ||
+                           y == y1 - 1;
+          // a row of the shell: whole on its rim, else its two ends
+          for (int x = x0; x < x1; x += rim ? 1 : x1 - 1 - x0)
+            t.at[n++] = (short)(x + RX * (y + RY * z));
+        }
+      k0 += (Shell(s) + NT - 1) / NT;
+      for (; n < k0 * NT; ++n) t.at[n] = -1;
+    }
+    return t;
+  }
+};
+
+template <typename TILE>
+struct TileTable {
+  static __device__ const typename TILE::Table value;
+};
+template <typename TILE>
+__device__ const typename TILE::Table TileTable<TILE>::value = TILE::Make();
+
+// One owned point: its LDS offset and its coordinates in the grid.
+struct TilePoint {
+  int at, x, y, z;
+};
+template <typename TILE>
+__device__ __forceinline__ TilePoint OwnedPoint(int k, int x0, int y0, int z0) {
+  TilePoint p;
+  p.at = TileTable<TILE>::value.at[k * TILE::NT + threadIdx.x];
+  const int a = p.at < 0 ? 0 : p.at;
+  const int r = a / TILE::RX, z = r / TILE::RY;
+  p.x = x0 - TILE::T + a - r * TILE::RX;
+  p.y = y0 - TILE::T + r - z * TILE::RY;
+  p.z = z0 - TILE::T + z;
+  return p;
+}
+
+// Loads the tile at (x0, y0, z0) with its halo; a periodic grid wraps, other
+// points outside the grid have no value that a map reads.
+template <typename TILE, bool PERIODIC, typename E>
+__device__ __forceinline__ void LoadTile(E *lds, const E *p, const int *dim,
+                                         int x0, int y0, int z0) {
+  const int n = dim[0] * dim[1] * dim[2];
+  const BufWin<E> w = BufWin<E>::Make(p, n, 0, n);
+  E v[TILE::kLoads][1];
+#pragma unroll
+  for (int k = 0; k < TILE::kLoads; ++k) {
+    const int e = k * TILE::NT + threadIdx.x;
+    const int r = e / TILE::RX, zz = r / TILE::RY;
+    int x = x0 - TILE::T + e - r * TILE::RX;
+    int y = y0 - TILE::T + r - zz * TILE::RY;
+    int z = z0 - TILE::T + zz;
+    bool in = e < TILE::kElems;
+    if (PERIODIC) {
+      x = WrapNear(x, dim[0]);
+      y = WrapNear(y, dim[1]);
+      z = WrapNear(z, dim[2]);
+    } else {
+      in = in && x >= 0 && x < dim[0] && y >= 0 && y < dim[1] && z >= 0 &&
+           z < dim[2];
+    }
+    w.template Load<1>(in ? x + dim[0] * (y + dim[1] * z) : kDrop, v[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < TILE::kLoads; ++k) {
+    const int e = k * TILE::NT + threadIdx.x;
+    if (e < TILE::kElems) lds[e] = v[k][0];
+  }
+}
+
+// ------------------------------------------------------ launch arithmetic
+// Tiles of one small grid per compute unit, and those of larger ones, whose
+// halo costs less.  Measured for T = 4 (us per sweep of the clamped 7-point
+// diffusion, small tile / mid tile / z-marching two-sweep passes): 64^3 1.94 /
+// 2.51 / 4.41, 80^3 2.75 / 2.63 / 5.27, 96^3 4.53 / 3.85 / 6.02, 128^3 7.97 /
+// 6.49 / 7.26, 144^3 11.1 / 8.83 / 8.89.  A kernel with the 12 centre-only
+// grids of the 19-point Jacobi sweep gains nothing (its tiles read the halo's
+// values of every one of them: 96^3 14.4 against 10.1).
+template <int T> using SmallTile = Tile<T, 16, 8, 8, 1024>;
+template <int T> using MidTile = Tile<T, 16, 16, 8, 1024>;
+constexpr int64_t kTileMaxPoints = 2200000;
+
+// Per-block partials of each sweep of a pass (NULL: none).
+struct TileReds {
+  void *p[4];
+};
+
+struct TileShape {
+  int tiles_x, tiles_y, blocks;
+};
+template <typename TILE>
+inline TileShape TileGrid(const __PSDomain &d) {
+  TileShape s = {0, 0, 0};
+  int n[3];
+  const int t[3] = {TILE::TX, TILE::TY, TILE::TZ};
+  for (int i = 0; i < 3; ++i) {
+    const int e = d.local_max[i] - d.local_min[i];
+    if (e <= 0) return s;
+    n[i] = (e + t[i] - 1) / t[i];
+  }
+  s.tiles_x = n[0];
+  s.tiles_y = n[1];
+  s.blocks = n[0] * n[1] * n[2];
+  return s;
+}
+
+// Whether a domain runs in small tiles (else in mid ones), and its blocks.
+inline bool InSmallTiles(const __PSDomain &d) {
+  return TileGrid<SmallTile<2>>(d).blocks <= __PSHipNumCUs();
+}
+inline int TileBlocks(const __PSDomain &d) {
+  return InSmallTiles(d) ? TileGrid<SmallTile<2>>(d).blocks
+                         : TileGrid<MidTile<2>>(d).blocks;
+}
+
+}  // namespace physis_hip
+
+#endif  // PHYSIS_HIP_TILE_H_

@@ -2708,7 +2708,8 @@ std::string Translator::EmitKernel(KernelInfo &k) {
   s += k.fast ? EmitFastRunKernel(k) : EmitGenericRunKernel(k);
   s += EmitLauncher(k);
   if (k.fusable || k.fuse_rb)
-    s += k.fuse_domain ? EmitFusedDomainKernel(k) : EmitFusedRunKernel(k);
+    s += (k.fuse_domain ? EmitFusedDomainKernel(k) : EmitFusedRunKernel(k)) +
+         (UsesTiles(k) ? EmitTileKernel(k) : "");
   return s;
 }
 
@@ -2727,20 +2728,57 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
     << T << ");\n"
     << "    " << V << " vt = va;\n"
     << "    vt.p = (" << T << " *)__PSHipScratch(8, bytes);\n";
+  // A small grid takes resident-tile passes of two pairs each, the first of
+  // one pair when the count is odd (and both when there are only two pairs,
+  // so that there are always two passes to ping-pong between).
+  const std::string &n = k.name;
+  const bool red = k.ret_type != "void";
+  const bool tiles = UsesTiles(k);
+  if (tiles)
+    o << "    const bool __small = s0." << gi.name
+      << "->num_elms <= physis_hip::kTileMaxPoints;\n"
+      << "    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);\n";
+  else
+    o << "    const int passes = iter;\n";
+  // one pass, pairs i and on (j: pass)
+  auto launch = [&](const std::string &src, const std::string &dst,
+                    const std::string &last) {
+    std::ostringstream f;
+    const std::string reds2 =
+        red ? "{red0.Slot(i), red1.Slot(i)}" : "{}";
+    const std::string reds4 =
+        red ? "{red0.Slot(i), red1.Slot(i), red0.Slot(i + 1), red1.Slot(i + 1)}"
+            : "{}";
+    if (tiles)
+      f << "      const int pairs = __small && iter > 2 && (j || iter % 2 == 0) ? 2 : 1;\n"
+           "      if (__small && pairs == 2)\n        __PSLaunchT_" << n << "<4>(s0, "
+        << src << ", " << dst << ", vb.p, " << last << ", stream, " << reds4
+        << ");\n      else if (__small)\n        __PSLaunchT_" << n << "<2>(s0, "
+        << src << ", " << dst << ", vb.p, " << last << ", stream, " << reds2
+        << ");\n      else\n  ";
+    else if (red)
+      f << "      const int pairs = 1;\n";
+    f << "      __PSLaunch2_" << n << "(s0, " << src << ", " << dst << ", "
+      << (k.fuse_domain
+              ? last + ", stream, " + (red ? "red0.Slot(i), red1.Slot(i)"
+                                           : "NULL, NULL")
+              : last + " ? vb.p : NULL, stream")
+      << ");\n";
+    if (red)
+      f << "      for (const int e = i + pairs; i < e; ++i) {\n"
+           "        red0.After(i);\n        red1.After(i);\n      }\n";
+    return f.str();
+  };
   if (!k.fuse_domain) {
-    // Each pass is one pair.  Even counts ping-pong a -> t -> a ...; odd
-    // counts (>= 3) send the first pass to b instead, a -> b -> t -> a ...
-    // (b is free until the last pass writes it).  Either way the last pass
-    // reads t and writes a, and its intermediate sweep to b.
+    // Even pass counts ping-pong a -> t -> a ...; odd counts (>= 3) send the
+    // first pass to b instead, a -> b -> t -> a ... (b is free until the
+    // last pass writes it).  Either way the last pass reads t and writes a,
+    // and its last but one sweep to b.
     o << "    " << V << " src = va;\n"
-      << "    int j = 0;\n"
-      << "    if (iter % 2) {\n"
-      << "      __PSLaunch2_" << k.name << "(s0, va, vb, NULL, stream);\n"
-      << "      src = vb;\n      j = 1;\n    }\n"
-      << "    for (; j < iter; ++j) {\n"
-      << "      const " << V << " dst = ((iter - 1 - j) % 2 == 0) ? va : vt;\n"
-      << "      __PSLaunch2_" << k.name
-      << "(s0, src, dst, j == iter - 1 ? vb.p : NULL, stream);\n"
+      << "    for (int j = 0; j < passes; ++j) {\n"
+      << "      const " << V << " dst = passes % 2 && j == 0 ? vb\n"
+         "          : ((passes - 1 - j) % 2 == 0) ? va : vt;\n"
+      << launch("src", "dst", "(j == passes - 1)")
       << "      src = dst;\n    }\n";
   } else {
     // Points outside the domain keep a's values in a, so the scratch grids
@@ -2748,21 +2786,18 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
     // domain).  Even counts ping-pong a -> t -> a ...; odd counts (>= 3) go
     // a -> t -> t2 -> a -> t -> a ... (b's values outside the domain are
     // read by every pass, so b cannot hold a pass).  The last pass writes a,
-    // and its intermediate sweep to b.
-    const bool red = k.ret_type != "void";
+    // and its last but one sweep to b.
     o << "    " << V << " vt2 = va;\n"
       << "    physis_hip::CopyDevice(vt.p, va.p, bytes, stream);\n"
-      << "    if (iter % 2) {\n"
+      << "    if (passes % 2) {\n"
       << "      vt2.p = (" << T << " *)__PSHipScratch(9, bytes);\n"
       << "      physis_hip::CopyDevice(vt2.p, va.p, bytes, stream);\n    }\n"
       << "    " << V << " src = va;\n"
-      << "    for (int j = 0; j < iter; ++j) {\n"
-      << "      " << V << " dst = (j % 2 == (iter % 2 ? 0 : 1)) ? va : vt;\n"
-      << "      if (iter % 2 && j < 2) dst = j == 0 ? vt : vt2;\n"
-      << "      __PSLaunch2_" << k.name << "(s0, src, dst, j == iter - 1, stream, "
-      << (red ? "red0.Slot(j), red1.Slot(j)" : "NULL, NULL") << ");\n";
-    if (red) o << "      red0.After(j);\n      red1.After(j);\n";
-    o << "      src = dst;\n    }\n";
+      << "    for (int j = 0" << (red ? ", i = 0" : "") << "; j < passes; ++j) {\n"
+      << "      " << V << " dst = (j % 2 == (passes % 2 ? 0 : 1)) ? va : vt;\n"
+      << "      if (passes % 2 && j < 2) dst = j == 0 ? vt : vt2;\n"
+      << launch("src", "dst", "(j == passes - 1)")
+      << "      src = dst;\n    }\n";
   }
   o << "    i0 = iter;\n  }\n";
   return o.str();
@@ -3110,6 +3145,214 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
   return o.str();
 }
 
+// Resident-tile passes of a fusable kernel (include/physis/hip/tile.h): T
+// sweeps of a map pair (or T / 2 red-black iterations) per launch for grids
+// too small to keep the z-marching passes busy, when the kernel has few
+// centre-only grids (UsesTiles).  The values of points
+// outside a map's domain alternate as the sweeps of the pair leave them: the
+// loaded grid's own after even sweeps (they stay in its LDS buffer), the other
+// grid's after odd ones.
+bool Translator::UsesTiles(const KernelInfo &k) {
+  int direct = 0;
+  for (auto &g : k.grids) direct += g.mode == GridParam::kDirect && g.read;
+  return (k.fusable || k.fuse_rb) && direct <= 4;
+}
+
+std::string Translator::EmitTileKernel(const KernelInfo &k) {
+  std::ostringstream o;
+  const std::string &n = k.name;
+  const GridParam &gi = k.grids[k.fuse_in], &go = k.grids[k.fuse_out];
+  const std::string T = gi.elem, V = gi.dev_view, I = gi.name, O = go.name;
+  const bool rb = k.fuse_rb, domain = k.fuse_domain;
+  const bool red = k.ret_type != "void";
+  const std::string RT = red ? k.ret_type : "float";
+  std::vector<const GridParam *> direct;
+  for (auto &g : k.grids)
+    if (g.mode == GridParam::kDirect && g.read) direct.push_back(&g);
+  std::vector<std::string> sp, sa;
+  for (auto &sc : k.scalars) {
+    sp.push_back(sc.type + " " + sc.name);
+    sa.push_back(sc.name);
+  }
+  std::string fa;
+  for (auto &a : sa) fa += ", " + a;
+  const std::string ACC = "physis_hip::ReduceOp<" + RT + ", RED < 0 ? 0 : RED>";
+  std::vector<std::string> args = {"__PSDomain dom"};
+  if (rb) args.push_back("__PSDomain gd");
+  args.push_back(V + " src");
+  args.push_back(V + " dst");
+  args.push_back(T + " *__restrict__ bg");
+  args.push_back("int store_mid");
+  for (auto *g : direct) args.push_back(g->dev_view + " " + g->name);
+  for (auto &x : sp) args.push_back(x);
+  args.push_back("int tiles_x");
+  args.push_back("int tiles_y");
+  args.push_back("physis_hip::TileReds red");
+  const std::string TD = rb ? "gd" : "dom";
+  o << "// Resident-tile pass of " << n << ": TILE::T sweeps of src per launch "
+       "into dst,\n// the one before the last into bg when store_mid.  red: "
+       "per-block partials of\n// each sweep.\n";
+  o << "template <typename TILE, int RED>\n__global__ __launch_bounds__(TILE::NT) "
+       "void __PSStencilRunT_" << n << "(\n    " << Join(args, ", ") << ") {\n"
+    << "  __shared__ " << T << " lds[2][TILE::kElems];\n"
+       "  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;\n"
+       "  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);\n"
+    << "  const int x0 = " << TD << ".local_min[0] + (b % tiles_x) * TILE::TX;\n"
+       "  b /= tiles_x;\n"
+    << "  const int y0 = " << TD << ".local_min[1] + (b % tiles_y) * TILE::TY;\n"
+    << "  const int z0 = " << TD << ".local_min[2] + (b / tiles_y) * TILE::TZ;\n"
+       "  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];\n"
+       "  const int n = nxy * src.dim[2];\n"
+    << "  const physis_hip::BufWin<" << T << "> dw = physis_hip::BufWin<" << T
+    << ">::Make(dst.p, n, 0, n);\n"
+    << "  const physis_hip::BufWin<" << T << "> bw = physis_hip::BufWin<" << T
+    << ">::Make(bg ? bg : dst.p, n, 0, n);\n";
+  o << "  physis_hip::TilePoint pt[K];\n"
+       "#pragma unroll\n  for (int k = 0; k < K; ++k)\n"
+       "    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);\n";
+  if (domain) {
+    for (auto *g : direct)
+      o << "  const physis_hip::BufWin<" << g->elem << "> " << g->name
+        << "_w = physis_hip::BufWin<" << g->elem << ">::Make(" << g->name
+        << ".p, n, 0, n);\n  " << g->elem << " " << g->name << "_c[K][1];\n";
+    o << "  " << T << " bg_c[K][1];\n  bool in[K];\n"
+         "#pragma unroll\n  for (int k = 0; k < K; ++k) {\n"
+         "    const physis_hip::TilePoint &p = pt[k];\n"
+         "    in[k] = p.at >= 0 && p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&\n"
+         "            p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&\n"
+         "            p.z >= dom.local_min[2] && p.z < dom.local_max[2];\n"
+         "    const bool grid = p.at >= 0 && p.x >= 0 && p.x < nx && p.y >= 0 &&\n"
+         "                      p.y < src.dim[1] && p.z >= 0 && p.z < src.dim[2];\n"
+         "    const int off = p.x + nx * p.y + nxy * p.z;\n"
+         "    bw.template Load<1>(grid && !in[k] ? off : physis_hip::kDrop, bg_c[k]);\n";
+    for (auto *g : direct)
+      o << "    " << g->name << "_w.template Load<1>(in[k] ? off : physis_hip::kDrop, "
+        << g->name << "_c[k]);\n";
+    o << "  }\n";
+  }
+  o << "  physis_hip::LoadTile<TILE, " << (gi.periodic ? "true" : "false")
+    << ">(lds[0], src.p, src.dim, x0, y0, z0);\n  __syncthreads();\n";
+  if (red)
+    o << "  " << RT << " acc[TILE::T];\n"
+         "#pragma unroll\n  for (int t = 0; t < TILE::T; ++t) {\n    acc[t] = 0;\n"
+         "    if constexpr (RED >= 0) acc[t] = " << ACC << "::identity();\n  }\n";
+  o << "  __PSCtx_" << n << " ctx;\n";
+  for (auto &g : k.grids) {
+    const std::string v = &g == &gi || rb ? "src" : (&g == &go ? "dst" : g.name);
+    if (!g.read && !g.emitted) continue;
+    o << "  ctx." << g.name << "_p = " << v << ".p;\n"
+      << "  for (int d = 0; d < 3; ++d) ctx." << g.name << "_dim[d] = "
+      << (domain ? v : "src") << ".dim[d];\n";
+  }
+  o << "#pragma unroll\n  for (int t = 1; t <= TILE::T; ++t) {\n"
+    << "    const " << T << " *const cur = lds[(t - 1) & 1];\n"
+    << "    " << T << " *const nxt = lds[t & 1];\n"
+       "#pragma unroll\n    for (int k = 0; k < TILE::Count(t); ++k) {\n"
+       "      const physis_hip::TilePoint &p = pt[k];\n"
+       "      if (p.at < 0) continue;\n";
+  for (size_t i = 0; i < gi.offsets.size(); ++i) {
+    const auto &off = gi.offsets[i];
+    o << "      ctx." << I << "[" << i << "] = cur[p.at + " << off[0] << " + RX * ("
+      << off[1] << " + RY * (" << off[2] << "))];\n";
+  }
+  for (auto *g : direct)
+    o << "      ctx." << g->name << "_c = " << g->name << "_c[k][0];\n";
+  o << "      ctx." << O << "_e = false;\n";
+  if (red)
+    o << "      const " << RT << " r = " << n << "(p.x, p.y, p.z, ctx" << fa
+      << ");\n      if constexpr (RED >= 0)\n"
+         "        if (k < TILE::Owned(0) && in[k]) acc[t - 1] = " << ACC
+      << "::apply(acc[t - 1], r);\n";
+  else
+    o << "      " << n << "(p.x, p.y, p.z, ctx" << fa << ");\n";
+  o << "      const int off = p.x + nx * p.y + nxy * p.z;\n";
+  if (domain) {
+    o << "      const bool keep = in[k];\n      const " << T << " v[1] = {ctx." << O
+      << "_v};\n"
+         "      if (t < TILE::T) {\n        if (keep)\n          nxt[p.at] = v[0];\n"
+         "        else if (t == 1)\n          nxt[p.at] = bg_c[k][0];\n      }\n";
+  } else if (rb) {
+    size_t c = 0;
+    for (size_t i = 0; i < gi.offsets.size(); ++i)
+      if (!gi.offsets[i][0] && !gi.offsets[i][1] && !gi.offsets[i][2]) c = i;
+    o << "      const bool upd = p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&\n"
+         "          p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&\n"
+         "          p.z >= dom.local_min[2] && p.z < dom.local_max[2] &&\n"
+         "          ((p.x + p.y + p.z + t - 1) & 1) == 0;\n"
+         "      const " << T << " v[1] = {upd ? ctx." << O << "_v : cur[p.at + 0]};\n"
+         "      if (t < TILE::T) nxt[p.at] = v[0];\n"
+         "      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];\n";
+    (void)c;
+  } else {
+    o << "      const " << T << " v[1] = {ctx." << O << "_v};\n"
+         "      if (t < TILE::T) nxt[p.at] = v[0];\n"
+         "      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];\n";
+  }
+  o << "      if (k < TILE::Owned(0)) {\n"
+       "        if (t == TILE::T)\n"
+       "          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);\n"
+       "        if (t == TILE::T - 1 && store_mid)\n"
+       "          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);\n"
+       "      }\n    }\n"
+       "    if (t < TILE::T) __syncthreads();\n  }\n";
+  if (red)
+    o << "  if constexpr (RED >= 0) {\n"
+      << "    __shared__ " << RT << " lds_red[TILE::T][TILE::NT / 64];\n"
+         "#pragma unroll\n    for (int t = 0; t < TILE::T; ++t) {\n"
+      << "      const " << RT << " r = physis_hip::BlockReduce<" << RT
+      << ", RED < 0 ? 0 : RED, TILE::NT>(acc[t], lds_red[t]);\n"
+         "      if (threadIdx.x == 0) ((" << RT << " *)red.p[t])[blockIdx.x] = r;\n"
+         "    }\n  }\n";
+  else
+    o << "  (void)red;\n";
+  o << "}\n\n";
+  // launcher
+  const std::string D = rb ? "physis_hip::WholeDomain(s." + I + ")" : "s.dom";
+  if (red)
+    o << "static int __PSBlocksT_" << n << "(const struct __PSStencil_" << n
+      << " &s) {\n  return physis_hip::TileBlocks(" << D << ");\n}\n\n";
+  std::vector<std::string> la = {"s.dom"};
+  if (rb) la.push_back("d");
+  la.push_back("src");
+  la.push_back("dst");
+  la.push_back("bg");
+  la.push_back("store_mid");
+  for (auto *g : direct)
+    la.push_back("physis_hip::DevView<" + g->dev_view + ">(s." + g->name + ")");
+  for (auto &a : sa) la.push_back("s." + a);
+  la.push_back("g.tiles_x");
+  la.push_back("g.tiles_y");
+  la.push_back("red");
+  const std::string LA = Join(la, ", ");
+  const std::string LP = "(const struct __PSStencil_" + n + " &s, const " + V +
+      " &src, const " + V + " &dst, " + T +
+      " *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {\n";
+  o << "template <typename TILE>\nstatic void __PSLaunchTile_" << n << LP
+    << "  const __PSDomain d = " << D << ";\n"
+       "  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);\n"
+       "  if (g.blocks == 0) return;\n";
+  if (red && k.used_reduce) {
+    o << "  switch (red.p[0] ? s.__reduce_op : -1) {\n";
+    for (const char *op : {"PS_MAX", "PS_MIN", "PS_SUM", "PS_PROD"})
+      o << "    case " << op << ":\n      hipLaunchKernelGGL((__PSStencilRunT_" << n
+        << "<TILE, " << op << ">), dim3(g.blocks), dim3(TILE::NT), 0, stream, " << LA
+        << ");\n      break;\n";
+    o << "    default:\n";
+  } else {
+    o << "  {\n";
+  }
+  o << "      hipLaunchKernelGGL((__PSStencilRunT_" << n
+    << "<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, " << LA
+    << ");\n  }\n}\n\n";
+  o << "template <int T>\nstatic void __PSLaunchT_" << n << LP
+    << "  if (physis_hip::InSmallTiles(" << D << "))\n"
+    << "    __PSLaunchTile_" << n
+    << "<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);\n"
+       "  else\n    __PSLaunchTile_" << n
+    << "<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);\n}\n\n";
+  return o.str();
+}
+
 std::string Translator::EmitRunFunction(const RunSite &r) {
   std::ostringstream o;
   std::vector<std::string> params = {"int iter"};
@@ -3138,8 +3381,12 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
     if (k.ret_type == "void") continue;
     std::string blocks = "__PSBlocks_" + k.name + "(" + si + ")";
     if (fused_pair && k.fuse_domain)
-      blocks = "(__fuse ? __PSBlocks2_" + k.name + "(" + si + ") : " + blocks +
-               ")";
+      blocks = "(!__fuse ? " + blocks +
+               (UsesTiles(k) ? " : " + si + "." + k.grids[k.fuse_in].name +
+                                   "->num_elms <= physis_hip::kTileMaxPoints ? "
+                                   "__PSBlocksT_" + k.name + "(" + si + ")"
+                             : "") +
+               " : __PSBlocks2_" + k.name + "(" + si + "))";
     o << "  physis_hip::MapReducer red" << i << "(" << si << ".__reduce_out, "
       << si << ".__reduce_op, " << PsTypeOf(k.ret_type) << ",\n      " << si
       << ".__reduce_out ? " << blocks << " : 0, iter, __slots);\n";
@@ -3165,10 +3412,21 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
       << "    " << V << " vt = va;\n"
       << "    vt.p = (" << T << " *)__PSHipScratch(8, bytes);\n"
       << "    " << V << " src = va;\n"
-      << "    for (int j = 0; j < iter; ++j) {\n"
+      << "    const bool __small = s0." << g.name
+      << "->num_elms <= physis_hip::kTileMaxPoints;\n"
+      << "    // two iterations a resident-tile pass, an even number of times, so that\n"
+         "    // the count of passes is odd when iter is\n"
+      << "    const int two = __small ? iter / 2 & ~1 : 0;\n"
+      << "    for (int i = 0, j = 0; i < iter; ++j) {\n"
       << "      const " << V << " dst = (j % 2 == 0) ? vt : va;\n"
-      << "      __PSLaunch2_" << k.name << "(s0, src, dst, NULL, stream);\n"
-      << "      src = dst;\n    }\n"
+      << "      const int its = j < two ? 2 : 1;\n"
+      << "      if (!__small)\n        __PSLaunch2_" << k.name
+      << "(s0, src, dst, NULL, stream);\n"
+      << "      else if (its == 2)\n        __PSLaunchT_" << k.name
+      << "<4>(s0, src, dst, NULL, 0, stream, {});\n"
+      << "      else\n        __PSLaunchT_" << k.name
+      << "<2>(s0, src, dst, NULL, 0, stream, {});\n"
+      << "      src = dst;\n      i += its;\n    }\n"
       << "    if (iter % 2) physis_hip::CopyDevice(va.p, vt.p, bytes, stream);\n"
       << "    i0 = iter;\n  }\n";
   }
@@ -3370,7 +3628,8 @@ std::string Translator::Translate() {
   std::ostringstream out;
   out << "// Generated by physisc-hip from " << prog_.file << ".\n"
       << "#define PHYSIS_HIP\n#include \"physis/physis.h\"\n"
-      << "#include \"physis/hip/stencil.h\"\n#include \"physis/hip/run.h\"\n";
+      << "#include \"physis/hip/stencil.h\"\n#include \"physis/hip/run.h\"\n"
+         "#include \"physis/hip/tile.h\"\n";
   for (auto &it : prog_.items)
     if (it.kind == TopItem::kInclude) out << it.include_line << "\n";
   out << "\n#pragma clang fp contract(off)\n\n";

@@ -155,6 +155,8 @@ class Translator {
   std::string EmitLauncher(const KernelInfo &k);
   std::string EmitFusedRunKernel(const KernelInfo &k);
   std::string EmitFusedDomainKernel(const KernelInfo &k);
+  std::string EmitTileKernel(const KernelInfo &k);
+  static bool UsesTiles(const KernelInfo &k);
   // the run-function branch that runs a fusable pair as two-sweep passes
   std::string EmitFusedRun(const KernelInfo &k);
   // Interior split of a wave step at rows y, plane z: the wave-uniform

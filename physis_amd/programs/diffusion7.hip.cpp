@@ -3,6 +3,7 @@
 #include "physis/physis.h"
 #include "physis/hip/stencil.h"
 #include "physis/hip/run.h"
+#include "physis/hip/tile.h"
 
 
 #pragma clang fp contract(off)
@@ -436,6 +437,85 @@ static bool __PSFusable2_diffusion7_kernel(const struct __PSStencil_diffusion7_k
   return true;
 }
 
+// Resident-tile pass of diffusion7_kernel: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_diffusion7_kernel(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, float ce, float cw, float cn, float cs, float ct, float cb, float cc, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_diffusion7_kernel ctx;
+  ctx.g1_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g1_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = src.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g1[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g1[1] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g1[2] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g1[3] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g1[4] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g1[5] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g1[6] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g2_e = false;
+      diffusion7_kernel(p.x, p.y, p.z, ctx, ce, cw, cn, cs, ct, cb, cc);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) nxt[p.at] = v[0];
+      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_diffusion7_kernel<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_diffusion7_kernel<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_diffusion7_kernel<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
+}
+
 // ---------------------------------------------- stencil diffusion7_periodic_kernel
 struct __PSStencil_diffusion7_periodic_kernel {
   __PSDomain dom;
@@ -816,6 +896,85 @@ static bool __PSFusable2_diffusion7_periodic_kernel(const struct __PSStencil_dif
   return true;
 }
 
+// Resident-tile pass of diffusion7_periodic_kernel: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_diffusion7_periodic_kernel(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, float ce, float cw, float cn, float cs, float ct, float cb, float cc, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  physis_hip::LoadTile<TILE, true>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_diffusion7_periodic_kernel ctx;
+  ctx.g1_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g1_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = src.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g1[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g1[1] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g1[2] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g1[3] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g1[4] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g1[5] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g1[6] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g2_e = false;
+      diffusion7_periodic_kernel(p.x, p.y, p.z, ctx, ce, cw, cn, cs, ct, cb, cc);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) nxt[p.at] = v[0];
+      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_diffusion7_periodic_kernel<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_diffusion7_periodic_kernel<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_diffusion7_periodic_kernel<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
+}
+
 static void __PSStencilRun_0(int iter, struct __PSStencil_diffusion7_kernel s0, struct __PSStencil_diffusion7_kernel s1) {
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("diffusion7_kernel, diffusion7_kernel");
@@ -830,16 +989,19 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_diffusion7_kernel s0, 
     const size_t bytes = (size_t)s0.g1->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
+    const bool __small = s0.g1->num_elms <= physis_hip::kTileMaxPoints;
+    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev src = va;
-    int j = 0;
-    if (iter % 2) {
-      __PSLaunch2_diffusion7_kernel(s0, va, vb, NULL, stream);
-      src = vb;
-      j = 1;
-    }
-    for (; j < iter; ++j) {
-      const __PSGrid3DFloat_dev dst = ((iter - 1 - j) % 2 == 0) ? va : vt;
-      __PSLaunch2_diffusion7_kernel(s0, src, dst, j == iter - 1 ? vb.p : NULL, stream);
+    for (int j = 0; j < passes; ++j) {
+      const __PSGrid3DFloat_dev dst = passes % 2 && j == 0 ? vb
+          : ((passes - 1 - j) % 2 == 0) ? va : vt;
+      const int pairs = __small && iter > 2 && (j || iter % 2 == 0) ? 2 : 1;
+      if (__small && pairs == 2)
+        __PSLaunchT_diffusion7_kernel<4>(s0, src, dst, vb.p, (j == passes - 1), stream, {});
+      else if (__small)
+        __PSLaunchT_diffusion7_kernel<2>(s0, src, dst, vb.p, (j == passes - 1), stream, {});
+      else
+        __PSLaunch2_diffusion7_kernel(s0, src, dst, (j == passes - 1) ? vb.p : NULL, stream);
       src = dst;
     }
     i0 = iter;
@@ -874,16 +1036,19 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_diffusion7_periodic_ke
     const size_t bytes = (size_t)s0.g1->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
+    const bool __small = s0.g1->num_elms <= physis_hip::kTileMaxPoints;
+    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev src = va;
-    int j = 0;
-    if (iter % 2) {
-      __PSLaunch2_diffusion7_periodic_kernel(s0, va, vb, NULL, stream);
-      src = vb;
-      j = 1;
-    }
-    for (; j < iter; ++j) {
-      const __PSGrid3DFloat_dev dst = ((iter - 1 - j) % 2 == 0) ? va : vt;
-      __PSLaunch2_diffusion7_periodic_kernel(s0, src, dst, j == iter - 1 ? vb.p : NULL, stream);
+    for (int j = 0; j < passes; ++j) {
+      const __PSGrid3DFloat_dev dst = passes % 2 && j == 0 ? vb
+          : ((passes - 1 - j) % 2 == 0) ? va : vt;
+      const int pairs = __small && iter > 2 && (j || iter % 2 == 0) ? 2 : 1;
+      if (__small && pairs == 2)
+        __PSLaunchT_diffusion7_periodic_kernel<4>(s0, src, dst, vb.p, (j == passes - 1), stream, {});
+      else if (__small)
+        __PSLaunchT_diffusion7_periodic_kernel<2>(s0, src, dst, vb.p, (j == passes - 1), stream, {});
+      else
+        __PSLaunch2_diffusion7_periodic_kernel(s0, src, dst, (j == passes - 1) ? vb.p : NULL, stream);
       src = dst;
     }
     i0 = iter;

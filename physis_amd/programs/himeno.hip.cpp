@@ -3,6 +3,7 @@
 #include "physis/physis.h"
 #include "physis/hip/stencil.h"
 #include "physis/hip/run.h"
+#include "physis/hip/tile.h"
 
 
 #pragma clang fp contract(off)
@@ -891,9 +892,9 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_jacobi_kernel s0, stru
   physis_hip::ReduceSlots __slots;
   const bool __fuse = iter >= 2 && __PSFusable2_jacobi_kernel(s0, s1);
   physis_hip::MapReducer red0(s0.__reduce_out, s0.__reduce_op, PS_FLOAT,
-      s0.__reduce_out ? (__fuse ? __PSBlocks2_jacobi_kernel(s0) : __PSBlocks_jacobi_kernel(s0)) : 0, iter, __slots);
+      s0.__reduce_out ? (!__fuse ? __PSBlocks_jacobi_kernel(s0) : __PSBlocks2_jacobi_kernel(s0)) : 0, iter, __slots);
   physis_hip::MapReducer red1(s1.__reduce_out, s1.__reduce_op, PS_FLOAT,
-      s1.__reduce_out ? (__fuse ? __PSBlocks2_jacobi_kernel(s1) : __PSBlocks_jacobi_kernel(s1)) : 0, iter, __slots);
+      s1.__reduce_out ? (!__fuse ? __PSBlocks_jacobi_kernel(s1) : __PSBlocks2_jacobi_kernel(s1)) : 0, iter, __slots);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.p0, PS_FLOAT);
@@ -903,19 +904,23 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_jacobi_kernel s0, stru
     const size_t bytes = (size_t)s0.p0->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
+    const int passes = iter;
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyDevice(vt.p, va.p, bytes, stream);
-    if (iter % 2) {
+    if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
       physis_hip::CopyDevice(vt2.p, va.p, bytes, stream);
     }
     __PSGrid3DFloat_dev src = va;
-    for (int j = 0; j < iter; ++j) {
-      __PSGrid3DFloat_dev dst = (j % 2 == (iter % 2 ? 0 : 1)) ? va : vt;
-      if (iter % 2 && j < 2) dst = j == 0 ? vt : vt2;
-      __PSLaunch2_jacobi_kernel(s0, src, dst, j == iter - 1, stream, red0.Slot(j), red1.Slot(j));
-      red0.After(j);
-      red1.After(j);
+    for (int j = 0, i = 0; j < passes; ++j) {
+      __PSGrid3DFloat_dev dst = (j % 2 == (passes % 2 ? 0 : 1)) ? va : vt;
+      if (passes % 2 && j < 2) dst = j == 0 ? vt : vt2;
+      const int pairs = 1;
+      __PSLaunch2_jacobi_kernel(s0, src, dst, (j == passes - 1), stream, red0.Slot(i), red1.Slot(i));
+      for (const int e = i + pairs; i < e; ++i) {
+        red0.After(i);
+        red1.After(i);
+      }
       src = dst;
     }
     i0 = iter;
@@ -947,9 +952,9 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_jacobi_kernel s0, stru
   physis_hip::ReduceSlots __slots;
   const bool __fuse = iter >= 2 && __PSFusable2_jacobi_kernel(s0, s1);
   physis_hip::MapReducer red0(s0.__reduce_out, s0.__reduce_op, PS_FLOAT,
-      s0.__reduce_out ? (__fuse ? __PSBlocks2_jacobi_kernel(s0) : __PSBlocks_jacobi_kernel(s0)) : 0, iter, __slots);
+      s0.__reduce_out ? (!__fuse ? __PSBlocks_jacobi_kernel(s0) : __PSBlocks2_jacobi_kernel(s0)) : 0, iter, __slots);
   physis_hip::MapReducer red1(s1.__reduce_out, s1.__reduce_op, PS_FLOAT,
-      s1.__reduce_out ? (__fuse ? __PSBlocks2_jacobi_kernel(s1) : __PSBlocks_jacobi_kernel(s1)) : 0, iter, __slots);
+      s1.__reduce_out ? (!__fuse ? __PSBlocks_jacobi_kernel(s1) : __PSBlocks2_jacobi_kernel(s1)) : 0, iter, __slots);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.p0, PS_FLOAT);
@@ -959,19 +964,23 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_jacobi_kernel s0, stru
     const size_t bytes = (size_t)s0.p0->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
+    const int passes = iter;
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyDevice(vt.p, va.p, bytes, stream);
-    if (iter % 2) {
+    if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
       physis_hip::CopyDevice(vt2.p, va.p, bytes, stream);
     }
     __PSGrid3DFloat_dev src = va;
-    for (int j = 0; j < iter; ++j) {
-      __PSGrid3DFloat_dev dst = (j % 2 == (iter % 2 ? 0 : 1)) ? va : vt;
-      if (iter % 2 && j < 2) dst = j == 0 ? vt : vt2;
-      __PSLaunch2_jacobi_kernel(s0, src, dst, j == iter - 1, stream, red0.Slot(j), red1.Slot(j));
-      red0.After(j);
-      red1.After(j);
+    for (int j = 0, i = 0; j < passes; ++j) {
+      __PSGrid3DFloat_dev dst = (j % 2 == (passes % 2 ? 0 : 1)) ? va : vt;
+      if (passes % 2 && j < 2) dst = j == 0 ? vt : vt2;
+      const int pairs = 1;
+      __PSLaunch2_jacobi_kernel(s0, src, dst, (j == passes - 1), stream, red0.Slot(i), red1.Slot(i));
+      for (const int e = i + pairs; i < e; ++i) {
+        red0.After(i);
+        red1.After(i);
+      }
       src = dst;
     }
     i0 = iter;

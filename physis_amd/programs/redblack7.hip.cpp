@@ -3,6 +3,7 @@
 #include "physis/physis.h"
 #include "physis/hip/stencil.h"
 #include "physis/hip/run.h"
+#include "physis/hip/tile.h"
 
 
 #pragma clang fp contract(off)
@@ -396,6 +397,87 @@ static bool __PSFusableRB_redblack7_kernel(const struct __PSStencil_redblack7_ke
   return true;
 }
 
+// Resident-tile pass of redblack7_kernel: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_redblack7_kernel(
+    __PSDomain dom, __PSDomain gd, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, float ce, float cw, float cn, float cs, float ct, float cb, float cc, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = gd.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = gd.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = gd.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_redblack7_kernel ctx;
+  ctx.g_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g[1] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g[2] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g[3] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g[4] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g[5] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g[6] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g_e = false;
+      redblack7_kernel(p.x, p.y, p.z, ctx, ce, cw, cn, cs, ct, cb, cc);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const bool upd = p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&
+          p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&
+          p.z >= dom.local_min[2] && p.z < dom.local_max[2] &&
+          ((p.x + p.y + p.z + t - 1) & 1) == 0;
+      const float v[1] = {upd ? ctx.g_v : cur[p.at + 0]};
+      if (t < TILE::T) nxt[p.at] = v[0];
+      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = physis_hip::WholeDomain(s.g);
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_redblack7_kernel<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, d, src, dst, bg, store_mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(physis_hip::WholeDomain(s.g)))
+    __PSLaunchTile_redblack7_kernel<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_redblack7_kernel<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
+}
+
 static void __PSStencilRun_0(int iter, struct __PSStencil_redblack7_kernel s0) {
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("redblack7_kernel");
@@ -408,10 +490,21 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_redblack7_kernel s0) {
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
-    for (int j = 0; j < iter; ++j) {
+    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    // two iterations a resident-tile pass, an even number of times, so that
+    // the count of passes is odd when iter is
+    const int two = __small ? iter / 2 & ~1 : 0;
+    for (int i = 0, j = 0; i < iter; ++j) {
       const __PSGrid3DFloat_dev dst = (j % 2 == 0) ? vt : va;
-      __PSLaunch2_redblack7_kernel(s0, src, dst, NULL, stream);
+      const int its = j < two ? 2 : 1;
+      if (!__small)
+        __PSLaunch2_redblack7_kernel(s0, src, dst, NULL, stream);
+      else if (its == 2)
+        __PSLaunchT_redblack7_kernel<4>(s0, src, dst, NULL, 0, stream, {});
+      else
+        __PSLaunchT_redblack7_kernel<2>(s0, src, dst, NULL, 0, stream, {});
       src = dst;
+      i += its;
     }
     if (iter % 2) physis_hip::CopyDevice(va.p, vt.p, bytes, stream);
     i0 = iter;

@@ -3,6 +3,7 @@
 #include "physis/physis.h"
 #include "physis/hip/stencil.h"
 #include "physis/hip/run.h"
+#include "physis/hip/tile.h"
 
 
 #pragma clang fp contract(off)
@@ -424,6 +425,103 @@ static bool __PSFusable2_corners(const struct __PSStencil_corners &s0, const str
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
   return true;
+}
+
+// Resident-tile pass of corners: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_corners(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  float bg_c[K][1];
+  bool in[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const physis_hip::TilePoint &p = pt[k];
+    in[k] = p.at >= 0 && p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&
+            p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&
+            p.z >= dom.local_min[2] && p.z < dom.local_max[2];
+    const bool grid = p.at >= 0 && p.x >= 0 && p.x < nx && p.y >= 0 &&
+                      p.y < src.dim[1] && p.z >= 0 && p.z < src.dim[2];
+    const int off = p.x + nx * p.y + nxy * p.z;
+    bw.template Load<1>(grid && !in[k] ? off : physis_hip::kDrop, bg_c[k]);
+  }
+  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_corners ctx;
+  ctx.g_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = dst.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g[1] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g[2] = cur[p.at + 1 + RX * (-1 + RY * (0))];
+      ctx.g[3] = cur[p.at + -1 + RX * (1 + RY * (0))];
+      ctx.g[4] = cur[p.at + 1 + RX * (1 + RY * (1))];
+      ctx.g[5] = cur[p.at + -1 + RX * (-1 + RY * (-1))];
+      ctx.g[6] = cur[p.at + 1 + RX * (0 + RY * (-1))];
+      ctx.g2_e = false;
+      corners(p.x, p.y, p.z, ctx);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const bool keep = in[k];
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) {
+        if (keep)
+          nxt[p.at] = v[0];
+        else if (t == 1)
+          nxt[p.at] = bg_c[k][0];
+      }
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_corners(const struct __PSStencil_corners &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_corners<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_corners(const struct __PSStencil_corners &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_corners<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_corners<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
 }
 
 // ---------------------------------------------- stencil corners_double
@@ -1360,6 +1458,101 @@ static bool __PSFusable2_inner(const struct __PSStencil_inner &s0, const struct 
   return true;
 }
 
+// Resident-tile pass of inner: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_inner(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, float w, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  float bg_c[K][1];
+  bool in[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const physis_hip::TilePoint &p = pt[k];
+    in[k] = p.at >= 0 && p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&
+            p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&
+            p.z >= dom.local_min[2] && p.z < dom.local_max[2];
+    const bool grid = p.at >= 0 && p.x >= 0 && p.x < nx && p.y >= 0 &&
+                      p.y < src.dim[1] && p.z >= 0 && p.z < src.dim[2];
+    const int off = p.x + nx * p.y + nxy * p.z;
+    bw.template Load<1>(grid && !in[k] ? off : physis_hip::kDrop, bg_c[k]);
+  }
+  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_inner ctx;
+  ctx.g_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = dst.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g[1] = cur[p.at + 1 + RX * (-1 + RY * (0))];
+      ctx.g[2] = cur[p.at + -1 + RX * (1 + RY * (0))];
+      ctx.g[3] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g[4] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g2_e = false;
+      inner(p.x, p.y, p.z, ctx, w);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const bool keep = in[k];
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) {
+        if (keep)
+          nxt[p.at] = v[0];
+        else if (t == 1)
+          nxt[p.at] = bg_c[k][0];
+      }
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_inner(const struct __PSStencil_inner &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_inner<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, s.w, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_inner(const struct __PSStencil_inner &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_inner<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_inner<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
+}
+
 extern "C" {
 
 static PSDomain3D whole(PSGrid3DFloat g) {
@@ -1456,17 +1649,25 @@ static void __PSStencilRun_4(int iter, struct __PSStencil_inner s0, struct __PSS
     const size_t bytes = (size_t)s0.g->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
+    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyDevice(vt.p, va.p, bytes, stream);
-    if (iter % 2) {
+    if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
       physis_hip::CopyDevice(vt2.p, va.p, bytes, stream);
     }
     __PSGrid3DFloat_dev src = va;
-    for (int j = 0; j < iter; ++j) {
-      __PSGrid3DFloat_dev dst = (j % 2 == (iter % 2 ? 0 : 1)) ? va : vt;
-      if (iter % 2 && j < 2) dst = j == 0 ? vt : vt2;
-      __PSLaunch2_inner(s0, src, dst, j == iter - 1, stream, NULL, NULL);
+    for (int j = 0; j < passes; ++j) {
+      __PSGrid3DFloat_dev dst = (j % 2 == (passes % 2 ? 0 : 1)) ? va : vt;
+      if (passes % 2 && j < 2) dst = j == 0 ? vt : vt2;
+      const int pairs = __small && iter > 2 && (j || iter % 2 == 0) ? 2 : 1;
+      if (__small && pairs == 2)
+        __PSLaunchT_inner<4>(s0, src, dst, vb.p, (j == passes - 1), stream, {});
+      else if (__small)
+        __PSLaunchT_inner<2>(s0, src, dst, vb.p, (j == passes - 1), stream, {});
+      else
+        __PSLaunch2_inner(s0, src, dst, (j == passes - 1), stream, NULL, NULL);
       src = dst;
     }
     i0 = iter;

@@ -3,6 +3,7 @@
 #include "physis/physis.h"
 #include "physis/hip/stencil.h"
 #include "physis/hip/run.h"
+#include "physis/hip/tile.h"
 
 
 #pragma clang fp contract(off)
@@ -421,6 +422,103 @@ static bool __PSFusable2_k7(const struct __PSStencil_k7 &s0, const struct __PSSt
   return true;
 }
 
+// Resident-tile pass of k7: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_k7(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  float bg_c[K][1];
+  bool in[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const physis_hip::TilePoint &p = pt[k];
+    in[k] = p.at >= 0 && p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&
+            p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&
+            p.z >= dom.local_min[2] && p.z < dom.local_max[2];
+    const bool grid = p.at >= 0 && p.x >= 0 && p.x < nx && p.y >= 0 &&
+                      p.y < src.dim[1] && p.z >= 0 && p.z < src.dim[2];
+    const int off = p.x + nx * p.y + nxy * p.z;
+    bw.template Load<1>(grid && !in[k] ? off : physis_hip::kDrop, bg_c[k]);
+  }
+  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_k7 ctx;
+  ctx.g_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = dst.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g[1] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g[2] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g[3] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g[4] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g[5] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g[6] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g2_e = false;
+      k7(p.x, p.y, p.z, ctx);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const bool keep = in[k];
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) {
+        if (keep)
+          nxt[p.at] = v[0];
+        else if (t == 1)
+          nxt[p.at] = bg_c[k][0];
+      }
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_k7(const struct __PSStencil_k7 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_k7<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_k7(const struct __PSStencil_k7 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_k7<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_k7<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
+}
+
 // ---------------------------------------------- stencil k7p
 struct __PSStencil_k7p {
   __PSDomain dom;
@@ -779,6 +877,85 @@ static bool __PSFusable2_k7p(const struct __PSStencil_k7p &s0, const struct __PS
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
   return true;
+}
+
+// Resident-tile pass of k7p: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_k7p(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  physis_hip::LoadTile<TILE, true>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_k7p ctx;
+  ctx.g_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = src.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g[1] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g[2] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g[3] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g[4] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g[5] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g[6] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g2_e = false;
+      k7p(p.x, p.y, p.z, ctx);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) nxt[p.at] = v[0];
+      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_k7p<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_k7p<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_k7p<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
 }
 
 // ---------------------------------------------- stencil k7n
@@ -1195,6 +1372,85 @@ static bool __PSFusable2_k7n(const struct __PSStencil_k7n &s0, const struct __PS
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
   return true;
+}
+
+// Resident-tile pass of k7n: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_k7n(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_k7n ctx;
+  ctx.g1_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g1_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = src.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g1[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g1[1] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g1[2] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g1[3] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g1[4] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g1[5] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g1[6] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g2_e = false;
+      k7n(p.x, p.y, p.z, ctx);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) nxt[p.at] = v[0];
+      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_k7n<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_k7n<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_k7n<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
 }
 
 // ---------------------------------------------- stencil kasym
@@ -2048,6 +2304,123 @@ static bool __PSFusable2_k27(const struct __PSStencil_k27 &s0, const struct __PS
   return true;
 }
 
+// Resident-tile pass of k27: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_k27(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  float bg_c[K][1];
+  bool in[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const physis_hip::TilePoint &p = pt[k];
+    in[k] = p.at >= 0 && p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&
+            p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&
+            p.z >= dom.local_min[2] && p.z < dom.local_max[2];
+    const bool grid = p.at >= 0 && p.x >= 0 && p.x < nx && p.y >= 0 &&
+                      p.y < src.dim[1] && p.z >= 0 && p.z < src.dim[2];
+    const int off = p.x + nx * p.y + nxy * p.z;
+    bw.template Load<1>(grid && !in[k] ? off : physis_hip::kDrop, bg_c[k]);
+  }
+  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_k27 ctx;
+  ctx.g_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = dst.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g[1] = cur[p.at + 1 + RX * (0 + RY * (-1))];
+      ctx.g[2] = cur[p.at + -1 + RX * (0 + RY * (-1))];
+      ctx.g[3] = cur[p.at + 0 + RX * (1 + RY * (-1))];
+      ctx.g[4] = cur[p.at + 1 + RX * (1 + RY * (-1))];
+      ctx.g[5] = cur[p.at + -1 + RX * (1 + RY * (-1))];
+      ctx.g[6] = cur[p.at + 0 + RX * (-1 + RY * (-1))];
+      ctx.g[7] = cur[p.at + 1 + RX * (-1 + RY * (-1))];
+      ctx.g[8] = cur[p.at + -1 + RX * (-1 + RY * (-1))];
+      ctx.g[9] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g[10] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g[11] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g[12] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g[13] = cur[p.at + 1 + RX * (1 + RY * (0))];
+      ctx.g[14] = cur[p.at + -1 + RX * (1 + RY * (0))];
+      ctx.g[15] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g[16] = cur[p.at + 1 + RX * (-1 + RY * (0))];
+      ctx.g[17] = cur[p.at + -1 + RX * (-1 + RY * (0))];
+      ctx.g[18] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g[19] = cur[p.at + 1 + RX * (0 + RY * (1))];
+      ctx.g[20] = cur[p.at + -1 + RX * (0 + RY * (1))];
+      ctx.g[21] = cur[p.at + 0 + RX * (1 + RY * (1))];
+      ctx.g[22] = cur[p.at + 1 + RX * (1 + RY * (1))];
+      ctx.g[23] = cur[p.at + -1 + RX * (1 + RY * (1))];
+      ctx.g[24] = cur[p.at + 0 + RX * (-1 + RY * (1))];
+      ctx.g[25] = cur[p.at + 1 + RX * (-1 + RY * (1))];
+      ctx.g[26] = cur[p.at + -1 + RX * (-1 + RY * (1))];
+      ctx.g2_e = false;
+      k27(p.x, p.y, p.z, ctx);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const bool keep = in[k];
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) {
+        if (keep)
+          nxt[p.at] = v[0];
+        else if (t == 1)
+          nxt[p.at] = bg_c[k][0];
+      }
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_k27(const struct __PSStencil_k27 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_k27<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_k27(const struct __PSStencil_k27 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_k27<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_k27<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
+}
+
 // ---------------------------------------------- stencil k27p
 struct __PSStencil_k27p {
   __PSDomain dom;
@@ -2511,6 +2884,105 @@ static bool __PSFusable2_k27p(const struct __PSStencil_k27p &s0, const struct __
   return true;
 }
 
+// Resident-tile pass of k27p: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_k27p(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  physis_hip::LoadTile<TILE, true>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_k27p ctx;
+  ctx.g_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
+  ctx.g2_p = dst.p;
+  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = src.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g[1] = cur[p.at + 1 + RX * (0 + RY * (-1))];
+      ctx.g[2] = cur[p.at + -1 + RX * (0 + RY * (-1))];
+      ctx.g[3] = cur[p.at + 0 + RX * (1 + RY * (-1))];
+      ctx.g[4] = cur[p.at + 1 + RX * (1 + RY * (-1))];
+      ctx.g[5] = cur[p.at + -1 + RX * (1 + RY * (-1))];
+      ctx.g[6] = cur[p.at + 0 + RX * (-1 + RY * (-1))];
+      ctx.g[7] = cur[p.at + 1 + RX * (-1 + RY * (-1))];
+      ctx.g[8] = cur[p.at + -1 + RX * (-1 + RY * (-1))];
+      ctx.g[9] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g[10] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g[11] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g[12] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g[13] = cur[p.at + 1 + RX * (1 + RY * (0))];
+      ctx.g[14] = cur[p.at + -1 + RX * (1 + RY * (0))];
+      ctx.g[15] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g[16] = cur[p.at + 1 + RX * (-1 + RY * (0))];
+      ctx.g[17] = cur[p.at + -1 + RX * (-1 + RY * (0))];
+      ctx.g[18] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g[19] = cur[p.at + 1 + RX * (0 + RY * (1))];
+      ctx.g[20] = cur[p.at + -1 + RX * (0 + RY * (1))];
+      ctx.g[21] = cur[p.at + 0 + RX * (1 + RY * (1))];
+      ctx.g[22] = cur[p.at + 1 + RX * (1 + RY * (1))];
+      ctx.g[23] = cur[p.at + -1 + RX * (1 + RY * (1))];
+      ctx.g[24] = cur[p.at + 0 + RX * (-1 + RY * (1))];
+      ctx.g[25] = cur[p.at + 1 + RX * (-1 + RY * (1))];
+      ctx.g[26] = cur[p.at + -1 + RX * (-1 + RY * (1))];
+      ctx.g2_e = false;
+      k27p(p.x, p.y, p.z, ctx);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const float v[1] = {ctx.g2_v};
+      if (t < TILE::T) nxt[p.at] = v[0];
+      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = s.dom;
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_k27p<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(s.dom))
+    __PSLaunchTile_k27p<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_k27p<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
+}
+
 // ---------------------------------------------- stencil k27i
 struct __PSStencil_k27i {
   __PSDomain dom;
@@ -2878,17 +3350,25 @@ static void __PSStencilRun_7(int iter, struct __PSStencil_k7 s0, struct __PSSten
     const size_t bytes = (size_t)s0.g->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
+    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyDevice(vt.p, va.p, bytes, stream);
-    if (iter % 2) {
+    if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
       physis_hip::CopyDevice(vt2.p, va.p, bytes, stream);
     }
     __PSGrid3DFloat_dev src = va;
-    for (int j = 0; j < iter; ++j) {
-      __PSGrid3DFloat_dev dst = (j % 2 == (iter % 2 ? 0 : 1)) ? va : vt;
-      if (iter % 2 && j < 2) dst = j == 0 ? vt : vt2;
-      __PSLaunch2_k7(s0, src, dst, j == iter - 1, stream, NULL, NULL);
+    for (int j = 0; j < passes; ++j) {
+      __PSGrid3DFloat_dev dst = (j % 2 == (passes % 2 ? 0 : 1)) ? va : vt;
+      if (passes % 2 && j < 2) dst = j == 0 ? vt : vt2;
+      const int pairs = __small && iter > 2 && (j || iter % 2 == 0) ? 2 : 1;
+      if (__small && pairs == 2)
+        __PSLaunchT_k7<4>(s0, src, dst, vb.p, (j == passes - 1), stream, {});
+      else if (__small)
+        __PSLaunchT_k7<2>(s0, src, dst, vb.p, (j == passes - 1), stream, {});
+      else
+        __PSLaunch2_k7(s0, src, dst, (j == passes - 1), stream, NULL, NULL);
       src = dst;
     }
     i0 = iter;
@@ -3354,6 +3834,87 @@ static bool __PSFusableRB_krb(const struct __PSStencil_krb &s0) {
   return true;
 }
 
+// Resident-tile pass of krb: TILE::T sweeps of src per launch into dst,
+// the one before the last into bg when store_mid.  red: per-block partials of
+// each sweep.
+template <typename TILE, int RED>
+__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_krb(
+    __PSDomain dom, __PSDomain gd, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
+  __shared__ float lds[2][TILE::kElems];
+  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
+  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
+  const int x0 = gd.local_min[0] + (b % tiles_x) * TILE::TX;
+  b /= tiles_x;
+  const int y0 = gd.local_min[1] + (b % tiles_y) * TILE::TY;
+  const int z0 = gd.local_min[2] + (b / tiles_y) * TILE::TZ;
+  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
+  const int n = nxy * src.dim[2];
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
+  physis_hip::TilePoint pt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
+  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
+  __syncthreads();
+  __PSCtx_krb ctx;
+  ctx.g_p = src.p;
+  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
+#pragma unroll
+  for (int t = 1; t <= TILE::T; ++t) {
+    const float *const cur = lds[(t - 1) & 1];
+    float *const nxt = lds[t & 1];
+#pragma unroll
+    for (int k = 0; k < TILE::Count(t); ++k) {
+      const physis_hip::TilePoint &p = pt[k];
+      if (p.at < 0) continue;
+      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (0))];
+      ctx.g[1] = cur[p.at + 1 + RX * (0 + RY * (0))];
+      ctx.g[2] = cur[p.at + -1 + RX * (0 + RY * (0))];
+      ctx.g[3] = cur[p.at + 0 + RX * (1 + RY * (0))];
+      ctx.g[4] = cur[p.at + 0 + RX * (-1 + RY * (0))];
+      ctx.g[5] = cur[p.at + 0 + RX * (0 + RY * (-1))];
+      ctx.g[6] = cur[p.at + 0 + RX * (0 + RY * (1))];
+      ctx.g_e = false;
+      krb(p.x, p.y, p.z, ctx);
+      const int off = p.x + nx * p.y + nxy * p.z;
+      const bool upd = p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&
+          p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&
+          p.z >= dom.local_min[2] && p.z < dom.local_max[2] &&
+          ((p.x + p.y + p.z + t - 1) & 1) == 0;
+      const float v[1] = {upd ? ctx.g_v : cur[p.at + 0]};
+      if (t < TILE::T) nxt[p.at] = v[0];
+      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
+      if (k < TILE::Owned(0)) {
+        if (t == TILE::T)
+          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+        if (t == TILE::T - 1 && store_mid)
+          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
+      }
+    }
+    if (t < TILE::T) __syncthreads();
+  }
+  (void)red;
+}
+
+template <typename TILE>
+static void __PSLaunchTile_krb(const struct __PSStencil_krb &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  const __PSDomain d = physis_hip::WholeDomain(s.g);
+  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
+  if (g.blocks == 0) return;
+  {
+      hipLaunchKernelGGL((__PSStencilRunT_krb<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, d, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
+  }
+}
+
+template <int T>
+static void __PSLaunchT_krb(const struct __PSStencil_krb &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
+  if (physis_hip::InSmallTiles(physis_hip::WholeDomain(s.g)))
+    __PSLaunchTile_krb<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
+  else
+    __PSLaunchTile_krb<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
+}
+
 // ---------------------------------------------- stencil krbp
 struct __PSStencil_krbp {
   __PSDomain dom;
@@ -3564,10 +4125,21 @@ static void __PSStencilRun_10(int iter, struct __PSStencil_krb s0) {
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
-    for (int j = 0; j < iter; ++j) {
+    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    // two iterations a resident-tile pass, an even number of times, so that
+    // the count of passes is odd when iter is
+    const int two = __small ? iter / 2 & ~1 : 0;
+    for (int i = 0, j = 0; i < iter; ++j) {
       const __PSGrid3DFloat_dev dst = (j % 2 == 0) ? vt : va;
-      __PSLaunch2_krb(s0, src, dst, NULL, stream);
+      const int its = j < two ? 2 : 1;
+      if (!__small)
+        __PSLaunch2_krb(s0, src, dst, NULL, stream);
+      else if (its == 2)
+        __PSLaunchT_krb<4>(s0, src, dst, NULL, 0, stream, {});
+      else
+        __PSLaunchT_krb<2>(s0, src, dst, NULL, 0, stream, {});
       src = dst;
+      i += its;
     }
     if (iter % 2) physis_hip::CopyDevice(va.p, vt.p, bytes, stream);
     i0 = iter;
