@@ -103,6 +103,19 @@ __device__ __forceinline__ T BlockReduce(T v, T *lds) {
   return r;
 }
 
+// The value of the lane before / after this one (undefined in the first /
+// last lane of the wave): one DPP move.
+__device__ __forceinline__ float LaneBefore(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138,
+                                         0xf, 0xf, true));  // wave_shr:1
+}
+__device__ __forceinline__ float LaneAfter(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130,
+                                         0xf, 0xf, true));  // wave_shl:1
+}
+
 // ------------------------------------------------------- XCD-aware numbering
 // Hardware dispatch places block b on XCD (b % 8).  Renumbering so that each
 // XCD receives a contiguous range of logical tiles keeps a tile's y- and

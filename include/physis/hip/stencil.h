@@ -482,6 +482,23 @@ __device__ __forceinline__ int RingSlot(int base, int k) {
   return s >= NSLOT ? s - NSLOT : s;
 }
 
+// ------------------------------------------------------------ rows passes
+// Columns of a rows pass (several sweeps of a 2-D map pair in registers, one
+// wave per block): of the wave's 256 columns the four at either end go stale
+// sweep by sweep, so that tiles lie 248 apart.
+constexpr int kRowsTX = 248, kRowsHalo = 4;
+
+// A row in registers: the lane's four points and the points beside them.
+struct RowRegs {
+  float v[6];
+  __device__ __forceinline__ void Set(const float (&own)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[1 + i] = own[i];
+    v[0] = LaneBefore(own[3]);
+    v[5] = LaneAfter(own[0]);
+  }
+};
+
 // ------------------------------------------------------ launch arithmetic
 // Host-side tile counts of a run kernel over a domain.
 struct RunShape {

@@ -1118,12 +1118,12 @@ void Translator::AnalyzeFusion(KernelInfo &k) {
   auto no = [&](const std::string &w) { k.fuse_why = w; };
   if (!cfg_.two_sweep) return no("HIP_TWO_SWEEP = false");
   if (!k.fast) return no("not a 2.5D run kernel");
-  if (k.rows2d) return no("a 2-D map");
   if (k.index_rebound) return no("an index parameter is rebound");
   if (k.used_rb) {
     // one pass per red-black iteration: the map reads only the grid it
     // updates, at offsets of at most one point including the centre, and
     // emits it once, unconditionally, at the top of its body
+    if (k.rows2d) return no("a 2-D red-black map");
     if (k.ret_type != "void") return no("a reducing red-black map");
     int gi = -1;
     for (int i = 0; i < (int)k.grids.size(); ++i) {
@@ -1193,6 +1193,13 @@ void Translator::AnalyzeFusion(KernelInfo &k) {
   if (!top) return no("the emit is conditional");
   k.fuse_in = in;
   k.fuse_out = out;
+  if (k.rows2d) {
+    // pairs over a domain inside the grid, several sweeps in registers
+    if (direct || k.ret_type != "void" || g.periodic)
+      return no("a 2-D map with centre-only grids, periodic gets or a result");
+    k.fusable = k.fuse_domain = true;
+    return;
+  }
   std::string whole_why;
   if (direct == 0 && k.ret_type == "void") {
     FuseScan scan(k);
@@ -2707,7 +2714,9 @@ std::string Translator::EmitKernel(KernelInfo &k) {
   s += EmitDeviceFunction(k);
   s += k.fast ? EmitFastRunKernel(k) : EmitGenericRunKernel(k);
   s += EmitLauncher(k);
-  if (k.fusable || k.fuse_rb)
+  if (k.fusable && k.rows2d)
+    s += EmitRowsKernel(k);
+  else if (k.fusable || k.fuse_rb)
     s += (k.fuse_domain ? EmitFusedDomainKernel(k) : EmitFusedRunKernel(k)) +
          (UsesTiles(k) ? EmitTileKernel(k) : "");
   return s;
@@ -2716,6 +2725,7 @@ std::string Translator::EmitKernel(KernelInfo &k) {
 // The run-function branch of a fusable pair (s0, s1) = k(a -> b), k(b -> a):
 // every pair of the run is one two-sweep pass when __fuse holds.
 std::string Translator::EmitFusedRun(const KernelInfo &k) {
+  if (k.rows2d) return EmitFusedRowsRun(k);
   std::ostringstream o;
   const GridParam &gi = k.grids[k.fuse_in], &go = k.grids[k.fuse_out];
   const std::string V = gi.dev_view, T = gi.elem;
@@ -2782,16 +2792,18 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
       << "      src = dst;\n    }\n";
   } else {
     // Points outside the domain keep a's values in a, so the scratch grids
-    // the passes write start as copies of a (stores stay inside the
+    // the passes write start with a's values there (stores stay inside the
     // domain).  Even counts ping-pong a -> t -> a ...; odd counts (>= 3) go
     // a -> t -> t2 -> a -> t -> a ... (b's values outside the domain are
     // read by every pass, so b cannot hold a pass).  The last pass writes a,
     // and its last but one sweep to b.
     o << "    " << V << " vt2 = va;\n"
-      << "    physis_hip::CopyDevice(vt.p, va.p, bytes, stream);\n"
+      << "    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], "
+         "s0.dom, stream);\n"
       << "    if (passes % 2) {\n"
       << "      vt2.p = (" << T << " *)__PSHipScratch(9, bytes);\n"
-      << "      physis_hip::CopyDevice(vt2.p, va.p, bytes, stream);\n    }\n"
+      << "      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], "
+         "s0.dom, stream);\n    }\n"
       << "    " << V << " src = va;\n"
       << "    for (int j = 0" << (red ? ", i = 0" : "") << "; j < passes; ++j) {\n"
       << "      " << V << " dst = (j % 2 == (passes % 2 ? 0 : 1)) ? va : vt;\n"
@@ -3155,7 +3167,7 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
 bool Translator::UsesTiles(const KernelInfo &k) {
   int direct = 0;
   for (auto &g : k.grids) direct += g.mode == GridParam::kDirect && g.read;
-  return (k.fusable || k.fuse_rb) && direct <= 4;
+  return (k.fusable || k.fuse_rb) && !k.rows2d && direct <= 4;
 }
 
 std::string Translator::EmitTileKernel(const KernelInfo &k) {
@@ -3350,6 +3362,179 @@ std::string Translator::EmitTileKernel(const KernelInfo &k) {
     << "<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);\n"
        "  else\n    __PSLaunchTile_" << n
     << "<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);\n}\n\n";
+  return o.str();
+}
+
+// Rows pass of a fusable 2-D map pair over a domain inside the grid: T sweeps
+// per launch in the registers of one wave, no LDS and no barrier.  The wave
+// marches y over a 256-column tile; sweep t's newest three rows are a register
+// queue (the row of step s - 2, s - 1 and s in slots (k + 1) % 3, (k + 2) % 3
+// and k), the points beside a lane's four come from its neighbours by DPP, and
+// sweep t computes row s - t from sweep t - 1's queue.  A point outside the
+// domain has the other grid's value after odd sweeps (b's, loaded) and its own
+// after even ones: from the third row of the queue two sweeps up.
+std::string Translator::EmitRowsKernel(const KernelInfo &k) {
+  std::ostringstream o;
+  const std::string &n = k.name;
+  const GridParam &gi = k.grids[k.fuse_in], &go = k.grids[k.fuse_out];
+  const std::string V = gi.dev_view, I = gi.name, O = go.name;
+  std::vector<std::string> args = {"__PSDomain dom", V + " src", V + " dst",
+                                   "float *__restrict__ bg", "int store_mid"};
+  std::string fa;
+  std::vector<std::string> la = {"d", "src", "dst", "bg", "store_mid"};
+  for (auto &sc : k.scalars) {
+    args.push_back(sc.type + " " + sc.name);
+    fa += ", " + sc.name;
+    la.push_back("s." + sc.name);
+  }
+  args.push_back("physis_hip::RunShape sh");
+  la.push_back("sh");
+  o << "// Rows pass of " << n << ": T sweeps of src into dst, the one before the\n"
+       "// last into bg when store_mid.\n"
+    << "template <int T>\n__global__ __launch_bounds__(64) void __PSStencilRunR_" << n
+    << "(\n    " << Join(args, ", ") << ") {\n"
+       "  constexpr int PD = 3;\n"
+       "  const int lane = threadIdx.x;\n"
+       "  const physis_hip::TileCoord tc = physis_hip::TileOf(sh.tiles_x, 1);\n"
+       "  const int xs = (sh.x_first_tile + tc.bx) * physis_hip::kRowsTX -\n"
+       "                 physis_hip::kRowsHalo + lane * 4;\n"
+       "  const int zb = dom.local_min[2] + tc.bz * sh.zchunk;\n"
+       "  const int ze = min(zb + sh.zchunk, dom.local_max[2]);\n"
+       "  if (zb >= ze) return;\n"
+       "  const int nx = src.dim[0], n = nx * src.dim[2];\n"
+       "  const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, "
+       "(long)(zb - T - 1) * nx, (long)(ze + T + 1) * nx);\n"
+       "  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg, n, "
+       "(long)(zb - T - 1) * nx, (long)(ze + T + 1) * nx);\n"
+       "  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, "
+       "(long)zb * nx, (long)ze * nx);\n"
+       "  const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(bg, n, "
+       "(long)zb * nx, (long)ze * nx);\n"
+       "  unsigned xm = 0;  // the lane's points inside the domain's columns\n"
+       "#pragma unroll\n  for (int i = 0; i < 4; ++i)\n"
+       "    if (xs + i >= dom.local_min[0] && xs + i < dom.local_max[0]) xm |= 1u << i;\n"
+       "  const bool xin = __all(xm == 15u);\n"
+       "  const unsigned om = lane >= 1 && lane <= 62 ? xm : 0u;\n"
+       "  const auto zin = [&](int z) { return z >= dom.local_min[2] && z < dom.local_max[2]; };\n"
+       "  float ld[PD][4], lb[PD][4];\n"
+       "  // row z of src, and of b one row behind where the domain leaves points out\n"
+       "  const auto load = [&](int z, int k) {\n"
+       "    aw.template Load<4>(xs + z * nx, ld[k]);\n"
+       "    bw.template Load<4>(xm == 15u && zin(z - 1) ? physis_hip::kDrop\n"
+       "                                                : xs + (z - 1) * nx, lb[k]);\n"
+       "  };\n"
+       "  physis_hip::RowRegs q[T][3];\n"
+       "#pragma unroll\n  for (int t = 0; t < T; ++t)\n"
+       "#pragma unroll\n    for (int k = 0; k < 3; ++k)\n"
+       "#pragma unroll\n      for (int i = 0; i < 6; ++i) q[t][k].v[i] = 0.0f;\n"
+    << "  __PSCtx_" << n << " ctx;\n";
+  for (const GridParam *g : {&gi, &go})
+    o << "  ctx." << g->name << "_p = " << (g == &gi ? "src" : "dst") << ".p;\n"
+      << "  ctx." << g->name << "_dim[0] = nx;\n"
+      << "  ctx." << g->name << "_dim[1] = src.dim[2];\n"
+      << "  ctx." << g->name << "_dim[2] = 1;\n";
+  o << "#pragma unroll\n  for (int k = 0; k < PD; ++k) load(zb - T + k, k);\n"
+       "  for (int sc = zb - T; sc < ze + T; sc += 3) {\n"
+       "#pragma unroll\n    for (int k = 0; k < 3; ++k) {\n"
+       "      const int s = sc + k;\n"
+       "      q[0][k].Set(ld[k]);\n"
+       "      float b[4];\n"
+       "#pragma unroll\n      for (int i = 0; i < 4; ++i) b[i] = lb[k][i];\n"
+       "      load(s + PD, k);\n"
+       "#pragma unroll\n      for (int t = 1; t <= T; ++t) {\n"
+       "        const int z = s - t;\n"
+       "        float v[4];\n"
+       "        const auto pts = [&](auto inside) {\n"
+       "#pragma unroll\n          for (int i = 0; i < 4; ++i) {\n";
+  for (size_t i = 0; i < gi.offsets.size(); ++i) {
+    const auto &off = gi.offsets[i];
+    o << "            ctx." << I << "[" << i << "] = q[t - 1][(k + "
+      << (off[2] == 0 ? 2 : (off[2] > 0 ? 0 : 1)) << ") % 3].v[1 + i + " << off[0]
+      << "];\n";
+  }
+  o << "            ctx." << O << "_e = false;\n"
+    << "            " << n << "(xs + i, z, ctx" << fa << ");\n"
+    << "            v[i] = ctx." << O << "_v;\n"
+       "            if constexpr (!decltype(inside)::value)\n"
+       "              if (!((xm >> i) & 1u && zin(z)))\n"
+       "                v[i] = t == 1 ? b[i] : q[t == 1 ? 0 : t - 2][(k + 1) % 3].v[1 + i];\n"
+       "          }\n        };\n"
+       "        if (xin && zin(z))\n          pts(physis_hip::Flag<true>{});\n"
+       "        else\n          pts(physis_hip::Flag<false>{});\n"
+       "        if (t < T) q[t == T ? 0 : t][k].Set(v);\n"
+       "        if (om && z >= zb && z < ze) {\n"
+       "          if (t == T)\n"
+       "            physis_hip::StoreMasked<float, 4>(dw, xs + z * nx, v, om);\n"
+       "          else if (t == T - 1 && store_mid)\n"
+       "            physis_hip::StoreMasked<float, 4>(mw, xs + z * nx, v, om);\n"
+       "        }\n      }\n    }\n  }\n}\n\n";
+  o << "template <int T>\nstatic void __PSLaunchR_" << n << "(const struct __PSStencil_"
+    << n << " &s, const " << V << " &src, const " << V
+    << " &dst, float *bg, int store_mid, hipStream_t stream) {\n"
+    << "  const __PSDomain d = physis_hip::RowDomain(s.dom);\n"
+       "  static int per_cu = physis_hip::BlocksPerCU((const void *)__PSStencilRunR_"
+    << n << "<T>, 64);\n"
+    << "  const physis_hip::RunShape sh = physis_hip::PlanRun(d, physis_hip::kRowsTX, 1, "
+       "per_cu,\n      physis_hip::WindowChunkLimitRows({s." << I << ", s." << O
+    << "}, T + 1), 2 * T + 3);\n"
+       "  if (sh.blocks == 0) return;\n"
+       "  hipLaunchKernelGGL(__PSStencilRunR_" << n << "<T>, dim3(sh.blocks), dim3(64), 0, "
+       "stream, " << Join(la, ", ") << ");\n}\n\n";
+  o << "// The pair (s0, s1) is " << n << "(a -> b), " << n
+    << "(b -> a) over one domain strictly\n// inside the grids, with the same "
+       "scalars: it may run as rows passes.\n"
+    << "static bool __PSFusable2_" << n << "(const struct __PSStencil_" << n
+    << " &s0, const struct __PSStencil_" << n << " &s1) {\n"
+    << "  static const bool off = getenv(\"PHYSIS_HIP_NO_FUSE\") != NULL;\n"
+    << "  const __PSGrid *a = s0." << I << ", *b = s0." << O << ";\n"
+    << "  if (off || !a || !b || a == b || s1." << I << " != b || s1." << O
+    << " != a) return false;\n"
+       "  if (a->num_dims != 2 || b->num_dims != 2) return false;\n"
+       "  for (int d = 0; d < 2; ++d) {\n"
+       "    if (a->dim[d] != b->dim[d]) return false;\n"
+       "    if (s0.dom.local_min[d] != s1.dom.local_min[d] ||\n"
+       "        s0.dom.local_max[d] != s1.dom.local_max[d]) return false;\n"
+       "    if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||\n"
+       "        s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;\n"
+       "  }\n";
+  for (auto &sc : k.scalars)
+    o << "  if (__builtin_memcmp(&s0." << sc.name << ", &s1." << sc.name
+      << ", sizeof(s0." << sc.name << "))) return false;\n";
+  o << "  return true;\n}\n\n";
+  return o.str();
+}
+
+// The run-function branch of a 2-D pair: rows passes of two pairs each (four
+// sweeps), the first of one pair when the count is odd and both when there
+// are only two, ping-ponging as the passes of a 3-D pair over a domain do.
+std::string Translator::EmitFusedRowsRun(const KernelInfo &k) {
+  std::ostringstream o;
+  const GridParam &gi = k.grids[k.fuse_in], &go = k.grids[k.fuse_out];
+  const std::string V = gi.dev_view, &n = k.name;
+  o << "  int i0 = 0;\n  if (__fuse) {\n"
+    << "    physis_hip::CheckGrid3D(s0." << gi.name << ", " << gi.ps_type << ");\n"
+    << "    physis_hip::CheckGrid3D(s0." << go.name << ", " << go.ps_type << ");\n"
+    << "    const " << V << " va = physis_hip::RowView<" << V << ">(s0." << gi.name << ");\n"
+    << "    float *const b = physis_hip::RowView<" << V << ">(s0." << go.name << ").p;\n"
+    << "    const size_t bytes = (size_t)s0." << gi.name << "->num_elms * sizeof(float);\n"
+    << "    const int passes = iter == 2 ? 2 : (iter + 1) / 2;\n"
+    << "    " << V << " vt = va, vt2 = va;\n"
+    << "    vt.p = (float *)__PSHipScratch(8, bytes);\n"
+    << "    const __PSDomain d = physis_hip::RowDomain(s0.dom);\n"
+    << "    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], 1, va.dim[2], d, stream);\n"
+    << "    if (passes % 2) {\n"
+    << "      vt2.p = (float *)__PSHipScratch(9, bytes);\n"
+    << "      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], 1, va.dim[2], d, stream);\n    }\n"
+    << "    " << V << " src = va;\n"
+    << "    for (int j = 0; j < passes; ++j) {\n"
+    << "      " << V << " dst = (j % 2 == (passes % 2 ? 0 : 1)) ? va : vt;\n"
+    << "      if (passes % 2 && j < 2) dst = j == 0 ? vt : vt2;\n"
+    << "      if (iter > 2 && (j || iter % 2 == 0))\n"
+    << "        __PSLaunchR_" << n << "<4>(s0, src, dst, b, j == passes - 1, stream);\n"
+    << "      else\n"
+    << "        __PSLaunchR_" << n << "<2>(s0, src, dst, b, j == passes - 1, stream);\n"
+    << "      src = dst;\n    }\n"
+    << "    i0 = iter;\n  }\n";
   return o.str();
 }
 

@@ -156,6 +156,8 @@ class Translator {
   std::string EmitFusedRunKernel(const KernelInfo &k);
   std::string EmitFusedDomainKernel(const KernelInfo &k);
   std::string EmitTileKernel(const KernelInfo &k);
+  std::string EmitRowsKernel(const KernelInfo &k);
+  std::string EmitFusedRowsRun(const KernelInfo &k);
   static bool UsesTiles(const KernelInfo &k);
   // the run-function branch that runs a fusable pair as two-sweep passes
   std::string EmitFusedRun(const KernelInfo &k);

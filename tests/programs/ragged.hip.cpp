@@ -721,7 +721,7 @@ static struct __PSStencil_corners2d __PSStencilMap_corners2d(
 //   g  staged x[-1,1] y[-0,0] z[-1,1] non-periodic
 //     offsets 0:(0,0,0) 1:(1,0,-1) 2:(-1,0,1) 3:(1,0,0)
 //   g2  not read, emitted
-//   two-sweep fusion of map pairs: no (a 2-D map)
+//   two-sweep fusion of map pairs: yes, over a domain inside the grid
 struct __PSCtx_corners2d {
   float g[4];
   const float *g_p;
@@ -874,6 +874,127 @@ static int __PSRun_corners2d(const struct __PSStencil_corners2d &s, hipStream_t 
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_corners2d<4>(s, stream, red)
          : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_corners2d<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_corners2d<1>(s, stream, red);
+}
+
+// Rows pass of corners2d: T sweeps of src into dst, the one before the
+// last into bg when store_mid.
+template <int T>
+__global__ __launch_bounds__(64) void __PSStencilRunR_corners2d(
+    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, physis_hip::RunShape sh) {
+  constexpr int PD = 3;
+  const int lane = threadIdx.x;
+  const physis_hip::TileCoord tc = physis_hip::TileOf(sh.tiles_x, 1);
+  const int xs = (sh.x_first_tile + tc.bx) * physis_hip::kRowsTX -
+                 physis_hip::kRowsHalo + lane * 4;
+  const int zb = dom.local_min[2] + tc.bz * sh.zchunk;
+  const int ze = min(zb + sh.zchunk, dom.local_max[2]);
+  if (zb >= ze) return;
+  const int nx = src.dim[0], n = nx * src.dim[2];
+  const physis_hip::BufWin<float> aw = physis_hip::BufWin<float>::Make(src.p, n, (long)(zb - T - 1) * nx, (long)(ze + T + 1) * nx);
+  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg, n, (long)(zb - T - 1) * nx, (long)(ze + T + 1) * nx);
+  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, (long)zb * nx, (long)ze * nx);
+  const physis_hip::BufWin<float> mw = physis_hip::BufWin<float>::Make(bg, n, (long)zb * nx, (long)ze * nx);
+  unsigned xm = 0;  // the lane's points inside the domain's columns
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (xs + i >= dom.local_min[0] && xs + i < dom.local_max[0]) xm |= 1u << i;
+  const bool xin = __all(xm == 15u);
+  const unsigned om = lane >= 1 && lane <= 62 ? xm : 0u;
+  const auto zin = [&](int z) { return z >= dom.local_min[2] && z < dom.local_max[2]; };
+  float ld[PD][4], lb[PD][4];
+  // row z of src, and of b one row behind where the domain leaves points out
+  const auto load = [&](int z, int k) {
+    aw.template Load<4>(xs + z * nx, ld[k]);
+    bw.template Load<4>(xm == 15u && zin(z - 1) ? physis_hip::kDrop
+                                                : xs + (z - 1) * nx, lb[k]);
+  };
+  physis_hip::RowRegs q[T][3];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int i = 0; i < 6; ++i) q[t][k].v[i] = 0.0f;
+  __PSCtx_corners2d ctx;
+  ctx.g_p = src.p;
+  ctx.g_dim[0] = nx;
+  ctx.g_dim[1] = src.dim[2];
+  ctx.g_dim[2] = 1;
+  ctx.g2_p = dst.p;
+  ctx.g2_dim[0] = nx;
+  ctx.g2_dim[1] = src.dim[2];
+  ctx.g2_dim[2] = 1;
+#pragma unroll
+  for (int k = 0; k < PD; ++k) load(zb - T + k, k);
+  for (int sc = zb - T; sc < ze + T; sc += 3) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int s = sc + k;
+      q[0][k].Set(ld[k]);
+      float b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[i] = lb[k][i];
+      load(s + PD, k);
+#pragma unroll
+      for (int t = 1; t <= T; ++t) {
+        const int z = s - t;
+        float v[4];
+        const auto pts = [&](auto inside) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            ctx.g[0] = q[t - 1][(k + 2) % 3].v[1 + i + 0];
+            ctx.g[1] = q[t - 1][(k + 1) % 3].v[1 + i + 1];
+            ctx.g[2] = q[t - 1][(k + 0) % 3].v[1 + i + -1];
+            ctx.g[3] = q[t - 1][(k + 2) % 3].v[1 + i + 1];
+            ctx.g2_e = false;
+            corners2d(xs + i, z, ctx);
+            v[i] = ctx.g2_v;
+            if constexpr (!decltype(inside)::value)
+              if (!((xm >> i) & 1u && zin(z)))
+                v[i] = t == 1 ? b[i] : q[t == 1 ? 0 : t - 2][(k + 1) % 3].v[1 + i];
+          }
+        };
+        if (xin && zin(z))
+          pts(physis_hip::Flag<true>{});
+        else
+          pts(physis_hip::Flag<false>{});
+        if (t < T) q[t == T ? 0 : t][k].Set(v);
+        if (om && z >= zb && z < ze) {
+          if (t == T)
+            physis_hip::StoreMasked<float, 4>(dw, xs + z * nx, v, om);
+          else if (t == T - 1 && store_mid)
+            physis_hip::StoreMasked<float, 4>(mw, xs + z * nx, v, om);
+        }
+      }
+    }
+  }
+}
+
+template <int T>
+static void __PSLaunchR_corners2d(const struct __PSStencil_corners2d &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream) {
+  const __PSDomain d = physis_hip::RowDomain(s.dom);
+  static int per_cu = physis_hip::BlocksPerCU((const void *)__PSStencilRunR_corners2d<T>, 64);
+  const physis_hip::RunShape sh = physis_hip::PlanRun(d, physis_hip::kRowsTX, 1, per_cu,
+      physis_hip::WindowChunkLimitRows({s.g, s.g2}, T + 1), 2 * T + 3);
+  if (sh.blocks == 0) return;
+  hipLaunchKernelGGL(__PSStencilRunR_corners2d<T>, dim3(sh.blocks), dim3(64), 0, stream, d, src, dst, bg, store_mid, sh);
+}
+
+// The pair (s0, s1) is corners2d(a -> b), corners2d(b -> a) over one domain strictly
+// inside the grids, with the same scalars: it may run as rows passes.
+static bool __PSFusable2_corners2d(const struct __PSStencil_corners2d &s0, const struct __PSStencil_corners2d &s1) {
+  static const bool off = getenv("PHYSIS_HIP_NO_FUSE") != NULL;
+  const __PSGrid *a = s0.g, *b = s0.g2;
+  if (off || !a || !b || a == b || s1.g != b || s1.g2 != a) return false;
+  if (a->num_dims != 2 || b->num_dims != 2) return false;
+  for (int d = 0; d < 2; ++d) {
+    if (a->dim[d] != b->dim[d]) return false;
+    if (s0.dom.local_min[d] != s1.dom.local_min[d] ||
+        s0.dom.local_max[d] != s1.dom.local_max[d]) return false;
+    if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
+        s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
+  }
+  return true;
 }
 
 // ---------------------------------------------- stencil wrap2
@@ -1652,10 +1773,10 @@ static void __PSStencilRun_4(int iter, struct __PSStencil_inner s0, struct __PSS
     const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
-    physis_hip::CopyDevice(vt.p, va.p, bytes, stream);
+    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
-      physis_hip::CopyDevice(vt2.p, va.p, bytes, stream);
+      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     }
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {
