@@ -3721,8 +3721,13 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
       float a_r4[VX + 0];
       SA::template ReadRow<0, 0>(a_lds + sp * SA::kPlane, wave + 0, lane, a_r4);
       float uo[VX];
+      auto __half = [&](auto __odd) {
+      constexpr int __p = decltype(__odd)::value ? 1 : 0;
 #pragma unroll
-      for (int i = 0; i < VX; ++i) {
+      for (int i = 1 - __p; i < VX; i += 2) uo[i] = a_r0[i + 1];
+      __builtin_assume(((yrow + s + 0) & 1) == __p);
+#pragma unroll
+      for (int i = __p; i < VX; i += 2) {
         ctx.g[0] = a_r0[i + 1];
         ctx.g[1] = a_r0[i + 2];
         ctx.g[2] = a_r0[i + 0];
@@ -3734,6 +3739,11 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
         krb(xs + i, yrow, s, ctx);
         uo[i] = ((xs + i) >= dom.local_min[0] && (xs + i) < dom.local_max[0] && yrow >= dom.local_min[1] && yrow < dom.local_max[1] && s >= dom.local_min[2] && s < dom.local_max[2] && (((xs + i) + yrow + s + 0) & 1) == 0) ? ctx.g_v : a_r0[i + 1];
       }
+      };
+      if ((yrow + s + 0) & 1)
+        __half(physis_hip::Flag<true>{});
+      else
+        __half(physis_hip::Flag<false>{});
       SB::WriteRow(b_lds + bo * SB::kPlane, wave, lane, uo);
       if (mid && out_row && s >= zb && s < ze) {
         unsigned m = 0;
@@ -3755,7 +3765,9 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
       ctx.g[6] = a_lds[sp * SA::kPlane + (hr + 0) * SA::kRow + SA::kPad + px + 0];
       ctx.g_e = false;
       krb(x0 + px, y0 - 2 + hr, s, ctx);
-      b_lds[bo * SB::kPlane + hr * SB::kRow + SB::kPad + px] = ((x0 + px) >= dom.local_min[0] && (x0 + px) < dom.local_max[0] && (y0 - 2 + hr) >= dom.local_min[1] && (y0 - 2 + hr) < dom.local_max[1] && s >= dom.local_min[2] && s < dom.local_max[2] && (((x0 + px) + (y0 - 2 + hr) + s + 0) & 1) == 0) ? ctx.g_v : a_lds[sc * SA::kPlane + hr * SA::kRow + SA::kPad + px];
+      const float old = a_lds[sc * SA::kPlane + hr * SA::kRow + SA::kPad + px];
+      const float now = ctx.g_v;
+      b_lds[bo * SB::kPlane + hr * SB::kRow + SB::kPad + px] = ((x0 + px) >= dom.local_min[0] && (x0 + px) < dom.local_max[0] && (y0 - 2 + hr) >= dom.local_min[1] && (y0 - 2 + hr) < dom.local_max[1] && s >= dom.local_min[2] && s < dom.local_max[2] && (((x0 + px) + (y0 - 2 + hr) + s + 0) & 1) == 0) ? now : old;
     }
   };
   auto __udouble = [&](const int z, const int sm, const int sc, const int sp) {
@@ -3772,8 +3784,13 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
       SB::template ReadRow<0, 0>(b_lds + sp * SB::kPlane, wave + 0, lane, b_r4);
       float uu[VX];
       unsigned m = 0;
+      auto __half = [&](auto __odd) {
+      constexpr int __p = decltype(__odd)::value ? 1 : 0;
 #pragma unroll
-      for (int i = 0; i < VX; ++i) {
+      for (int i = 1 - __p; i < VX; i += 2) uu[i] = b_r0[i + 1];
+      __builtin_assume(((yrow + z + 1) & 1) == __p);
+#pragma unroll
+      for (int i = __p; i < VX; i += 2) {
         ctx.g[0] = b_r0[i + 1];
         ctx.g[1] = b_r0[i + 2];
         ctx.g[2] = b_r0[i + 0];
@@ -3784,8 +3801,15 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
         ctx.g_e = false;
         krb(xs + i, yrow, z, ctx);
         uu[i] = ((xs + i) >= dom.local_min[0] && (xs + i) < dom.local_max[0] && yrow >= dom.local_min[1] && yrow < dom.local_max[1] && z >= dom.local_min[2] && z < dom.local_max[2] && (((xs + i) + yrow + z + 1) & 1) == 0) ? ctx.g_v : b_r0[i + 1];
-        m |= (xs + i >= gd.local_min[0] && xs + i < gd.local_max[0]) ? 1u << i : 0u;
       }
+      };
+      if ((yrow + z + 1) & 1)
+        __half(physis_hip::Flag<true>{});
+      else
+        __half(physis_hip::Flag<false>{});
+#pragma unroll
+      for (int i = 0; i < VX; ++i)
+        m |= (xs + i >= gd.local_min[0] && xs + i < gd.local_max[0]) ? 1u << i : 0u;
       physis_hip::StoreMasked<float, VX>(dw, xs + yrow * nx + z * nxy, uu, m);
     }
   };
