@@ -165,6 +165,18 @@ inline RunShape PlanRun(const __PSDomain &dom, int tx, int ty, int per_cu,
                     extra);
 }
 
+// Points per lane (4 or 2) of a whole-grid two-sweep pass over rows of nx
+// points: tiles of 256 points, or of 128 where those pad the rows so much
+// less that they win although a point costs 1.2 times as much in them (its
+// row's loads, addresses and masks are shared by half as many points).
+// us a sweep at 4 and 2 points, clamped 7-point map: 256^3 19.4 and 23.3,
+// 257^3 38.6 and 31.5, 384^3 74.2 and 66.6, 512^3 116 and 145; red-black
+// iteration: 256^3 39.1 and 44.9, 257^3 73.2 and 62.1, 384^3 147 and 130.
+inline int PairVX(int nx) {
+  const long wide = (nx + 255) / 256 * 256L, narrow = (nx + 127) / 128 * 128L;
+  return narrow * 5 < wide * 4 ? 2 : 4;
+}
+
 // A 3-D grid argument must be live, of the stencil's element type, and small
 // enough for 32-bit PSIndex offsets (the reference's default index type).
 inline void CheckGrid3D(const __PSGrid *g, int type) {

@@ -14,6 +14,7 @@
 
 #include <cstdint>
 
+#include "physis/hip/run.h"
 #include "physis/hip/stencil.h"
 #include "physis/physis_hip.h"
 
@@ -131,14 +132,33 @@ __device__ __forceinline__ void LoadTile(E *lds, const E *p, const int *dim,
 // ------------------------------------------------------ launch arithmetic
 // Tiles of one small grid per compute unit, and those of larger ones, whose
 // halo costs less.  Measured for T = 4 (us per sweep of the clamped 7-point
-// diffusion, small tile / mid tile / z-marching two-sweep passes): 64^3 1.94 /
-// 2.51 / 4.41, 80^3 2.75 / 2.63 / 5.27, 96^3 4.53 / 3.85 / 6.02, 128^3 7.97 /
-// 6.49 / 7.26, 144^3 11.1 / 8.83 / 8.89.  A kernel with the 12 centre-only
+// diffusion, small tile / mid tile): 64^3 1.94 / 2.51, 80^3 2.75 / 2.63, 96^3
+// 4.53 / 3.85, 128^3 7.97 / 6.49.  A kernel with the 12 centre-only
 // grids of the 19-point Jacobi sweep gains nothing (its tiles read the halo's
 // values of every one of them: 96^3 14.4 against 10.1).
 template <int T> using SmallTile = Tile<T, 16, 8, 8, 1024>;
 template <int T> using MidTile = Tile<T, 16, 16, 8, 1024>;
+// The largest grid of a pass over part of a grid (EmitFusedDomainKernel's
+// pairs beside it).
 constexpr int64_t kTileMaxPoints = 2200000;
+// Whether a pass over a whole grid runs in tiles: both kinds of pass cost by
+// the points of their padded tiles, us a sweep about 1.4 + 2.5 per million
+// points here and 4.3 + 1 in a z-marching pair (0.83 at four points per
+// lane), so that the line follows the width as much as the size.  Tiles and
+// pairs, clamped 7-point map (red-black iterations cost twice as much and
+// fall on the same sides): 112^3 5.2 and 6.3, 128^3 6.4 and 6.0, 150^3 11.3
+// and 9.3, 250x80x80 6.5 and 5.7, 250x64x64 4.0 and 4.9, 64x256x256 11.4 and
+// 11.9, 100x180x180 11.3 and 8.6, 16x400x400 8.1 and 22.7, 48x300x300 12.5
+// and 15.3.  Past 16 million points (a grid of 64 MB) nothing was measured,
+// and the tiles' halos no longer come from the cache.
+inline bool TilesBeatPairs(const int *dim) {
+  const auto up = [](double n, int t) { return (double)(((long)n + t - 1) / t * t); };
+  const bool narrow = PairVX(dim[0]) == 2;
+  const double tile = up(dim[0], 16) * up(dim[1], 16) * up(dim[2], 8) * 1e-6;
+  const double pair = (narrow ? up(dim[0], 128) : up(dim[0], 256) * 0.83) *
+                      up(dim[1], 8) * dim[2] * 1e-6;
+  return tile <= 16 && 2.5 * tile - pair < 2.2;
+}
 
 // Per-block partials of each sweep of a pass (NULL: none).
 struct TileReds {

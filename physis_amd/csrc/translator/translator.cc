@@ -2455,28 +2455,29 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
        "      st[0].Load(aw, src.p, src.dim, ra, s0 + 5);\n"
        "      st[1].Load(aw, src.p, src.dim, ra, s0 + 6);\n"
        "    }\n  }\n}\n\n";
-  // launcher.  Launch shape: 4 points per lane in 12-wave blocks (8
-  // output rows; the two six-slot rings take 152 KB of LDS, one block per
-  // CU); measured on the 512^3 clamped kernel: 239 us per launch, against
-  // 374 us in 8-wave blocks, and 257 us for one plane per barrier in
-  // 16-wave blocks with four-slot rings.
-  const int vx = 4, by = 12;
-  o << "static constexpr int __PS2VX_" << n << " = " << vx << ", __PS2BY_"
-    << n << " = " << by << ";\n";
+  // launcher.  Launch shape: 12-wave blocks (8 output rows; at 4 points per
+  // lane the two six-slot rings take 152 KB of LDS, one block per CU);
+  // measured on the 512^3 clamped kernel: 239 us per launch, against 374 us
+  // in 8-wave blocks, and 257 us for one plane per barrier in 16-wave blocks
+  // with four-slot rings.  Points per lane by the padded width (PairVX).
+  const int by = 12;
   std::vector<std::string> largs = {"s.dom", "src", "dst", "mid"};
   if (rb) largs = {"s.dom", "gd", "src", "dst", "mid"};
   for (auto &a : sa) largs.push_back("s." + a);
   largs.push_back("sh");
-  o << "static void __PSLaunch2_" << n << "(const struct __PSStencil_" << n
+  o << "template <int VX>\nstatic void __PSLaunch2V_" << n
+    << "(const struct __PSStencil_" << n
     << " &s, const " << V << " &src, const " << V << " &dst, " << T
     << " *mid, hipStream_t stream) {\n"
-    << "  constexpr int VX = __PS2VX_" << n << ", BY = __PS2BY_" << n << ";\n"
+    << "  constexpr int BY = " << by << ";\n"
     << (rb ? "  const __PSDomain gd = physis_hip::WholeDomain(s." + I + ");\n" : "")
     << "  static int per_cu = physis_hip::BlocksPerCU(\n"
        "      (const void *)__PSStencilRun2_" << n << "<VX, BY, false>, 64 * BY);\n"
+    // (a pass steps over its chunk and four planes; two, the default, cost
+    // 600x200x200 6 % of a sweep in a last wave of blocks)
     << "  const physis_hip::RunShape sh = physis_hip::PlanRun("
     << (rb ? "gd" : "s.dom") << ", 64 * VX, BY - 4, per_cu,\n"
-       "      physis_hip::WindowChunkLimit({s." << I << "}, 3));\n"
+       "      physis_hip::WindowChunkLimit({s." << I << "}, 3), 4);\n"
     << "  if (sh.blocks == 0) return;\n"
     << "  if (s." << I << "->dim[0] % VX == 0)\n"
     << "    hipLaunchKernelGGL((__PSStencilRun2_" << n << "<VX, BY, false>), "
@@ -2484,7 +2485,13 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
     << Join(largs, ", ") << ");\n  else\n"
     << "    hipLaunchKernelGGL((__PSStencilRun2_" << n << "<VX, BY, true>), "
        "dim3(sh.blocks), dim3(64 * BY), 0, stream, "
-    << Join(largs, ", ") << ");\n}\n\n";
+    << Join(largs, ", ") << ");\n}\n\n"
+    << "static void __PSLaunch2_" << n << "(const struct __PSStencil_" << n
+    << " &s, const " << V << " &src, const " << V << " &dst, " << T
+    << " *mid, hipStream_t stream) {\n"
+    << "  if (physis_hip::PairVX(s." << I << "->dim[0]) == 4)\n    __PSLaunch2V_"
+    << n << "<4>(s, src, dst, mid, stream);\n  else\n    __PSLaunch2V_" << n
+    << "<2>(s, src, dst, mid, stream);\n}\n\n";
   // run-time check
   if (rb) {
     // one map of both colours over a domain at least one point inside the
@@ -2776,9 +2783,11 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
   const bool red = k.ret_type != "void";
   const bool tiles = UsesTiles(k);
   if (tiles)
-    o << "    const bool __small = s0." << gi.name
-      << "->num_elms <= physis_hip::kTileMaxPoints;\n"
-      << "    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);\n";
+    o << "    const bool __small = "
+      << (k.fuse_domain
+              ? "s0." + gi.name + "->num_elms <= physis_hip::kTileMaxPoints"
+              : "physis_hip::TilesBeatPairs(s0." + gi.name + "->dim)")
+      << ";\n    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);\n";
   else
     o << "    const int passes = iter;\n";
   // one pass, pairs i and on (j: pass)
@@ -3628,8 +3637,8 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
       << "    " << V << " vt = va;\n"
       << "    vt.p = (" << T << " *)__PSHipScratch(8, bytes);\n"
       << "    " << V << " src = va;\n"
-      << "    const bool __small = s0." << g.name
-      << "->num_elms <= physis_hip::kTileMaxPoints;\n"
+      << "    const bool __small = physis_hip::TilesBeatPairs(s0." << g.name
+      << "->dim);\n"
       << "    // two iterations a resident-tile pass, an even number of times, so that\n"
          "    // the count of passes is odd when iter is\n"
       << "    const int two = __small ? iter / 2 & ~1 : 0;\n"

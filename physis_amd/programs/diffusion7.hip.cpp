@@ -401,18 +401,25 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_kernel(
   }
 }
 
-static constexpr int __PS2VX_diffusion7_kernel = 4, __PS2BY_diffusion7_kernel = 12;
-static void __PSLaunch2_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  constexpr int VX = __PS2VX_diffusion7_kernel, BY = __PS2BY_diffusion7_kernel;
+template <int VX>
+static void __PSLaunch2V_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  constexpr int BY = 12;
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun2_diffusion7_kernel<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
-      physis_hip::WindowChunkLimit({s.g1}, 3));
+      physis_hip::WindowChunkLimit({s.g1}, 3), 4);
   if (sh.blocks == 0) return;
   if (s.g1->dim[0] % VX == 0)
     hipLaunchKernelGGL((__PSStencilRun2_diffusion7_kernel<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
   else
     hipLaunchKernelGGL((__PSStencilRun2_diffusion7_kernel<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+}
+
+static void __PSLaunch2_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  if (physis_hip::PairVX(s.g1->dim[0]) == 4)
+    __PSLaunch2V_diffusion7_kernel<4>(s, src, dst, mid, stream);
+  else
+    __PSLaunch2V_diffusion7_kernel<2>(s, src, dst, mid, stream);
 }
 
 // The pair (s0, s1) is diffusion7_kernel(a -> b), diffusion7_kernel(b -> a) over the whole grid with the
@@ -860,18 +867,25 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_diffusion7_periodic_k
   }
 }
 
-static constexpr int __PS2VX_diffusion7_periodic_kernel = 4, __PS2BY_diffusion7_periodic_kernel = 12;
-static void __PSLaunch2_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  constexpr int VX = __PS2VX_diffusion7_periodic_kernel, BY = __PS2BY_diffusion7_periodic_kernel;
+template <int VX>
+static void __PSLaunch2V_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  constexpr int BY = 12;
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun2_diffusion7_periodic_kernel<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
-      physis_hip::WindowChunkLimit({s.g1}, 3));
+      physis_hip::WindowChunkLimit({s.g1}, 3), 4);
   if (sh.blocks == 0) return;
   if (s.g1->dim[0] % VX == 0)
     hipLaunchKernelGGL((__PSStencilRun2_diffusion7_periodic_kernel<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
   else
     hipLaunchKernelGGL((__PSStencilRun2_diffusion7_periodic_kernel<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+}
+
+static void __PSLaunch2_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  if (physis_hip::PairVX(s.g1->dim[0]) == 4)
+    __PSLaunch2V_diffusion7_periodic_kernel<4>(s, src, dst, mid, stream);
+  else
+    __PSLaunch2V_diffusion7_periodic_kernel<2>(s, src, dst, mid, stream);
 }
 
 // The pair (s0, s1) is diffusion7_periodic_kernel(a -> b), diffusion7_periodic_kernel(b -> a) over the whole grid with the
@@ -989,7 +1003,7 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_diffusion7_kernel s0, 
     const size_t bytes = (size_t)s0.g1->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = s0.g1->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {
@@ -1036,7 +1050,7 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_diffusion7_periodic_ke
     const size_t bytes = (size_t)s0.g1->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = s0.g1->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {

@@ -394,19 +394,26 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_redblack7_kernel(
   }
 }
 
-static constexpr int __PS2VX_redblack7_kernel = 4, __PS2BY_redblack7_kernel = 12;
-static void __PSLaunch2_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  constexpr int VX = __PS2VX_redblack7_kernel, BY = __PS2BY_redblack7_kernel;
+template <int VX>
+static void __PSLaunch2V_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  constexpr int BY = 12;
   const __PSDomain gd = physis_hip::WholeDomain(s.g);
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun2_redblack7_kernel<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(gd, 64 * VX, BY - 4, per_cu,
-      physis_hip::WindowChunkLimit({s.g}, 3));
+      physis_hip::WindowChunkLimit({s.g}, 3), 4);
   if (sh.blocks == 0) return;
   if (s.g->dim[0] % VX == 0)
     hipLaunchKernelGGL((__PSStencilRun2_redblack7_kernel<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
   else
     hipLaunchKernelGGL((__PSStencilRun2_redblack7_kernel<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, s.ce, s.cw, s.cn, s.cs, s.ct, s.cb, s.cc, sh);
+}
+
+static void __PSLaunch2_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  if (physis_hip::PairVX(s.g->dim[0]) == 4)
+    __PSLaunch2V_redblack7_kernel<4>(s, src, dst, mid, stream);
+  else
+    __PSLaunch2V_redblack7_kernel<2>(s, src, dst, mid, stream);
 }
 
 // The red-black map s0 may run as one pass per iteration: both colours, a domain
@@ -514,7 +521,7 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_redblack7_kernel s0) {
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
-    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim);
     // two iterations a resident-tile pass, an even number of times, so that
     // the count of passes is odd when iter is
     const int two = __small ? iter / 2 & ~1 : 0;

@@ -850,18 +850,25 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7p(
   }
 }
 
-static constexpr int __PS2VX_k7p = 4, __PS2BY_k7p = 12;
-static void __PSLaunch2_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  constexpr int VX = __PS2VX_k7p, BY = __PS2BY_k7p;
+template <int VX>
+static void __PSLaunch2V_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  constexpr int BY = 12;
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun2_k7p<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
-      physis_hip::WindowChunkLimit({s.g}, 3));
+      physis_hip::WindowChunkLimit({s.g}, 3), 4);
   if (sh.blocks == 0) return;
   if (s.g->dim[0] % VX == 0)
     hipLaunchKernelGGL((__PSStencilRun2_k7p<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
   else
     hipLaunchKernelGGL((__PSStencilRun2_k7p<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+}
+
+static void __PSLaunch2_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  if (physis_hip::PairVX(s.g->dim[0]) == 4)
+    __PSLaunch2V_k7p<4>(s, src, dst, mid, stream);
+  else
+    __PSLaunch2V_k7p<2>(s, src, dst, mid, stream);
 }
 
 // The pair (s0, s1) is k7p(a -> b), k7p(b -> a) over the whole grid with the
@@ -1345,18 +1352,25 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k7n(
   }
 }
 
-static constexpr int __PS2VX_k7n = 4, __PS2BY_k7n = 12;
-static void __PSLaunch2_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  constexpr int VX = __PS2VX_k7n, BY = __PS2BY_k7n;
+template <int VX>
+static void __PSLaunch2V_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  constexpr int BY = 12;
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun2_k7n<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
-      physis_hip::WindowChunkLimit({s.g1}, 3));
+      physis_hip::WindowChunkLimit({s.g1}, 3), 4);
   if (sh.blocks == 0) return;
   if (s.g1->dim[0] % VX == 0)
     hipLaunchKernelGGL((__PSStencilRun2_k7n<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
   else
     hipLaunchKernelGGL((__PSStencilRun2_k7n<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+}
+
+static void __PSLaunch2_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  if (physis_hip::PairVX(s.g1->dim[0]) == 4)
+    __PSLaunch2V_k7n<4>(s, src, dst, mid, stream);
+  else
+    __PSLaunch2V_k7n<2>(s, src, dst, mid, stream);
 }
 
 // The pair (s0, s1) is k7n(a -> b), k7n(b -> a) over the whole grid with the
@@ -2855,18 +2869,25 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_k27p(
   }
 }
 
-static constexpr int __PS2VX_k27p = 4, __PS2BY_k27p = 12;
-static void __PSLaunch2_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  constexpr int VX = __PS2VX_k27p, BY = __PS2BY_k27p;
+template <int VX>
+static void __PSLaunch2V_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  constexpr int BY = 12;
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun2_k27p<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(s.dom, 64 * VX, BY - 4, per_cu,
-      physis_hip::WindowChunkLimit({s.g}, 3));
+      physis_hip::WindowChunkLimit({s.g}, 3), 4);
   if (sh.blocks == 0) return;
   if (s.g->dim[0] % VX == 0)
     hipLaunchKernelGGL((__PSStencilRun2_k27p<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
   else
     hipLaunchKernelGGL((__PSStencilRun2_k27p<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, src, dst, mid, sh);
+}
+
+static void __PSLaunch2_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  if (physis_hip::PairVX(s.g->dim[0]) == 4)
+    __PSLaunch2V_k27p<4>(s, src, dst, mid, stream);
+  else
+    __PSLaunch2V_k27p<2>(s, src, dst, mid, stream);
 }
 
 // The pair (s0, s1) is k27p(a -> b), k27p(b -> a) over the whole grid with the
@@ -3831,19 +3852,26 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun2_krb(
   }
 }
 
-static constexpr int __PS2VX_krb = 4, __PS2BY_krb = 12;
-static void __PSLaunch2_krb(const struct __PSStencil_krb &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  constexpr int VX = __PS2VX_krb, BY = __PS2BY_krb;
+template <int VX>
+static void __PSLaunch2V_krb(const struct __PSStencil_krb &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  constexpr int BY = 12;
   const __PSDomain gd = physis_hip::WholeDomain(s.g);
   static int per_cu = physis_hip::BlocksPerCU(
       (const void *)__PSStencilRun2_krb<VX, BY, false>, 64 * BY);
   const physis_hip::RunShape sh = physis_hip::PlanRun(gd, 64 * VX, BY - 4, per_cu,
-      physis_hip::WindowChunkLimit({s.g}, 3));
+      physis_hip::WindowChunkLimit({s.g}, 3), 4);
   if (sh.blocks == 0) return;
   if (s.g->dim[0] % VX == 0)
     hipLaunchKernelGGL((__PSStencilRun2_krb<VX, BY, false>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, sh);
   else
     hipLaunchKernelGGL((__PSStencilRun2_krb<VX, BY, true>), dim3(sh.blocks), dim3(64 * BY), 0, stream, s.dom, gd, src, dst, mid, sh);
+}
+
+static void __PSLaunch2_krb(const struct __PSStencil_krb &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
+  if (physis_hip::PairVX(s.g->dim[0]) == 4)
+    __PSLaunch2V_krb<4>(s, src, dst, mid, stream);
+  else
+    __PSLaunch2V_krb<2>(s, src, dst, mid, stream);
 }
 
 // The red-black map s0 may run as one pass per iteration: both colours, a domain
@@ -4149,7 +4177,7 @@ static void __PSStencilRun_10(int iter, struct __PSStencil_krb s0) {
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
-    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim);
     // two iterations a resident-tile pass, an even number of times, so that
     // the count of passes is odd when iter is
     const int two = __small ? iter / 2 & ~1 : 0;

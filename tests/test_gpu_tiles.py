@@ -1,8 +1,8 @@
 """Resident-tile passes (include/physis/hip/tile.h: small grids, four sweeps
 of a fused pair or two red-black iterations per launch) against the oracle,
 bit for bit on both grids: extents below the halo, at and one off the tiles'
-edges, on both sides of the tile-size and of the grid-size rule; odd and even
-counts."""
+edges, on both sides of the tile-size and of the grid-size rule, where
+whole-grid pairs take two and four points per lane; odd and even counts."""
 import ctypes as C
 
 import numpy as np
@@ -15,7 +15,10 @@ pytestmark = pytest.mark.gpu
 COEF = (0.11, 0.09, 0.12, 0.08, 0.105, 0.095, 0.39)
 SHAPES = [(1, 2, 1), (2, 3, 1), (3, 3, 3), (5, 4, 6), (15, 7, 7), (16, 8, 8),
           (17, 9, 9), (33, 17, 12), (64, 64, 64), (65, 64, 64), (96, 40, 70),
-          (130, 130, 130), (131, 130, 130)]
+          (130, 130, 130), (131, 130, 130),
+          # thin grids in tiles, and pairs at two points per lane
+          (16, 300, 290), (47, 260, 181), (121, 120, 123), (127, 153, 139),
+          (257, 90, 101), (383, 70, 122), (385, 70, 122)]
 
 
 def _bits(a):
