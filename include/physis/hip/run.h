@@ -172,9 +172,13 @@ inline RunShape PlanRun(const __PSDomain &dom, int tx, int ty, int per_cu,
 // us a sweep at 4 and 2 points, clamped 7-point map: 256^3 19.4 and 23.3,
 // 257^3 38.6 and 31.5, 384^3 74.2 and 66.6, 512^3 116 and 145; red-black
 // iteration: 256^3 39.1 and 44.9, 257^3 73.2 and 62.1, 384^3 147 and 130.
-inline int PairVX(int nx) {
+// Periodic planes are loaded through a window of their own each, twice as
+// often per point in the narrow tiles: a point costs 1.2 to 1.36 times as much
+// (181x163x137 10.2 and 12.5, 321x190x157 20.9 and 21.4).
+inline int PairVX(int nx, bool periodic) {
   const long wide = (nx + 255) / 256 * 256L, narrow = (nx + 127) / 128 * 128L;
-  return narrow * 5 < wide * 4 ? 2 : 4;
+  return periodic ? (narrow * 7 < wide * 5 ? 2 : 4)
+                  : (narrow * 5 < wide * 4 ? 2 : 4);
 }
 
 // A 3-D grid argument must be live, of the stencil's element type, and small

@@ -151,9 +151,9 @@ constexpr int64_t kTileMaxPoints = 2200000;
 // 11.9, 100x180x180 11.3 and 8.6, 16x400x400 8.1 and 22.7, 48x300x300 12.5
 // and 15.3.  Past 16 million points (a grid of 64 MB) nothing was measured,
 // and the tiles' halos no longer come from the cache.
-inline bool TilesBeatPairs(const int *dim) {
+inline bool TilesBeatPairs(const int *dim, bool periodic) {
   const auto up = [](double n, int t) { return (double)(((long)n + t - 1) / t * t); };
-  const bool narrow = PairVX(dim[0]) == 2;
+  const bool narrow = PairVX(dim[0], periodic) == 2;
   const double tile = up(dim[0], 16) * up(dim[1], 16) * up(dim[2], 8) * 1e-6;
   const double pair = (narrow ? up(dim[0], 128) : up(dim[0], 256) * 0.83) *
                       up(dim[1], 8) * dim[2] * 1e-6;

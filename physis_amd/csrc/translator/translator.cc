@@ -2268,8 +2268,9 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
   };
   // A red-black row updates every other point: those at i = __p, __p + 2 of
   // the lane's points, __p by the row's parity (uniform over the wave, whose
-  // tile starts at an even x), so that only they are computed (256^3
-  // iterations: all points computed and half dropped took 42 us).
+  // tile starts at an even x), so that only they are computed (us an
+  // iteration, all points computed and half dropped before: 192^3 27.3 ->
+  // 25.8, 384^3 163 -> 154).
   auto half_begin = [&](const std::string &z, int c, const std::string &out,
                         const std::string &pre) {
     return "      auto __half = [&](auto __odd) {\n"
@@ -2333,9 +2334,11 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
     << "  const physis_hip::BufWin<" << T << "> mw = physis_hip::BufWin<" << T
     << ">::Make(mid ? mid : dst.p, n, (long)zb * nxy, (long)ze * nxy);\n"
     // A red-black pass issues every load of the prologue before the first
-    // one is stored (512^3 iterations 4% faster); a map pair stores each
-    // plane before the next is loaded: with all of them in flight the
-    // compiler schedules the loop worse (512^3 passes 8% slower).
+    // one is stored (us an iteration: 192^3 28.7 -> 27.3, 384^3 166 -> 163);
+    // a map pair stores each plane before the next is loaded: with all of
+    // them in flight the compiler takes 110 VGPRs instead of 100 and
+    // schedules the loop worse (us a sweep: 256^3 19.2 -> 21.0, 384^3 74.2
+    // -> 81.7).
     << "  SA st[PD]" << (rb ? ", pro[4]" : "") << ";\n"
        "  const typename SA::Addr ra = SA::Prepare(src.dim, x0, yrow, lane);\n"
     << (rb ? "#pragma unroll\n  for (int k = 0; k < 4; ++k)\n"
@@ -2489,7 +2492,7 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
     << "static void __PSLaunch2_" << n << "(const struct __PSStencil_" << n
     << " &s, const " << V << " &src, const " << V << " &dst, " << T
     << " *mid, hipStream_t stream) {\n"
-    << "  if (physis_hip::PairVX(s." << I << "->dim[0]) == 4)\n    __PSLaunch2V_"
+    << "  if (physis_hip::PairVX(s." << I << "->dim[0], " << per << ") == 4)\n    __PSLaunch2V_"
     << n << "<4>(s, src, dst, mid, stream);\n  else\n    __PSLaunch2V_" << n
     << "<2>(s, src, dst, mid, stream);\n}\n\n";
   // run-time check
@@ -2786,7 +2789,8 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
     o << "    const bool __small = "
       << (k.fuse_domain
               ? "s0." + gi.name + "->num_elms <= physis_hip::kTileMaxPoints"
-              : "physis_hip::TilesBeatPairs(s0." + gi.name + "->dim)")
+              : "physis_hip::TilesBeatPairs(s0." + gi.name + "->dim, " +
+                    (gi.periodic ? "true" : "false") + ")")
       << ";\n    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);\n";
   else
     o << "    const int passes = iter;\n";
@@ -3638,7 +3642,7 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
       << "    vt.p = (" << T << " *)__PSHipScratch(8, bytes);\n"
       << "    " << V << " src = va;\n"
       << "    const bool __small = physis_hip::TilesBeatPairs(s0." << g.name
-      << "->dim);\n"
+      << "->dim, " << (g.periodic ? "true" : "false") << ");\n"
       << "    // two iterations a resident-tile pass, an even number of times, so that\n"
          "    // the count of passes is odd when iter is\n"
       << "    const int two = __small ? iter / 2 & ~1 : 0;\n"

@@ -416,7 +416,7 @@ static void __PSLaunch2V_diffusion7_kernel(const struct __PSStencil_diffusion7_k
 }
 
 static void __PSLaunch2_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g1->dim[0]) == 4)
+  if (physis_hip::PairVX(s.g1->dim[0], false) == 4)
     __PSLaunch2V_diffusion7_kernel<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_diffusion7_kernel<2>(s, src, dst, mid, stream);
@@ -882,7 +882,7 @@ static void __PSLaunch2V_diffusion7_periodic_kernel(const struct __PSStencil_dif
 }
 
 static void __PSLaunch2_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g1->dim[0]) == 4)
+  if (physis_hip::PairVX(s.g1->dim[0], true) == 4)
     __PSLaunch2V_diffusion7_periodic_kernel<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_diffusion7_periodic_kernel<2>(s, src, dst, mid, stream);
@@ -1003,7 +1003,7 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_diffusion7_kernel s0, 
     const size_t bytes = (size_t)s0.g1->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim);
+    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim, false);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {
@@ -1050,7 +1050,7 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_diffusion7_periodic_ke
     const size_t bytes = (size_t)s0.g1->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim);
+    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim, true);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {

@@ -410,7 +410,7 @@ static void __PSLaunch2V_redblack7_kernel(const struct __PSStencil_redblack7_ker
 }
 
 static void __PSLaunch2_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g->dim[0]) == 4)
+  if (physis_hip::PairVX(s.g->dim[0], false) == 4)
     __PSLaunch2V_redblack7_kernel<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_redblack7_kernel<2>(s, src, dst, mid, stream);
@@ -521,7 +521,7 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_redblack7_kernel s0) {
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
-    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim);
+    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim, false);
     // two iterations a resident-tile pass, an even number of times, so that
     // the count of passes is odd when iter is
     const int two = __small ? iter / 2 & ~1 : 0;

@@ -865,7 +865,7 @@ static void __PSLaunch2V_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFl
 }
 
 static void __PSLaunch2_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g->dim[0]) == 4)
+  if (physis_hip::PairVX(s.g->dim[0], true) == 4)
     __PSLaunch2V_k7p<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_k7p<2>(s, src, dst, mid, stream);
@@ -1367,7 +1367,7 @@ static void __PSLaunch2V_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFl
 }
 
 static void __PSLaunch2_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g1->dim[0]) == 4)
+  if (physis_hip::PairVX(s.g1->dim[0], false) == 4)
     __PSLaunch2V_k7n<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_k7n<2>(s, src, dst, mid, stream);
@@ -2884,7 +2884,7 @@ static void __PSLaunch2V_k27p(const struct __PSStencil_k27p &s, const __PSGrid3D
 }
 
 static void __PSLaunch2_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g->dim[0]) == 4)
+  if (physis_hip::PairVX(s.g->dim[0], true) == 4)
     __PSLaunch2V_k27p<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_k27p<2>(s, src, dst, mid, stream);
@@ -3868,7 +3868,7 @@ static void __PSLaunch2V_krb(const struct __PSStencil_krb &s, const __PSGrid3DFl
 }
 
 static void __PSLaunch2_krb(const struct __PSStencil_krb &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g->dim[0]) == 4)
+  if (physis_hip::PairVX(s.g->dim[0], false) == 4)
     __PSLaunch2V_krb<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_krb<2>(s, src, dst, mid, stream);
@@ -4177,7 +4177,7 @@ static void __PSStencilRun_10(int iter, struct __PSStencil_krb s0) {
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
-    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim);
+    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim, false);
     // two iterations a resident-tile pass, an even number of times, so that
     // the count of passes is odd when iter is
     const int two = __small ? iter / 2 & ~1 : 0;

@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
 
 STORAGE_NAMES = {0: "fp32", 1: "bf16", 2: "fp16"}
 # (shape, nbatch): odd sizes, a batch of two, and a wide grid that takes the
-# 4-points-per-lane sweep (nx > 128, nx % 4 == 0) with a ragged second tile
+# 2-points-per-lane 16-bit sweep (128-point tiles) with a ragged last tile
 CASES = [((40, 22, 18), 1), ((34, 14, 18), 2), ((260, 14, 10), 1)]
 
 

@@ -17,8 +17,8 @@ def rb(ps):
     return RedBlack7()
 
 
-# x extents that are multiples of 4 run one pass per iteration (odd counts
-# end with a copy back), the others two colour sweeps
+# one pass per iteration, two per pass on small grids (an odd count of passes
+# ends with a copy back)
 @pytest.mark.parametrize("shape,count", [((130, 66, 40), 3), ((36, 9, 7), 2),
                                          ((64, 64, 64), 1), ((33, 17, 20), 2),
                                          ((128, 96, 80), 3),

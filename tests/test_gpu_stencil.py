@@ -92,8 +92,7 @@ def test_shapes(ps, d7, shape, periodic):
 @pytest.mark.parametrize("periodic", [False, True])
 def test_two_sweep_passes_leave_both_grids(ps, d7, shape, pairs, periodic):
     """PSStencilRun(m12, m21, pairs) of the 7-point kernels runs as two-sweep
-    passes when x is a multiple of 4 (an odd pair count starts with one plain
-    pair): g1 must hold sweep 2*pairs and g2 sweep 2*pairs - 1, bit-exact,
+    passes or, on small grids, as resident-tile passes of four: g1 must hold sweep 2*pairs and g2 sweep 2*pairs - 1, bit-exact,
     across tile edges in x (260 = 256 + 4), y (not a multiple of the 12-row
     tile) and z chunks."""
     from physis_amd.seeded import uniform01

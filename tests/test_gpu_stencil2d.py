@@ -1,8 +1,8 @@
 """2-D 5- and 9-point maps (physis_amd/programs/stencil2d.c), which run on
 the 2.5D kernel over the grids' rows view (nx x 1 x ny, y marched as z), on
 the GPU against oracle_stencil2d_run, bit for bit on both grids: ragged
-shapes, x extents that are not multiples of 4 (one point per lane), single
-sweeps and pairs, and 16384^2."""
+shapes, x extents that are not multiples of 4 (the ragged form), single
+sweeps and pairs (four sweeps per launch), and 16384^2."""
 import numpy as np
 import pytest
 
