@@ -423,6 +423,10 @@ struct InputSrc {
 // What becomes of a convolution's results (COUT 8 or 24 channels).
 enum Epi {
   kEpiStore,    // + bias, ReLU when RELU, rounded and stored
+  kEpiPool,     // stored, and averaged over the 4x4x4 cells of the coarse grid
+                // (8 x 128^3: a pass of its own read the tensor again, 58 us
+                // of a prediction's 744; the sums of rounded values here, in
+                // another order, are what that pass summed)
   kEpiGate,     // gated by act > 0 (the ReLU whose input gradient this is)
   kEpiPredict,  // + bias, ReLU, rounded, 1x1 head, p = scale out bnd
   kEpiUpSkip    // 24 channels: 16 summed over the 4x4x4 cells of the coarse
@@ -432,7 +436,7 @@ struct EpiArgs {
   const float *bias = nullptr;
   u16 *y = nullptr;            // stored channels (kEpiUpSkip: the last 8)
   const u16 *act = nullptr;    // kEpiGate, kEpiUpSkip
-  u16 *coarse = nullptr;       // kEpiUpSkip
+  u16 *coarse = nullptr;       // kEpiPool, kEpiUpSkip
   const float *head = nullptr; // kEpiPredict: 8 weights and the bias
   const float *bnd = nullptr;  // kEpiPredict, from element off, as p
   void *p = nullptr;
@@ -473,7 +477,8 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
   constexpr int XS = XT + 2, RS = ROWS + 2;
   constexpr int PLANE = RS * XS * CIN;  // u16 elements of a staged plane
   constexpr int SEG = XT / 16;
-  constexpr bool kCells = EPI == kEpiUpSkip;  // sums over 4x4x4 cells
+  // sums over 4x4x4 cells
+  constexpr bool kCells = EPI == kEpiPool || EPI == kEpiUpSkip;
   __shared__ __attribute__((aligned(16))) u16 ring[2 * PLANE];
   __shared__ __attribute__((aligned(16))) float cells[kCells ? TY / 2 : 1]
       [kCells ? SEG : 1][kCells ? 64 : 1];
@@ -641,6 +646,13 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
           w2.x = GateWord(w2.x, av[i].x);
           w2.y = GateWord(w2.y, av[i].y);
         }
+        if constexpr (EPI == kEpiPool) {
+          if (done)
+            csum[i] += f32x4{__uint_as_float(w2.x << 16),
+                             __uint_as_float(w2.x & 0xffff0000u),
+                             __uint_as_float(w2.y << 16),
+                             __uint_as_float(w2.y & 0xffff0000u)};
+        }
         if constexpr (EPI == kEpiPredict) {
           float s = hw[0] * __uint_as_float(w2.x << 16);
           s += hw[1] * __uint_as_float(w2.x & 0xffff0000u);
@@ -667,8 +679,9 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
           acc[i][s][(j + 1) % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
       if constexpr (kCells) {
-        // the last plane of a row of cells: sums over 4 x (lanes) and over
-        // the rows of a pair of waves (LDS), in a fixed order
+        // the last plane of a row of cells: sums over 4 x (lanes), over a
+        // wave's two rows where lanes hold them apart, and over the rows of a
+        // pair of waves (LDS), in a fixed order
         if (done && (z & (kPool - 1)) == kPool - 1) {  // uniform
 #pragma unroll
           for (int i = 0; i < SEG; ++i) {
@@ -676,6 +689,8 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
             for (int e = 0; e < 4; ++e) {
               csum[i][e] += __shfl_xor(csum[i][e], 1, 64);
               csum[i][e] += __shfl_xor(csum[i][e], 2, 64);
+              if constexpr (EPI == kEpiPool)
+                csum[i][e] += __shfl_xor(csum[i][e], 32, 64);
             }
             if ((wv & 1) && (r & 3) == 0)
               *reinterpret_cast<f32x4 *>(&cells[wv >> 1][i][4 * (4 * g + (r >> 2))]) =
@@ -692,11 +707,20 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
               if ((r & 3) == 0 && xo < W && yw < H) {
                 const f32x4 v = csum[i] + *reinterpret_cast<const f32x4 *>(
                     &cells[wv >> 1][i][4 * (4 * g + (r >> 2))]);
-                const long o = (crow + xo / kPool) * 16 + 4 * g;
-                const uint2 a = *reinterpret_cast<const uint2 *>(ep.act + o);
-                *reinterpret_cast<uint2 *>(ep.coarse + o) =
-                    make_uint2(GateWord(Pack2(v[0], v[1]), a.x),
-                               GateWord(Pack2(v[2], v[3]), a.y));
+                if constexpr (EPI == kEpiPool) {
+                  constexpr float q = 1.0f / (kPool * kPool * kPool);
+                  if (g < 2)
+                    *reinterpret_cast<uint2 *>(
+                        ep.coarse + (crow + xo / kPool) * 8 + 4 * g) =
+                        make_uint2(Pack2(q * v[0], q * v[1]),
+                                   Pack2(q * v[2], q * v[3]));
+                } else {
+                  const long o = (crow + xo / kPool) * 16 + 4 * g;
+                  const uint2 a = *reinterpret_cast<const uint2 *>(ep.act + o);
+                  *reinterpret_cast<uint2 *>(ep.coarse + o) =
+                      make_uint2(GateWord(Pack2(v[0], v[1]), a.x),
+                                 GateWord(Pack2(v[2], v[3]), a.y));
+                }
               }
             }
           }
@@ -1360,7 +1384,7 @@ void ConvMLaunchXT(const SrcArgs &src, const u16 *wt, const EpiArgs &ep, int N,
   const long tiles = (long)((W + XT - 1) / XT) * ((H + 2 * TY - 1) / (2 * TY));
   int tz, zchunk;
   ZChunks(tiles, N, D, kConvMWavesPerCU / TY, &tz, &zchunk);
-  if (EPI == kEpiUpSkip) {  // whole cells
+  if (EPI == kEpiPool || EPI == kEpiUpSkip) {  // whole cells
     zchunk = (zchunk + kPool - 1) / kPool * kPool;
     tz = (D + zchunk - 1) / zchunk;
   }
@@ -1633,6 +1657,19 @@ void ConvSrc(const __PSUNet *net, int l, const SrcArgs &src, u16 *out, int N,
   ConvMLaunch<CIN, 8, true, SRC, kEpiStore>(src, L.wt, ep, N, D, H, W);
 }
 
+// An 8-channel layer and its 4x4x4 average pool (a prediction of 8 x 128^3
+// 744 -> 697 us).
+void ConvPool(const __PSUNet *net, int l, const u16 *x, u16 *out, u16 *pool,
+              int N, int D, int H, int W) {
+  const Layer &L = net->layers[l];
+  EpiArgs ep;
+  ep.bias = net->params + L.b_off;
+  ep.y = out;
+  ep.coarse = pool;
+  ConvMLaunch<8, 8, true, PlainSrc, kEpiPool>(SrcArgs{x, nullptr, 0}, L.wt, ep,
+                                              N, D, H, W);
+}
+
 // The last layer, the head and the scaled, masked prediction into p.
 template <typename T>
 void ConvPredict(const __PSUNet *net, const __PSGrid *bnd, __PSGrid *p,
@@ -1661,10 +1698,7 @@ void Forward(__PSUNet *net, const __PSGrid *rhs, const __PSGrid *bnd,
   const long off = (long)first * net->nx * net->ny * net->nzs;
   ConvSrc<2, InputSrc>(net, 0, SrcArgs{rhs->p, bnd->p, off}, net->a[0], d.N,
                        d.D1, d.H1, d.W1);
-  ConvL(net, 1, net->a[0], net->a[1], d.N, d.D1, d.H1, d.W1);
-  hipLaunchKernelGGL(PoolKernel, dim3(Blocks(d.P2)), dim3(256), 0, Stream(),
-                     net->a[1], net->q1, 8, d.D2, d.H2, d.W2, (int)d.P2);
-  Check();
+  ConvPool(net, 1, net->a[0], net->a[1], net->q1, d.N, d.D1, d.H1, d.W1);
   ConvL(net, 2, net->q1, net->a[2], d.N, d.D2, d.H2, d.W2);
   ConvL(net, 3, net->a[2], net->a[3], d.N, d.D2, d.H2, d.W2);
   hipLaunchKernelGGL(PoolKernel, dim3(Blocks(d.P3 * 2)), dim3(256), 0,

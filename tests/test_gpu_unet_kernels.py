@@ -55,7 +55,8 @@ def test_layer(ps, dims):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("shape,problems,first,count",
                          [((16, 16, 16), 3, 1, 2), ((48, 16, 32), 2, 1, 1),
-                          ((80, 32, 16), 2, 0, 2), ((32, 48, 16), 3, 2, 1)])
+                          ((80, 32, 16), 2, 0, 2), ((32, 48, 16), 3, 2, 1),
+                          ((112, 16, 48), 1, 0, 1)])
 def test_network(ps, shape, problems, first, count, dtype):
     """Gradient and prediction of problems [first, first + count): bounds as
     for the 32^3 network (tests/test_gpu_unet.py); the other problems of the
