@@ -9,8 +9,8 @@ counters' units), at 512^3 24 two-sweep launches of the 7-point clamped
 kernel, five single sweeps of it, 10 periodic sweeps (five two-sweep
 launches), 3 PSReduce SUMs at 512^3, 10 Himeno sweeps at 512x256x256 (five
 two-sweep launches) and three pairs of single Himeno sweeps, and the
-precision tier at 512^3: 10 BF16 inner sweeps (one pair of single sweeps,
-four two-sweep launches) and 3 fused FP64 update + residual passes.
+precision tier at 512^3: 10 BF16 inner sweeps (five two-sweep launches)
+and 3 fused FP64 update + residual passes.
 Then `python3 -m physis_amd.profile_summary OUT_fetch OUT_write` writes the
 per-kernel HBM traffic summary.
 
