@@ -454,7 +454,12 @@ struct EpiArgs {
 // taps, whose sums live in registers and rotate.  A rows: with 8 output
 // channels, 8 h + co of output row y + h (zero where ry - h is no tap); with
 // 24, sets 0 and 1 hold channels 0 .. 15 of the two rows and set 2 channels
-// 16 .. 23 of both.  With 2 input channels k = (4 ry + dx) 2 + ci, one K step.
+// 16 .. 23 of both.  With 2 staged input channels the B operand's other six
+// are zeros, so that the sums are those of the layer's 8 channels to the bit:
+// one K step of 4 ry x 3 dx x 2 channels sums in another order, and the BF16
+// roundings of ten layers make 6e-4 of a prediction of those last bits (its
+// error against 64 bits, 2.8e-3, stays the same).  That costs 34 us of 731 at
+// 8 x 128^3; held to four waves per SIMD (130 VGPRs without) 14 less.
 // The kernel it replaces held a ring of planes and read every B operand
 // three times: LDS reads bounded it (24 -> 8 at 8 x 128^3: 184 us of LDS
 // time in 396 us, now 245 with the concatenation read in place, which was
@@ -464,7 +469,7 @@ struct EpiArgs {
 template <int CIN, int COUT, bool RELU, int XT, int TY,
           template <int, int, int, int> class SRC, int EPI,
           typename PT = double>
-__global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
+__global__ __launch_bounds__(64 * TY, CIN == 2 ? 4 : 1) void ConvMKernel(
     SrcArgs src, const u16 *__restrict__ wt, EpiArgs ep, int D, int H, int W,
     int tz, int zchunk) {
   static_assert(COUT == 8 || COUT == 24, "output channels");
@@ -472,7 +477,7 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
   constexpr int S = COUT == 8 ? 1 : 3;  // A operands per B operand
   constexpr int WC = CIN == 2 ? 8 : CIN;  // channels of the stored weights
   constexpr int KPW = KPad(WC);
-  constexpr int KS = CIN == 2 ? 1 : 12 * CIN / 32;  // K steps per plane
+  constexpr int KS = 12 * WC / 32;  // K steps per plane
   constexpr int NTH = 64 * TY, ROWS = 2 * TY;
   constexpr int XS = XT + 2, RS = ROWS + 2;
   constexpr int PLANE = RS * XS * CIN;  // u16 elements of a staged plane
@@ -506,9 +511,9 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
 #pragma unroll
   for (int kb = 0; kb < KS; ++kb) {
     const int k0 = kb * 32 + 8 * g;
-    const int cell = CIN == 2 ? 0 : k0 / CIN, ci0 = k0 - cell * CIN;
-    const int ry = CIN == 2 ? g : cell / 3, dx = CIN == 2 ? 0 : cell % 3;
-    boff[kb] = (ry * XS + dx) * CIN + (CIN == 2 ? 0 : ci0);
+    const int cell = k0 / WC, ci0 = k0 - cell * WC;
+    const int ry = cell / 3, dx = cell % 3;
+    boff[kb] = (ry * XS + dx) * CIN + ci0;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int h = COUT == 8 || s == 2 ? r >> 3 : s;
@@ -516,21 +521,10 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
       const int dy = ry - h;
 #pragma unroll
       for (int t = 0; t < 3; ++t) {
-        bf16x8 a = Zero8();
-        if (dy >= 0 && dy <= 2) {
-          const u16 *w = wt + (long)co * KPW + (9 * t + 3 * dy + dx) * WC;
-          if constexpr (CIN == 2) {
-            unsigned v[4];
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-              v[d] = *reinterpret_cast<const unsigned *>(w + d * WC);
-            v[3] = 0;
-            a = __builtin_bit_cast(bf16x8, make_uint4(v[0], v[1], v[2], v[3]));
-          } else {
-            a = Load8(w + ci0);
-          }
-        }
-        aw[s][t][kb] = a;
+        aw[s][t][kb] =
+            dy >= 0 && dy <= 2
+                ? Load8(wt + (long)co * KPW + (9 * t + 3 * dy + dx) * WC + ci0)
+                : Zero8();
       }
     }
   }
@@ -596,10 +590,10 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
         for (int kb = 0; kb < KS; ++kb) {
           bf16x8 bo;
           if constexpr (CIN == 2) {
-            const unsigned *w = reinterpret_cast<const unsigned *>(
-                rb + 16 * i * CIN + boff[kb]);
-            // (the fourth position has no weight)
-            bo = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], 0u));
+            bo = __builtin_bit_cast(
+                bf16x8, make_uint4(*reinterpret_cast<const unsigned *>(
+                                       rb + 16 * i * CIN + boff[kb]),
+                                   0u, 0u, 0u));
           } else {
             bo = *reinterpret_cast<const bf16x8 *>(rb + 16 * i * CIN + boff[kb]);
           }
@@ -654,11 +648,17 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 3 : 1) void ConvMKernel(
                              __uint_as_float(w2.y & 0xffff0000u)};
         }
         if constexpr (EPI == kEpiPredict) {
-          float s = hw[0] * __uint_as_float(w2.x << 16);
-          s += hw[1] * __uint_as_float(w2.x & 0xffff0000u);
-          s += hw[2] * __uint_as_float(w2.y << 16);
-          s += hw[3] * __uint_as_float(w2.y & 0xffff0000u);
-          pv[i] = s + __shfl_xor(s, 16, 64);
+          // channel by channel: the even lane's four, then the odd lane's
+          const auto dot = [&](float s) {
+            s += hw[0] * __uint_as_float(w2.x << 16);
+            s += hw[1] * __uint_as_float(w2.x & 0xffff0000u);
+            s += hw[2] * __uint_as_float(w2.y << 16);
+            s += hw[3] * __uint_as_float(w2.y & 0xffff0000u);
+            return s;
+          };
+          const float all = dot(__shfl_xor(dot(0.0f), 16, 64));  // odd lanes'
+          const float below = __shfl_xor(all, 16, 64);
+          pv[i] = g & 1 ? all : below;
           if (i % 2 == 1 || i == SEG - 1) {  // the pair's stores
             const int xp = x0 + 16 * (i & ~1) + r + px;
             const float q = (g & 1) && i % 2 == 1 ? pv[i] : pv[i & ~1];
@@ -1372,9 +1372,10 @@ void ConvZLaunch(const u16 *x, const u16 *wt, const float *b, bool relu,
 // The input-marching convolution (8 or 24 output channels).  Block shapes
 // (XT positions by 2 TY rows) measured at 8 x 128^3, us, of 64x8, 32x8, 64x16
 // and 32x16: plain 8 -> 8 115 / 102 / 131 / 109; gated 164 / 216 / 177 / 150;
-// prediction 202 / 228 / 201 / 143; network input 91 / 113 / 101 / 118;
-// 24 -> 8 (32x8, 32x16) 234 / 267; 8 -> 24 with cell sums 401 / 288.  Rows of
-// at most 16 positions take XT = 16.
+// prediction 202 / 228 / 201 / 143; network input (a whole prediction) 731 /
+// 736 / 741 / 736; 24 -> 8 (32x8, 32x16) 234 / 267; 8 -> 24 with cell sums 401
+// / 288.  Other sizes take the same shapes unmeasured, but rows of at most 16
+// positions XT = 16.
 constexpr int kConvMWavesPerCU = 16;
 template <int CIN, int COUT, bool RELU, int XT, int TY,
           template <int, int, int, int> class SRC, int EPI, typename PT>

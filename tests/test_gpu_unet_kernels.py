@@ -2,7 +2,9 @@
 (oracle/unet_ref.py): convolutions of 8 and 24 output channels and filter
 gradients on rows one off a tile's width, heights one off its rows and few
 planes; whole networks on problems whose rows are not multiples of the tiles,
-over a window of the problems of a grid."""
+over a window of the problems of a grid; and the fused passes (network input,
+pool, concatenation, gate, head) against the layers they are made of, to the
+bit."""
 import os
 import sys
 
@@ -101,3 +103,113 @@ def test_network(ps, shape, problems, first, count, dtype):
         net.free()
         for g in grids + [p]:
             ps.PSGridFree(g)
+
+
+def _round(a):
+    return U.bf16_float(U.bf16_bits(a)).reshape(a.shape)
+
+
+def _up(a):
+    for axis in (1, 2, 3):
+        a = a.repeat(4, axis)
+    return a
+
+
+def _pool(a, wave):
+    """4x4x4 means of BF16 values, summed in FP32 one after another, or (wave)
+    as the first pool sums: planes, then pairs of columns, then of rows."""
+    n, d, h, w, c = a.shape
+    a = a.reshape(n, d // 4, 4, h // 4, 4, w // 4, 4, c)
+    if wave:
+        s = ((a[:, :, 0] + a[:, :, 1]) + a[:, :, 2]) + a[:, :, 3]
+        s = (s[..., 0, :] + s[..., 1, :]) + (s[..., 2, :] + s[..., 3, :])
+        s = (s[:, :, :, 0] + s[:, :, :, 1]) + (s[:, :, :, 2] + s[:, :, :, 3])
+    else:
+        s = np.zeros((n, d // 4, h // 4, w // 4, c), np.float32)
+        for z in range(4):
+            for y in range(4):
+                for x in range(4):
+                    s += a[:, :, z, :, y, :, x]
+    return _round(s * np.float32(1 / 64))
+
+
+@pytest.mark.parametrize("shape,batch", [((16, 16, 16), 2), ((48, 32, 16), 1),
+                                         ((80, 16, 32), 1)])
+def test_network_is_its_layers(ps, shape, batch):
+    """The prediction, and the gradients of the last two layers, are to the
+    bit what the layers give one after another on whole 8-channel tensors:
+    the network input as a tensor of 8 channels, pools, upsampling,
+    concatenation, gate and head in numpy."""
+    from physis_amd.warmstart import (UNet, conv_backward_data_host,
+                                      conv_backward_filter_host,
+                                      conv_forward_host)
+    print(f"layers of {shape} x {batch}", flush=True)
+    nx, ny, nzs = shape
+    m = nx * ny * nzs * batch
+    coefs = poisson_problem(nx, ny, nzs, nbatch=batch, gaussians=(3, 6),
+                            sigma=(2.0, 5.0), seed=11)
+    rhs, bnd = coefs[11].reshape(-1), coefs[10].reshape(-1)
+    target = (np.random.default_rng(3).standard_normal(m) * bnd) \
+        .astype(np.float32)
+    grids = []
+    for a in (rhs, bnd, target):
+        grids.append(ps.PSGridNew((nx, ny, nzs * batch)))
+        ps.PSGridCopyin(grids[-1], a)
+    p = ps.PSGridNew((nx, ny, nzs * batch), np.float64)
+    scale = np.float32(4.0)
+    net = UNet(nx, ny, nzs, batch, float(scale), seed=5)
+    try:
+        par = net.get_params()
+        _, grad = net.loss_grad(*grids, 0, batch)
+        net.predict(grids[0], grids[1], 0, batch, p)
+        got = ps.PSGridCopyout(p)
+    finally:
+        net.free()
+        for g in grids + [p]:
+            ps.PSGridFree(g)
+    off, layers = 0, []
+    for ci, co in ((8, 8), (8, 8), (8, 16), (16, 16), (16, 32), (32, 32),
+                   (48, 16), (16, 16), (24, 8), (8, 8)):
+        k = co * 27 * ci
+        layers.append((ci, co, U.bf16_bits(par[off:off + k]),
+                       par[off + k:off + k + co],
+                       slice(off, off + k), slice(off + k, off + k + co)))
+        off += k + co
+    head = par[off:off + 9]
+
+    def conv(l, a):
+        ci, co, w, b = layers[l][:4]
+        y = conv_forward_host(U.bf16_bits(a.reshape(-1)), w, b, True,
+                              *a.shape[:4], ci, co)
+        return U.bf16_float(y).reshape(a.shape[:4] + (co,))
+
+    x = np.zeros((batch, nzs, ny, nx, 8), np.float32)
+    x[..., 0] = _round(rhs).reshape(x.shape[:4])
+    x[..., 1] = _round(bnd).reshape(x.shape[:4])
+    a1 = conv(1, conv(0, x))
+    a3 = conv(3, conv(2, _pool(a1, True)))
+    a5 = conv(5, conv(4, _pool(a3, False)))
+    a7 = conv(7, conv(6, np.concatenate([_up(a5), a3], 4)))
+    c1 = np.concatenate([_up(a7), a1], 4)
+    a8 = conv(8, c1)
+    a9 = conv(9, a8)
+    out = np.zeros(a9.shape[:4], np.float32)
+    for c in range(8):
+        out += head[c] * a9[..., c]
+    out = (out + head[8]).reshape(-1)
+    assert np.array_equal(got, (scale * out).astype(np.float64) * bnd)
+    # the head's gradient, through the gates of the last two layers
+    g = np.float32(2.0) * (out - target * (np.float32(1) / scale)) / \
+        np.float32(m)
+    dz = _round(np.where(a9 > 0, head[:8] * g.reshape(a9.shape[:4] + (1,)),
+                         np.float32(0)))
+    for l, below in ((9, a8), (8, c1)):
+        ci, co, w, _, ws, bs = layers[l]
+        dims = below.shape[:4] + (ci, co)
+        bits = U.bf16_bits(dz.reshape(-1))
+        dw, db = conv_backward_filter_host(U.bf16_bits(below.reshape(-1)),
+                                           bits, *dims)
+        assert np.array_equal(grad[ws], dw) and np.array_equal(grad[bs], db)
+        if l == 9:
+            dx = U.bf16_float(conv_backward_data_host(bits, w, *dims))
+            dz = np.where(below > 0, dx.reshape(below.shape), np.float32(0))
