@@ -438,12 +438,14 @@ class ReduceSlots {
   int next_ = 1;
 };
 
-// Partial results of a PSStencilMapReduce map inside one run function.  The
-// run kernel of execution i writes one partial per block into Slot(i);
-// After(i) queues the fold of every completed batch of executions into pinned
-// memory, and Finish() waits and hands the results to the user's array
-// (out[i] = reduction of execution i).  A NULL out makes it a no-op.  (A wait
-// and a copy per map and batch cost 50 us each.)
+// Partial results of a PSStencilMapReduce map inside one run function.  A
+// launch of executions i, i + 1 (a pass of several pairs; else i alone) writes
+// one partial per block into Slot(i), Slot(i + 1); After(last of them) queues
+// the fold of the executions so far into pinned memory once they are a batch
+// (one slot is to spare for the launch that goes past it), and Finish() waits
+// and hands the results to the user's array (out[i] = reduction of execution
+// i).  A NULL out makes it a no-op.  (A wait and a copy per map and batch cost
+// 50 us each.)
 class MapReducer {
  public:
   MapReducer(void *out, int op, int type, int nblocks, int iter,
@@ -455,22 +457,22 @@ class MapReducer {
       return;
     }
     elm_ = (type == PS_DOUBLE || type == PS_LONG) ? 8 : 4;
-    batch_ = iter < kBatch ? iter : kBatch;
     const int slot = slots.Next();
-    base_ = (char *)__PSHipScratch(slot, (size_t)batch_ * nblocks_ * elm_);
+    const int held = iter <= kBatch ? iter : kBatch + 1;
+    base_ = (char *)__PSHipScratch(slot, (size_t)held * nblocks_ * elm_);
     pinned_ = (char *)__PSHipPinned(slot, (size_t)iter * elm_);
   }
   void *Slot(int i) const {
     if (!out_) return nullptr;
-    return base_ + (size_t)(i % batch_) * nblocks_ * elm_;
+    return base_ + (size_t)(i - first_) * nblocks_ * elm_;
   }
   void After(int i) {
     if (!out_) return;
-    if ((i + 1) % batch_ != 0 && i + 1 != iter_) return;
-    const int first = i - (i % batch_);
-    const int count = i + 1 - first;
+    const int count = i + 1 - first_;
+    if (count < kBatch && i + 1 != iter_) return;
     __PSHipReduceFoldAsync(type_, op_, base_, nblocks_, count,
-                           pinned_ + (size_t)first * elm_);
+                           pinned_ + (size_t)first_ * elm_);
+    first_ = i + 1;
   }
   void Finish(hipStream_t stream) {
     if (!out_) return;
@@ -487,7 +489,7 @@ class MapReducer {
   static constexpr int kBatch = 256;
   char *out_;
   int op_, type_, nblocks_, iter_;
-  int elm_ = 4, batch_ = 1;
+  int elm_ = 4, first_ = 0;  // first execution not folded yet
   char *base_ = nullptr, *pinned_ = nullptr;
 };
 

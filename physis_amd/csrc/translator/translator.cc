@@ -2819,8 +2819,7 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
               : last + " ? vb.p : NULL, stream")
       << ");\n";
     if (red)
-      f << "      for (const int e = i + pairs; i < e; ++i) {\n"
-           "        red0.After(i);\n        red1.After(i);\n      }\n";
+      f << "      i += pairs;\n      red0.After(i - 1);\n      red1.After(i - 1);\n";
     return f.str();
   };
   if (!k.fuse_domain) {

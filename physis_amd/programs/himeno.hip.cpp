@@ -917,10 +917,9 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_jacobi_kernel s0, stru
       if (passes % 2 && j < 2) dst = j == 0 ? vt : vt2;
       const int pairs = 1;
       __PSLaunch2_jacobi_kernel(s0, src, dst, (j == passes - 1), stream, red0.Slot(i), red1.Slot(i));
-      for (const int e = i + pairs; i < e; ++i) {
-        red0.After(i);
-        red1.After(i);
-      }
+      i += pairs;
+      red0.After(i - 1);
+      red1.After(i - 1);
       src = dst;
     }
     i0 = iter;
@@ -977,10 +976,9 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_jacobi_kernel s0, stru
       if (passes % 2 && j < 2) dst = j == 0 ? vt : vt2;
       const int pairs = 1;
       __PSLaunch2_jacobi_kernel(s0, src, dst, (j == passes - 1), stream, red0.Slot(i), red1.Slot(i));
-      for (const int e = i + pairs; i < e; ++i) {
-        red0.After(i);
-        red1.After(i);
-      }
+      i += pairs;
+      red0.After(i - 1);
+      red1.After(i - 1);
       src = dst;
     }
     i0 = iter;

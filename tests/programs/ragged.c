@@ -1,7 +1,8 @@
 /* Maps that read past the ends of rows whose extents are multiples of
  * nothing: non-periodic gets over the whole grid (an index past the end of a
  * row names the next row's points, one outside the grid 0), periodic gets
- * two points away, and a map pair over the interior. */
+ * two points away, a map pair over the interior, and pairs over a box of the
+ * grid whose kernels return the change of each point. */
 #include "physis/physis.h"
 
 static void corners(const int x, const int y, const int z, PSGrid3DFloat g,
@@ -51,6 +52,27 @@ static void inner(const int x, const int y, const int z, PSGrid3DFloat g,
   PSGridEmit(g2, v * w);
 }
 
+static float settle(const int x, const int y, const int z, PSGrid3DFloat g,
+                    PSGrid3DFloat g2, PSGrid3DFloat c, float w) {
+  float u = PSGridGet(g, x, y, z);
+  float v = u + PSGridGet(g, x+1, y-1, z) + PSGridGet(g, x-1, y+1, z) +
+            PSGridGet(g, x, y, z+1) + PSGridGet(g, x, y, z-1);
+  v = v * w + PSGridGet(c, x, y, z);
+  PSGridEmit(g2, v);
+  return v - u;
+}
+
+static double settle_square(const int x, const int y, const int z,
+                            PSGrid3DFloat g, PSGrid3DFloat g2, float w) {
+  float u = PSGridGet(g, x, y, z);
+  float v = u + PSGridGet(g, x+1, y-1, z) + PSGridGet(g, x-1, y+1, z) +
+            PSGridGet(g, x, y, z+1) + PSGridGet(g, x, y, z-1);
+  v = v * w;
+  PSGridEmit(g2, v);
+  double d = v - u;
+  return d * d;
+}
+
 static PSDomain3D whole(PSGrid3DFloat g) {
   return PSDomain3DNew(0, PSGridDim(g, 0), 0, PSGridDim(g, 1), 0,
                        PSGridDim(g, 2));
@@ -81,5 +103,26 @@ void ragged_inner(PSGrid3DFloat g, PSGrid3DFloat g2, int count, float w) {
   PSDomain3D d = PSDomain3DNew(1, PSGridDim(g, 0) - 1, 1, PSGridDim(g, 1) - 1,
                                1, PSGridDim(g, 2) - 1);
   PSStencilRun(PSStencilMap(inner, d, g, g2, w), PSStencilMap(inner, d, g2, g, w),
+               count);
+}
+
+/* count pairs over the box; more[i] and back[i]: the largest change of the
+ * sweeps of pair i. */
+void ragged_settle(PSGrid3DFloat g, PSGrid3DFloat g2, PSGrid3DFloat c, int x0,
+                   int x1, int y0, int y1, int z0, int z1, int count, float w,
+                   float *more, float *back) {
+  PSDomain3D d = PSDomain3DNew(x0, x1, y0, y1, z0, z1);
+  PSStencilRun(PSStencilMapReduce(more, PS_MAX, settle, d, g, g2, c, w),
+               PSStencilMapReduce(back, PS_MAX, settle, d, g2, g, c, w),
+               count);
+}
+
+/* The same without the third grid; the sums of the squared changes. */
+void ragged_settle_square(PSGrid3DFloat g, PSGrid3DFloat g2, int x0, int x1,
+                          int y0, int y1, int z0, int z1, int count, float w,
+                          double *more, double *back) {
+  PSDomain3D d = PSDomain3DNew(x0, x1, y0, y1, z0, z1);
+  PSStencilRun(PSStencilMapReduce(more, PS_SUM, settle_square, d, g, g2, w),
+               PSStencilMapReduce(back, PS_SUM, settle_square, d, g2, g, w),
                count);
 }

@@ -2,7 +2,8 @@
 of a fused pair or two red-black iterations per launch) against the oracle,
 bit for bit on both grids: extents below the halo, at and one off the tiles'
 edges, on both sides of the tile-size and of the grid-size rule, where
-whole-grid pairs take two and four points per lane; odd and even counts."""
+whole-grid pairs take two and four points per lane; odd and even counts; pairs
+over a box of the grid and their results per sweep, against numpy."""
 import ctypes as C
 
 import numpy as np
@@ -93,3 +94,66 @@ def test_interior_pairs(ps, shape):
         assert np.array_equal(ps.PSGridCopyout(g2), u[1].reshape(-1)), count
     ps.PSGridFree(g)
     ps.PSGridFree(g2)
+
+
+# (shape, box): the interior, boxes off the grid's origin in tiles of both
+# sizes, and one in a grid too large for tiles (z-marching passes)
+BOXES = [((18, 10, 10), None), ((70, 40, 30), (21, 58, 9, 31, 5, 24)),
+         ((130, 128, 128), None), ((130, 128, 128), (5, 126, 3, 67, 60, 127)),
+         ((260, 100, 90), (130, 171, 50, 61, 33, 45))]
+
+
+@pytest.mark.parametrize("square", [False, True])
+@pytest.mark.parametrize("shape,box,counts",
+                         [s + ((1, 2, 3, 4, 5),) for s in BOXES] +
+                         # more executions than fold at once (256), from an
+                         # even and from an odd first pass
+                         [BOXES[0] + ((256, 257, 258, 513),)])
+def test_reducing_pairs(ps, shape, box, counts, square):
+    """Pairs over a box, with a result per sweep: every result, and both
+    grids bit for bit."""
+    L = ps.load_program("ragged")
+    G, N = ps.PSGridPtr, [C.c_int] * 7 + [C.c_float, C.c_void_p, C.c_void_p]
+    L.ragged_settle.argtypes = [G, G, G] + N
+    L.ragged_settle_square.argtypes = [G, G] + N
+    nx, ny, nz = shape
+    x0, x1, y0, y1, z0, z1 = box = box or (1, nx - 1, 1, ny - 1, 1, nz - 1)
+    rng = np.random.default_rng(nx + x0)
+    a, b, c = rng.standard_normal((3, nz, ny, nx)).astype(np.float32)
+    w, dtype = np.float32(0.2), np.float64 if square else np.float32
+    i = (slice(z0, z1), slice(y0, y1), slice(x0, x1))
+    u, want, ends = [a.copy(), b.copy()], [], {}
+    for k in range(2 * max(counts)):
+        s = u[k % 2]
+        v = s[i] + s[z0:z1, y0 - 1:y1 - 1, x0 + 1:x1 + 1] + \
+            s[z0:z1, y0 + 1:y1 + 1, x0 - 1:x1 - 1] + \
+            s[z0 + 1:z1 + 1, y0:y1, x0:x1] + s[z0 - 1:z1 - 1, y0:y1, x0:x1]
+        v = v * w if square else v * w + c[i]
+        d = v - s[i]
+        want.append(np.sum(d.astype(np.float64) ** 2) if square else d.max())
+        u[1 - k % 2][i] = v
+        if (k + 1) % 2 == 0 and (k + 1) // 2 in counts:
+            ends[(k + 1) // 2] = [x.copy() for x in u]
+    grids = [ps.PSGridNew(shape) for _ in range(3)]
+    ps.PSGridCopyin(grids[2], c)
+    for count in counts:
+        print(f"reducing {shape} {box} x {count} square={square}", flush=True)
+        for g, x in zip(grids, (a, b)):
+            ps.PSGridCopyin(g, x)
+        got = np.full((2, count), -1, dtype)
+        args = list(box) + [count, w, got[0].ctypes.data, got[1].ctypes.data]
+        if square:
+            L.ragged_settle_square(*[g.handle for g in grids[:2]], *args)
+        else:
+            L.ragged_settle(*[g.handle for g in grids], *args)
+        for g, x in zip(grids, ends[count]):
+            assert np.array_equal(ps.PSGridCopyout(g), x.reshape(-1)), count
+        ref = np.array(want[:2 * count], dtype).reshape(count, 2).T
+        if square:  # FP64 sums of (at most) this many terms, all positive
+            err = np.abs(got - ref)
+            assert np.all(err <= d.size * 2.0 ** -53 * ref), \
+                (count, np.argwhere(err > d.size * 2.0 ** -53 * ref))
+        else:
+            assert np.array_equal(got, ref), (count, np.argwhere(got != ref))
+    for g in grids:
+        ps.PSGridFree(g)
