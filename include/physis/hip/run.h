@@ -215,13 +215,13 @@ inline void CopyDevice(void *dst, const void *src, size_t bytes,
   }
 }
 
-// Copies the points of an nx x ny x nz grid outside a domain inside it: one
-// thread per row of the domain copies its ends, then one block per row that
-// lies outside.
+// Copies the points of an nx x ny x nz grid view that lie outside a domain and
+// at most one point from it: one thread per row of the domain copies the point
+// beyond either end, then one thread per point the rows of the shell.
 template <typename T>
-__global__ __launch_bounds__(256) void CopyOutsideKernel(
-    T *__restrict__ dst, const T *__restrict__ src, int nx, int ny, int nz,
-    __PSDomain d, int row_blocks) {
+__global__ __launch_bounds__(256) void CopyShellKernel(
+    T *__restrict__ dst, const T *__restrict__ src, int nx, int ny,
+    __PSDomain d, __PSDomain box, int row_blocks, int outer) {
   const int x0 = d.local_min[0], x1 = d.local_max[0];
   const int y0 = d.local_min[1], dy = d.local_max[1] - y0;
   const int z0 = d.local_min[2], dz = d.local_max[2] - z0;
@@ -229,38 +229,56 @@ __global__ __launch_bounds__(256) void CopyOutsideKernel(
     const int r = blockIdx.x * 256 + threadIdx.x;
     if (r >= dy * dz) return;
     const long row = ((long)(z0 + r / dy) * ny + y0 + r % dy) * nx;
-    for (int x = 0; x < x0; ++x) dst[row + x] = src[row + x];
-    for (int x = x1; x < nx; ++x) dst[row + x] = src[row + x];
+    if (x0 > box.local_min[0]) dst[row + x0 - 1] = src[row + x0 - 1];
+    if (x1 < box.local_max[0]) dst[row + x1] = src[row + x1];
     return;
   }
-  int r = blockIdx.x - row_blocks, y, z;
-  if (r < (nz - dz) * ny) {  // a plane outside
-    z = r / ny;
-    y = r - z * ny;
-    z = z < z0 ? z : z + dz;
+  const int bx = box.local_max[0] - box.local_min[0];
+  const int by = box.local_max[1] - box.local_min[1];
+  const int bz = box.local_max[2] - box.local_min[2];
+  const int i = (blockIdx.x - row_blocks) * 256 + threadIdx.x;
+  if (i >= outer) return;
+  int r = i / bx, y, z;  // row of the shell
+  if (r < (bz - dz) * by) {  // in a plane before or behind the domain's
+    z = r / by;
+    y = box.local_min[1] + r - z * by;
+    z = box.local_min[2] + z;
+    if (z >= z0) z += dz;
   } else {
-    r -= (nz - dz) * ny;
-    z = r / (ny - dy);
-    y = r - z * (ny - dy);
-    y = y < y0 ? y : y + dy;
+    r -= (bz - dz) * by;
+    z = r / (by - dy);
+    y = box.local_min[1] + r - z * (by - dy);
+    if (y >= y0) y += dy;
     z += z0;
   }
-  const long row = ((long)z * ny + y) * nx;
-  for (int x = threadIdx.x; x < nx; x += 256) dst[row + x] = src[row + x];
+  const long at = ((long)z * ny + y) * nx + box.local_min[0] + i % bx;
+  dst[at] = src[at];
 }
 
-// The points of grid view src outside domain d into dst (the scratch grids
-// of passes over a domain: stores stay inside it, so that only these have to
-// be there).  Copying whole grids took 34 us of the 10 sweeps of a 4096^2 map.
+// Grid view src's points around domain d into dst: what the passes over a
+// domain need of a scratch grid they write (stores stay inside the domain, and
+// a point reads no further than one beyond it).  The rest of the scratch grid
+// stays as it is: copying whole grids took 34 us of the 10 sweeps of a 4096^2
+// map, and copying every point outside the domain 3.6 ms of two pairs over 100 x
+// 100 points of 16384^2 (15 us now) and 354 us of two over 64^3 points of 512^3
+// (30 now).
 template <typename T>
-inline void CopyOutside(T *dst, const T *src, int nx, int ny, int nz,
-                        const __PSDomain &d, hipStream_t stream) {
-  const int dy = d.local_max[1] - d.local_min[1];
-  const int dz = d.local_max[2] - d.local_min[2];
-  const int row_blocks = (dy * dz + 255) / 256;
-  const int outside = (nz - dz) * ny + dz * (ny - dy);
-  hipLaunchKernelGGL(CopyOutsideKernel<T>, dim3(row_blocks + outside),
-                     dim3(256), 0, stream, dst, src, nx, ny, nz, d, row_blocks);
+inline void CopyShell(T *dst, const T *src, int nx, int ny, int nz,
+                      const __PSDomain &d, hipStream_t stream) {
+  const int n[3] = {nx, ny, nz};
+  __PSDomain box = d;
+  int e[3], b[3];
+  for (int i = 0; i < 3; ++i) {
+    if (box.local_min[i] > 0) --box.local_min[i];
+    if (box.local_max[i] < n[i]) ++box.local_max[i];
+    e[i] = d.local_max[i] - d.local_min[i];
+    b[i] = box.local_max[i] - box.local_min[i];
+  }
+  const int row_blocks = (e[1] * e[2] + 255) / 256;
+  const int outer = ((b[2] - e[2]) * b[1] + e[2] * (b[1] - e[1])) * b[0];
+  hipLaunchKernelGGL(CopyShellKernel<T>, dim3(row_blocks + (outer + 255) / 256),
+                     dim3(256), 0, stream, dst, src, nx, ny, d, box, row_blocks,
+                     outer);
 }
 
 // The domain of a map must lie inside every grid the map emits to; the run

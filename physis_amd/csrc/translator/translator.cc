@@ -2835,17 +2835,17 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
       << "      src = dst;\n    }\n";
   } else {
     // Points outside the domain keep a's values in a, so the scratch grids
-    // the passes write start with a's values there (stores stay inside the
-    // domain).  Even counts ping-pong a -> t -> a ...; odd counts (>= 3) go
+    // the passes write start with a's values around it (stores stay inside the
+    // domain, and no point reads further than one beyond it).  Even counts ping-pong a -> t -> a ...; odd counts (>= 3) go
     // a -> t -> t2 -> a -> t -> a ... (b's values outside the domain are
     // read by every pass, so b cannot hold a pass).  The last pass writes a,
     // and its last but one sweep to b.
     o << "    " << V << " vt2 = va;\n"
-      << "    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], "
+      << "    physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], "
          "s0.dom, stream);\n"
       << "    if (passes % 2) {\n"
       << "      vt2.p = (" << T << " *)__PSHipScratch(9, bytes);\n"
-      << "      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], "
+      << "      physis_hip::CopyShell(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], "
          "s0.dom, stream);\n    }\n"
       << "    " << V << " src = va;\n"
       << "    for (int j = 0" << (red ? ", i = 0" : "") << "; j < passes; ++j) {\n"
@@ -3564,10 +3564,10 @@ std::string Translator::EmitFusedRowsRun(const KernelInfo &k) {
     << "    " << V << " vt = va, vt2 = va;\n"
     << "    vt.p = (float *)__PSHipScratch(8, bytes);\n"
     << "    const __PSDomain d = physis_hip::RowDomain(s0.dom);\n"
-    << "    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], 1, va.dim[2], d, stream);\n"
+    << "    physis_hip::CopyShell(vt.p, va.p, va.dim[0], 1, va.dim[2], d, stream);\n"
     << "    if (passes % 2) {\n"
     << "      vt2.p = (float *)__PSHipScratch(9, bytes);\n"
-    << "      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], 1, va.dim[2], d, stream);\n    }\n"
+    << "      physis_hip::CopyShell(vt2.p, va.p, va.dim[0], 1, va.dim[2], d, stream);\n    }\n"
     << "    " << V << " src = va;\n"
     << "    for (int j = 0; j < passes; ++j) {\n"
     << "      " << V << " dst = (j % 2 == (passes % 2 ? 0 : 1)) ? va : vt;\n"

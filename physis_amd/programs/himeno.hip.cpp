@@ -906,10 +906,10 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_jacobi_kernel s0, stru
     vt.p = (float *)__PSHipScratch(8, bytes);
     const int passes = iter;
     __PSGrid3DFloat_dev vt2 = va;
-    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
+    physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
-      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
+      physis_hip::CopyShell(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     }
     __PSGrid3DFloat_dev src = va;
     for (int j = 0, i = 0; j < passes; ++j) {
@@ -965,10 +965,10 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_jacobi_kernel s0, stru
     vt.p = (float *)__PSHipScratch(8, bytes);
     const int passes = iter;
     __PSGrid3DFloat_dev vt2 = va;
-    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
+    physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
-      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
+      physis_hip::CopyShell(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     }
     __PSGrid3DFloat_dev src = va;
     for (int j = 0, i = 0; j < passes; ++j) {

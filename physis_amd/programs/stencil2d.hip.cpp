@@ -630,10 +630,10 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_s2d5 s0, struct __PSSt
     __PSGrid3DFloat_dev vt = va, vt2 = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const __PSDomain d = physis_hip::RowDomain(s0.dom);
-    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], 1, va.dim[2], d, stream);
+    physis_hip::CopyShell(vt.p, va.p, va.dim[0], 1, va.dim[2], d, stream);
     if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
-      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], 1, va.dim[2], d, stream);
+      physis_hip::CopyShell(vt2.p, va.p, va.dim[0], 1, va.dim[2], d, stream);
     }
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {
@@ -670,10 +670,10 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_s2d9 s0, struct __PSSt
     __PSGrid3DFloat_dev vt = va, vt2 = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const __PSDomain d = physis_hip::RowDomain(s0.dom);
-    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], 1, va.dim[2], d, stream);
+    physis_hip::CopyShell(vt.p, va.p, va.dim[0], 1, va.dim[2], d, stream);
     if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
-      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], 1, va.dim[2], d, stream);
+      physis_hip::CopyShell(vt2.p, va.p, va.dim[0], 1, va.dim[2], d, stream);
     }
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {

@@ -73,6 +73,14 @@ static double settle_square(const int x, const int y, const int z,
   return d * d;
 }
 
+static void inner2d(const int x, const int y, PSGrid2DFloat g,
+                    PSGrid2DFloat g2, float w) {
+  float v = PSGridGet(g, x, y) + PSGridGet(g, x+1, y-1) +
+            PSGridGet(g, x-1, y+1) + PSGridGet(g, x-1, y) +
+            PSGridGet(g, x+1, y+1);
+  PSGridEmit(g2, v * w);
+}
+
 static PSDomain3D whole(PSGrid3DFloat g) {
   return PSDomain3DNew(0, PSGridDim(g, 0), 0, PSGridDim(g, 1), 0,
                        PSGridDim(g, 2));
@@ -125,4 +133,19 @@ void ragged_settle_square(PSGrid3DFloat g, PSGrid3DFloat g2, int x0, int x1,
   PSStencilRun(PSStencilMapReduce(more, PS_SUM, settle_square, d, g, g2, w),
                PSStencilMapReduce(back, PS_SUM, settle_square, d, g2, g, w),
                count);
+}
+
+/* count pairs of sweeps over a box, without results. */
+void ragged_box(PSGrid3DFloat g, PSGrid3DFloat g2, int x0, int x1, int y0,
+                int y1, int z0, int z1, int count, float w) {
+  PSDomain3D d = PSDomain3DNew(x0, x1, y0, y1, z0, z1);
+  PSStencilRun(PSStencilMap(inner, d, g, g2, w), PSStencilMap(inner, d, g2, g, w),
+               count);
+}
+
+void ragged_box2d(PSGrid2DFloat g, PSGrid2DFloat g2, int x0, int x1, int y0,
+                  int y1, int count, float w) {
+  PSDomain2D d = PSDomain2DNew(x0, x1, y0, y1);
+  PSStencilRun(PSStencilMap(inner2d, d, g, g2, w),
+               PSStencilMap(inner2d, d, g2, g, w), count);
 }

@@ -3374,10 +3374,10 @@ static void __PSStencilRun_7(int iter, struct __PSStencil_k7 s0, struct __PSSten
     const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
-    physis_hip::CopyOutside(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
+    physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
       vt2.p = (float *)__PSHipScratch(9, bytes);
-      physis_hip::CopyOutside(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
+      physis_hip::CopyShell(vt2.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     }
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {

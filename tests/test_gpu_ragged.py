@@ -2,7 +2,7 @@
 (tests/programs/ragged.c), bit for bit against numpy: the points past the
 end of a row (the next row's, 0 outside the grid, the wrapped ones of a
 periodic get) at the sizes where a lane's vector hangs over a row's end, a
-tile's end or the grid's end."""
+tile's end or the grid's end; and pairs over boxes anywhere in a grid."""
 import ctypes as C
 
 import numpy as np
@@ -21,6 +21,8 @@ def prog(ps):
     for f in ("corners", "corners_double", "corners2d", "wrap2"):
         getattr(L, "ragged_" + f).argtypes = [G, G]
     L.ragged_inner.argtypes = [G, G, C.c_int, C.c_float]
+    L.ragged_box.argtypes = [G, G] + [C.c_int] * 7 + [C.c_float]
+    L.ragged_box2d.argtypes = [G, G] + [C.c_int] * 5 + [C.c_float]
     return L
 
 
@@ -138,3 +140,54 @@ def test_interior_pairs(ps, prog, shape, count):
         u[1 - k % 2][1:-1, 1:-1, 1:-1] = v * w
     for k in range(2):
         assert np.array_equal(got[k], u[k].reshape(-1)), k
+
+
+# In 2-D: rows passes whose first column tile is not the grid's, boxes that
+# begin and end inside a lane's four points or cross a column tile (248
+# points), thin and single-point ones.  In 3-D: resident tiles of both sizes,
+# z-marching passes in a grid too large for them, a box crossing x tiles.
+BOXES = [((300, 40), (1, 299, 1, 39)), ((301, 40), (5, 9, 3, 36)),
+         ((700, 90), (301, 650, 17, 80)), ((520, 300), (242, 262, 1, 299)),
+         ((64, 1000), (3, 61, 400, 410)), ((9, 9), (4, 5, 4, 5)),
+         ((30, 20, 25), (7, 12, 2, 19, 11, 24)),
+         ((97, 90, 80), (30, 96, 20, 81, 1, 79)),
+         ((300, 90, 90), (250, 270, 30, 50, 7, 9)),
+         ((515, 140, 60), (3, 512, 2, 137, 1, 59)),
+         ((40, 9, 9), (20, 21, 4, 5, 4, 5))]
+
+
+@pytest.mark.parametrize("shape,box", BOXES)
+def test_pairs_over_a_box(ps, prog, shape, box):
+    """1 to 7 pairs (odd and even counts of passes), both grids.  The passes'
+    scratch grids hold NaN from a run over such grids before."""
+    dims = len(shape)
+    run = prog.ragged_box if dims == 3 else prog.ragged_box2d
+    rng = np.random.default_rng(sum(shape))
+    a, b = rng.standard_normal((2,) + shape[::-1]).astype(np.float32)
+    w = np.float32(0.2)
+    offsets = [(0, 0, 0), (1, -1, 0), (-1, 1, 0), (0, 0, 1), (0, 0, -1)] \
+        if dims == 3 else [(0, 0), (1, -1), (-1, 1), (-1, 0), (1, 1)]
+
+    def at(u, d):
+        return u[tuple(slice(box[2 * k] + d[k], box[2 * k + 1] + d[k])
+                       for k in reversed(range(dims)))]
+
+    g, g2 = ps.PSGridNew(shape, np.float32), ps.PSGridNew(shape, np.float32)
+    all_of = sum(([1, n - 1] for n in shape), [])
+    u = [a.copy(), b.copy()]
+    for count in range(1, 8):
+        print(f"box {box} of {shape} x {count}", flush=True)
+        for x in (g, g2):
+            ps.PSGridCopyin(x, np.full(shape[::-1], np.nan, np.float32))
+        run(g.handle, g2.handle, *all_of, 5, w)  # both scratch grids
+        ps.PSGridCopyin(g, a)
+        ps.PSGridCopyin(g2, b)
+        run(g.handle, g2.handle, *box, count, w)
+        for k in range(2):  # the pair
+            v = _sum(lambda d: at(u[k], d), [(None, d) for d in offsets],
+                     np.float32)
+            at(u[1 - k], (0,) * dims)[...] = v * w
+        for x, want in zip((g, g2), u):
+            assert np.array_equal(ps.PSGridCopyout(x), want.reshape(-1)), count
+    ps.PSGridFree(g)
+    ps.PSGridFree(g2)
