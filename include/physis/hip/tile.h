@@ -138,9 +138,6 @@ __device__ __forceinline__ void LoadTile(E *lds, const E *p, const int *dim,
 // values of every one of them: 96^3 14.4 against 10.1).
 template <int T> using SmallTile = Tile<T, 16, 8, 8, 1024>;
 template <int T> using MidTile = Tile<T, 16, 16, 8, 1024>;
-// The largest grid of a pass over part of a grid (EmitFusedDomainKernel's
-// pairs beside it).
-constexpr int64_t kTileMaxPoints = 2200000;
 // Whether a pass over a whole grid runs in tiles: both kinds of pass cost by
 // the points of their padded tiles, us a sweep about 1.4 + 2.5 per million
 // points here and 4.3 + 1 in a z-marching pair (0.83 at four points per
@@ -158,6 +155,30 @@ inline bool TilesBeatPairs(const int *dim, bool periodic) {
   const double pair = (narrow ? up(dim[0], 128) : up(dim[0], 256) * 0.83) *
                       up(dim[1], 8) * dim[2] * 1e-6;
   return tile <= 16 && 2.5 * tile - pair < 2.2;
+}
+
+// Whether a pass over a domain inside a grid of `points` points runs in tiles,
+// beside EmitFusedDomainKernel's pairs (tiles of 256 x 12 points): us a sweep
+// about 1.4 + 2.5 per million points of the padded tiles here and 4.3 + 0.83
+// there.  Tiles and pairs, 5-point map over the interior, no results, 80 sweeps:
+// 256x60x60 3.8 and 5.3, 512x40x40 3.8 and 5.5, 128x130x130 6.3 and 7.8,
+// 24x300x300 8.8 and 21.5, 260x92x90 7.6 and 7.9, 300x100x70 7.8 and 7.7,
+// 512x128x32 6.3 and 6.6, 512x66x62 6.4 and 6.0, 256x92x92 7.4 and 5.7,
+// 1024x46x46 7.5 and 6.4; with a centre-only grid and a result per sweep both
+// cost about 1.4 times as much (256x92x92 9.8 and 8.5).  Past kTileMaxPoints
+// nothing was measured; the byte offsets of a grid of kTileMaxGrid 8-byte points
+// stay within a buffer window.
+constexpr long kTileMaxPoints = 2200000;
+constexpr int64_t kTileMaxGrid = 1 << 27;
+inline bool TilesBeatDomainPairs(const __PSDomain &d, int64_t points) {
+  const auto up = [](int n, int t) { return (double)((n + t - 1) / t * t); };
+  long e[3];
+  for (int i = 0; i < 3; ++i) e[i] = d.local_max[i] - d.local_min[i];
+  if (points > kTileMaxGrid || e[0] * e[1] * e[2] > kTileMaxPoints) return false;
+  const double tile = up(e[0], 16) * up(e[1], 16) * up(e[2], 8) * 1e-6;
+  const double wide = up(d.local_max[0], 256) - d.local_min[0] / 256 * 256;
+  const double pair = wide * up(e[1], 12) * e[2] * 1e-6;
+  return 2.5 * tile - 0.83 * pair < 2.9;
 }
 
 // Per-block partials of each sweep of a pass (NULL: none).

@@ -2788,7 +2788,7 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
   if (tiles)
     o << "    const bool __small = "
       << (k.fuse_domain
-              ? "s0." + gi.name + "->num_elms <= physis_hip::kTileMaxPoints"
+              ? "physis_hip::TilesBeatDomainPairs(s0.dom, s0." + gi.name + "->num_elms)"
               : "physis_hip::TilesBeatPairs(s0." + gi.name + "->dim, " +
                     (gi.periodic ? "true" : "false") + ")")
       << ";\n    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);\n";
@@ -3610,9 +3610,9 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
     std::string blocks = "__PSBlocks_" + k.name + "(" + si + ")";
     if (fused_pair && k.fuse_domain)
       blocks = "(!__fuse ? " + blocks +
-               (UsesTiles(k) ? " : " + si + "." + k.grids[k.fuse_in].name +
-                                   "->num_elms <= physis_hip::kTileMaxPoints ? "
-                                   "__PSBlocksT_" + k.name + "(" + si + ")"
+               (UsesTiles(k) ? " : physis_hip::TilesBeatDomainPairs(" + si + ".dom, " +
+                                   si + "." + k.grids[k.fuse_in].name +
+                                   "->num_elms) ? __PSBlocksT_" + k.name + "(" + si + ")"
                              : "") +
                " : __PSBlocks2_" + k.name + "(" + si + "))";
     o << "  physis_hip::MapReducer red" << i << "(" << si << ".__reduce_out, "

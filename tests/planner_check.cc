@@ -1,10 +1,14 @@
 // Host-only check of the run-kernel launch planner (include/physis/hip/run.h):
-// prints, for each case, the z chunk and window bytes that PlanRunFor picks.
-// Built and run by tests/test_planner.py; no device is touched.
+// prints, for each case, the z chunk and window bytes that PlanRunFor picks;
+// "tiles": whether pairs over a domain run in resident tiles
+// (include/physis/hip/tile.h).  Built and run by tests/test_planner.py; no
+// device is touched.
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 
 #include "physis/hip/run.h"
+#include "physis/hip/tile.h"
 
 namespace {
 
@@ -44,6 +48,15 @@ void Case(int nx, int ny, int nz, int elm, int margin, int tx, int ty,
 }  // namespace
 
 int main(int argc, char **argv) {
+  if (argc == 9 && std::strcmp(argv[1], "tiles") == 0) {
+    __PSDomain dom = {};
+    for (int d = 0; d < 3; ++d) {
+      dom.local_min[d] = std::atoi(argv[2 + 2 * d]);
+      dom.local_max[d] = std::atoi(argv[3 + 2 * d]);
+    }
+    std::printf("%d\n", physis_hip::TilesBeatDomainPairs(dom, std::atol(argv[8])));
+    return 0;
+  }
   if (argc > 1) {
     // one case from the command line (the rejection path exits here)
     if (argc != 9) return 2;

@@ -3275,7 +3275,7 @@ static void __PSStencilRun_4(int iter, struct __PSStencil_inner s0, struct __PSS
     const size_t bytes = (size_t)s0.g->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
@@ -3321,9 +3321,9 @@ static void __PSStencilRun_5(int iter, struct __PSStencil_settle s0, struct __PS
   physis_hip::ReduceSlots __slots;
   const bool __fuse = iter >= 2 && __PSFusable2_settle(s0, s1);
   physis_hip::MapReducer red0(s0.__reduce_out, s0.__reduce_op, PS_FLOAT,
-      s0.__reduce_out ? (!__fuse ? __PSBlocks_settle(s0) : s0.g->num_elms <= physis_hip::kTileMaxPoints ? __PSBlocksT_settle(s0) : __PSBlocks2_settle(s0)) : 0, iter, __slots);
+      s0.__reduce_out ? (!__fuse ? __PSBlocks_settle(s0) : physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? __PSBlocksT_settle(s0) : __PSBlocks2_settle(s0)) : 0, iter, __slots);
   physis_hip::MapReducer red1(s1.__reduce_out, s1.__reduce_op, PS_FLOAT,
-      s1.__reduce_out ? (!__fuse ? __PSBlocks_settle(s1) : s1.g->num_elms <= physis_hip::kTileMaxPoints ? __PSBlocksT_settle(s1) : __PSBlocks2_settle(s1)) : 0, iter, __slots);
+      s1.__reduce_out ? (!__fuse ? __PSBlocks_settle(s1) : physis_hip::TilesBeatDomainPairs(s1.dom, s1.g->num_elms) ? __PSBlocksT_settle(s1) : __PSBlocks2_settle(s1)) : 0, iter, __slots);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g, PS_FLOAT);
@@ -3333,7 +3333,7 @@ static void __PSStencilRun_5(int iter, struct __PSStencil_settle s0, struct __PS
     const size_t bytes = (size_t)s0.g->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
@@ -3386,9 +3386,9 @@ static void __PSStencilRun_6(int iter, struct __PSStencil_settle_square s0, stru
   physis_hip::ReduceSlots __slots;
   const bool __fuse = iter >= 2 && __PSFusable2_settle_square(s0, s1);
   physis_hip::MapReducer red0(s0.__reduce_out, s0.__reduce_op, PS_DOUBLE,
-      s0.__reduce_out ? (!__fuse ? __PSBlocks_settle_square(s0) : s0.g->num_elms <= physis_hip::kTileMaxPoints ? __PSBlocksT_settle_square(s0) : __PSBlocks2_settle_square(s0)) : 0, iter, __slots);
+      s0.__reduce_out ? (!__fuse ? __PSBlocks_settle_square(s0) : physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? __PSBlocksT_settle_square(s0) : __PSBlocks2_settle_square(s0)) : 0, iter, __slots);
   physis_hip::MapReducer red1(s1.__reduce_out, s1.__reduce_op, PS_DOUBLE,
-      s1.__reduce_out ? (!__fuse ? __PSBlocks_settle_square(s1) : s1.g->num_elms <= physis_hip::kTileMaxPoints ? __PSBlocksT_settle_square(s1) : __PSBlocks2_settle_square(s1)) : 0, iter, __slots);
+      s1.__reduce_out ? (!__fuse ? __PSBlocks_settle_square(s1) : physis_hip::TilesBeatDomainPairs(s1.dom, s1.g->num_elms) ? __PSBlocksT_settle_square(s1) : __PSBlocks2_settle_square(s1)) : 0, iter, __slots);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g, PS_FLOAT);
@@ -3398,7 +3398,7 @@ static void __PSStencilRun_6(int iter, struct __PSStencil_settle_square s0, stru
     const size_t bytes = (size_t)s0.g->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
@@ -3458,7 +3458,7 @@ static void __PSStencilRun_7(int iter, struct __PSStencil_inner s0, struct __PSS
     const size_t bytes = (size_t)s0.g->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);

@@ -3371,7 +3371,7 @@ static void __PSStencilRun_7(int iter, struct __PSStencil_k7 s0, struct __PSSten
     const size_t bytes = (size_t)s0.g->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = s0.g->num_elms <= physis_hip::kTileMaxPoints;
+    const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
     const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);

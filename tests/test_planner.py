@@ -21,7 +21,8 @@ def planner(tmp_path_factory):
     if not os.path.exists(HIPCC):
         pytest.skip("hipcc not available")
     out = str(tmp_path_factory.mktemp("planner") / "planner_check")
-    subprocess.run([HIPCC, "-std=c++17", "-O1", f"-I{ROOT}/include",
+    subprocess.run([HIPCC, "-x", "hip", "--offload-arch=gfx950", "-std=c++17",
+                    "-O1", f"-I{ROOT}/include",
                     os.path.join(ROOT, "tests", "planner_check.cc"), "-o",
                     out], check=True, capture_output=True)
     return out
@@ -57,3 +58,19 @@ def test_plane_beyond_reach_is_rejected(planner):
                         "256"], capture_output=True, text=True)
     assert r.returncode != 0
     assert "2 GiB reach of a buffer window" in r.stderr
+
+
+# Pairs over a domain, by the side measured faster (include/physis/hip/tile.h):
+# the domain counts and not its grid, and rows that fill the 256-point tiles of
+# a z-marching pass as much as the number of points.
+@pytest.mark.parametrize("box,points,tiles", [
+    ((1, 63) * 3, 64 ** 3, True), ((1, 255, 1, 59, 1, 59), 921600, True),
+    ((1, 23, 1, 299, 1, 299), 2160000, True),
+    ((40, 72) * 3, 512 ** 3, True), ((40, 72) * 3, 512 ** 3 + 1, False),
+    ((1, 255, 1, 91, 1, 91), 2166784, False),
+    ((1, 1023, 1, 45, 1, 45), 2166784, False),
+    ((1, 255) * 3, 256 ** 3, False), ((1, 511) * 3, 512 ** 3, False)])
+def test_tiles_for_pairs_over_a_domain(planner, box, points, tiles):
+    r = subprocess.run([planner, "tiles", *map(str, box), str(points)],
+                       check=True, capture_output=True, text=True)
+    assert int(r.stdout) == tiles
