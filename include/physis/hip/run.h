@@ -68,13 +68,18 @@ inline int BlocksPerCU(const void *kernel, int threads) {
 // reach; a grid of which not even one such window fits is rejected (the
 // reference's 32-bit PSIndex, include/physis/physis_common.h:33-55, bounds
 // elements, not bytes).
-inline int WindowChunkLimit(const __PSGrid *g, int margin) {
+inline int64_t WindowPlanes(const __PSGrid *g, int margin) {
   if (!g) return INT32_MAX;
   int64_t plane = (int64_t)g->elm_size;
   for (int d = 0; d < g->num_dims && d < 2; ++d) plane *= g->dim[d];
   if (plane <= 0) return INT32_MAX;
-  const int64_t planes = (int64_t)INT32_MAX / plane - 2 * (int64_t)margin;
+  return (int64_t)INT32_MAX / plane - 2 * (int64_t)margin;
+}
+inline int WindowChunkLimit(const __PSGrid *g, int margin) {
+  const int64_t planes = WindowPlanes(g, margin);
   if (planes < 1) {
+    int64_t plane = (int64_t)g->elm_size;
+    for (int d = 0; d < g->num_dims && d < 2; ++d) plane *= g->dim[d];
     std::fprintf(stderr,
                  "[physis-hip] a %lld-byte plane (with %d halo planes per "
                  "side) exceeds the 2 GiB reach of a buffer window\n",
@@ -82,6 +87,19 @@ inline int WindowChunkLimit(const __PSGrid *g, int margin) {
     std::exit(EXIT_FAILURE);
   }
   return planes > INT32_MAX ? INT32_MAX : (int)planes;
+}
+// Whether a pass with `margin` planes (rows of a 2-D grid in the rows view) per
+// side has a window at all: passes of several sweeps reach further than single
+// sweeps, which serve the grids whose planes are too large for them.
+inline bool WindowsFit(std::initializer_list<const __PSGrid *> grids,
+                       int margin, bool rows = false) {
+  for (const __PSGrid *g : grids) {
+    if (!g) continue;
+    __PSGrid w = *g;
+    if (rows) w.num_dims = 1;
+    if (WindowPlanes(&w, margin) < 1) return false;
+  }
+  return true;
 }
 inline int WindowChunkLimit(std::initializer_list<const __PSGrid *> grids,
                             int margin) {

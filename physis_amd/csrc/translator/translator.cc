@@ -2511,7 +2511,7 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
       << "  for (int d = 0; d < 3; ++d)\n"
          "    if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||\n"
          "        s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;\n"
-      << "  return true;\n}\n\n";
+      << "  return physis_hip::WindowsFit({a}, 3);\n}\n\n";
     return o.str();
   }
   o << "// The pair (s0, s1) is " << n << "(a -> b), " << n
@@ -2532,7 +2532,7 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
   for (auto &a : sa)
     o << "  if (__builtin_memcmp(&s0." << a << ", &s1." << a << ", sizeof(s0." << a
       << "))) return false;\n";
-  o << "  return true;\n}\n\n";
+  o << "  return physis_hip::WindowsFit({a}, 3);\n}\n\n";
   return o.str();
 }
 
@@ -3118,6 +3118,8 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
     << " = " << kBY << ";\n";
   std::vector<std::string> wgrids = {"s." + I, "s." + O};
   for (auto *g : direct) wgrids.push_back("s." + g->name);
+  std::vector<std::string> wgrids0 = {"a", "b"};
+  for (auto *g : direct) wgrids0.push_back("s0." + g->name);
   o << "template <int VX, int BY>\nstatic physis_hip::RunShape __PSShape2_" << n
     << "(const struct __PSStencil_" << n << " &s) {\n"
     << "  static int per_cu = physis_hip::BlocksPerCU(\n"
@@ -3196,7 +3198,7 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
   if (red)
     o << "  if ((s0.__reduce_out == NULL) != (s1.__reduce_out == NULL) ||\n"
          "      (s0.__reduce_out && s0.__reduce_op != s1.__reduce_op)) return false;\n";
-  o << "  return true;\n}\n\n";
+  o << "  return physis_hip::WindowsFit({" << Join(wgrids0, ", ") << "}, 3);\n}\n\n";
   return o.str();
 }
 
@@ -3543,7 +3545,7 @@ std::string Translator::EmitRowsKernel(const KernelInfo &k) {
   for (auto &sc : k.scalars)
     o << "  if (__builtin_memcmp(&s0." << sc.name << ", &s1." << sc.name
       << ", sizeof(s0." << sc.name << "))) return false;\n";
-  o << "  return true;\n}\n\n";
+  o << "  return physis_hip::WindowsFit({a, b}, 5, true);\n}\n\n";
   return o.str();
 }
 

@@ -882,7 +882,7 @@ static bool __PSFusable2_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s
   if (__builtin_memcmp(&s0.omega, &s1.omega, sizeof(s0.omega))) return false;
   if ((s0.__reduce_out == NULL) != (s1.__reduce_out == NULL) ||
       (s0.__reduce_out && s0.__reduce_op != s1.__reduce_op)) return false;
-  return true;
+  return physis_hip::WindowsFit({a, b, s0.a0, s0.a1, s0.a2, s0.a3, s0.b0, s0.b1, s0.b2, s0.c0, s0.c1, s0.c2, s0.bnd, s0.wrk1}, 3);
 }
 
 static void __PSStencilRun_0(int iter, struct __PSStencil_jacobi_kernel s0, struct __PSStencil_jacobi_kernel s1) {

@@ -304,7 +304,7 @@ static bool __PSFusable2_s2d5(const struct __PSStencil_s2d5 &s0, const struct __
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
-  return true;
+  return physis_hip::WindowsFit({a, b}, 5, true);
 }
 
 // ---------------------------------------------- stencil s2d9
@@ -611,7 +611,7 @@ static bool __PSFusable2_s2d9(const struct __PSStencil_s2d9 &s0, const struct __
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
-  return true;
+  return physis_hip::WindowsFit({a, b}, 5, true);
 }
 
 static void __PSStencilRun_0(int iter, struct __PSStencil_s2d5 s0, struct __PSStencil_s2d5 s1) {

@@ -1,7 +1,7 @@
 // Host-only check of the run-kernel launch planner (include/physis/hip/run.h):
 // prints, for each case, the z chunk and window bytes that PlanRunFor picks;
 // "tiles": whether pairs over a domain run in resident tiles
-// (include/physis/hip/tile.h).  Built and run by tests/test_planner.py; no
+// (include/physis/hip/tile.h); "fits": whether a pass has a window at all.  Built and run by tests/test_planner.py; no
 // device is touched.
 #include <cstdio>
 #include <cstdlib>
@@ -55,6 +55,13 @@ int main(int argc, char **argv) {
       dom.local_max[d] = std::atoi(argv[3 + 2 * d]);
     }
     std::printf("%d\n", physis_hip::TilesBeatDomainPairs(dom, std::atol(argv[8])));
+    return 0;
+  }
+  if (argc == 8 && std::strcmp(argv[1], "fits") == 0) {
+    __PSGrid g = MakeGrid(std::atoi(argv[2]), std::atoi(argv[3]),
+                          std::atoi(argv[4]), std::atoi(argv[5]));
+    std::printf("%d\n", physis_hip::WindowsFit({&g}, std::atoi(argv[6]),
+                                               std::atoi(argv[7]) != 0));
     return 0;
   }
   if (argc > 1) {

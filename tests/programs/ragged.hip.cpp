@@ -424,7 +424,7 @@ static bool __PSFusable2_corners(const struct __PSStencil_corners &s0, const str
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
-  return true;
+  return physis_hip::WindowsFit({a, b}, 3);
 }
 
 // Resident-tile pass of corners: TILE::T sweeps of src per launch into dst,
@@ -994,7 +994,7 @@ static bool __PSFusable2_corners2d(const struct __PSStencil_corners2d &s0, const
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
-  return true;
+  return physis_hip::WindowsFit({a, b}, 5, true);
 }
 
 // ---------------------------------------------- stencil wrap2
@@ -1576,7 +1576,7 @@ static bool __PSFusable2_inner(const struct __PSStencil_inner &s0, const struct 
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
-  return true;
+  return physis_hip::WindowsFit({a, b}, 3);
 }
 
 // Resident-tile pass of inner: TILE::T sweeps of src per launch into dst,
@@ -2160,7 +2160,7 @@ static bool __PSFusable2_settle(const struct __PSStencil_settle &s0, const struc
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
   if ((s0.__reduce_out == NULL) != (s1.__reduce_out == NULL) ||
       (s0.__reduce_out && s0.__reduce_op != s1.__reduce_op)) return false;
-  return true;
+  return physis_hip::WindowsFit({a, b, s0.c}, 3);
 }
 
 // Resident-tile pass of settle: TILE::T sweeps of src per launch into dst,
@@ -2750,7 +2750,7 @@ static bool __PSFusable2_settle_square(const struct __PSStencil_settle_square &s
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
   if ((s0.__reduce_out == NULL) != (s1.__reduce_out == NULL) ||
       (s0.__reduce_out && s0.__reduce_op != s1.__reduce_op)) return false;
-  return true;
+  return physis_hip::WindowsFit({a, b}, 3);
 }
 
 // Resident-tile pass of settle_square: TILE::T sweeps of src per launch into dst,
@@ -3176,7 +3176,7 @@ static bool __PSFusable2_inner2d(const struct __PSStencil_inner2d &s0, const str
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
-  return true;
+  return physis_hip::WindowsFit({a, b}, 5, true);
 }
 
 extern "C" {

@@ -419,7 +419,7 @@ static bool __PSFusable2_k7(const struct __PSStencil_k7 &s0, const struct __PSSt
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
-  return true;
+  return physis_hip::WindowsFit({a, b}, 3);
 }
 
 // Resident-tile pass of k7: TILE::T sweeps of src per launch into dst,
@@ -883,7 +883,7 @@ static bool __PSFusable2_k7p(const struct __PSStencil_k7p &s0, const struct __PS
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  return true;
+  return physis_hip::WindowsFit({a}, 3);
 }
 
 // Resident-tile pass of k7p: TILE::T sweeps of src per launch into dst,
@@ -1385,7 +1385,7 @@ static bool __PSFusable2_k7n(const struct __PSStencil_k7n &s0, const struct __PS
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  return true;
+  return physis_hip::WindowsFit({a}, 3);
 }
 
 // Resident-tile pass of k7n: TILE::T sweeps of src per launch into dst,
@@ -2315,7 +2315,7 @@ static bool __PSFusable2_k27(const struct __PSStencil_k27 &s0, const struct __PS
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
-  return true;
+  return physis_hip::WindowsFit({a, b}, 3);
 }
 
 // Resident-tile pass of k27: TILE::T sweeps of src per launch into dst,
@@ -2902,7 +2902,7 @@ static bool __PSFusable2_k27p(const struct __PSStencil_k27p &s0, const struct __
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  return true;
+  return physis_hip::WindowsFit({a}, 3);
 }
 
 // Resident-tile pass of k27p: TILE::T sweeps of src per launch into dst,
@@ -3883,7 +3883,7 @@ static bool __PSFusableRB_krb(const struct __PSStencil_krb &s0) {
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
-  return true;
+  return physis_hip::WindowsFit({a}, 3);
 }
 
 // Resident-tile pass of krb: TILE::T sweeps of src per launch into dst,
@@ -4634,7 +4634,7 @@ static bool __PSFusable2_k5(const struct __PSStencil_k5 &s0, const struct __PSSt
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
-  return true;
+  return physis_hip::WindowsFit({a, b}, 5, true);
 }
 
 static void __PSStencilRun_13(int iter, struct __PSStencil_k3 s0) {

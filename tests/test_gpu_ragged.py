@@ -191,3 +191,29 @@ def test_pairs_over_a_box(ps, prog, shape, box):
             assert np.array_equal(ps.PSGridCopyout(x), want.reshape(-1)), count
     ps.PSGridFree(g)
     ps.PSGridFree(g2)
+
+
+def test_rows_too_long_for_passes(ps, prog):
+    """Rows whose windows fit single sweeps but not a rows pass: the pair runs
+    as single sweeps."""
+    nx, x0, x1, w = 60_000_000, 29_999_900, 30_000_100, np.float32(0.2)
+    print(f"pairs over rows of {nx}", flush=True)
+    n = x1 - x0 + 2
+    a = np.zeros((3, nx), np.float32)
+    a[:, x0 - 1:x1 + 1] = np.random.default_rng(1).standard_normal((3, n))
+    g, g2 = ps.PSGridNew((nx, 3)), ps.PSGridNew((nx, 3))
+    ps.PSGridCopyin(g, a)
+    ps.PSGridCopyin(g2, a)
+    prog.ragged_box2d(g.handle, g2.handle, x0, x1, 1, 2, 3, w)
+    got = [ps.PSGridCopyout(x).reshape(3, nx) for x in (g, g2)]
+    ps.PSGridFree(g)
+    ps.PSGridFree(g2)
+    u = [a[:, x0 - 1:x1 + 1].copy() for _ in range(2)]
+    for k in range(6):
+        s = u[k % 2]
+        v = s[1, 1:-1] + s[0, 2:] + s[2, :-2] + s[1, :-2] + s[2, 2:]
+        u[1 - k % 2][1, 1:-1] = v * w
+    for k in range(2):
+        assert np.array_equal(got[k][:, x0 - 1:x1 + 1], u[k]), k
+        a[:, x0 - 1:x1 + 1] = got[k][:, x0 - 1:x1 + 1]
+        assert np.array_equal(got[k], a)

@@ -74,3 +74,18 @@ def test_tiles_for_pairs_over_a_domain(planner, box, points, tiles):
     r = subprocess.run([planner, "tiles", *map(str, box), str(points)],
                        check=True, capture_output=True, text=True)
     assert int(r.stdout) == tiles
+
+
+# Passes of several sweeps reach further than single sweeps: where their
+# windows do not fit, the run takes single sweeps (it must not be refused).
+@pytest.mark.parametrize("grid,elm,margin,rows,fits", [
+    ((512, 512, 512), 4, 3, 0, True), ((8755, 8755, 8), 4, 3, 0, True),
+    ((9001, 9001, 8), 4, 3, 0, False), ((9001, 9001, 8), 4, 2, 0, True),
+    ((6500, 6500, 8), 8, 3, 0, False), ((48000000, 3, 1), 4, 5, 1, True),
+    ((49000000, 3, 1), 4, 5, 1, False), ((60000000, 3, 1), 4, 2, 1, True)])
+def test_passes_of_several_sweeps_within_reach(planner, grid, elm, margin,
+                                               rows, fits):
+    r = subprocess.run([planner, "fits", *map(str, grid), str(elm),
+                        str(margin), str(rows)], check=True,
+                       capture_output=True, text=True)
+    assert int(r.stdout) == fits
