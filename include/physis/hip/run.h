@@ -454,6 +454,14 @@ class RunTimer {
   hipEvent_t start_ = nullptr, stop_ = nullptr;
 };
 
+// Whether the device holds the scratch grids (slot 8, and 9 when `second`) of
+// passes of several sweeps.  Where it does not, a run takes single sweeps,
+// which need none.
+inline bool HaveScratch(size_t bytes, bool second) {
+  return __PSHipTryScratch(8, bytes) &&
+         (!second || __PSHipTryScratch(9, bytes));
+}
+
 // Scratch slots of the reducing maps of one run function: runtime scratch
 // areas 1..7 (__PSHipScratch), one per map that reduces, in map order, so
 // no two maps of a run share partials.

@@ -171,6 +171,8 @@ extern int __PSHipNumCUs(void);
  * two-sweep (temporally blocked) runs in slots 8 and 9; slot 0 is
  * PSReduce's own. */
 extern void *__PSHipScratch(int slot, size_t bytes);
+/* The same, or NULL when the device memory is out. */
+extern void *__PSHipTryScratch(int slot, size_t bytes);
 /* Folds the per-block partial results of a PSStencilMapReduce map: row r of
  * the device array partials (count rows of nparts elements of `type`) is
  * reduced with op into host_out[r]; float sums accumulate in double.

@@ -39,7 +39,7 @@ void EnsureInit() {
   r.initialized = true;
 }
 
-void *Scratch(int slot, size_t bytes) {
+void *TryScratch(int slot, size_t bytes) {
   Runtime &r = rt();
   EnsureInit();
   if (slot < 0 || slot >= Runtime::kScratchSlots)
@@ -48,12 +48,26 @@ void *Scratch(int slot, size_t bytes) {
     if (r.scratch[slot]) {
       PS_HIP_CHECK(hipStreamSynchronize(r.stream));
       PS_HIP_CHECK(hipFree(r.scratch[slot]));
+      r.scratch[slot] = nullptr;
+      r.scratch_bytes[slot] = 0;
     }
     size_t cap = bytes < (1u << 20) ? (1u << 20) : bytes;
-    PS_HIP_CHECK(hipMalloc(&r.scratch[slot], cap));
+    const hipError_t e = hipMalloc(&r.scratch[slot], cap);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      r.scratch[slot] = nullptr;
+      return nullptr;
+    }
+    PS_HIP_CHECK(e);
     r.scratch_bytes[slot] = cap;
   }
   return r.scratch[slot];
+}
+
+void *Scratch(int slot, size_t bytes) {
+  void *p = TryScratch(slot, bytes);
+  if (!p) PS_FATAL("out of device memory: %zu bytes of scratch", bytes);
+  return p;
 }
 
 void *HostResultSlot() {
@@ -412,6 +426,9 @@ int __PSHipNumCUs(void) {
 }
 
 void *__PSHipScratch(int slot, size_t bytes) { return Scratch(slot, bytes); }
+void *__PSHipTryScratch(int slot, size_t bytes) {
+  return TryScratch(slot, bytes);
+}
 
 void *__PSHipPinned(int slot, size_t bytes) { return Pinned(slot, bytes); }
 

@@ -51,6 +51,7 @@ Runtime &rt();
 // test programs do) still work.
 void EnsureInit();
 void *Scratch(int slot, size_t bytes);
+void *TryScratch(int slot, size_t bytes);  // NULL when out of device memory
 void *HostResultSlot();
 void *Pinned(int slot, size_t bytes);
 

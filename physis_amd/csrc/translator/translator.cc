@@ -2511,7 +2511,9 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
       << "  for (int d = 0; d < 3; ++d)\n"
          "    if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||\n"
          "        s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;\n"
-      << "  return physis_hip::WindowsFit({a}, 3);\n}\n\n";
+      << "  return physis_hip::WindowsFit({a}, 3) &&\n"
+         "         physis_hip::HaveScratch((size_t)a->num_elms * sizeof(" << T
+      << "), false);\n}\n\n";
     return o.str();
   }
   o << "// The pair (s0, s1) is " << n << "(a -> b), " << n
@@ -2763,6 +2765,19 @@ std::string Translator::EmitKernel(KernelInfo &k) {
   return s;
 }
 
+std::string Translator::SmallExpr(const KernelInfo &k) {
+  const GridParam &g = k.grids[k.fuse_in];
+  return k.fuse_domain ? "physis_hip::TilesBeatDomainPairs(s0.dom, s0." + g.name +
+                             "->num_elms)"
+                       : "physis_hip::TilesBeatPairs(s0." + g.name + "->dim, " +
+                             (g.periodic ? "true" : "false") + ")";
+}
+std::string Translator::PassesExpr(const KernelInfo &k) {
+  if (!k.rows2d && !UsesTiles(k)) return "iter";
+  return (k.rows2d ? "" : "!" + SmallExpr(k) + " ? iter : ") +
+         std::string("iter == 2 ? 2 : (iter + 1) / 2");
+}
+
 // The run-function branch of a fusable pair (s0, s1) = k(a -> b), k(b -> a):
 // every pair of the run is one two-sweep pass when __fuse holds.
 std::string Translator::EmitFusedRun(const KernelInfo &k) {
@@ -2785,15 +2800,8 @@ std::string Translator::EmitFusedRun(const KernelInfo &k) {
   const std::string &n = k.name;
   const bool red = k.ret_type != "void";
   const bool tiles = UsesTiles(k);
-  if (tiles)
-    o << "    const bool __small = "
-      << (k.fuse_domain
-              ? "physis_hip::TilesBeatDomainPairs(s0.dom, s0." + gi.name + "->num_elms)"
-              : "physis_hip::TilesBeatPairs(s0." + gi.name + "->dim, " +
-                    (gi.periodic ? "true" : "false") + ")")
-      << ";\n    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);\n";
-  else
-    o << "    const int passes = iter;\n";
+  if (tiles) o << "    const bool __small = " << SmallExpr(k) << ";\n";
+  o << "    const int passes = " << PassesExpr(k) << ";\n";
   // one pass, pairs i and on (j: pass)
   auto launch = [&](const std::string &src, const std::string &dst,
                     const std::string &last) {
@@ -3562,7 +3570,7 @@ std::string Translator::EmitFusedRowsRun(const KernelInfo &k) {
     << "    const " << V << " va = physis_hip::RowView<" << V << ">(s0." << gi.name << ");\n"
     << "    float *const b = physis_hip::RowView<" << V << ">(s0." << go.name << ").p;\n"
     << "    const size_t bytes = (size_t)s0." << gi.name << "->num_elms * sizeof(float);\n"
-    << "    const int passes = iter == 2 ? 2 : (iter + 1) / 2;\n"
+    << "    const int passes = " << PassesExpr(k) << ";\n"
     << "    " << V << " vt = va, vt2 = va;\n"
     << "    vt.p = (float *)__PSHipScratch(8, bytes);\n"
     << "    const __PSDomain d = physis_hip::RowDomain(s0.dom);\n"
@@ -3602,9 +3610,15 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
   const bool fused_pair = r.kernels.size() == 2 &&
                           r.kernels[0] == r.kernels[1] &&
                           kernels_.at(r.kernels[0]).fusable;
-  if (fused_pair)
-    o << "  const bool __fuse = iter >= 2 && __PSFusable2_" << r.kernels[0]
-      << "(s0, s1);\n";
+  if (fused_pair) {
+    const KernelInfo &k = kernels_.at(r.kernels[0]);
+    const GridParam &g = k.grids[k.fuse_in];
+    // (passes over a domain take a second scratch grid when their count is odd)
+    o << "  const bool __fuse = iter >= 2 && __PSFusable2_" << k.name
+      << "(s0, s1) &&\n      physis_hip::HaveScratch((size_t)s0." << g.name
+      << "->num_elms * sizeof(" << g.elem << "), "
+      << (k.fuse_domain ? "(" + PassesExpr(k) + ") % 2 != 0" : "false") << ");\n";
+  }
   for (size_t i = 0; i < r.kernels.size(); ++i) {
     const KernelInfo &k = kernels_.at(r.kernels[i]);
     std::string si = "s" + std::to_string(i);
@@ -3642,8 +3656,7 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
       << "    " << V << " vt = va;\n"
       << "    vt.p = (" << T << " *)__PSHipScratch(8, bytes);\n"
       << "    " << V << " src = va;\n"
-      << "    const bool __small = physis_hip::TilesBeatPairs(s0." << g.name
-      << "->dim, " << (g.periodic ? "true" : "false") << ");\n"
+      << "    const bool __small = " << SmallExpr(k) << ";\n"
       << "    // two iterations a resident-tile pass, an even number of times, so that\n"
          "    // the count of passes is odd when iter is\n"
       << "    const int two = __small ? iter / 2 & ~1 : 0;\n"

@@ -161,6 +161,9 @@ class Translator {
   static bool UsesTiles(const KernelInfo &k);
   // the run-function branch that runs a fusable pair as two-sweep passes
   std::string EmitFusedRun(const KernelInfo &k);
+  // of the pair s0, s1: whether it runs in small-grid passes, and its passes
+  static std::string SmallExpr(const KernelInfo &k);
+  static std::string PassesExpr(const KernelInfo &k);
   // Interior split of a wave step at rows y, plane z: the wave-uniform
   // condition and the facts assumed under it ("" when the body compares
   // neither y nor z).

@@ -993,7 +993,8 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_diffusion7_kernel s0, 
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("diffusion7_kernel, diffusion7_kernel");
   physis_hip::RunTimer timer(stream);
-  const bool __fuse = iter >= 2 && __PSFusable2_diffusion7_kernel(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_diffusion7_kernel(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g1->num_elms * sizeof(float), false);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g1, PS_FLOAT);
@@ -1004,7 +1005,7 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_diffusion7_kernel s0, 
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim, false);
-    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
+    const int passes = !physis_hip::TilesBeatPairs(s0.g1->dim, false) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {
       const __PSGrid3DFloat_dev dst = passes % 2 && j == 0 ? vb
@@ -1040,7 +1041,8 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_diffusion7_periodic_ke
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("diffusion7_periodic_kernel, diffusion7_periodic_kernel");
   physis_hip::RunTimer timer(stream);
-  const bool __fuse = iter >= 2 && __PSFusable2_diffusion7_periodic_kernel(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_diffusion7_periodic_kernel(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g1->num_elms * sizeof(float), false);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g1, PS_FLOAT);
@@ -1051,7 +1053,7 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_diffusion7_periodic_ke
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim, true);
-    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
+    const int passes = !physis_hip::TilesBeatPairs(s0.g1->dim, true) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {
       const __PSGrid3DFloat_dev dst = passes % 2 && j == 0 ? vb

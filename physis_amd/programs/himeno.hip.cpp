@@ -890,7 +890,8 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_jacobi_kernel s0, stru
   __PSTraceStencilPre("jacobi_kernel, jacobi_kernel");
   physis_hip::RunTimer timer(stream);
   physis_hip::ReduceSlots __slots;
-  const bool __fuse = iter >= 2 && __PSFusable2_jacobi_kernel(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_jacobi_kernel(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.p0->num_elms * sizeof(float), (iter) % 2 != 0);
   physis_hip::MapReducer red0(s0.__reduce_out, s0.__reduce_op, PS_FLOAT,
       s0.__reduce_out ? (!__fuse ? __PSBlocks_jacobi_kernel(s0) : __PSBlocks2_jacobi_kernel(s0)) : 0, iter, __slots);
   physis_hip::MapReducer red1(s1.__reduce_out, s1.__reduce_op, PS_FLOAT,
@@ -949,7 +950,8 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_jacobi_kernel s0, stru
   __PSTraceStencilPre("jacobi_kernel, jacobi_kernel");
   physis_hip::RunTimer timer(stream);
   physis_hip::ReduceSlots __slots;
-  const bool __fuse = iter >= 2 && __PSFusable2_jacobi_kernel(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_jacobi_kernel(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.p0->num_elms * sizeof(float), (iter) % 2 != 0);
   physis_hip::MapReducer red0(s0.__reduce_out, s0.__reduce_op, PS_FLOAT,
       s0.__reduce_out ? (!__fuse ? __PSBlocks_jacobi_kernel(s0) : __PSBlocks2_jacobi_kernel(s0)) : 0, iter, __slots);
   physis_hip::MapReducer red1(s1.__reduce_out, s1.__reduce_op, PS_FLOAT,

@@ -618,7 +618,8 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_s2d5 s0, struct __PSSt
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("s2d5, s2d5");
   physis_hip::RunTimer timer(stream);
-  const bool __fuse = iter >= 2 && __PSFusable2_s2d5(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_s2d5(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g->num_elms * sizeof(float), (iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g, PS_FLOAT);
@@ -658,7 +659,8 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_s2d9 s0, struct __PSSt
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("s2d9, s2d9");
   physis_hip::RunTimer timer(stream);
-  const bool __fuse = iter >= 2 && __PSFusable2_s2d9(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_s2d9(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g->num_elms * sizeof(float), (iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g, PS_FLOAT);

@@ -3265,7 +3265,8 @@ static void __PSStencilRun_4(int iter, struct __PSStencil_inner s0, struct __PSS
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("inner, inner");
   physis_hip::RunTimer timer(stream);
-  const bool __fuse = iter >= 2 && __PSFusable2_inner(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_inner(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g->num_elms * sizeof(float), (!physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g, PS_FLOAT);
@@ -3276,7 +3277,7 @@ static void __PSStencilRun_4(int iter, struct __PSStencil_inner s0, struct __PSS
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
-    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
+    const int passes = !physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
@@ -3319,7 +3320,8 @@ static void __PSStencilRun_5(int iter, struct __PSStencil_settle s0, struct __PS
   __PSTraceStencilPre("settle, settle");
   physis_hip::RunTimer timer(stream);
   physis_hip::ReduceSlots __slots;
-  const bool __fuse = iter >= 2 && __PSFusable2_settle(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_settle(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g->num_elms * sizeof(float), (!physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0);
   physis_hip::MapReducer red0(s0.__reduce_out, s0.__reduce_op, PS_FLOAT,
       s0.__reduce_out ? (!__fuse ? __PSBlocks_settle(s0) : physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? __PSBlocksT_settle(s0) : __PSBlocks2_settle(s0)) : 0, iter, __slots);
   physis_hip::MapReducer red1(s1.__reduce_out, s1.__reduce_op, PS_FLOAT,
@@ -3334,7 +3336,7 @@ static void __PSStencilRun_5(int iter, struct __PSStencil_settle s0, struct __PS
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
-    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
+    const int passes = !physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
@@ -3384,7 +3386,8 @@ static void __PSStencilRun_6(int iter, struct __PSStencil_settle_square s0, stru
   __PSTraceStencilPre("settle_square, settle_square");
   physis_hip::RunTimer timer(stream);
   physis_hip::ReduceSlots __slots;
-  const bool __fuse = iter >= 2 && __PSFusable2_settle_square(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_settle_square(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g->num_elms * sizeof(float), (!physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0);
   physis_hip::MapReducer red0(s0.__reduce_out, s0.__reduce_op, PS_DOUBLE,
       s0.__reduce_out ? (!__fuse ? __PSBlocks_settle_square(s0) : physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? __PSBlocksT_settle_square(s0) : __PSBlocks2_settle_square(s0)) : 0, iter, __slots);
   physis_hip::MapReducer red1(s1.__reduce_out, s1.__reduce_op, PS_DOUBLE,
@@ -3399,7 +3402,7 @@ static void __PSStencilRun_6(int iter, struct __PSStencil_settle_square s0, stru
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
-    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
+    const int passes = !physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
@@ -3448,7 +3451,8 @@ static void __PSStencilRun_7(int iter, struct __PSStencil_inner s0, struct __PSS
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("inner, inner");
   physis_hip::RunTimer timer(stream);
-  const bool __fuse = iter >= 2 && __PSFusable2_inner(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_inner(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g->num_elms * sizeof(float), (!physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g, PS_FLOAT);
@@ -3459,7 +3463,7 @@ static void __PSStencilRun_7(int iter, struct __PSStencil_inner s0, struct __PSS
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
-    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
+    const int passes = !physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
@@ -3501,7 +3505,8 @@ static void __PSStencilRun_8(int iter, struct __PSStencil_inner2d s0, struct __P
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("inner2d, inner2d");
   physis_hip::RunTimer timer(stream);
-  const bool __fuse = iter >= 2 && __PSFusable2_inner2d(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_inner2d(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g->num_elms * sizeof(float), (iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g, PS_FLOAT);

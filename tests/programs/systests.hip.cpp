@@ -3361,7 +3361,8 @@ static void __PSStencilRun_7(int iter, struct __PSStencil_k7 s0, struct __PSSten
   hipStream_t stream = (hipStream_t)__PSHipStream();
   __PSTraceStencilPre("k7, k7");
   physis_hip::RunTimer timer(stream);
-  const bool __fuse = iter >= 2 && __PSFusable2_k7(s0, s1);
+  const bool __fuse = iter >= 2 && __PSFusable2_k7(s0, s1) &&
+      physis_hip::HaveScratch((size_t)s0.g->num_elms * sizeof(float), (!physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0);
   int i0 = 0;
   if (__fuse) {
     physis_hip::CheckGrid3D(s0.g, PS_FLOAT);
@@ -3372,7 +3373,7 @@ static void __PSStencilRun_7(int iter, struct __PSStencil_k7 s0, struct __PSSten
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     const bool __small = physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms);
-    const int passes = !__small ? iter : (iter == 2 ? 2 : (iter + 1) / 2);
+    const int passes = !physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev vt2 = va;
     physis_hip::CopyShell(vt.p, va.p, va.dim[0], va.dim[1], va.dim[2], s0.dom, stream);
     if (passes % 2) {
@@ -3883,7 +3884,8 @@ static bool __PSFusableRB_krb(const struct __PSStencil_krb &s0) {
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
-  return physis_hip::WindowsFit({a}, 3);
+  return physis_hip::WindowsFit({a}, 3) &&
+         physis_hip::HaveScratch((size_t)a->num_elms * sizeof(float), false);
 }
 
 // Resident-tile pass of krb: TILE::T sweeps of src per launch into dst,

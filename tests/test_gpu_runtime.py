@@ -54,3 +54,18 @@ def test_oversized_allocation_returns_invalid_grid(ps):
         ps.PSGridNew((1 << 14, 1 << 13, 1 << 13))
     g = ps.PSGridNew((8, 8, 8))   # the runtime is still usable
     ps.PSGridFree(g)
+
+
+def test_scratch_that_does_not_fit(ps):
+    """A scratch area that the device cannot hold is NULL, not the end of the
+    program, and its slot is usable again afterwards."""
+    import ctypes as C
+    rt = ps.runtime()
+    rt.__PSHipTryScratch.argtypes = rt.__PSHipScratch.argtypes = [C.c_int,
+                                                                  C.c_size_t]
+    rt.__PSHipTryScratch.restype = rt.__PSHipScratch.restype = C.c_void_p
+    for slot in (8, 9):
+        assert rt.__PSHipTryScratch(slot, 1 << 20)
+        assert rt.__PSHipTryScratch(slot, 1 << 48) is None
+        p = rt.__PSHipTryScratch(slot, 1 << 20)
+        assert p and p == rt.__PSHipScratch(slot, 4096)

@@ -2,6 +2,7 @@
 translator produces, the stencil analysis finds the reference's offsets,
 and unsupported constructs are rejected with an error."""
 import os
+import re
 import subprocess
 import tempfile
 
@@ -12,7 +13,8 @@ PHYSISC = os.path.join(ROOT, "physis_amd", "bin", "physisc-hip")
 SOURCES = [os.path.join(ROOT, "physis_amd", "programs", f)
            for f in ("diffusion7.c", "himeno.c", "redblack7.c", "udt7.c",
                      "stencil2d.c", "mixed7.c")] + \
-          [os.path.join(ROOT, "tests", "programs", "systests.c")]
+          [os.path.join(ROOT, "tests", "programs", f)
+           for f in ("systests.c", "ragged.c")]
 
 
 def translate(src, text=None):
@@ -530,3 +532,26 @@ void run(PSGrid3DFloat a, PSGrid3DFloat b) {
     rc, code, err = translate(None, src)
     assert rc == 0, err
     assert "a  staged x[-1,1]" in code
+
+
+@pytest.mark.parametrize("program,second", [
+    ("diffusion7", "false"), ("redblack7", "false"),
+    ("himeno", "(iter) % 2 != 0"),
+    ("stencil2d", "(iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0"),
+    ("ragged", "(!physis_hip::TilesBeatDomainPairs(s0.dom, s0.g->num_elms) ? "
+               "iter : iter == 2 ? 2 : (iter + 1) / 2) % 2 != 0")])
+def test_passes_of_several_sweeps_need_their_scratch_grids(program, second):
+    """The passes are taken only where the device has room for the scratch
+    grids they ping-pong with (two for an odd count over a domain); single
+    sweeps, which need none, otherwise."""
+    src = [f for f in SOURCES if os.path.basename(f) == program + ".c"][0]
+    rc, code, err = translate(src)
+    assert rc == 0, err
+    asked = re.findall(r"const bool __fuse = (.*?);", code, re.S) + \
+        re.findall(r"return (physis_hip::WindowsFit\(\{a\}, 3\) &&.*?);", code,
+                   re.S)
+    asked = [re.sub(r"\s+", " ", c) for c in asked]
+    assert asked
+    for c in asked:
+        assert "&& physis_hip::HaveScratch((size_t)" in c, c
+    assert any("sizeof(float), " + second + ")" in c for c in asked), asked
