@@ -88,8 +88,11 @@ constexpr int KPad(int cin) { return ((27 * cin + 31) / 32) * 32; }
 // The GEMM is D[cout][16 x] = W[cout][32 k] X[32 k][16 x]: the weights are
 // the A operand (registers, or LDS when they are many), the staged input the
 // B operand (one aligned 16-byte LDS read per lane), and a lane's result is
-// four consecutive channels of one position, stored as one 8-byte word.
-template <int CIN, int COUT, bool RELU, int XT, int TY>
+// four consecutive channels of one position, stored as one 8-byte word.  GATE:
+// the results are gated by act > 0 (the ReLU whose input gradient they are); as
+// a run-time choice it cost 16 -> 48 at rows of 32 positions its registers (112
+// VGPRs -> 256 and 9 spilled).
+template <int CIN, int COUT, bool RELU, bool GATE, int XT, int TY>
 __global__ __launch_bounds__(64 * TY) void ConvZKernel(
     const u16 *__restrict__ x, const u16 *__restrict__ wt,
     const float *__restrict__ bias, const u16 *__restrict__ act,
@@ -264,7 +267,7 @@ __global__ __launch_bounds__(64 * TY) void ConvZKernel(
               }
               w2[h] = (unsigned)F2Bf(v0) | ((unsigned)F2Bf(v1) << 16);
             }
-            if (act) {  // gated by the ReLU whose input gradient this is
+            if constexpr (GATE) {
               const uint2 a = *reinterpret_cast<const uint2 *>(
                   act + (row + xo) * COUT + co);
               w2[0] = GateWord(w2[0], a.x);
@@ -1360,12 +1363,11 @@ void ConvZLaunch(const u16 *x, const u16 *wt, const float *b, bool relu,
   int tz, zchunk;
   ZChunks(tiles, N, D, kConvZBlocksPerCU, &tz, &zchunk);
   const dim3 grid(tiles, N * tz), block(64 * TY);
-  if (relu)
-    hipLaunchKernelGGL((ConvZKernel<CIN, COUT, true, XT, TY>), grid, block, 0,
-                       Stream(), x, wt, b, act, y, D, H, W, tz, zchunk);
-  else
-    hipLaunchKernelGGL((ConvZKernel<CIN, COUT, false, XT, TY>), grid, block,
-                       0, Stream(), x, wt, b, act, y, D, H, W, tz, zchunk);
+  const auto kernel = relu  ? ConvZKernel<CIN, COUT, true, false, XT, TY>
+                      : act ? ConvZKernel<CIN, COUT, false, true, XT, TY>
+                            : ConvZKernel<CIN, COUT, false, false, XT, TY>;
+  hipLaunchKernelGGL(kernel, grid, block, 0, Stream(), x, wt, b, act, y, D, H,
+                     W, tz, zchunk);
   Check();
 }
 
@@ -1526,6 +1528,8 @@ void SumParts(const float *part, long n, float *out, const float *part2,
 
 void Conv(int cin, int cout, const u16 *x, const u16 *wt, const float *b,
           bool relu, const u16 *act, u16 *y, int N, int D, int H, int W) {
+  if (act && (relu || b || cout == 24))
+    PS_FATAL("no gated convolution kernel with a bias, a ReLU or 24 channels");
 #define PS_CASE(I, O) \
   if (cin == I && cout == O) \
     return ConvT<I, O>(x, wt, b, relu, act, y, N, D, H, W);
