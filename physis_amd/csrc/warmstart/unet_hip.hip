@@ -292,37 +292,47 @@ __global__ __launch_bounds__(64 * TY) void ConvZKernel(
 // 16 bytes per thread and load; the tensor has the staged resolution, or
 // (UP) a quarter of it per axis, read once per fine position: an upsampled
 // tensor is never written out.  Positions outside the grid are zero: the
-// loads are range-checked buffer loads over one plane (none of it for a
-// plane outside the problem), whose offsets are computed once.
-constexpr int kOutside = (int)0x80000000u;
+// loads are range-checked buffer loads over the rows of one plane that the
+// block reads (none of a plane outside the problem), whose offsets are computed
+// once.  The rows and not the plane, so that only their bytes have to stay
+// below kReach (CheckRows on the host).
+constexpr unsigned kOutside = 0xfffffff0u, kReach = 0xfffffff0u;
+// `rows` rows of W positions of `channels` from row y of H on, in bytes.
+__device__ __forceinline__ unsigned RowBytes(int y, int rows, int H, int W,
+                                             int channels) {
+  return (unsigned)min(rows, H - y) * (unsigned)W * (unsigned)(channels * 2);
+}
 
 template <int CIN, int NCH, int COFF, bool UP, int RS, int XS, int NTH>
 struct PlaneStream {
   static constexpr int NV = NCH / 8, SV = RS * XS * NV;
   static constexpr int VPT = (SV + NTH - 1) / NTH;
-  int off[VPT];  // byte offset within a plane, kOutside outside the grid
+  static constexpr int Q = UP ? kPool : 1;
+  unsigned off[VPT];  // bytes from row yb, kOutside outside the grid
+  unsigned bytes;     // of the rows from yb on
+  int yb;
   uint4 buf[VPT];
 
   __device__ __forceinline__ void Init(int y0, int x0, int H, int W) {
+    yb = max(y0 - 1, 0) / Q;
+    bytes = RowBytes(yb, RS, H / Q, W / Q, NCH);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int v = threadIdx.x + i * NTH;
       const int c8 = v % NV, t = v / NV;
       const int yy = y0 - 1 + t / XS, xx = x0 - 1 + t % XS;
       const bool in = v < SV && yy >= 0 && yy < H && xx >= 0 && xx < W;
-      const int pos = UP ? (yy / kPool) * (W / kPool) + xx / kPool
-                         : yy * W + xx;
+      const unsigned pos = (yy / Q - yb) * (W / Q) + xx / Q;
       off[i] = in ? (pos * NCH + c8 * 8) * 2 : kOutside;
     }
   }
   __device__ __forceinline__ void Fetch(const u16 *p, int n, int z, int D,
                                         int H, int W) {
     const bool in = z >= 0 && z < D;
-    const int q = UP ? kPool : 1;
-    const int plane = (H / q) * (W / q) * NCH;
+    const long row = ((long)n * (D / Q) + z / Q) * (H / Q) + yb;
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<u16 *>(p) + (in ? ((long)n * (D / q) + z / q) * plane : 0),
-        0, in ? plane * 2 : 0, physis_hip::kBufDword3);
+        const_cast<u16 *>(p) + (in ? row * (W / Q) * NCH : 0), 0,
+        in ? bytes : 0, physis_hip::kBufDword3);
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
       buf[i] = __builtin_bit_cast(
@@ -383,7 +393,7 @@ template <int CIN, int RS, int XS, int NTH>
 struct InputSrc {
   static_assert(CIN == 2 || CIN == 4, "rhs and bnd");
   static constexpr int SV = RS * XS, VPT = (SV + NTH - 1) / NTH;
-  int off[VPT];
+  unsigned off[VPT];
   float r[VPT], m[VPT];
   __device__ __forceinline__ void Init(int y0, int x0, int H, int W) {
 #pragma unroll
@@ -833,21 +843,22 @@ __global__ __launch_bounds__(64 * NW) void WgradZKernel(
     in.Init(y0, x0, H, W);
     // output-gradient plane zz (zeros outside [zb, ze))
     uint4 bd[DVT];
-    int doff[DVT];
+    unsigned doff[DVT];  // from row y0
+    const unsigned dbytes = RowBytes(y0, ROWS, H, W, COUT);
 #pragma unroll
     for (int i = 0; i < DVT; ++i) {
       const int v = threadIdx.x + i * NTH, t = v / (COUT / 8);
       const int yy = y0 + t / XT, xx = x0 + t % XT;
       doff[i] = v < DV && yy < H && xx < W
-                    ? ((yy * W + xx) * COUT + v % (COUT / 8) * 8) * 2
+                    ? ((unsigned)(t / XT * W + xx) * COUT + v % (COUT / 8) * 8) * 2
                     : kOutside;
     }
     auto fetchd = [&](int zz) {
       const bool ok = zz >= zb && zz < ze;
-      const int plane = H * W * COUT;
+      const long row = ((long)n * D + zz) * H + y0;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<u16 *>(dz) + (ok ? ((long)n * D + zz) * plane : 0), 0,
-          ok ? plane * 2 : 0, physis_hip::kBufDword3);
+          const_cast<u16 *>(dz) + (ok ? row * W * COUT : 0), 0, ok ? dbytes : 0,
+          physis_hip::kBufDword3);
 #pragma unroll
       for (int i = 0; i < DVT; ++i)
         bd[i] = __builtin_bit_cast(
@@ -1356,6 +1367,14 @@ void ZChunks(long tiles, int N, int D, int per_cu, int *tz, int *zchunk) {
   *tz = (D + *zchunk - 1) / *zchunk;
 }
 
+// The rows of a plane that a block reads through one buffer descriptor.
+void CheckRows(int rows, int H, int W, int channels) {
+  const long bytes = (long)std::min(rows, H) * W * channels * 2;
+  if (bytes > (long)kReach)
+    PS_FATAL("convolution: %d rows of %d positions of %d channels exceed the "
+             "reach of a buffer descriptor", std::min(rows, H), W, channels);
+}
+
 template <int CIN, int COUT, int XT, int TY>
 void ConvZLaunch(const u16 *x, const u16 *wt, const float *b, bool relu,
                  const u16 *act, u16 *y, int N, int D, int H, int W) {
@@ -1384,6 +1403,7 @@ template <int CIN, int COUT, bool RELU, int XT, int TY,
 void ConvMLaunchXT(const SrcArgs &src, const u16 *wt, const EpiArgs &ep, int N,
                    int D, int H, int W) {
   static_assert(EPI != kEpiPredict || XT == 16 || XT % 32 == 0, "pairs");
+  CheckRows(2 * TY + 2, H, W, CIN);
   const long tiles = (long)((W + XT - 1) / XT) * ((H + 2 * TY - 1) / (2 * TY));
   int tz, zchunk;
   ZChunks(tiles, N, D, kConvMWavesPerCU / TY, &tz, &zchunk);
@@ -1494,6 +1514,7 @@ void WgradZLaunch(const SrcArgs &src, const u16 *dz, float *part, float *bpart,
     PS_FATAL("filter gradient: %ld partial blocks exceed the %ld allocated",
              nb, capacity);
   constexpr int R = WgradZRows(CIN), NW = kWgradZWaves;
+  CheckRows(R + 2, H, W, std::max(CIN, COUT));
   const dim3 grid((unsigned)nb), block(64 * NW);
   if (WgradZXT(CIN, W) == 64) {
     if constexpr (CIN <= 24)

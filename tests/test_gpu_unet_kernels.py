@@ -213,3 +213,40 @@ def test_network_is_its_layers(ps, shape, batch):
         if l == 9:
             dx = U.bf16_float(conv_backward_data_host(bits, w, *dims))
             dz = np.where(below > 0, dx.reshape(below.shape), np.float32(0))
+
+
+def test_planes_of_more_than_2_gib(ps):
+    """Positions outside a plane of more than 2 GiB are zeros like any others:
+    convolutions and filter gradients of ones count the taps inside."""
+    from physis_amd.warmstart import (conv_backward_filter_host,
+                                      conv_forward_host)
+    one = np.uint16(0x3f80)
+    h, w, cin, cout = 6800, 6700, 24, 8
+    print(f"forward {h} x {w} x {cin}", flush=True)
+    assert h * w * cin * 2 > 2 ** 31
+    y = conv_forward_host(np.full(h * w * cin, one),
+                          U.bf16_bits(np.full(cout * 27 * cin, 1 / 256)),
+                          np.zeros(cout, np.float32), True, 1, 1, h, w, cin,
+                          cout).reshape(h, w, cout)
+    rows = np.full(h, 3)
+    rows[[0, -1]] = 2
+    cols = np.full(w, 3)
+    cols[[0, -1]] = 2
+    want = U.bf16_bits(rows[:, None] * cols[None, :] * (cin / 256)) \
+        .reshape(h, w)
+    assert all(np.array_equal(y[:, :, c], want) for c in range(cout))
+    h, w, cin, cout = 4800, 4700, 16, 48
+    print(f"filter gradient {h} x {w} x {cout}", flush=True)
+    assert h * w * cout * 2 > 2 ** 31
+    dw, db = conv_backward_filter_host(np.full(h * w * cin, one),
+                                       np.full(h * w * cout, one),
+                                       1, 1, h, w, cin, cout)
+    k = np.array([h - 1, h, h - 1], np.float64)[:, None] * \
+        np.array([w - 1, w, w - 1])[None, :]
+    ref = np.zeros((3, 3, 3))
+    ref[1] = k  # one plane: no taps in z
+    dw = dw.reshape(cout, 27, cin)
+    # FP32 sums of whole numbers: exact below 2^24, then half a unit each for
+    # the last few additions
+    assert np.all(np.abs(dw - ref.reshape(1, 27, 1)) <= 1e-6 * h * w)
+    assert np.all(np.abs(db - h * w) <= 1e-6 * h * w)
