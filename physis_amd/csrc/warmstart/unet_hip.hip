@@ -464,7 +464,9 @@ struct EpiArgs {
 // output planes it reaches: the B operand of a K step (8 channels of one
 // staged position per lane: k = (3 ry + dx) CIN + ci over the four input rows
 // ry of the two output rows) is read from LDS once and feeds the three z
-// taps, whose sums live in registers and rotate.  A rows: with 8 output
+// taps, whose sums live in registers and rotate.  (An input that is not finite
+// makes NaN of the zero weights of the row beyond a tap's reach: a result then
+// depends on one row more than it should.)  A rows: with 8 output
 // channels, 8 h + co of output row y + h (zero where ry - h is no tap); with
 // 24, sets 0 and 1 hold channels 0 .. 15 of the two rows and set 2 channels
 // 16 .. 23 of both.  With 2 staged input channels the B operand's other six
@@ -485,8 +487,7 @@ template <int CIN, int COUT, bool RELU, int XT, int TY,
 __global__ __launch_bounds__(64 * TY, CIN == 2 ? 4 : 1) void ConvMKernel(
     SrcArgs src, const u16 *__restrict__ wt, EpiArgs ep, int D, int H, int W,
     int tz, int zchunk) {
-  static_assert(COUT == 8 || COUT == 24, "output channels");
-  static_assert(EPI == kEpiStore || (EPI == kEpiUpSkip) == (COUT == 24), "");
+  static_assert(COUT == (EPI == kEpiUpSkip ? 24 : 8), "output channels");
   constexpr int S = COUT == 8 ? 1 : 3;  // A operands per B operand
   constexpr int WC = CIN == 2 ? 8 : CIN;  // channels of the stored weights
   constexpr int KPW = KPad(WC);
@@ -541,13 +542,10 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 4 : 1) void ConvMKernel(
       }
     }
   }
-  // bias of the lane's four channels of the paired results, and of sets 0, 1
-  float bb[4], ba[S == 1 ? 1 : 4];
+  float bb[4];  // bias of the lane's four channels of the paired results
 #pragma unroll
-  for (int v = 0; v < 4; ++v) {
+  for (int v = 0; v < 4; ++v)
     bb[v] = ep.bias ? ep.bias[COUT - 8 + 4 * (g & 1) + v] : 0.0f;
-    if constexpr (S > 1) ba[v] = ep.bias ? ep.bias[4 * g + v] : 0.0f;
-  }
   float hw[4], hb = 0.0f;  // head weights of the lane's four channels
   if constexpr (EPI == kEpiPredict) {
 #pragma unroll
@@ -626,22 +624,6 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 4 : 1) void ConvMKernel(
         if constexpr (EPI == kEpiUpSkip) {
           if (done) csum[i] += acc[i][0][(j + 1) % 3] + acc[i][1][(j + 1) % 3];
         }
-        if constexpr (COUT == 24 && EPI == kEpiStore) {
-#pragma unroll
-          for (int s = 0; s < 2; ++s) {
-            if (done && yw + s < H && xo < W) {
-              f32x4 v = acc[i][s][(j + 1) % 3];
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                v[e] += ba[e];
-                if (RELU) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
-              }
-              *reinterpret_cast<uint2 *>(
-                  ep.y + ((((long)n * D + z) * H + yw + s) * W + xo) * 24 +
-                  4 * g) = make_uint2(Pack2(v[0], v[1]), Pack2(v[2], v[3]));
-            }
-          }
-        }
         f32x4 v = acc[i][S - 1][(j + 1) % 3];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -680,12 +662,7 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 4 : 1) void ConvMKernel(
                   (PT)(ep.scale * (q + hb)) * (PT)bv[i / 2];
           }
         } else if (in_row) {
-          if constexpr (COUT == 24 && EPI == kEpiStore)
-            *reinterpret_cast<uint2 *>(ep.y + (row + xo) * 24 + 16 +
-                                       4 * (g & 1)) = w2;
-          else
-            *reinterpret_cast<uint2 *>(ep.y + (row + xo) * 8 + 4 * (g & 1)) =
-                w2;
+          *reinterpret_cast<uint2 *>(ep.y + (row + xo) * 8 + 4 * (g & 1)) = w2;
         }
 #pragma unroll
         for (int s = 0; s < S; ++s)
@@ -1390,7 +1367,7 @@ void ConvZLaunch(const u16 *x, const u16 *wt, const float *b, bool relu,
   Check();
 }
 
-// The input-marching convolution (8 or 24 output channels).  Block shapes
+// The input-marching convolution.  Block shapes
 // (XT positions by 2 TY rows) measured at 8 x 128^3, us, of 64x8, 32x8, 64x16
 // and 32x16: plain 8 -> 8 115 / 102 / 131 / 109; gated 164 / 216 / 177 / 150;
 // prediction 202 / 228 / 201 / 143; network input (a whole prediction) 731 /
@@ -1431,31 +1408,26 @@ void ConvMLaunch(const SrcArgs &src, const u16 *wt, const EpiArgs &ep, int N,
                                                         W);
 }
 
-// A convolution of whole tensors; act: gate of the results, or NULL.  8 and
-// 24 output channels march the input planes (ConvMKernel); more keep the
-// ring of planes: x tile of 64 positions below 24 input channels, else 32,
-// 16 for rows of at most 16; 8 rows per block below 24 input channels, else
-// 4 (the ring of 4 staged planes then stays within LDS).
+// A convolution of whole tensors; act: gate of the results, or NULL.  8 output
+// channels march the input planes (ConvMKernel); more keep the ring of planes:
+// x tile of 64 positions below 24 input channels, else 32, 16 for rows of at
+// most 16; 8 rows per block below 24 input channels, else 4 (the ring of 4
+// staged planes then stays within LDS).
 template <int CIN, int COUT>
 void ConvT(const u16 *x, const u16 *wt, const float *b, bool relu,
            const u16 *act, u16 *y, int N, int D, int H, int W) {
-  if constexpr (COUT == 8 || COUT == 24) {
+  if constexpr (COUT == 8) {
     SrcArgs src{x, nullptr, 0};
     EpiArgs ep;
     ep.bias = b;
     ep.act = act;
     ep.y = y;
-    if constexpr (COUT == 8) {
-      if (act)
-        return ConvMLaunch<CIN, 8, false, PlainSrc, kEpiGate>(src, wt, ep, N,
-                                                              D, H, W);
-    }
-    if (relu)
-      ConvMLaunch<CIN, COUT, true, PlainSrc, kEpiStore>(src, wt, ep, N, D, H,
-                                                        W);
+    if (act)
+      ConvMLaunch<CIN, 8, false, PlainSrc, kEpiGate>(src, wt, ep, N, D, H, W);
+    else if (relu)
+      ConvMLaunch<CIN, 8, true, PlainSrc, kEpiStore>(src, wt, ep, N, D, H, W);
     else
-      ConvMLaunch<CIN, COUT, false, PlainSrc, kEpiStore>(src, wt, ep, N, D, H,
-                                                         W);
+      ConvMLaunch<CIN, 8, false, PlainSrc, kEpiStore>(src, wt, ep, N, D, H, W);
   } else {
     constexpr int TY = CIN < 24 ? 8 : 4;
     if constexpr (CIN < 24) {
@@ -1549,8 +1521,8 @@ void SumParts(const float *part, long n, float *out, const float *part2,
 
 void Conv(int cin, int cout, const u16 *x, const u16 *wt, const float *b,
           bool relu, const u16 *act, u16 *y, int N, int D, int H, int W) {
-  if (act && (relu || b || cout == 24))
-    PS_FATAL("no gated convolution kernel with a bias, a ReLU or 24 channels");
+  if (act && (relu || b))
+    PS_FATAL("no gated convolution kernel with a bias or a ReLU");
 #define PS_CASE(I, O) \
   if (cin == I && cout == O) \
     return ConvT<I, O>(x, wt, b, relu, act, y, N, D, H, W);

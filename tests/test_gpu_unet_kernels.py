@@ -250,3 +250,22 @@ def test_planes_of_more_than_2_gib(ps):
     # the last few additions
     assert np.all(np.abs(dw - ref.reshape(1, 27, 1)) <= 1e-6 * h * w)
     assert np.all(np.abs(db - h * w) <= 1e-6 * h * w)
+
+
+def test_infinite_input_reaches_its_taps_only(ps):
+    """8 -> 24 channels: results that no tap leads to stay finite."""
+    from physis_amd.warmstart import conv_forward_host
+    n, d, h, w, cin, cout = dims = (1, 5, 9, 40, 8, 24)
+    rng = np.random.default_rng(2)
+    x = rng.standard_normal((d, h, w, cin)).astype(np.float32)
+    wt = U.bf16_bits(rng.standard_normal(cout * 27 * cin))
+    for at in ((2, 4, 20), (2, 5, 31), (0, 0, 0), (4, 8, 39)):
+        print(f"infinite at {at}", flush=True)
+        xi = x.copy()
+        xi[at + (3,)] = np.inf
+        y = U.bf16_float(conv_forward_host(
+            U.bf16_bits(xi.reshape(-1)), wt, np.zeros(cout, np.float32), False,
+            *dims)).reshape(d, h, w, cout)
+        near = np.zeros((d, h, w), bool)
+        near[tuple(slice(max(c - 1, 0), c + 2) for c in at)] = True
+        assert np.all(np.isfinite(y).all(3) == ~near)
