@@ -1137,6 +1137,7 @@ void Translator::AnalyzeFusion(KernelInfo &k) {
     }
     if (gi < 0) return no("a red-black map reading no grid");
     const GridParam &g = k.grids[gi];
+    if (g.elem != "float") return no("not a float grid");
     bool centre = false;
     for (auto &o : g.offsets) centre = centre || (!o[0] && !o[1] && !o[2]);
     if (!centre) return no("a red-black map not reading its centre");

@@ -1,8 +1,9 @@
 /* Maps that read past the ends of rows whose extents are multiples of
  * nothing: non-periodic gets over the whole grid (an index past the end of a
  * row names the next row's points, one outside the grid 0), periodic gets
- * two points away, a map pair over the interior, and pairs over a box of the
- * grid whose kernels return the change of each point. */
+ * two points away, a map pair over the interior, pairs over a box of the
+ * grid whose kernels return the change of each point, and a red-black map of
+ * an 8-byte grid. */
 #include "physis/physis.h"
 
 static void corners(const int x, const int y, const int z, PSGrid3DFloat g,
@@ -81,6 +82,15 @@ static void inner2d(const int x, const int y, PSGrid2DFloat g,
   PSGridEmit(g2, v * w);
 }
 
+static void relax_double(const int x, const int y, const int z,
+                         PSGrid3DDouble g) {
+  double v = PSGridGet(g, x, y, z) + PSGridGet(g, x+1, y, z) +
+             PSGridGet(g, x-1, y, z) + PSGridGet(g, x, y+1, z) +
+             PSGridGet(g, x, y-1, z) + PSGridGet(g, x, y, z+1) +
+             PSGridGet(g, x, y, z-1);
+  PSGridEmit(g, v * 0.125);
+}
+
 static PSDomain3D whole(PSGrid3DFloat g) {
   return PSDomain3DNew(0, PSGridDim(g, 0), 0, PSGridDim(g, 1), 0,
                        PSGridDim(g, 2));
@@ -148,4 +158,10 @@ void ragged_box2d(PSGrid2DFloat g, PSGrid2DFloat g2, int x0, int x1, int y0,
   PSDomain2D d = PSDomain2DNew(x0, x1, y0, y1);
   PSStencilRun(PSStencilMap(inner2d, d, g, g2, w),
                PSStencilMap(inner2d, d, g2, g, w), count);
+}
+
+void ragged_relax_double(PSGrid3DDouble g, int count) {
+  PSDomain3D d = PSDomain3DNew(1, PSGridDim(g, 0) - 1, 1, PSGridDim(g, 1) - 1,
+                               1, PSGridDim(g, 2) - 1);
+  PSStencilRun(PSStencilMapRedBlack(relax_double, d, g), count);
 }

@@ -3179,6 +3179,197 @@ static bool __PSFusable2_inner2d(const struct __PSStencil_inner2d &s0, const str
   return physis_hip::WindowsFit({a, b}, 5, true);
 }
 
+// ---------------------------------------------- stencil relax_double
+struct __PSStencil_relax_double {
+  __PSDomain dom;
+  __PSGrid *g;
+  int __g_index;
+  int __rb;  // -1 all points, 0 red, 1 black, 2 red then black
+};
+
+static struct __PSStencil_relax_double __PSStencilMap_relax_double(
+    __PSDomain __dom, __PSGrid *g) {
+  struct __PSStencil_relax_double __s = {__dom, g, __PSGridGetID(g), -1};
+  return __s;
+}
+
+static struct __PSStencil_relax_double __PSStencilMapRed_relax_double(
+    __PSDomain __dom, __PSGrid *g) {
+  struct __PSStencil_relax_double __s = __PSStencilMap_relax_double(__dom, g);
+  __s.__rb = 0;
+  return __s;
+}
+
+static struct __PSStencil_relax_double __PSStencilMapBlack_relax_double(
+    __PSDomain __dom, __PSGrid *g) {
+  struct __PSStencil_relax_double __s = __PSStencilMap_relax_double(__dom, g);
+  __s.__rb = 1;
+  return __s;
+}
+
+static struct __PSStencil_relax_double __PSStencilMapRedBlack_relax_double(
+    __PSDomain __dom, __PSGrid *g) {
+  struct __PSStencil_relax_double __s = __PSStencilMap_relax_double(__dom, g);
+  __s.__rb = 2;
+  return __s;
+}
+
+// Stencil analysis of relax_double (2.5D run kernel):
+//   g  staged x[-1,1] y[-1,1] z[-1,1] non-periodic, emitted
+//     offsets 0:(0,0,0) 1:(1,0,0) 2:(-1,0,0) 3:(0,1,0) 4:(0,-1,0) 5:(0,0,1) 6:(0,0,-1)
+//   red-black: in-place colour sweep reads only the other colour
+//   two-sweep fusion of map pairs: no (not a float grid)
+struct __PSCtx_relax_double {
+  double g[7];
+  double g_v;
+  bool g_e;
+  const double *g_p;
+  int g_dim[3];
+};
+
+__device__ __forceinline__ void relax_double(
+    const int x, const int y, const int z, __PSCtx_relax_double &__ctx) {
+  double v = __ctx.g[0] + __ctx.g[1] + __ctx.g[2] + __ctx.g[3] + __ctx.g[4] + __ctx.g[5] + __ctx.g[6];
+  (__ctx.g_v = (v * 0.125), __ctx.g_e = true);
+}
+
+// Run kernel: VX points per lane, BY waves per block (the first and
+// last 1 load halo rows), staged planes PD steps ahead,
+// centre-only grids one step ahead.  RED: reduction operator of a
+// PSStencilMapReduce execution, or -1.
+// FORM: VX, plus kRagged for x extents that are not multiples of VX.
+template <int FORM, int BY, int RED>
+__global__ __launch_bounds__(64 * BY) void __PSStencilRun_relax_double(
+    __PSDomain dom, __PSGrid3DDouble_dev g, physis_hip::RunShape sh, float *__restrict__ __red, int __rb) {
+  constexpr int VX = physis_hip::FormVX(FORM);
+  constexpr bool RAGGED = physis_hip::FormRagged(FORM);
+  constexpr int PD = 2;
+  constexpr int HY = 1;
+  constexpr int TX = 64 * VX, TY = BY - 2 * HY;
+  typedef physis_hip::Stage<double, VX, BY, 1, HY, 4, false, double, RAGGED> S_g;
+  __shared__ __attribute__((aligned(16))) double g_lds[S_g::kLdsElems];
+  const int lane = threadIdx.x % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const physis_hip::TileCoord tc = physis_hip::TileOf(sh.tiles_x, sh.tiles_y);
+  const int x0 = (sh.x_first_tile + tc.bx) * TX;
+  const int y0 = dom.local_min[1] + tc.by * TY;
+  const int zb = dom.local_min[2] + tc.bz * sh.zchunk;
+  const int ze = min(zb + sh.zchunk, dom.local_max[2]);
+  if (zb < ze) {
+    const int yrow = y0 - HY + wave;
+    const bool computes = wave >= HY && wave < BY - HY && yrow < dom.local_max[1];
+    const int xs = x0 + lane * VX;
+    const int g_nxy = g.dim[0] * g.dim[1];
+    const physis_hip::BufWin<double> g_w = physis_hip::BufWin<double>::Make(g.p, g_nxy * g.dim[2], (long)(zb + -2) * g_nxy, (long)(ze + 2) * g_nxy);
+    S_g g_st[PD];
+    const typename S_g::Addr g_ra = S_g::Prepare(g.dim, x0, yrow, lane);
+    S_g g_pro[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Load(g_w, g.p, g.dim, g_ra, zb + -1 + k);
+#pragma unroll
+    for (int k = 0; k < PD; ++k)
+      g_st[k].Load(g_w, g.p, g.dim, g_ra, zb + 2 + k);
+    int g_base = 0;
+    const int g_enx = g.dim[0], g_enxy = g.dim[0] * g.dim[1];
+    const physis_hip::BufWin<double> g_ew = physis_hip::BufWin<double>::Make(g.p, g_enxy * g.dim[2], (long)zb * g_enxy, (long)ze * g_enxy);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      g_pro[k].Store(g_lds + k * S_g::kPlane, wave, lane, g_ra);
+    __syncthreads();
+    __PSCtx_relax_double ctx;
+    ctx.g_p = g.p;
+    for (int d = 0; d < 3; ++d) ctx.g_dim[d] = g.dim[d];
+    if constexpr (VX > 1) __builtin_assume((xs & (VX - 1)) == 0);
+    if constexpr (VX > 1 && !RAGGED) {
+      __builtin_assume((ctx.g_dim[0] & 3) == 0);
+    }
+    constexpr int U = 2;
+    for (int zc = zb; zc < ze; zc += U) {
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const int z = zc + k;
+        const int cur = k & 1, nxt = cur ^ 1;
+        (void)cur; (void)nxt;
+        if (computes && z < ze) {
+          double g_r0[VX + 2];
+          S_g::template ReadRow<-1, 1>(g_lds + physis_hip::RingSlot<4>(g_base, 1) * S_g::kPlane, wave + 0, lane, g_r0);
+          double g_r1[VX + 0];
+          S_g::template ReadRow<0, 0>(g_lds + physis_hip::RingSlot<4>(g_base, 1) * S_g::kPlane, wave + 1, lane, g_r1);
+          double g_r2[VX + 0];
+          S_g::template ReadRow<0, 0>(g_lds + physis_hip::RingSlot<4>(g_base, 1) * S_g::kPlane, wave + -1, lane, g_r2);
+          double g_r3[VX + 0];
+          S_g::template ReadRow<0, 0>(g_lds + physis_hip::RingSlot<4>(g_base, 2) * S_g::kPlane, wave + 0, lane, g_r3);
+          double g_r4[VX + 0];
+          S_g::template ReadRow<0, 0>(g_lds + physis_hip::RingSlot<4>(g_base, 0) * S_g::kPlane, wave + 0, lane, g_r4);
+          double g_out[VX];
+          unsigned g_mask = 0;
+#pragma unroll
+          for (int i = 0; i < VX; ++i) {
+            const int x = xs + i;
+            const bool __in = x >= dom.local_min[0] && x < dom.local_max[0] &&
+                (__rb < 0 || ((x + yrow + z + __rb) & 1) == 0);
+            {
+              ctx.g[0] = g_r0[i + 1];
+              ctx.g[1] = g_r0[i + 2];
+              ctx.g[2] = g_r0[i + 0];
+              ctx.g[3] = g_r1[i + 0];
+              ctx.g[4] = g_r2[i + 0];
+              ctx.g[5] = g_r3[i + 0];
+              ctx.g[6] = g_r4[i + 0];
+              ctx.g_e = false;
+              relax_double(x, yrow, z, ctx);
+              g_out[i] = ctx.g_v;
+              g_mask |= (__in && ctx.g_e) ? 1u << i : 0u;
+            }
+          }
+          physis_hip::StoreMasked<double, VX>(g_ew, xs + yrow * g_enx + z * g_enxy, g_out, g_mask);
+        }
+        g_st[k % PD].Store(g_lds + physis_hip::RingSlot<4>(g_base, 3) * S_g::kPlane, wave, lane, g_ra);
+        __syncthreads();
+        g_st[k % PD].Load(g_w, g.p, g.dim, g_ra, z + 2 + PD);
+        g_base = physis_hip::RingSlot<4>(g_base, 1);
+      }
+    }
+  }
+  (void)__red;
+}
+
+template <int VX>
+static physis_hip::RunShape __PSShape_relax_double(const struct __PSStencil_relax_double &s) {
+  static int per_cu = physis_hip::BlocksPerCU(
+      (const void *)__PSStencilRun_relax_double<VX, 8, -1>, 64 * 8);
+  return physis_hip::PlanRun(s.dom, 64 * physis_hip::FormVX(VX), 8 - 2 * 1, per_cu, physis_hip::WindowChunkLimit({s.g}, 2));
+}
+
+template <int VX>
+static int __PSLaunch_relax_double(const struct __PSStencil_relax_double &s, hipStream_t stream, void *red) {
+  const physis_hip::RunShape sh = __PSShape_relax_double<VX>(s);
+  if (sh.blocks == 0) return 0;
+  const dim3 grid(sh.blocks), block(64 * 8);
+  for (int __c = s.__rb == 2 ? 0 : s.__rb; __c <= (s.__rb == 2 ? 1 : s.__rb); ++__c) {
+  (void)red;
+  {
+      hipLaunchKernelGGL((__PSStencilRun_relax_double<VX, 8, -1>), grid, block, 0, stream, s.dom, physis_hip::DevView<__PSGrid3DDouble_dev>(s.g), sh, (float *)NULL, __c);
+  }
+  }
+  return sh.blocks;
+}
+
+static int __PSBlocks_relax_double(const struct __PSStencil_relax_double &s) {
+  return (s.g->dim[0] % 4 == 0) ? __PSShape_relax_double<4>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_relax_double<4 + physis_hip::kRagged>(s).blocks
+         : __PSShape_relax_double<1>(s).blocks;
+}
+
+static int __PSRun_relax_double(const struct __PSStencil_relax_double &s, hipStream_t stream, void *red) {
+  physis_hip::CheckGrid3D(s.g, PS_DOUBLE);
+  physis_hip::CheckEmitDomain(s.dom, s.g);
+  return (s.g->dim[0] % 4 == 0) ? __PSLaunch_relax_double<4>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_relax_double<4 + physis_hip::kRagged>(s, stream, red)
+         : __PSLaunch_relax_double<1>(s, stream, red);
+}
+
 extern "C" {
 
 static PSDomain3D whole(PSGrid3DFloat g) {
@@ -3547,6 +3738,25 @@ extern "C" {
 void ragged_box2d(PSGrid2DFloat g, PSGrid2DFloat g2, int x0, int x1, int y0, int y1, int count, float w) {
   PSDomain2D d = PSDomain2DNew(x0, x1, y0, y1);
   __PSStencilRun_8(count, __PSStencilMap_inner2d(d, g, g2, w), __PSStencilMap_inner2d(d, g2, g, w));
+}
+
+}  // extern "C"
+
+static void __PSStencilRun_9(int iter, struct __PSStencil_relax_double s0) {
+  hipStream_t stream = (hipStream_t)__PSHipStream();
+  __PSTraceStencilPre("relax_double");
+  physis_hip::RunTimer timer(stream);
+  for (int i = 0; i < iter; ++i) {
+    __PSRun_relax_double(s0, stream, NULL);
+  }
+  __PSTraceStencilPost(timer.Stop());
+}
+
+extern "C" {
+
+void ragged_relax_double(PSGrid3DDouble g, int count) {
+  PSDomain3D d = PSDomain3DNew(1, PSGridDim(g, 0) - 1, 1, PSGridDim(g, 1) - 1, 1, PSGridDim(g, 2) - 1);
+  __PSStencilRun_9(count, __PSStencilMapRedBlack_relax_double(d, g));
 }
 
 }  // extern "C"

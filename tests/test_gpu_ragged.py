@@ -217,3 +217,29 @@ def test_rows_too_long_for_passes(ps, prog):
         assert np.array_equal(got[k][:, x0 - 1:x1 + 1], u[k]), k
         a[:, x0 - 1:x1 + 1] = got[k][:, x0 - 1:x1 + 1]
         assert np.array_equal(got[k], a)
+
+
+@pytest.mark.parametrize("shape", [(9, 7, 5), (66, 33, 20), (257, 30, 9)])
+def test_red_black_double(ps, prog, shape):
+    """A red-black map of an 8-byte grid (its colour sweeps are not fused: two
+    rings of 8-byte planes do not fit LDS)."""
+    print(f"red-black double {shape}", flush=True)
+    nx, ny, nz = shape
+    a = np.random.default_rng(nx).standard_normal((nz, ny, nx))
+    z, y, x = np.meshgrid(*map(np.arange, a.shape), indexing="ij")
+    inside = np.zeros(a.shape, bool)
+    inside[1:-1, 1:-1, 1:-1] = True
+    prog.ragged_relax_double.argtypes = [ps.PSGridPtr, C.c_int]
+    for count in (1, 2, 3):
+        g = ps.PSGridNew(shape, np.float64)
+        ps.PSGridCopyin(g, a)
+        prog.ragged_relax_double(g.handle, count)
+        got = ps.PSGridCopyout(g)
+        ps.PSGridFree(g)
+        u = a.copy()
+        for k in range(2 * count):
+            v = u.copy()
+            for axis, d in ((2, -1), (2, 1), (1, -1), (1, 1), (0, -1), (0, 1)):
+                v += np.roll(u, d, axis)
+            u = np.where(inside & ((x + y + z + k) % 2 == 0), v * 0.125, u)
+        assert np.array_equal(got, u.reshape(-1)), count
