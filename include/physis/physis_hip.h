@@ -182,7 +182,8 @@ extern void __PSHipReduceFold(int type, int op, const void *partials,
 /* Pinned host area number `slot` (0 <= slot < 10) of at least `bytes`, kept
  * and grown across calls: kernels write it, the host reads it after a wait
  * on the runtime stream.  Generated run functions keep the results of fused
- * reductions in slots 1..7; slot 0 is __PSHipReduceFold's own. */
+ * reductions in slots 1..7; slot 0 is __PSHipReduceFold's own (the waiting form,
+ * for callers of their own: generated run functions use the one below). */
 extern void *__PSHipPinned(int slot, size_t bytes);
 /* __PSHipReduceFold without the wait: the results are in `out` (pinned or
  * device memory) once the runtime stream has drained. */

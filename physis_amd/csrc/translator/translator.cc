@@ -3338,17 +3338,13 @@ std::string Translator::EmitTileKernel(const KernelInfo &k) {
          "      if (t < TILE::T) {\n        if (keep)\n          nxt[p.at] = v[0];\n"
          "        else if (t == 1)\n          nxt[p.at] = bg_c[k][0];\n      }\n";
   } else if (rb) {
-    size_t c = 0;
-    for (size_t i = 0; i < gi.offsets.size(); ++i)
-      if (!gi.offsets[i][0] && !gi.offsets[i][1] && !gi.offsets[i][2]) c = i;
     o << "      const bool upd = p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&\n"
          "          p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&\n"
          "          p.z >= dom.local_min[2] && p.z < dom.local_max[2] &&\n"
          "          ((p.x + p.y + p.z + t - 1) & 1) == 0;\n"
-         "      const " << T << " v[1] = {upd ? ctx." << O << "_v : cur[p.at + 0]};\n"
+         "      const " << T << " v[1] = {upd ? ctx." << O << "_v : cur[p.at]};\n"
          "      if (t < TILE::T) nxt[p.at] = v[0];\n"
          "      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];\n";
-    (void)c;
   } else {
     o << "      const " << T << " v[1] = {ctx." << O << "_v};\n"
          "      if (t < TILE::T) nxt[p.at] = v[0];\n"

@@ -747,6 +747,9 @@ __global__ __launch_bounds__(64 * TY, CIN == 2 ? 4 : 1) void ConvMKernel(
 // and shifted B by register: at 8 x 128^3 24 -> 8 took 471 us, now 249, and
 // 8 -> 8 207, now 122 (92 us of bytes); rows that are not multiples of 32 ran
 // on a kernel that gathered its operands 2 bytes at a time.
+// An input that is not finite times the zeros of gradient planes outside a chunk
+// is NaN: gradients of taps that lead out of the grid are then NaN too (as they
+// were for rows of multiples of 32).
 __device__ __forceinline__ bf16x8 ReadTr(const u16 *a, const u16 *b) {
   typedef __attribute__((address_space(3))) s16x4 *P;
   const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)a);
@@ -1580,7 +1583,7 @@ struct __PSUNet {
   long step = 0;
   // activations (BF16) at batch max_batch
   u16 *a[10] = {}, *q1 = nullptr, *q2 = nullptr, *c2 = nullptr;
-  float *out = nullptr;
+  float *out = nullptr;  // head outputs, for the smooth loss terms alone
   // gradient scratch
   u16 *g1a = nullptr, *g1b = nullptr, *gc1 = nullptr;  // level 1
   u16 *g2a = nullptr, *g2b = nullptr, *gc2 = nullptr;  // level 2
@@ -1970,11 +1973,9 @@ __PSUNet *PSUNetNew(int nx, int ny, int nzs, int max_batch, float out_scale,
   size_t pe = (size_t)kHeadBlocks * 9, be = 0;
   for (int l = 0; l < 10; ++l) {
     const int lv = l < 2 || l > 7 ? 1 : (l < 4 || l > 5 ? 2 : 3);
-    const long P = lv == 1 ? d.P1 : (lv == 2 ? d.P2 : d.P3);
     const int W = lv == 1 ? d.W1 : (lv == 2 ? d.W2 : d.W3);
     const int H = lv == 1 ? d.H1 : (lv == 2 ? d.H2 : d.H3);
     const int D = lv == 1 ? d.D1 : (lv == 2 ? d.D2 : d.D3);
-    (void)P;
     // the block count depends on the batch: the largest over every batch a
     // call may use
     size_t nb = 0;

@@ -3936,7 +3936,7 @@ __global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_krb(
           p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&
           p.z >= dom.local_min[2] && p.z < dom.local_max[2] &&
           ((p.x + p.y + p.z + t - 1) & 1) == 0;
-      const float v[1] = {upd ? ctx.g_v : cur[p.at + 0]};
+      const float v[1] = {upd ? ctx.g_v : cur[p.at]};
       if (t < TILE::T) nxt[p.at] = v[0];
       const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
       if (k < TILE::Owned(0)) {
