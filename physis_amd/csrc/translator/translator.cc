@@ -1788,6 +1788,9 @@ std::vector<Row> RowsOf(const GridParam &g) {
 
 std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
   std::ostringstream o;
+  int centre_only = 0;
+  for (auto &g : k.grids) centre_only += g.mode == GridParam::kDirect && g.read;
+  const bool batch = centre_only <= 4;
   const std::string &n = k.name;
   const bool red = k.ret_type != "void";
   const std::string RT = red ? k.ret_type : "float";
@@ -1853,11 +1856,21 @@ std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
       o << "    const typename S_" << G << "::Addr " << G << "_ra = S_" << G
         << "::Prepare(" << G << ".dim, x0, yrow, lane);\n";
       // every load of the prologue is issued before the first one is
-      // stored: a short z chunk then waits for memory once
-      o << "    S_" << G << " " << G << "_pro[" << nslot - 1 << "];\n"
-        << "#pragma unroll\n    for (int k = 0; k < " << nslot - 1 << "; ++k)\n"
-        << "      " << G << "_pro[k].Load(" << G << "_w, " << G << ".p, " << G
-        << ".dim, " << G << "_ra, zb + " << g.zl << " + k);\n";
+      // stored: a short z chunk then waits for memory once (a kernel with
+      // many centre-only grids loads those after them and loses: two 19-point
+      // sweeps of 32x256x200 184 us with the batch and 174 without, 132x60x60
+      // 29.1 and 27.2, 256x128x100 81.6 and 79.4, 512x256x200 590 and 583)
+      if (batch)
+        o << "    S_" << G << " " << G << "_pro[" << nslot - 1 << "];\n"
+          << "#pragma unroll\n    for (int k = 0; k < " << nslot - 1 << "; ++k)\n"
+          << "      " << G << "_pro[k].Load(" << G << "_w, " << G << ".p, " << G
+          << ".dim, " << G << "_ra, zb + " << g.zl << " + k);\n";
+      else
+        o << "#pragma unroll\n    for (int k = 0; k < " << nslot - 1
+          << "; ++k) {\n      " << G << "_st[0].Load(" << G << "_w, " << G
+          << ".p, " << G << ".dim, " << G << "_ra, zb + " << g.zl << " + k);\n"
+          << "      " << G << "_st[0].Store(" << G << "_lds + k * S_" << G
+          << "::kPlane, wave, lane, " << G << "_ra);\n    }\n";
       o << "#pragma unroll\n    for (int k = 0; k < PD; ++k)\n      " << G
         << "_st[k].Load(" << G << "_w, " << G << ".p, " << G << ".dim, " << G
         << "_ra, zb + " << g.zr + 1 << " + k);\n";
@@ -1884,7 +1897,7 @@ std::string Translator::EmitFastRunKernel(const KernelInfo &k) {
     }
   }
   for (auto &g : k.grids)
-    if (g.mode == GridParam::kStaged)
+    if (g.mode == GridParam::kStaged && batch)
       o << "#pragma unroll\n    for (int k = 0; k < " << g.zr - g.zl + 1
         << "; ++k)\n      " << g.name << "_pro[k].Store(" << g.name
         << "_lds + k * S_" << g.name << "::kPlane, wave, lane, " << g.name

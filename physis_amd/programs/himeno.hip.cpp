@@ -167,10 +167,11 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_jacobi_kernel(
     const physis_hip::BufWin<float> p0_w = physis_hip::BufWin<float>::Make(p0.p, p0_nxy * p0.dim[2], (long)(zb + -2) * p0_nxy, (long)(ze + 2) * p0_nxy);
     S_p0 p0_st[PD];
     const typename S_p0::Addr p0_ra = S_p0::Prepare(p0.dim, x0, yrow, lane);
-    S_p0 p0_pro[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-      p0_pro[k].Load(p0_w, p0.p, p0.dim, p0_ra, zb + -1 + k);
+    for (int k = 0; k < 3; ++k) {
+      p0_st[0].Load(p0_w, p0.p, p0.dim, p0_ra, zb + -1 + k);
+      p0_st[0].Store(p0_lds + k * S_p0::kPlane, wave, lane, p0_ra);
+    }
 #pragma unroll
     for (int k = 0; k < PD; ++k)
       p0_st[k].Load(p0_w, p0.p, p0.dim, p0_ra, zb + 2 + k);
@@ -225,9 +226,6 @@ __global__ __launch_bounds__(64 * BY) void __PSStencilRun_jacobi_kernel(
     const physis_hip::BufWin<float> wrk1_w = physis_hip::BufWin<float>::Make(wrk1.p, wrk1_nxy * wrk1.dim[2], (long)zb * wrk1_nxy, (long)ze * wrk1_nxy);
     float wrk1_dv[2][VX];
     wrk1_w.template Load<VX, physis_hip::kStreamLoad>(xs + drow * wrk1_nx + zb * wrk1_nxy, wrk1_dv[0]);
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      p0_pro[k].Store(p0_lds + k * S_p0::kPlane, wave, lane, p0_ra);
     __syncthreads();
     __PSCtx_jacobi_kernel ctx;
     ctx.p0_p = p0.p;

@@ -555,3 +555,16 @@ def test_passes_of_several_sweeps_need_their_scratch_grids(program, second):
     for c in asked:
         assert "&& physis_hip::HaveScratch((size_t)" in c, c
     assert any("sizeof(float), " + second + ")" in c for c in asked), asked
+
+
+def test_prologue_loads_are_batched_where_that_pays():
+    """A run kernel issues every load of its prologue before the first store,
+    unless many centre-only grids' loads come after them."""
+    for src, fn, batched in ((SOURCES[0], "diffusion7_kernel", True),
+                             (SOURCES[1], "jacobi_kernel", False)):
+        rc, code, err = translate(src)
+        assert rc == 0, err
+        kernel = code[code.index("void __PSStencilRun_" + fn + "("):]
+        kernel = kernel[:kernel.index("__syncthreads();")]
+        assert ("_pro[k].Load(" in kernel) == batched
+        assert ("_st[0].Store(" in kernel) != batched
