@@ -183,6 +183,35 @@ inline RunShape PlanRun(const __PSDomain &dom, int tx, int ty, int per_cu,
                     extra);
 }
 
+// Whether a single sweep over rows whose extents are not multiples of 4 runs
+// at one point per lane (tiles of 64 points) and not in the ragged form at four
+// (tiles of 256): it does where it covers the domain with so many fewer lanes
+// that the work shared by a lane's four points does not count.  Periodic planes
+// are loaded through a window of their own each, four times as often per point,
+// but small grids still gain from the blocks (77x60x60 12.1 and 13, 222x60x60 12.9
+// and 13.4).
+// us at one point and ragged, rows of 63, 127, 191, 255 and 290 points by
+// 256 x 200: 7-point clamped diffusion 11.1 and 16.9, 19.2 and 20.3, 27.1 and
+// 23.3, 33 and 27, 36 and 37; periodic 15.3 and 18.9, 23 and 20, 33 and 24;
+// 7-point over user points 58 and 92, 81 and 94, 117 and 99, 136 and 110, 150
+// and 170; 19-point 49 and 103, 104 and 119, 151 and 139, 208 and 171, 245 and
+// 242; 7 gets at corners 10 and 17, 13 and 17, 18 and 18, 22 and 20, 25 and 33.
+// (8-byte grids always do: 14 and 49, 24 and 50, 30 and 50, 42 and 51, 45 and
+// 98; four of their points are two 16-byte vectors, and LDS holds half as many
+// blocks.)
+// A colour sweep leaves every other point of a lane's four as it is: large ones
+// run at one point per lane (255^3 63 and 70 an iteration, 383x200x150 48 and 51;
+// 150^3 26 and 23).
+inline bool OnePointRows(const __PSDomain &d, bool periodic, bool colour) {
+  const auto tiles = [&](int t) {
+    return (d.local_max[0] + t - 1) / t - d.local_min[0] / t;
+  };
+  double points = 1;
+  for (int i = 0; i < 3; ++i) points *= d.local_max[i] - d.local_min[i];
+  if (periodic) return tiles(64) <= tiles(256) || points < 1.5e6;
+  return 2 * tiles(64) <= 5 * tiles(256) || (colour && points >= 8e6);
+}
+
 // Points per lane (4 or 2) of a whole-grid two-sweep pass over rows of nx
 // points: tiles of 256 points, or of 128 where those pad the rows so much
 // less that they win although a point costs 1.2 times as much in them (its
@@ -220,8 +249,7 @@ inline void CheckGrid3D(const __PSGrid *g, int type) {
   }
 }
 
-// Device-to-device copy of `bytes` on `stream` (scratch grids of two-sweep
-// runs start as copies of the grid they stand in for); aborts on an error.
+// Device-to-device copy of `bytes` on `stream`; aborts on an error.
 inline void CopyDevice(void *dst, const void *src, size_t bytes,
                        hipStream_t stream) {
   const hipError_t e =

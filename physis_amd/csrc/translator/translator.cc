@@ -2683,11 +2683,25 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
         add(emit_checks,
             "physis_hip::CheckEmitDomain(s.dom, " + HostGrid(k, g) + ")");
     }
+    // ... and so does one that fewer lanes cover at one point each
+    // (OnePointRows), and always an 8-byte grid
+    bool wide = false, periodic = false;
+    for (auto &g : k.grids) {
+      if ((!g.read && !g.emitted) || g.user) continue;
+      wide = wide || g.elem == "double" || g.elem == "long";
+      periodic = periodic || (g.mode == GridParam::kStaged && g.periodic);
+    }
+    if (!wide)
+      add(rconds, "!physis_hip::OnePointRows(" + D + ", " +
+                      (periodic ? "true" : "false") + ", " +
+                      (k.used_rb ? "true" : "false") + ")");
     std::string vec = conds.empty() ? "true" : Join(conds, " && ");
     std::string rag = rconds.empty() ? "true" : Join(rconds, " && ");
     auto pick = [&](const std::string &f, const std::string &tail) {
-      return "  return (" + vec + ") ? " + f + "<4>" + tail + "\n         : (" +
-             rag + ") ? " + f + "<4 + physis_hip::kRagged>" + tail +
+      return "  return (" + vec + ") ? " + f + "<4>" + tail +
+             (wide ? ""
+                   : "\n         : (" + rag + ") ? " + f +
+                         "<4 + physis_hip::kRagged>" + tail) +
              "\n         : " + f + "<1>" + tail + ";\n";
     };
     o << "static int __PSBlocks_" << n << "(const struct __PSStencil_" << n

@@ -217,7 +217,7 @@ static int __PSLaunch_diffusion7_kernel(const struct __PSStencil_diffusion7_kern
 
 static int __PSBlocks_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s) {
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_diffusion7_kernel<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_diffusion7_kernel<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_diffusion7_kernel<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_diffusion7_kernel<1>(s).blocks;
 }
 
@@ -226,7 +226,7 @@ static int __PSRun_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel 
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_diffusion7_kernel<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_diffusion7_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_diffusion7_kernel<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_diffusion7_kernel<1>(s, stream, red);
 }
 
@@ -701,7 +701,7 @@ static int __PSLaunch_diffusion7_periodic_kernel(const struct __PSStencil_diffus
 
 static int __PSBlocks_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s) {
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_diffusion7_periodic_kernel<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_diffusion7_periodic_kernel<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSShape_diffusion7_periodic_kernel<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_diffusion7_periodic_kernel<1>(s).blocks;
 }
 
@@ -710,7 +710,7 @@ static int __PSRun_diffusion7_periodic_kernel(const struct __PSStencil_diffusion
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_diffusion7_periodic_kernel<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_diffusion7_periodic_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSLaunch_diffusion7_periodic_kernel<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_diffusion7_periodic_kernel<1>(s, stream, red);
 }
 

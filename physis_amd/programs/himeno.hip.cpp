@@ -407,7 +407,7 @@ static int __PSLaunch_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, h
 
 static int __PSBlocks_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s) {
   return (s.p0->dim[0] % 4 == 0 && s.p1->dim[0] % 4 == 0 && s.a0->dim[0] % 4 == 0 && s.a1->dim[0] % 4 == 0 && s.a2->dim[0] % 4 == 0 && s.a3->dim[0] % 4 == 0 && s.b0->dim[0] % 4 == 0 && s.b1->dim[0] % 4 == 0 && s.b2->dim[0] % 4 == 0 && s.c0->dim[0] % 4 == 0 && s.c1->dim[0] % 4 == 0 && s.c2->dim[0] % 4 == 0 && s.bnd->dim[0] % 4 == 0 && s.wrk1->dim[0] % 4 == 0) ? __PSShape_jacobi_kernel<4>(s).blocks
-         : (s.dom.local_max[0] <= s.p0->dim[0]) ? __PSShape_jacobi_kernel<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.p0->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_jacobi_kernel<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_jacobi_kernel<1>(s).blocks;
 }
 
@@ -428,7 +428,7 @@ static int __PSRun_jacobi_kernel(const struct __PSStencil_jacobi_kernel &s, hipS
   physis_hip::CheckGrid3D(s.wrk1, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.p1);
   return (s.p0->dim[0] % 4 == 0 && s.p1->dim[0] % 4 == 0 && s.a0->dim[0] % 4 == 0 && s.a1->dim[0] % 4 == 0 && s.a2->dim[0] % 4 == 0 && s.a3->dim[0] % 4 == 0 && s.b0->dim[0] % 4 == 0 && s.b1->dim[0] % 4 == 0 && s.b2->dim[0] % 4 == 0 && s.c0->dim[0] % 4 == 0 && s.c1->dim[0] % 4 == 0 && s.c2->dim[0] % 4 == 0 && s.bnd->dim[0] % 4 == 0 && s.wrk1->dim[0] % 4 == 0) ? __PSLaunch_jacobi_kernel<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.p0->dim[0]) ? __PSLaunch_jacobi_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.p0->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_jacobi_kernel<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_jacobi_kernel<1>(s, stream, red);
 }
 

@@ -202,7 +202,7 @@ static int __PSLaunch_redblack7_kernel(const struct __PSStencil_redblack7_kernel
 
 static int __PSBlocks_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s) {
   return (s.g->dim[0] % 4 == 0) ? __PSShape_redblack7_kernel<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_redblack7_kernel<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, true)) ? __PSShape_redblack7_kernel<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_redblack7_kernel<1>(s).blocks;
 }
 
@@ -210,7 +210,7 @@ static int __PSRun_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g);
   return (s.g->dim[0] % 4 == 0) ? __PSLaunch_redblack7_kernel<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_redblack7_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, true)) ? __PSLaunch_redblack7_kernel<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_redblack7_kernel<1>(s, stream, red);
 }
 

@@ -171,7 +171,7 @@ static int __PSLaunch_s2d5(const struct __PSStencil_s2d5 &s, hipStream_t stream,
 
 static int __PSBlocks_s2d5(const struct __PSStencil_s2d5 &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_s2d5<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_s2d5<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSShape_s2d5<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_s2d5<1>(s).blocks;
 }
 
@@ -180,7 +180,7 @@ static int __PSRun_s2d5(const struct __PSStencil_s2d5 &s, hipStream_t stream, vo
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_s2d5<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_s2d5<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSLaunch_s2d5<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_s2d5<1>(s, stream, red);
 }
 
@@ -474,7 +474,7 @@ static int __PSLaunch_s2d9(const struct __PSStencil_s2d9 &s, hipStream_t stream,
 
 static int __PSBlocks_s2d9(const struct __PSStencil_s2d9 &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_s2d9<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_s2d9<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSShape_s2d9<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_s2d9<1>(s).blocks;
 }
 
@@ -483,7 +483,7 @@ static int __PSRun_s2d9(const struct __PSStencil_s2d9 &s, hipStream_t stream, vo
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_s2d9<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_s2d9<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSLaunch_s2d9<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_s2d9<1>(s, stream, red);
 }
 

@@ -233,7 +233,7 @@ static int __PSLaunch_udt7_kernel(const struct __PSStencil_udt7_kernel &s, hipSt
 
 static int __PSBlocks_udt7_kernel(const struct __PSStencil_udt7_kernel &s) {
   return (s.g->dim[0] % 4 == 0) ? __PSShape_udt7_kernel<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_udt7_kernel<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_udt7_kernel<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_udt7_kernel<1>(s).blocks;
 }
 
@@ -241,7 +241,7 @@ static int __PSRun_udt7_kernel(const struct __PSStencil_udt7_kernel &s, hipStrea
   physis_hip::CheckUserGrid3D(s.g);
   physis_hip::CheckEmitDomain(s.dom, s.g);
   return (s.g->dim[0] % 4 == 0) ? __PSLaunch_udt7_kernel<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_udt7_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_udt7_kernel<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_udt7_kernel<1>(s, stream, red);
 }
 
@@ -443,7 +443,7 @@ static int __PSLaunch_udt7_whole_kernel(const struct __PSStencil_udt7_whole_kern
 
 static int __PSBlocks_udt7_whole_kernel(const struct __PSStencil_udt7_whole_kernel &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_udt7_whole_kernel<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_udt7_whole_kernel<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_udt7_whole_kernel<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_udt7_whole_kernel<1>(s).blocks;
 }
 
@@ -452,7 +452,7 @@ static int __PSRun_udt7_whole_kernel(const struct __PSStencil_udt7_whole_kernel 
   physis_hip::CheckUserGrid3D(s.g2);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_udt7_whole_kernel<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_udt7_whole_kernel<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_udt7_whole_kernel<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_udt7_whole_kernel<1>(s, stream, red);
 }
 

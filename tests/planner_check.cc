@@ -1,7 +1,8 @@
 // Host-only check of the run-kernel launch planner (include/physis/hip/run.h):
 // prints, for each case, the z chunk and window bytes that PlanRunFor picks;
 // "tiles": whether pairs over a domain run in resident tiles
-// (include/physis/hip/tile.h); "fits": whether a pass has a window at all.  Built and run by tests/test_planner.py; no
+// (include/physis/hip/tile.h); "fits": whether a pass has a window at all; "one":
+// whether a single sweep runs at one point per lane.  Built and run by tests/test_planner.py; no
 // device is touched.
 #include <cstdio>
 #include <cstdlib>
@@ -55,6 +56,13 @@ int main(int argc, char **argv) {
       dom.local_max[d] = std::atoi(argv[3 + 2 * d]);
     }
     std::printf("%d\n", physis_hip::TilesBeatDomainPairs(dom, std::atol(argv[8])));
+    return 0;
+  }
+  if (argc == 7 && std::strcmp(argv[1], "one") == 0) {
+    __PSDomain dom = {};
+    for (int d = 0; d < 3; ++d) dom.local_max[d] = std::atoi(argv[2 + d]);
+    std::printf("%d\n", physis_hip::OnePointRows(dom, std::atoi(argv[5]) != 0,
+                                                 std::atoi(argv[6]) != 0));
     return 0;
   }
   if (argc == 8 && std::strcmp(argv[1], "fits") == 0) {

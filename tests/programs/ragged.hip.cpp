@@ -174,7 +174,7 @@ static int __PSLaunch_corners(const struct __PSStencil_corners &s, hipStream_t s
 
 static int __PSBlocks_corners(const struct __PSStencil_corners &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_corners<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_corners<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_corners<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_corners<1>(s).blocks;
 }
 
@@ -183,7 +183,7 @@ static int __PSRun_corners(const struct __PSStencil_corners &s, hipStream_t stre
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_corners<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_corners<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_corners<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_corners<1>(s, stream, red);
 }
 
@@ -689,7 +689,6 @@ static int __PSLaunch_corners_double(const struct __PSStencil_corners_double &s,
 
 static int __PSBlocks_corners_double(const struct __PSStencil_corners_double &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_corners_double<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_corners_double<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_corners_double<1>(s).blocks;
 }
 
@@ -698,7 +697,6 @@ static int __PSRun_corners_double(const struct __PSStencil_corners_double &s, hi
   physis_hip::CheckGrid3D(s.g2, PS_DOUBLE);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_corners_double<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_corners_double<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_corners_double<1>(s, stream, red);
 }
 
@@ -863,7 +861,7 @@ static int __PSLaunch_corners2d(const struct __PSStencil_corners2d &s, hipStream
 
 static int __PSBlocks_corners2d(const struct __PSStencil_corners2d &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_corners2d<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_corners2d<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSShape_corners2d<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_corners2d<1>(s).blocks;
 }
 
@@ -872,7 +870,7 @@ static int __PSRun_corners2d(const struct __PSStencil_corners2d &s, hipStream_t 
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_corners2d<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_corners2d<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSLaunch_corners2d<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_corners2d<1>(s, stream, red);
 }
 
@@ -1159,7 +1157,7 @@ static int __PSLaunch_wrap2(const struct __PSStencil_wrap2 &s, hipStream_t strea
 
 static int __PSBlocks_wrap2(const struct __PSStencil_wrap2 &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_wrap2<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_wrap2<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSShape_wrap2<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_wrap2<1>(s).blocks;
 }
 
@@ -1168,7 +1166,7 @@ static int __PSRun_wrap2(const struct __PSStencil_wrap2 &s, hipStream_t stream, 
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_wrap2<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_wrap2<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSLaunch_wrap2<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_wrap2<1>(s, stream, red);
 }
 
@@ -1335,7 +1333,7 @@ static int __PSLaunch_inner(const struct __PSStencil_inner &s, hipStream_t strea
 
 static int __PSBlocks_inner(const struct __PSStencil_inner &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_inner<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_inner<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_inner<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_inner<1>(s).blocks;
 }
 
@@ -1344,7 +1342,7 @@ static int __PSRun_inner(const struct __PSStencil_inner &s, hipStream_t stream, 
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_inner<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_inner<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_inner<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_inner<1>(s, stream, red);
 }
 
@@ -1888,7 +1886,7 @@ static int __PSLaunch_settle(const struct __PSStencil_settle &s, hipStream_t str
 
 static int __PSBlocks_settle(const struct __PSStencil_settle &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0 && s.c->dim[0] % 4 == 0) ? __PSShape_settle<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_settle<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_settle<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_settle<1>(s).blocks;
 }
 
@@ -1898,7 +1896,7 @@ static int __PSRun_settle(const struct __PSStencil_settle &s, hipStream_t stream
   physis_hip::CheckGrid3D(s.c, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0 && s.c->dim[0] % 4 == 0) ? __PSLaunch_settle<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_settle<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_settle<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_settle<1>(s, stream, red);
 }
 
@@ -2492,7 +2490,7 @@ static int __PSLaunch_settle_square(const struct __PSStencil_settle_square &s, h
 
 static int __PSBlocks_settle_square(const struct __PSStencil_settle_square &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_settle_square<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_settle_square<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_settle_square<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_settle_square<1>(s).blocks;
 }
 
@@ -2501,7 +2499,7 @@ static int __PSRun_settle_square(const struct __PSStencil_settle_square &s, hipS
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_settle_square<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_settle_square<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_settle_square<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_settle_square<1>(s, stream, red);
 }
 
@@ -3043,7 +3041,7 @@ static int __PSLaunch_inner2d(const struct __PSStencil_inner2d &s, hipStream_t s
 
 static int __PSBlocks_inner2d(const struct __PSStencil_inner2d &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_inner2d<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_inner2d<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSShape_inner2d<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_inner2d<1>(s).blocks;
 }
 
@@ -3052,7 +3050,7 @@ static int __PSRun_inner2d(const struct __PSStencil_inner2d &s, hipStream_t stre
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_inner2d<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_inner2d<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSLaunch_inner2d<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_inner2d<1>(s, stream, red);
 }
 
@@ -3358,7 +3356,6 @@ static int __PSLaunch_relax_double(const struct __PSStencil_relax_double &s, hip
 
 static int __PSBlocks_relax_double(const struct __PSStencil_relax_double &s) {
   return (s.g->dim[0] % 4 == 0) ? __PSShape_relax_double<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_relax_double<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_relax_double<1>(s).blocks;
 }
 
@@ -3366,7 +3363,6 @@ static int __PSRun_relax_double(const struct __PSStencil_relax_double &s, hipStr
   physis_hip::CheckGrid3D(s.g, PS_DOUBLE);
   physis_hip::CheckEmitDomain(s.dom, s.g);
   return (s.g->dim[0] % 4 == 0) ? __PSLaunch_relax_double<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_relax_double<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_relax_double<1>(s, stream, red);
 }
 

@@ -173,7 +173,7 @@ static int __PSLaunch_k7(const struct __PSStencil_k7 &s, hipStream_t stream, voi
 
 static int __PSBlocks_k7(const struct __PSStencil_k7 &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k7<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_k7<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_k7<1>(s).blocks;
 }
 
@@ -182,7 +182,7 @@ static int __PSRun_k7(const struct __PSStencil_k7 &s, hipStream_t stream, void *
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k7<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_k7<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_k7<1>(s, stream, red);
 }
 
@@ -684,7 +684,7 @@ static int __PSLaunch_k7p(const struct __PSStencil_k7p &s, hipStream_t stream, v
 
 static int __PSBlocks_k7p(const struct __PSStencil_k7p &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7p<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k7p<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSShape_k7p<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_k7p<1>(s).blocks;
 }
 
@@ -693,7 +693,7 @@ static int __PSRun_k7p(const struct __PSStencil_k7p &s, hipStream_t stream, void
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7p<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k7p<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSLaunch_k7p<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_k7p<1>(s, stream, red);
 }
 
@@ -1168,7 +1168,7 @@ static int __PSLaunch_k7n(const struct __PSStencil_k7n &s, hipStream_t stream, v
 
 static int __PSBlocks_k7n(const struct __PSStencil_k7n &s) {
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k7n<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_k7n<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_k7n<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_k7n<1>(s).blocks;
 }
 
@@ -1177,7 +1177,7 @@ static int __PSRun_k7n(const struct __PSStencil_k7n &s, hipStream_t stream, void
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k7n<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_k7n<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_k7n<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_k7n<1>(s, stream, red);
 }
 
@@ -1623,7 +1623,7 @@ static int __PSLaunch_kasym(const struct __PSStencil_kasym &s, hipStream_t strea
 
 static int __PSBlocks_kasym(const struct __PSStencil_kasym &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kasym<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_kasym<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_kasym<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kasym<1>(s).blocks;
 }
 
@@ -1632,7 +1632,7 @@ static int __PSRun_kasym(const struct __PSStencil_kasym &s, hipStream_t stream, 
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kasym<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_kasym<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_kasym<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kasym<1>(s, stream, red);
 }
 
@@ -1788,7 +1788,7 @@ static int __PSLaunch_kasymp(const struct __PSStencil_kasymp &s, hipStream_t str
 
 static int __PSBlocks_kasymp(const struct __PSStencil_kasymp &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kasymp<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_kasymp<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSShape_kasymp<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kasymp<1>(s).blocks;
 }
 
@@ -1797,7 +1797,7 @@ static int __PSRun_kasymp(const struct __PSStencil_kasymp &s, hipStream_t stream
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kasymp<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_kasymp<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSLaunch_kasymp<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kasymp<1>(s, stream, red);
 }
 
@@ -1993,7 +1993,7 @@ static int __PSLaunch_k27(const struct __PSStencil_k27 &s, hipStream_t stream, v
 
 static int __PSBlocks_k27(const struct __PSStencil_k27 &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k27<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_k27<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_k27<1>(s).blocks;
 }
 
@@ -2002,7 +2002,7 @@ static int __PSRun_k27(const struct __PSStencil_k27 &s, hipStream_t stream, void
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k27<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_k27<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_k27<1>(s, stream, red);
 }
 
@@ -2627,7 +2627,7 @@ static int __PSLaunch_k27p(const struct __PSStencil_k27p &s, hipStream_t stream,
 
 static int __PSBlocks_k27p(const struct __PSStencil_k27p &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27p<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k27p<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSShape_k27p<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_k27p<1>(s).blocks;
 }
 
@@ -2636,7 +2636,7 @@ static int __PSRun_k27p(const struct __PSStencil_k27p &s, hipStream_t stream, vo
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27p<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k27p<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSLaunch_k27p<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_k27p<1>(s, stream, red);
 }
 
@@ -3196,7 +3196,7 @@ static int __PSLaunch_k27i(const struct __PSStencil_k27i &s, hipStream_t stream,
 
 static int __PSBlocks_k27i(const struct __PSStencil_k27i &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27i<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k27i<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_k27i<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_k27i<1>(s).blocks;
 }
 
@@ -3205,7 +3205,7 @@ static int __PSRun_k27i(const struct __PSStencil_k27i &s, hipStream_t stream, vo
   physis_hip::CheckGrid3D(s.g2, PS_INT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27i<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k27i<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_k27i<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_k27i<1>(s, stream, red);
 }
 
@@ -3661,7 +3661,7 @@ static int __PSLaunch_krb(const struct __PSStencil_krb &s, hipStream_t stream, v
 
 static int __PSBlocks_krb(const struct __PSStencil_krb &s) {
   return (s.g->dim[0] % 4 == 0) ? __PSShape_krb<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_krb<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, true)) ? __PSShape_krb<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_krb<1>(s).blocks;
 }
 
@@ -3669,7 +3669,7 @@ static int __PSRun_krb(const struct __PSStencil_krb &s, hipStream_t stream, void
   physis_hip::CheckGrid3D(s.g, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g);
   return (s.g->dim[0] % 4 == 0) ? __PSLaunch_krb<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_krb<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, true)) ? __PSLaunch_krb<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_krb<1>(s, stream, red);
 }
 
@@ -4150,7 +4150,7 @@ static int __PSLaunch_krbp(const struct __PSStencil_krbp &s, hipStream_t stream,
 
 static int __PSBlocks_krbp(const struct __PSStencil_krbp &s) {
   return (s.g->dim[0] % 4 == 0) ? __PSShape_krbp<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_krbp<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, true)) ? __PSShape_krbp<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_krbp<1>(s).blocks;
 }
 
@@ -4163,7 +4163,7 @@ static int __PSRun_krbp(const struct __PSStencil_krbp &s, hipStream_t stream, vo
   }
   physis_hip::CheckEmitDomain(s.dom, s.g);
   return (s.g->dim[0] % 4 == 0) ? __PSLaunch_krbp<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_krbp<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, true)) ? __PSLaunch_krbp<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_krbp<1>(s, stream, red);
 }
 
@@ -4504,7 +4504,7 @@ static int __PSLaunch_k5(const struct __PSStencil_k5 &s, hipStream_t stream, voi
 
 static int __PSBlocks_k5(const struct __PSStencil_k5 &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k5<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_k5<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSShape_k5<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_k5<1>(s).blocks;
 }
 
@@ -4513,7 +4513,7 @@ static int __PSRun_k5(const struct __PSStencil_k5 &s, hipStream_t stream, void *
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k5<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_k5<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(physis_hip::RowDomain(s.dom), false, false)) ? __PSLaunch_k5<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_k5<1>(s, stream, red);
 }
 
@@ -4880,7 +4880,7 @@ static int __PSLaunch_kmix(const struct __PSStencil_kmix &s, hipStream_t stream,
 
 static int __PSBlocks_kmix(const struct __PSStencil_kmix &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kmix<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_kmix<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_kmix<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kmix<1>(s).blocks;
 }
 
@@ -4891,7 +4891,7 @@ static int __PSRun_kmix(const struct __PSStencil_kmix &s, hipStream_t stream, vo
   physis_hip::CheckGrid3D(s.j, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kmix<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_kmix<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_kmix<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kmix<1>(s, stream, red);
 }
 
@@ -5090,7 +5090,7 @@ static int __PSLaunch_khole(const struct __PSStencil_khole &s, hipStream_t strea
 
 static int __PSBlocks_khole(const struct __PSStencil_khole &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_khole<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_khole<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_khole<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_khole<1>(s).blocks;
 }
 
@@ -5099,7 +5099,7 @@ static int __PSRun_khole(const struct __PSStencil_khole &s, hipStream_t stream, 
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_khole<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_khole<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_khole<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_khole<1>(s, stream, red);
 }
 
@@ -5460,7 +5460,7 @@ static int __PSLaunch_kvec3(const struct __PSStencil_kvec3 &s, hipStream_t strea
 
 static int __PSBlocks_kvec3(const struct __PSStencil_kvec3 &s) {
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kvec3<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_kvec3<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_kvec3<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kvec3<1>(s).blocks;
 }
 
@@ -5469,7 +5469,7 @@ static int __PSRun_kvec3(const struct __PSStencil_kvec3 &s, hipStream_t stream, 
   physis_hip::CheckUserGrid3D(s.g2);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kvec3<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_kvec3<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_kvec3<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kvec3<1>(s, stream, red);
 }
 
@@ -5756,7 +5756,7 @@ static int __PSLaunch_ktensor(const struct __PSStencil_ktensor &s, hipStream_t s
 
 static int __PSBlocks_ktensor(const struct __PSStencil_ktensor &s) {
   return (s.g->dim[0] % 4 == 0) ? __PSShape_ktensor<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSShape_ktensor<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_ktensor<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_ktensor<1>(s).blocks;
 }
 
@@ -5764,7 +5764,7 @@ static int __PSRun_ktensor(const struct __PSStencil_ktensor &s, hipStream_t stre
   physis_hip::CheckUserGrid3D(s.g);
   physis_hip::CheckEmitDomain(s.dom, s.g);
   return (s.g->dim[0] % 4 == 0) ? __PSLaunch_ktensor<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0]) ? __PSLaunch_ktensor<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_ktensor<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_ktensor<1>(s, stream, red);
 }
 
@@ -6085,7 +6085,7 @@ static int __PSLaunch_kcplx(const struct __PSStencil_kcplx &s, hipStream_t strea
 
 static int __PSBlocks_kcplx(const struct __PSStencil_kcplx &s) {
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kcplx<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSShape_kcplx<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSShape_kcplx<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kcplx<1>(s).blocks;
 }
 
@@ -6094,7 +6094,7 @@ static int __PSRun_kcplx(const struct __PSStencil_kcplx &s, hipStream_t stream, 
   physis_hip::CheckUserGrid3D(s.g2);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g1->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kcplx<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g1->dim[0]) ? __PSLaunch_kcplx<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g1->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSLaunch_kcplx<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kcplx<1>(s, stream, red);
 }
 
@@ -6264,7 +6264,7 @@ static int __PSLaunch_kdouble(const struct __PSStencil_kdouble &s, hipStream_t s
 
 static int __PSBlocks_kdouble(const struct __PSStencil_kdouble &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kdouble<4>(s).blocks
-         : (true) ? __PSShape_kdouble<4 + physis_hip::kRagged>(s).blocks
+         : (!physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_kdouble<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kdouble<1>(s).blocks;
 }
 
@@ -6273,7 +6273,7 @@ static int __PSRun_kdouble(const struct __PSStencil_kdouble &s, hipStream_t stre
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kdouble<4>(s, stream, red)
-         : (true) ? __PSLaunch_kdouble<4 + physis_hip::kRagged>(s, stream, red)
+         : (!physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_kdouble<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kdouble<1>(s, stream, red);
 }
 
@@ -6439,7 +6439,7 @@ static int __PSLaunch_kshadow(const struct __PSStencil_kshadow &s, hipStream_t s
 
 static int __PSBlocks_kshadow(const struct __PSStencil_kshadow &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kshadow<4>(s).blocks
-         : (true) ? __PSShape_kshadow<4 + physis_hip::kRagged>(s).blocks
+         : (!physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_kshadow<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kshadow<1>(s).blocks;
 }
 
@@ -6448,7 +6448,7 @@ static int __PSRun_kshadow(const struct __PSStencil_kshadow &s, hipStream_t stre
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kshadow<4>(s, stream, red)
-         : (true) ? __PSLaunch_kshadow<4 + physis_hip::kRagged>(s, stream, red)
+         : (!physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_kshadow<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kshadow<1>(s, stream, red);
 }
 
@@ -6643,7 +6643,7 @@ static int __PSLaunch_kscaled(const struct __PSStencil_kscaled &s, hipStream_t s
 
 static int __PSBlocks_kscaled(const struct __PSStencil_kscaled &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kscaled<4>(s).blocks
-         : (true) ? __PSShape_kscaled<4 + physis_hip::kRagged>(s).blocks
+         : (!physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_kscaled<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kscaled<1>(s).blocks;
 }
 
@@ -6652,7 +6652,7 @@ static int __PSRun_kscaled(const struct __PSStencil_kscaled &s, hipStream_t stre
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kscaled<4>(s, stream, red)
-         : (true) ? __PSLaunch_kscaled<4 + physis_hip::kRagged>(s, stream, red)
+         : (!physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_kscaled<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kscaled<1>(s, stream, red);
 }
 

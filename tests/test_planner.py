@@ -89,3 +89,19 @@ def test_passes_of_several_sweeps_within_reach(planner, grid, elm, margin,
                         str(margin), str(rows)], check=True,
                        capture_output=True, text=True)
     assert int(r.stdout) == fits
+
+
+# Single sweeps over rows that are no multiples of 4, at one point per lane or
+# ragged at four: the side measured faster (include/physis/hip/run.h).
+@pytest.mark.parametrize("extents,periodic,colour,one", [
+    ((63, 256, 200), 0, 0, True), ((127, 256, 200), 0, 0, True),
+    ((191, 256, 200), 0, 0, False), ((255, 256, 200), 0, 0, False),
+    ((290, 256, 200), 0, 0, True), ((385, 256, 200), 0, 0, False),
+    ((63, 256, 200), 1, 0, True), ((127, 256, 200), 1, 0, False),
+    ((255, 256, 200), 1, 0, False), ((222, 60, 60), 1, 0, True),
+    ((150, 150, 150), 0, 1, False), ((255, 255, 255), 0, 1, True)])
+def test_points_per_lane_of_ragged_rows(planner, extents, periodic, colour, one):
+    r = subprocess.run([planner, "one", *map(str, extents), str(periodic),
+                        str(colour)], check=True, capture_output=True,
+                       text=True)
+    assert int(r.stdout) == one
