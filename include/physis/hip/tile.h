@@ -157,6 +157,25 @@ inline bool TilesBeatPairs(const int *dim, bool periodic) {
   return tile <= 16 && 2.5 * tile - pair < 2.2;
 }
 
+// Padded points (millions) of an extent box in tiles of tx x ty x tz.
+inline double PaddedMega(long ex, long ey, long ez, int tx, int ty, int tz) {
+  const auto up = [](long n, int t) { return (double)((n + t - 1) / t * t); };
+  return up(ex, tx) * up(ey, ty) * up(ez, tz) * 1e-6;
+}
+// Whether passes of several sweeps over a whole grid beat single sweeps.  Rows
+// that are no multiples of 4 and fit a 64-point tile run their single sweeps at
+// one point per lane there, half the lanes of the narrowest z-marching pass, and
+// those sweeps cost less than it (us a sweep, single and pair, clamped 7-point:
+// 41x700x700 47 and 73, 41x1000x1000 87 and 133; red-black iteration 54x292x284
+// 27 and 30); tiles beat them as long as the sweeps' latency counts (1.4 + 2.5
+// per million padded points against 6 + 1.5: 41x300x300 13 and 15, 33x500x500
+// 31 and 29).
+inline bool PassesPay(const int *dim, bool periodic) {
+  if (dim[0] % 4 == 0 || dim[0] > 64) return true;
+  return TilesBeatPairs(dim, periodic) &&
+         2.5 * PaddedMega(dim[0], dim[1], dim[2], 16, 16, 8) <
+             4.6 + 1.5 * PaddedMega(dim[0], dim[1], dim[2], 64, 1, 1);
+}
 // Whether a pass over a domain inside a grid of `points` points runs in tiles,
 // beside EmitFusedDomainKernel's pairs (tiles of 256 x 12 points): us a sweep
 // about 1.4 + 2.5 per million points of the padded tiles here and 4.3 + 0.83
@@ -179,6 +198,26 @@ inline bool TilesBeatDomainPairs(const __PSDomain &d, int64_t points) {
   const double wide = up(d.local_max[0], 256) - d.local_min[0] / 256 * 256;
   const double pair = wide * up(e[1], 12) * e[2] * 1e-6;
   return 2.5 * tile - 0.83 * pair < 2.9;
+}
+
+// Whether passes of a domain pair of 4 points per lane (EmitFusedDomainKernel's
+// with few centre-only grids, or tiles) beat single sweeps, on rows of nx points
+// that are no multiples of 4: single sweeps run at one point per lane in tiles
+// of 64 there.  Us a sweep, single and pair, 5-point map over the interior:
+// 41x300x300 12 and 27, 41x1000x1000 80 and 274, 97x300x300 23 and 29,
+// 129x400x400 48 and 57, 290x200x200 30 and 30, 257x200x200 and 161x300x300
+// faster as pairs; tiles as above.
+inline bool DomainPassesPay(const __PSDomain &d, int nx, int64_t points) {
+  if (nx % 4 == 0) return true;
+  long e[3];
+  for (int i = 0; i < 3; ++i) e[i] = d.local_max[i] - d.local_min[i];
+  const auto tiles = [&](int t) {
+    return (d.local_max[0] + t - 1) / t - d.local_min[0] / t;
+  };
+  if (TilesBeatDomainPairs(d, points))
+    return 2.5 * PaddedMega(e[0], e[1], e[2], 16, 16, 8) <
+           1.6 + 1.5 * tiles(64) * 64e-6 * e[1] * e[2];
+  return tiles(256) * 12 <= tiles(64) * 5;
 }
 
 // Per-block partials of each sweep of a pass (NULL: none).

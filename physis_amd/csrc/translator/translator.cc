@@ -2525,6 +2525,7 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
       << "  for (int d = 0; d < 3; ++d)\n"
          "    if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||\n"
          "        s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;\n"
+      << "  if (!physis_hip::PassesPay(a->dim, false)) return false;\n"
       << "  return physis_hip::WindowsFit({a}, 3) &&\n"
          "         physis_hip::HaveScratch((size_t)a->num_elms * sizeof(" << T
       << "), false);\n}\n\n";
@@ -2548,6 +2549,7 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
   for (auto &a : sa)
     o << "  if (__builtin_memcmp(&s0." << a << ", &s1." << a << ", sizeof(s0." << a
       << "))) return false;\n";
+  o << "  if (!physis_hip::PassesPay(a->dim, " << per << ")) return false;\n";
   o << "  return physis_hip::WindowsFit({a}, 3);\n}\n\n";
   return o.str();
 }
@@ -3234,6 +3236,9 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
   if (red)
     o << "  if ((s0.__reduce_out == NULL) != (s1.__reduce_out == NULL) ||\n"
          "      (s0.__reduce_out && s0.__reduce_op != s1.__reduce_op)) return false;\n";
+  if (kVX == 4)
+    o << "  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) "
+         "return false;\n";
   o << "  return physis_hip::WindowsFit({" << Join(wgrids0, ", ") << "}, 3);\n}\n\n";
   return o.str();
 }

@@ -2,7 +2,8 @@
 // prints, for each case, the z chunk and window bytes that PlanRunFor picks;
 // "tiles": whether pairs over a domain run in resident tiles
 // (include/physis/hip/tile.h); "fits": whether a pass has a window at all; "one":
-// whether a single sweep runs at one point per lane.  Built and run by tests/test_planner.py; no
+// whether a single sweep runs at one point per lane; "pay": whether passes over
+// a whole grid, and over its interior, beat single sweeps.  Built and run by tests/test_planner.py; no
 // device is touched.
 #include <cstdio>
 #include <cstdlib>
@@ -63,6 +64,19 @@ int main(int argc, char **argv) {
     for (int d = 0; d < 3; ++d) dom.local_max[d] = std::atoi(argv[2 + d]);
     std::printf("%d\n", physis_hip::OnePointRows(dom, std::atoi(argv[5]) != 0,
                                                  std::atoi(argv[6]) != 0));
+    return 0;
+  }
+  if (argc == 6 && std::strcmp(argv[1], "pay") == 0) {
+    __PSDomain dom = {};
+    int dim[3];
+    for (int d = 0; d < 3; ++d) {
+      dim[d] = std::atoi(argv[2 + d]);
+      dom.local_min[d] = 1;
+      dom.local_max[d] = dim[d] - 1;
+    }
+    std::printf("%d %d\n", physis_hip::PassesPay(dim, std::atoi(argv[5]) != 0),
+                physis_hip::DomainPassesPay(dom, dim[0],
+                                            (int64_t)dim[0] * dim[1] * dim[2]));
     return 0;
   }
   if (argc == 8 && std::strcmp(argv[1], "fits") == 0) {

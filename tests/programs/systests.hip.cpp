@@ -419,6 +419,7 @@ static bool __PSFusable2_k7(const struct __PSStencil_k7 &s0, const struct __PSSt
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
+  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) return false;
   return physis_hip::WindowsFit({a, b}, 3);
 }
 
@@ -883,6 +884,7 @@ static bool __PSFusable2_k7p(const struct __PSStencil_k7p &s0, const struct __PS
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
+  if (!physis_hip::PassesPay(a->dim, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -1385,6 +1387,7 @@ static bool __PSFusable2_k7n(const struct __PSStencil_k7n &s0, const struct __PS
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
+  if (!physis_hip::PassesPay(a->dim, false)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -2315,6 +2318,7 @@ static bool __PSFusable2_k27(const struct __PSStencil_k27 &s0, const struct __PS
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
+  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) return false;
   return physis_hip::WindowsFit({a, b}, 3);
 }
 
@@ -2902,6 +2906,7 @@ static bool __PSFusable2_k27p(const struct __PSStencil_k27p &s0, const struct __
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
+  if (!physis_hip::PassesPay(a->dim, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -3884,6 +3889,7 @@ static bool __PSFusableRB_krb(const struct __PSStencil_krb &s0) {
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
+  if (!physis_hip::PassesPay(a->dim, false)) return false;
   return physis_hip::WindowsFit({a}, 3) &&
          physis_hip::HaveScratch((size_t)a->num_elms * sizeof(float), false);
 }
