@@ -176,6 +176,30 @@ inline bool PassesPay(const int *dim, bool periodic) {
          2.5 * PaddedMega(dim[0], dim[1], dim[2], 16, 16, 8) <
              4.6 + 1.5 * PaddedMega(dim[0], dim[1], dim[2], 64, 1, 1);
 }
+// Whether the last of an odd number of red-black iterations runs as two colour
+// sweeps in place: a pass ends in the scratch grid there and takes a copy.  On
+// rows that are no multiples of 4 (us of one iteration, sweeps, pass and copy):
+// 129^3 20 and 23, 150^3 23 and 28, 257^3 63 and 81, 54x200x200 21 and 28, but
+// 255^3 63 and 59, 65^3 14 and 8, 383x200x150 48 and 50; the estimates fit these (sweeps 5.5 + 0.75 per
+// million points + 0.95 per million of the lanes, twice; copies 2.2 + 0.9 per MB
+// up to 8.5 + 0.155).  Rows of multiples of 4 take the pass, as measured faster
+// from 255^3 on.
+inline bool RedBlackLastAsSweeps(const int *dim, int iterations) {
+  if (iterations % 2 == 0 || dim[0] % 4 == 0) return false;
+  const bool narrow = PairVX(dim[0], false) == 2;
+  const double n = PaddedMega(dim[0], dim[1], dim[2], 1, 1, 1), mb = 4 * n;
+  const double sweeps = 2 * (5.5 + 0.75 * n + 0.95 * PaddedMega(dim[0], dim[1],
+                                                                 dim[2], 64, 1, 1));
+  const double pass =
+      TilesBeatPairs(dim, false)
+          ? 2 * (1.4 + 2.5 * PaddedMega(dim[0], dim[1], dim[2], 16, 16, 8))
+          : 2 * (4.3 + (narrow ? 1.0 : 0.83) *
+                           PaddedMega(dim[0], dim[1], dim[2], narrow ? 128 : 256, 8, 1));
+  const double copy = 2.2 + 0.9 * mb < 8.5 + 0.155 * mb ? 2.2 + 0.9 * mb
+                                                        : 8.5 + 0.155 * mb;
+  return sweeps < 1.08 * (pass + copy);
+}
+
 // Whether a pass over a domain inside a grid of `points` points runs in tiles,
 // beside EmitFusedDomainKernel's pairs (tiles of 256 x 12 points): us a sweep
 // about 1.4 + 2.5 per million points of the padded tiles here and 4.3 + 0.83

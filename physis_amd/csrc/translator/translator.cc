@@ -3686,6 +3686,9 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
       << "    vt.p = (" << T << " *)__PSHipScratch(8, bytes);\n"
       << "    " << V << " src = va;\n"
       << "    const bool __small = " << SmallExpr(k) << ";\n"
+      << "    // (the last iteration may be left to the colour sweeps below)\n"
+      << "    const int last = physis_hip::RedBlackLastAsSweeps(s0." << g.name
+      << "->dim, iter) ? 1 : 0;\n    iter -= last;\n"
       << "    // two iterations a resident-tile pass, an even number of times, so that\n"
          "    // the count of passes is odd when iter is\n"
       << "    const int two = __small ? iter / 2 & ~1 : 0;\n"
@@ -3700,7 +3703,7 @@ std::string Translator::EmitRunFunction(const RunSite &r) {
       << "<2>(s0, src, dst, NULL, 0, stream, {});\n"
       << "      src = dst;\n      i += its;\n    }\n"
       << "    if (iter % 2) physis_hip::CopyDevice(va.p, vt.p, bytes, stream);\n"
-      << "    i0 = iter;\n  }\n";
+      << "    i0 = iter;\n    iter += last;\n  }\n";
   }
   o << "  for (int i = " << (fuse || fuse_rb ? "i0" : "0") << "; i < iter; ++i) {\n";
   for (size_t i = 0; i < r.kernels.size(); ++i) {

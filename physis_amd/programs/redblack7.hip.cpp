@@ -524,6 +524,9 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_redblack7_kernel s0) {
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
     const bool __small = physis_hip::TilesBeatPairs(s0.g->dim, false);
+    // (the last iteration may be left to the colour sweeps below)
+    const int last = physis_hip::RedBlackLastAsSweeps(s0.g->dim, iter) ? 1 : 0;
+    iter -= last;
     // two iterations a resident-tile pass, an even number of times, so that
     // the count of passes is odd when iter is
     const int two = __small ? iter / 2 & ~1 : 0;
@@ -541,6 +544,7 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_redblack7_kernel s0) {
     }
     if (iter % 2) physis_hip::CopyDevice(va.p, vt.p, bytes, stream);
     i0 = iter;
+    iter += last;
   }
   for (int i = i0; i < iter; ++i) {
     __PSRun_redblack7_kernel(s0, stream, NULL);

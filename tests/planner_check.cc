@@ -3,7 +3,8 @@
 // "tiles": whether pairs over a domain run in resident tiles
 // (include/physis/hip/tile.h); "fits": whether a pass has a window at all; "one":
 // whether a single sweep runs at one point per lane; "pay": whether passes over
-// a whole grid, and over its interior, beat single sweeps.  Built and run by tests/test_planner.py; no
+// a whole grid, and over its interior, beat single sweeps, and whether the last
+// of one red-black iteration runs as colour sweeps.  Built and run by tests/test_planner.py; no
 // device is touched.
 #include <cstdio>
 #include <cstdlib>
@@ -74,9 +75,10 @@ int main(int argc, char **argv) {
       dom.local_min[d] = 1;
       dom.local_max[d] = dim[d] - 1;
     }
-    std::printf("%d %d\n", physis_hip::PassesPay(dim, std::atoi(argv[5]) != 0),
+    std::printf("%d %d %d\n", physis_hip::PassesPay(dim, std::atoi(argv[5]) != 0),
                 physis_hip::DomainPassesPay(dom, dim[0],
-                                            (int64_t)dim[0] * dim[1] * dim[2]));
+                                            (int64_t)dim[0] * dim[1] * dim[2]),
+                physis_hip::RedBlackLastAsSweeps(dim, 1));
     return 0;
   }
   if (argc == 8 && std::strcmp(argv[1], "fits") == 0) {

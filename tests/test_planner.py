@@ -120,4 +120,16 @@ def test_points_per_lane_of_ragged_rows(planner, extents, periodic, colour, one)
 def test_passes_where_they_pay(planner, extents, whole, interior):
     r = subprocess.run([planner, "pay", *map(str, extents), "0"], check=True,
                        capture_output=True, text=True)
-    assert [int(v) for v in r.stdout.split()] == [whole, interior]
+    assert [int(v) for v in r.stdout.split()][:2] == [whole, interior]
+
+
+# The last of an odd number of red-black iterations as a pass and a copy, or as
+# two colour sweeps: the side measured faster.
+@pytest.mark.parametrize("extents,sweeps", [
+    ((129, 129, 129), True), ((150, 150, 150), True), ((257, 257, 257), True),
+    ((54, 200, 200), True), ((383, 200, 150), True), ((255, 255, 255), False),
+    ((65, 65, 65), False), ((33, 100, 100), False), ((256, 256, 256), False)])
+def test_last_red_black_iteration(planner, extents, sweeps):
+    r = subprocess.run([planner, "pay", *map(str, extents), "0"], check=True,
+                       capture_output=True, text=True)
+    assert int(r.stdout.split()[2]) == sweeps
