@@ -2686,14 +2686,19 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
             "physis_hip::CheckEmitDomain(s.dom, " + HostGrid(k, g) + ")");
     }
     // ... and so does one that fewer lanes cover at one point each
-    // (OnePointRows), and always an 8-byte grid
-    bool wide = false, periodic = false;
+    // (OnePointRows).  Maps of 8-byte grids, and maps that read a grid through
+    // bounds-checked gets (each of a lane's points its own), have no ragged
+    // form: 7-point map with three 1-D coefficient grids, one point per lane
+    // and ragged, 191x256x200 30 and 43 us, 511x256x200 68 and 97.
+    bool one_point = false, periodic = false;
     for (auto &g : k.grids) {
       if ((!g.read && !g.emitted) || g.user) continue;
-      wide = wide || g.elem == "double" || g.elem == "long";
+      one_point = one_point || g.elem == "double" || g.elem == "long" ||
+                  (g.read && (g.irregular || (g.mode != GridParam::kStaged &&
+                                              g.mode != GridParam::kDirect)));
       periodic = periodic || (g.mode == GridParam::kStaged && g.periodic);
     }
-    if (!wide)
+    if (!one_point)
       add(rconds, "!physis_hip::OnePointRows(" + D + ", " +
                       (periodic ? "true" : "false") + ", " +
                       (k.used_rb ? "true" : "false") + ")");
@@ -2701,7 +2706,7 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
     std::string rag = rconds.empty() ? "true" : Join(rconds, " && ");
     auto pick = [&](const std::string &f, const std::string &tail) {
       return "  return (" + vec + ") ? " + f + "<4>" + tail +
-             (wide ? ""
+             (one_point ? ""
                    : "\n         : (" + rag + ") ? " + f +
                          "<4 + physis_hip::kRagged>" + tail) +
              "\n         : " + f + "<1>" + tail + ";\n";

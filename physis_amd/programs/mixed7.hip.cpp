@@ -193,7 +193,6 @@ static int __PSLaunch_mixed7_kernel(const struct __PSStencil_mixed7_kernel &s, h
 
 static int __PSBlocks_mixed7_kernel(const struct __PSStencil_mixed7_kernel &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_mixed7_kernel<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_mixed7_kernel<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_mixed7_kernel<1>(s).blocks;
 }
 
@@ -205,7 +204,6 @@ static int __PSRun_mixed7_kernel(const struct __PSStencil_mixed7_kernel &s, hipS
   physis_hip::CheckGrid3D(s.k, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_mixed7_kernel<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_mixed7_kernel<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_mixed7_kernel<1>(s, stream, red);
 }
 

@@ -4890,7 +4890,6 @@ static int __PSLaunch_kmix(const struct __PSStencil_kmix &s, hipStream_t stream,
 
 static int __PSBlocks_kmix(const struct __PSStencil_kmix &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kmix<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_kmix<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kmix<1>(s).blocks;
 }
 
@@ -4901,7 +4900,6 @@ static int __PSRun_kmix(const struct __PSStencil_kmix &s, hipStream_t stream, vo
   physis_hip::CheckGrid3D(s.j, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kmix<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_kmix<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kmix<1>(s, stream, red);
 }
 
@@ -6449,7 +6447,6 @@ static int __PSLaunch_kshadow(const struct __PSStencil_kshadow &s, hipStream_t s
 
 static int __PSBlocks_kshadow(const struct __PSStencil_kshadow &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_kshadow<4>(s).blocks
-         : (!physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_kshadow<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_kshadow<1>(s).blocks;
 }
 
@@ -6458,7 +6455,6 @@ static int __PSRun_kshadow(const struct __PSStencil_kshadow &s, hipStream_t stre
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_kshadow<4>(s, stream, red)
-         : (!physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_kshadow<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_kshadow<1>(s, stream, red);
 }
 

@@ -568,3 +568,21 @@ def test_prologue_loads_are_batched_where_that_pays():
         kernel = kernel[:kernel.index("__syncthreads();")]
         assert ("_pro[k].Load(" in kernel) == batched
         assert ("_st[0].Store(" in kernel) != batched
+
+
+def test_ragged_form_only_where_it_can_pay():
+    """Maps of 8-byte grids, and maps reading a grid through bounds-checked
+    gets, run ragged rows at one point per lane."""
+    for name, launch, ragged in (("mixed7.c", "__PSLaunch_mixed7", False),
+                                 ("udt7.c", "__PSLaunch_udt7_kernel", True),
+                                 ("ragged.c", "__PSLaunch_corners", True),
+                                 ("ragged.c", "__PSLaunch_corners_double",
+                                  False)):
+        src = [f for f in SOURCES if os.path.basename(f) == name][0]
+        rc, code, err = translate(src)
+        assert rc == 0, err
+        forms = set(re.findall(launch + r"\w*<([^>]*)>\(s, stream", code)) \
+            if name == "mixed7.c" else \
+            set(re.findall(launch + r"<([^>]*)>\(s, stream", code))
+        assert forms == {"4", "1"} | ({"4 + physis_hip::kRagged"} if ragged
+                                      else set()), (name, forms)
