@@ -135,7 +135,8 @@ __device__ __forceinline__ void LoadTile(E *lds, const E *p, const int *dim,
 // diffusion, small tile / mid tile): 64^3 1.94 / 2.51, 80^3 2.75 / 2.63, 96^3
 // 4.53 / 3.85, 128^3 7.97 / 6.49.  A kernel with the 12 centre-only
 // grids of the 19-point Jacobi sweep gains nothing (its tiles read the halo's
-// values of every one of them: 96^3 14.4 against 10.1).
+// values of every one of them: 96^3 14.4 against 10.1), nor does one of 27 points
+// (their halo's arithmetic: 256x60x60 9.5 against 8.4).
 template <int T> using SmallTile = Tile<T, 16, 8, 8, 1024>;
 template <int T> using MidTile = Tile<T, 16, 16, 8, 1024>;
 // Whether a pass over a whole grid runs in tiles: both kinds of pass cost by
@@ -169,9 +170,13 @@ inline double PaddedMega(long ex, long ey, long ez, int tx, int ty, int tz) {
 // 41x700x700 47 and 73, 41x1000x1000 87 and 133; red-black iteration 54x292x284
 // 27 and 30); tiles beat them as long as the sweeps' latency counts (1.4 + 2.5
 // per million padded points against 6 + 1.5: 41x300x300 13 and 15, 33x500x500
-// 31 and 29).
-inline bool PassesPay(const int *dim, bool periodic) {
-  if (dim[0] % 4 == 0 || dim[0] > 64) return true;
+// 31 and 29).  A kernel of many gets (`tiles` false) has no tiles and pays for
+// every lane: its passes have to cover the rows with no more of them.
+inline bool PassesPay(const int *dim, bool periodic, bool tiles) {
+  if (dim[0] % 4 == 0) return true;
+  const int wide = PairVX(dim[0], periodic) == 2 ? 128 : 256;
+  if (!tiles) return (dim[0] + wide - 1) / wide * wide <= (dim[0] + 63) / 64 * 64;
+  if (dim[0] > 64) return true;
   return TilesBeatPairs(dim, periodic) &&
          2.5 * PaddedMega(dim[0], dim[1], dim[2], 16, 16, 8) <
              4.6 + 1.5 * PaddedMega(dim[0], dim[1], dim[2], 64, 1, 1);
@@ -230,14 +235,19 @@ inline bool TilesBeatDomainPairs(const __PSDomain &d, int64_t points) {
 // of 64 there.  Us a sweep, single and pair, 5-point map over the interior:
 // 41x300x300 12 and 27, 41x1000x1000 80 and 274, 97x300x300 23 and 29,
 // 129x400x400 48 and 57, 290x200x200 30 and 30, 257x200x200 and 161x300x300
-// faster as pairs; tiles as above.
-inline bool DomainPassesPay(const __PSDomain &d, int nx, int64_t points) {
+// faster as pairs; tiles as above.  27 points (`tiles` false), 4 pairs: 191x256x200
+// 241 and 263 us, 321x256x200 400 and 471, 222x60x60 61 and 65, 255x256x200
+// faster as pairs.
+inline bool DomainPassesPay(const __PSDomain &d, int nx, int64_t points,
+                            bool use_tiles) {
   if (nx % 4 == 0) return true;
   long e[3];
   for (int i = 0; i < 3; ++i) e[i] = d.local_max[i] - d.local_min[i];
   const auto tiles = [&](int t) {
     return (d.local_max[0] + t - 1) / t - d.local_min[0] / t;
   };
+  if (!use_tiles)
+    return tiles(256) * 4 <= tiles(64) && e[0] * e[1] * e[2] >= 2000000;
   if (TilesBeatDomainPairs(d, points))
     return 2.5 * PaddedMega(e[0], e[1], e[2], 16, 16, 8) <
            1.6 + 1.5 * tiles(64) * 64e-6 * e[1] * e[2];

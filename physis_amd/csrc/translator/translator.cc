@@ -2525,7 +2525,8 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
       << "  for (int d = 0; d < 3; ++d)\n"
          "    if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||\n"
          "        s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;\n"
-      << "  if (!physis_hip::PassesPay(a->dim, false)) return false;\n"
+      << "  if (!physis_hip::PassesPay(a->dim, false, "
+      << (UsesTiles(k) ? "true" : "false") << ")) return false;\n"
       << "  return physis_hip::WindowsFit({a}, 3) &&\n"
          "         physis_hip::HaveScratch((size_t)a->num_elms * sizeof(" << T
       << "), false);\n}\n\n";
@@ -2549,7 +2550,8 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
   for (auto &a : sa)
     o << "  if (__builtin_memcmp(&s0." << a << ", &s1." << a << ", sizeof(s0." << a
       << "))) return false;\n";
-  o << "  if (!physis_hip::PassesPay(a->dim, " << per << ")) return false;\n";
+  o << "  if (!physis_hip::PassesPay(a->dim, " << per << ", "
+    << (UsesTiles(k) ? "true" : "false") << ")) return false;\n";
   o << "  return physis_hip::WindowsFit({a}, 3);\n}\n\n";
   return o.str();
 }
@@ -2696,7 +2698,10 @@ std::string Translator::EmitLauncher(const KernelInfo &k) {
       one_point = one_point || g.elem == "double" || g.elem == "long" ||
                   (g.read && (g.irregular || (g.mode != GridParam::kStaged &&
                                               g.mode != GridParam::kDirect)));
-      periodic = periodic || (g.mode == GridParam::kStaged && g.periodic);
+      // (the windows of periodic planes count beside few gets only: 27 points
+      // over 257x400x300 as for clamped ones, 119 us at one point and 127)
+      periodic = periodic || (g.mode == GridParam::kStaged && g.periodic &&
+                              g.offsets.size() <= 9);
     }
     if (!one_point)
       add(rconds, "!physis_hip::OnePointRows(" + D + ", " +
@@ -3242,8 +3247,8 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
     o << "  if ((s0.__reduce_out == NULL) != (s1.__reduce_out == NULL) ||\n"
          "      (s0.__reduce_out && s0.__reduce_op != s1.__reduce_op)) return false;\n";
   if (kVX == 4)
-    o << "  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) "
-         "return false;\n";
+    o << "  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms, "
+      << (UsesTiles(k) ? "true" : "false") << ")) return false;\n";
   o << "  return physis_hip::WindowsFit({" << Join(wgrids0, ", ") << "}, 3);\n}\n\n";
   return o.str();
 }
@@ -3251,14 +3256,15 @@ std::string Translator::EmitFusedDomainKernel(const KernelInfo &k) {
 // Resident-tile passes of a fusable kernel (include/physis/hip/tile.h): T
 // sweeps of a map pair (or T / 2 red-black iterations) per launch for grids
 // too small to keep the z-marching passes busy, when the kernel has few
-// centre-only grids (UsesTiles).  The values of points
+// centre-only grids and gets (UsesTiles).  The values of points
 // outside a map's domain alternate as the sweeps of the pair leave them: the
 // loaded grid's own after even sweeps (they stay in its LDS buffer), the other
 // grid's after odd ones.
 bool Translator::UsesTiles(const KernelInfo &k) {
   int direct = 0;
   for (auto &g : k.grids) direct += g.mode == GridParam::kDirect && g.read;
-  return (k.fusable || k.fuse_rb) && !k.rows2d && direct <= 4;
+  return (k.fusable || k.fuse_rb) && !k.rows2d && direct <= 4 &&
+         k.grids[k.fuse_in].offsets.size() <= 9;
 }
 
 std::string Translator::EmitTileKernel(const KernelInfo &k) {

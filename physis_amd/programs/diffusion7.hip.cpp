@@ -441,7 +441,7 @@ static bool __PSFusable2_diffusion7_kernel(const struct __PSStencil_diffusion7_k
   if (__builtin_memcmp(&s0.ct, &s1.ct, sizeof(s0.ct))) return false;
   if (__builtin_memcmp(&s0.cb, &s1.cb, sizeof(s0.cb))) return false;
   if (__builtin_memcmp(&s0.cc, &s1.cc, sizeof(s0.cc))) return false;
-  if (!physis_hip::PassesPay(a->dim, false)) return false;
+  if (!physis_hip::PassesPay(a->dim, false, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -908,7 +908,7 @@ static bool __PSFusable2_diffusion7_periodic_kernel(const struct __PSStencil_dif
   if (__builtin_memcmp(&s0.ct, &s1.ct, sizeof(s0.ct))) return false;
   if (__builtin_memcmp(&s0.cb, &s1.cb, sizeof(s0.cb))) return false;
   if (__builtin_memcmp(&s0.cc, &s1.cc, sizeof(s0.cc))) return false;
-  if (!physis_hip::PassesPay(a->dim, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, true, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 

@@ -425,7 +425,7 @@ static bool __PSFusableRB_redblack7_kernel(const struct __PSStencil_redblack7_ke
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
-  if (!physis_hip::PassesPay(a->dim, false)) return false;
+  if (!physis_hip::PassesPay(a->dim, false, true)) return false;
   return physis_hip::WindowsFit({a}, 3) &&
          physis_hip::HaveScratch((size_t)a->num_elms * sizeof(float), false);
 }

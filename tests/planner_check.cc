@@ -75,9 +75,10 @@ int main(int argc, char **argv) {
       dom.local_min[d] = 1;
       dom.local_max[d] = dim[d] - 1;
     }
-    std::printf("%d %d %d\n", physis_hip::PassesPay(dim, std::atoi(argv[5]) != 0),
+    std::printf("%d %d %d\n", physis_hip::PassesPay(dim, false, std::atoi(argv[5]) != 0),
                 physis_hip::DomainPassesPay(dom, dim[0],
-                                            (int64_t)dim[0] * dim[1] * dim[2]),
+                                            (int64_t)dim[0] * dim[1] * dim[2],
+                                            std::atoi(argv[5]) != 0),
                 physis_hip::RedBlackLastAsSweeps(dim, 1));
     return 0;
   }

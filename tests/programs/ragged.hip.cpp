@@ -424,7 +424,7 @@ static bool __PSFusable2_corners(const struct __PSStencil_corners &s0, const str
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
-  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) return false;
+  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms, true)) return false;
   return physis_hip::WindowsFit({a, b}, 3);
 }
 
@@ -1575,7 +1575,7 @@ static bool __PSFusable2_inner(const struct __PSStencil_inner &s0, const struct 
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
-  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) return false;
+  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms, true)) return false;
   return physis_hip::WindowsFit({a, b}, 3);
 }
 
@@ -2160,7 +2160,7 @@ static bool __PSFusable2_settle(const struct __PSStencil_settle &s0, const struc
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
   if ((s0.__reduce_out == NULL) != (s1.__reduce_out == NULL) ||
       (s0.__reduce_out && s0.__reduce_op != s1.__reduce_op)) return false;
-  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) return false;
+  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms, true)) return false;
   return physis_hip::WindowsFit({a, b, s0.c}, 3);
 }
 
@@ -2751,7 +2751,7 @@ static bool __PSFusable2_settle_square(const struct __PSStencil_settle_square &s
   if (__builtin_memcmp(&s0.w, &s1.w, sizeof(s0.w))) return false;
   if ((s0.__reduce_out == NULL) != (s1.__reduce_out == NULL) ||
       (s0.__reduce_out && s0.__reduce_op != s1.__reduce_op)) return false;
-  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) return false;
+  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms, true)) return false;
   return physis_hip::WindowsFit({a, b}, 3);
 }
 

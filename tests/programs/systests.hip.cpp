@@ -419,7 +419,7 @@ static bool __PSFusable2_k7(const struct __PSStencil_k7 &s0, const struct __PSSt
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
-  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) return false;
+  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms, true)) return false;
   return physis_hip::WindowsFit({a, b}, 3);
 }
 
@@ -884,7 +884,7 @@ static bool __PSFusable2_k7p(const struct __PSStencil_k7p &s0, const struct __PS
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  if (!physis_hip::PassesPay(a->dim, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, true, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -1387,7 +1387,7 @@ static bool __PSFusable2_k7n(const struct __PSStencil_k7n &s0, const struct __PS
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  if (!physis_hip::PassesPay(a->dim, false)) return false;
+  if (!physis_hip::PassesPay(a->dim, false, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -2318,125 +2318,8 @@ static bool __PSFusable2_k27(const struct __PSStencil_k27 &s0, const struct __PS
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
   }
-  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms)) return false;
+  if (!physis_hip::DomainPassesPay(s0.dom, a->dim[0], a->num_elms, false)) return false;
   return physis_hip::WindowsFit({a, b}, 3);
-}
-
-// Resident-tile pass of k27: TILE::T sweeps of src per launch into dst,
-// the one before the last into bg when store_mid.  red: per-block partials of
-// each sweep.
-template <typename TILE, int RED>
-__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_k27(
-    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
-  __shared__ float lds[2][TILE::kElems];
-  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
-  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
-  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
-  b /= tiles_x;
-  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
-  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
-  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
-  const int n = nxy * src.dim[2];
-  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
-  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
-  physis_hip::TilePoint pt[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
-  float bg_c[K][1];
-  bool in[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const physis_hip::TilePoint &p = pt[k];
-    in[k] = p.at >= 0 && p.x >= dom.local_min[0] && p.x < dom.local_max[0] &&
-            p.y >= dom.local_min[1] && p.y < dom.local_max[1] &&
-            p.z >= dom.local_min[2] && p.z < dom.local_max[2];
-    const bool grid = p.at >= 0 && p.x >= 0 && p.x < nx && p.y >= 0 &&
-                      p.y < src.dim[1] && p.z >= 0 && p.z < src.dim[2];
-    const int off = p.x + nx * p.y + nxy * p.z;
-    bw.template Load<1>(grid && !in[k] ? off : physis_hip::kDrop, bg_c[k]);
-  }
-  physis_hip::LoadTile<TILE, false>(lds[0], src.p, src.dim, x0, y0, z0);
-  __syncthreads();
-  __PSCtx_k27 ctx;
-  ctx.g_p = src.p;
-  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
-  ctx.g2_p = dst.p;
-  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = dst.dim[d];
-#pragma unroll
-  for (int t = 1; t <= TILE::T; ++t) {
-    const float *const cur = lds[(t - 1) & 1];
-    float *const nxt = lds[t & 1];
-#pragma unroll
-    for (int k = 0; k < TILE::Count(t); ++k) {
-      const physis_hip::TilePoint &p = pt[k];
-      if (p.at < 0) continue;
-      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (-1))];
-      ctx.g[1] = cur[p.at + 1 + RX * (0 + RY * (-1))];
-      ctx.g[2] = cur[p.at + -1 + RX * (0 + RY * (-1))];
-      ctx.g[3] = cur[p.at + 0 + RX * (1 + RY * (-1))];
-      ctx.g[4] = cur[p.at + 1 + RX * (1 + RY * (-1))];
-      ctx.g[5] = cur[p.at + -1 + RX * (1 + RY * (-1))];
-      ctx.g[6] = cur[p.at + 0 + RX * (-1 + RY * (-1))];
-      ctx.g[7] = cur[p.at + 1 + RX * (-1 + RY * (-1))];
-      ctx.g[8] = cur[p.at + -1 + RX * (-1 + RY * (-1))];
-      ctx.g[9] = cur[p.at + 0 + RX * (0 + RY * (0))];
-      ctx.g[10] = cur[p.at + 1 + RX * (0 + RY * (0))];
-      ctx.g[11] = cur[p.at + -1 + RX * (0 + RY * (0))];
-      ctx.g[12] = cur[p.at + 0 + RX * (1 + RY * (0))];
-      ctx.g[13] = cur[p.at + 1 + RX * (1 + RY * (0))];
-      ctx.g[14] = cur[p.at + -1 + RX * (1 + RY * (0))];
-      ctx.g[15] = cur[p.at + 0 + RX * (-1 + RY * (0))];
-      ctx.g[16] = cur[p.at + 1 + RX * (-1 + RY * (0))];
-      ctx.g[17] = cur[p.at + -1 + RX * (-1 + RY * (0))];
-      ctx.g[18] = cur[p.at + 0 + RX * (0 + RY * (1))];
-      ctx.g[19] = cur[p.at + 1 + RX * (0 + RY * (1))];
-      ctx.g[20] = cur[p.at + -1 + RX * (0 + RY * (1))];
-      ctx.g[21] = cur[p.at + 0 + RX * (1 + RY * (1))];
-      ctx.g[22] = cur[p.at + 1 + RX * (1 + RY * (1))];
-      ctx.g[23] = cur[p.at + -1 + RX * (1 + RY * (1))];
-      ctx.g[24] = cur[p.at + 0 + RX * (-1 + RY * (1))];
-      ctx.g[25] = cur[p.at + 1 + RX * (-1 + RY * (1))];
-      ctx.g[26] = cur[p.at + -1 + RX * (-1 + RY * (1))];
-      ctx.g2_e = false;
-      k27(p.x, p.y, p.z, ctx);
-      const int off = p.x + nx * p.y + nxy * p.z;
-      const bool keep = in[k];
-      const float v[1] = {ctx.g2_v};
-      if (t < TILE::T) {
-        if (keep)
-          nxt[p.at] = v[0];
-        else if (t == 1)
-          nxt[p.at] = bg_c[k][0];
-      }
-      if (k < TILE::Owned(0)) {
-        if (t == TILE::T)
-          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
-        if (t == TILE::T - 1 && store_mid)
-          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
-      }
-    }
-    if (t < TILE::T) __syncthreads();
-  }
-  (void)red;
-}
-
-template <typename TILE>
-static void __PSLaunchTile_k27(const struct __PSStencil_k27 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
-  const __PSDomain d = s.dom;
-  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
-  if (g.blocks == 0) return;
-  {
-      hipLaunchKernelGGL((__PSStencilRunT_k27<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
-  }
-}
-
-template <int T>
-static void __PSLaunchT_k27(const struct __PSStencil_k27 &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
-  if (physis_hip::InSmallTiles(s.dom))
-    __PSLaunchTile_k27<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
-  else
-    __PSLaunchTile_k27<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
 }
 
 // ---------------------------------------------- stencil k27p
@@ -2631,7 +2514,7 @@ static int __PSLaunch_k27p(const struct __PSStencil_k27p &s, hipStream_t stream,
 
 static int __PSBlocks_k27p(const struct __PSStencil_k27p &s) {
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSShape_k27p<4>(s).blocks
-         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSShape_k27p<4 + physis_hip::kRagged>(s).blocks
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSShape_k27p<4 + physis_hip::kRagged>(s).blocks
          : __PSShape_k27p<1>(s).blocks;
 }
 
@@ -2640,7 +2523,7 @@ static int __PSRun_k27p(const struct __PSStencil_k27p &s, hipStream_t stream, vo
   physis_hip::CheckGrid3D(s.g2, PS_FLOAT);
   physis_hip::CheckEmitDomain(s.dom, s.g2);
   return (s.g->dim[0] % 4 == 0 && s.g2->dim[0] % 4 == 0) ? __PSLaunch_k27p<4>(s, stream, red)
-         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, true, false)) ? __PSLaunch_k27p<4 + physis_hip::kRagged>(s, stream, red)
+         : (s.dom.local_max[0] <= s.g->dim[0] && !physis_hip::OnePointRows(s.dom, false, false)) ? __PSLaunch_k27p<4 + physis_hip::kRagged>(s, stream, red)
          : __PSLaunch_k27p<1>(s, stream, red);
 }
 
@@ -2906,107 +2789,8 @@ static bool __PSFusable2_k27p(const struct __PSStencil_k27p &s0, const struct __
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  if (!physis_hip::PassesPay(a->dim, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, true, false)) return false;
   return physis_hip::WindowsFit({a}, 3);
-}
-
-// Resident-tile pass of k27p: TILE::T sweeps of src per launch into dst,
-// the one before the last into bg when store_mid.  red: per-block partials of
-// each sweep.
-template <typename TILE, int RED>
-__global__ __launch_bounds__(TILE::NT) void __PSStencilRunT_k27p(
-    __PSDomain dom, __PSGrid3DFloat_dev src, __PSGrid3DFloat_dev dst, float *__restrict__ bg, int store_mid, int tiles_x, int tiles_y, physis_hip::TileReds red) {
-  __shared__ float lds[2][TILE::kElems];
-  constexpr int K = TILE::K, RX = TILE::RX, RY = TILE::RY;
-  int b = physis_hip::XcdLogicalBlock(blockIdx.x, gridDim.x);
-  const int x0 = dom.local_min[0] + (b % tiles_x) * TILE::TX;
-  b /= tiles_x;
-  const int y0 = dom.local_min[1] + (b % tiles_y) * TILE::TY;
-  const int z0 = dom.local_min[2] + (b / tiles_y) * TILE::TZ;
-  const int nx = src.dim[0], nxy = src.dim[0] * src.dim[1];
-  const int n = nxy * src.dim[2];
-  const physis_hip::BufWin<float> dw = physis_hip::BufWin<float>::Make(dst.p, n, 0, n);
-  const physis_hip::BufWin<float> bw = physis_hip::BufWin<float>::Make(bg ? bg : dst.p, n, 0, n);
-  physis_hip::TilePoint pt[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-    pt[k] = physis_hip::OwnedPoint<TILE>(k, x0, y0, z0);
-  physis_hip::LoadTile<TILE, true>(lds[0], src.p, src.dim, x0, y0, z0);
-  __syncthreads();
-  __PSCtx_k27p ctx;
-  ctx.g_p = src.p;
-  for (int d = 0; d < 3; ++d) ctx.g_dim[d] = src.dim[d];
-  ctx.g2_p = dst.p;
-  for (int d = 0; d < 3; ++d) ctx.g2_dim[d] = src.dim[d];
-#pragma unroll
-  for (int t = 1; t <= TILE::T; ++t) {
-    const float *const cur = lds[(t - 1) & 1];
-    float *const nxt = lds[t & 1];
-#pragma unroll
-    for (int k = 0; k < TILE::Count(t); ++k) {
-      const physis_hip::TilePoint &p = pt[k];
-      if (p.at < 0) continue;
-      ctx.g[0] = cur[p.at + 0 + RX * (0 + RY * (-1))];
-      ctx.g[1] = cur[p.at + 1 + RX * (0 + RY * (-1))];
-      ctx.g[2] = cur[p.at + -1 + RX * (0 + RY * (-1))];
-      ctx.g[3] = cur[p.at + 0 + RX * (1 + RY * (-1))];
-      ctx.g[4] = cur[p.at + 1 + RX * (1 + RY * (-1))];
-      ctx.g[5] = cur[p.at + -1 + RX * (1 + RY * (-1))];
-      ctx.g[6] = cur[p.at + 0 + RX * (-1 + RY * (-1))];
-      ctx.g[7] = cur[p.at + 1 + RX * (-1 + RY * (-1))];
-      ctx.g[8] = cur[p.at + -1 + RX * (-1 + RY * (-1))];
-      ctx.g[9] = cur[p.at + 0 + RX * (0 + RY * (0))];
-      ctx.g[10] = cur[p.at + 1 + RX * (0 + RY * (0))];
-      ctx.g[11] = cur[p.at + -1 + RX * (0 + RY * (0))];
-      ctx.g[12] = cur[p.at + 0 + RX * (1 + RY * (0))];
-      ctx.g[13] = cur[p.at + 1 + RX * (1 + RY * (0))];
-      ctx.g[14] = cur[p.at + -1 + RX * (1 + RY * (0))];
-      ctx.g[15] = cur[p.at + 0 + RX * (-1 + RY * (0))];
-      ctx.g[16] = cur[p.at + 1 + RX * (-1 + RY * (0))];
-      ctx.g[17] = cur[p.at + -1 + RX * (-1 + RY * (0))];
-      ctx.g[18] = cur[p.at + 0 + RX * (0 + RY * (1))];
-      ctx.g[19] = cur[p.at + 1 + RX * (0 + RY * (1))];
-      ctx.g[20] = cur[p.at + -1 + RX * (0 + RY * (1))];
-      ctx.g[21] = cur[p.at + 0 + RX * (1 + RY * (1))];
-      ctx.g[22] = cur[p.at + 1 + RX * (1 + RY * (1))];
-      ctx.g[23] = cur[p.at + -1 + RX * (1 + RY * (1))];
-      ctx.g[24] = cur[p.at + 0 + RX * (-1 + RY * (1))];
-      ctx.g[25] = cur[p.at + 1 + RX * (-1 + RY * (1))];
-      ctx.g[26] = cur[p.at + -1 + RX * (-1 + RY * (1))];
-      ctx.g2_e = false;
-      k27p(p.x, p.y, p.z, ctx);
-      const int off = p.x + nx * p.y + nxy * p.z;
-      const float v[1] = {ctx.g2_v};
-      if (t < TILE::T) nxt[p.at] = v[0];
-      const bool keep = p.x < nx && p.y < src.dim[1] && p.z < src.dim[2];
-      if (k < TILE::Owned(0)) {
-        if (t == TILE::T)
-          dw.template Store<1>(keep ? off : physis_hip::kDrop, v);
-        if (t == TILE::T - 1 && store_mid)
-          bw.template Store<1>(keep ? off : physis_hip::kDrop, v);
-      }
-    }
-    if (t < TILE::T) __syncthreads();
-  }
-  (void)red;
-}
-
-template <typename TILE>
-static void __PSLaunchTile_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
-  const __PSDomain d = s.dom;
-  const physis_hip::TileShape g = physis_hip::TileGrid<TILE>(d);
-  if (g.blocks == 0) return;
-  {
-      hipLaunchKernelGGL((__PSStencilRunT_k27p<TILE, -1>), dim3(g.blocks), dim3(TILE::NT), 0, stream, s.dom, src, dst, bg, store_mid, g.tiles_x, g.tiles_y, red);
-  }
-}
-
-template <int T>
-static void __PSLaunchT_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *bg, int store_mid, hipStream_t stream, const physis_hip::TileReds &red) {
-  if (physis_hip::InSmallTiles(s.dom))
-    __PSLaunchTile_k27p<physis_hip::SmallTile<T>>(s, src, dst, bg, store_mid, stream, red);
-  else
-    __PSLaunchTile_k27p<physis_hip::MidTile<T>>(s, src, dst, bg, store_mid, stream, red);
 }
 
 // ---------------------------------------------- stencil k27i
@@ -3889,7 +3673,7 @@ static bool __PSFusableRB_krb(const struct __PSStencil_krb &s0) {
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
-  if (!physis_hip::PassesPay(a->dim, false)) return false;
+  if (!physis_hip::PassesPay(a->dim, false, true)) return false;
   return physis_hip::WindowsFit({a}, 3) &&
          physis_hip::HaveScratch((size_t)a->num_elms * sizeof(float), false);
 }

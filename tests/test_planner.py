@@ -109,17 +109,20 @@ def test_points_per_lane_of_ragged_rows(planner, extents, periodic, colour, one)
 
 # Whole-grid and interior passes against single sweeps, which run in tiles of 64
 # points on rows that are no multiples of 4: the side measured faster
-# (include/physis/hip/tile.h).
-@pytest.mark.parametrize("extents,whole,interior", [
-    ((41, 100, 100), True, True), ((41, 300, 300), True, False),
-    ((41, 1000, 1000), False, False), ((33, 500, 500), False, False),
-    ((40, 1000, 1000), True, True), ((65, 500, 500), True, False),
-    ((97, 300, 300), True, False), ((129, 400, 400), True, False),
-    ((161, 300, 300), True, True), ((257, 200, 200), True, True),
-    ((321, 300, 200), True, True)])
-def test_passes_where_they_pay(planner, extents, whole, interior):
-    r = subprocess.run([planner, "pay", *map(str, extents), "0"], check=True,
-                       capture_output=True, text=True)
+# (include/physis/hip/tile.h); few: a kernel of few gets, which has tiles.
+@pytest.mark.parametrize("extents,whole,interior,few", [
+    ((41, 100, 100), True, True, 1), ((41, 300, 300), True, False, 1),
+    ((41, 1000, 1000), False, False, 1), ((33, 500, 500), False, False, 1),
+    ((40, 1000, 1000), True, True, 1), ((65, 500, 500), True, False, 1),
+    ((97, 300, 300), True, False, 1), ((129, 400, 400), True, False, 1),
+    ((161, 300, 300), True, True, 1), ((257, 200, 200), True, True, 1),
+    ((321, 300, 200), True, True, 1),
+    ((37, 256, 200), False, False, 0), ((191, 256, 200), False, False, 0),
+    ((255, 256, 200), True, True, 0), ((256, 60, 60), True, True, 0),
+    ((321, 256, 200), True, False, 0)])
+def test_passes_where_they_pay(planner, extents, whole, interior, few):
+    r = subprocess.run([planner, "pay", *map(str, extents), str(few)],
+                       check=True, capture_output=True, text=True)
     assert [int(v) for v in r.stdout.split()][:2] == [whole, interior]
 
 
