@@ -214,18 +214,23 @@ inline bool OnePointRows(const __PSDomain &d, bool periodic, bool colour) {
 
 // Points per lane (4 or 2) of a whole-grid two-sweep pass over rows of nx
 // points: tiles of 256 points, or of 128 where those pad the rows so much
-// less that they win although a point costs 1.2 times as much in them (its
-// row's loads, addresses and masks are shared by half as many points).
-// us a sweep at 4 and 2 points, clamped 7-point map: 256^3 19.4 and 23.3,
-// 257^3 38.6 and 31.5, 384^3 74.2 and 66.6, 512^3 116 and 145; red-black
-// iteration: 256^3 39.1 and 44.9, 257^3 73.2 and 62.1, 384^3 147 and 130.
-// Periodic planes are loaded through a window of their own each, twice as
-// often per point in the narrow tiles: a point costs 1.2 to 1.36 times as much
-// (181x163x137 10.2 and 12.5, 321x190x157 20.9 and 21.4).
-inline int PairVX(int nx, bool periodic) {
-  const long wide = (nx + 255) / 256 * 256L, narrow = (nx + 127) / 128 * 128L;
-  return periodic ? (narrow * 7 < wide * 5 ? 2 : 4)
-                  : (narrow * 5 < wide * 4 ? 2 : 4);
+// less that they win although a point costs more in them (its row's loads,
+// addresses and masks are shared by half as many points; periodic planes are
+// loaded through a window of their own each), and more the fewer planes a block
+// has.  us a sweep at 4 and 2 points, clamped 7-point map: 128x100x100 6.4 and
+// 5.9, 128x256x256 19.0 and 13.5; 384x60x60 5.7 and 6.1, 368x200x150 18.0 and
+// 18.9, 301x256x256 34.3 and 32.7, 384^3 74 and 67.  Periodic: 128x100x100 7.1 and
+// 7.6, 100x128x128 7.7 and 7.4, 128x256x256 19.8 and 15.1, 321x190x157 20.9 and
+// 21.4.  Red-black iteration: 128x164x65 11.4 and 11.8, 100x128x128 13.0 and 12.2,
+// 128x256x256 35 and 26; 384x60x60 10.0 and 12.1, 368x200x200 43 and 45,
+// 301x256x256 63 and 64, 384^3 147 and 130.
+inline int PairVX(const int *dim, bool periodic, bool colours) {
+  const long wide = (dim[0] + 255) / 256 * 256L, narrow = (dim[0] + 127) / 128 * 128L;
+  const double n = (double)dim[0] * dim[1] * dim[2];
+  if (narrow * 2 == wide)
+    return n >= (periodic || colours ? 1.5e6 : 0.0) ? 2 : 4;
+  if (periodic || narrow * 5 >= wide * 4) return 4;
+  return n >= (colours ? 3e7 : 1.6e7) ? 2 : 4;
 }
 
 // A 3-D grid argument must be live, of the stencil's element type, and small

@@ -139,23 +139,30 @@ __device__ __forceinline__ void LoadTile(E *lds, const E *p, const int *dim,
 // (their halo's arithmetic: 256x60x60 9.5 against 8.4).
 template <int T> using SmallTile = Tile<T, 16, 8, 8, 1024>;
 template <int T> using MidTile = Tile<T, 16, 16, 8, 1024>;
-// Whether a pass over a whole grid runs in tiles: both kinds of pass cost by
-// the points of their padded tiles, us a sweep about 1.4 + 2.5 per million
-// points here and 4.3 + 1 in a z-marching pair (0.83 at four points per
-// lane), so that the line follows the width as much as the size.  Tiles and
-// pairs, clamped 7-point map (red-black iterations cost twice as much and
-// fall on the same sides): 112^3 5.2 and 6.3, 128^3 6.4 and 6.0, 150^3 11.3
-// and 9.3, 250x80x80 6.5 and 5.7, 250x64x64 4.0 and 4.9, 64x256x256 11.4 and
-// 11.9, 100x180x180 11.3 and 8.6, 16x400x400 8.1 and 22.7, 48x300x300 12.5
-// and 15.3.  Past 16 million points (a grid of 64 MB) nothing was measured,
-// and the tiles' halos no longer come from the cache.
-inline bool TilesBeatPairs(const int *dim, bool periodic) {
-  const auto up = [](double n, int t) { return (double)(((long)n + t - 1) / t * t); };
-  const bool narrow = PairVX(dim[0], periodic) == 2;
-  const double tile = up(dim[0], 16) * up(dim[1], 16) * up(dim[2], 8) * 1e-6;
-  const double pair = (narrow ? up(dim[0], 128) : up(dim[0], 256) * 0.83) *
-                      up(dim[1], 8) * dim[2] * 1e-6;
-  return tile <= 16 && 2.5 * tile - pair < 2.2;
+// Whether a pass over a whole grid runs in tiles, from what a sweep costs in
+// either kind of pass (us): 1.5 + 1.2 per round of mid tiles (a block per CU; 23
+// to 24 for 18 rounds), and for z-marching pairs the lines below by the million
+// points of their padded tiles, fitted to 130 grids where the kinds lie close:
+// the rule's choice is 0.5 % slower than the better one in the mean, and 11 % at
+// most (red-black 112x230x33; clamped 180x191x27 7 %).  Tiles and pairs, clamped
+// 7-point map: 112^3 5.2 and 6.3, 128^3 6.4 and 6.0, 150^3 11.3 and 9.3, 250x80x80
+// 6.5 and 5.7, 250x64x64 4.0 and 4.9, 64x256x256 11.4 and 11.9, 80x137x356 11.3
+// and 10.7, 16x400x400 8.1 and 22.7, 48x300x300 12.5 and 15.3, 100x68x124 5.0 and
+// 5.7, 180x110x96 6.6 and 6.0, 148x124x87 6.5 and 6.2 (periodic 6.4 and 6.8,
+// red-black 6.4 and 5.6).  Past 16 million points (a grid of 64 MB) nothing was
+// measured, and the tiles' halos no longer come from the cache.
+inline bool TilesBeatPairs(const int *dim, bool periodic, bool colours) {
+  constexpr long kCUs = 256;
+  const auto in = [](long n, long t) { return (n + t - 1) / t; };
+  const long blocks = in(dim[0], 16) * in(dim[1], 16) * in(dim[2], 8);
+  if (blocks > 16000000 / 2048) return false;
+  const bool narrow = PairVX(dim, periodic, colours) == 2;
+  const int tx = narrow ? 128 : 256;
+  const double points = 1e-6 * in(dim[0], tx) * tx * in(dim[1], 8) * 8 * dim[2];
+  const double pair = colours    ? narrow ? 4.5 + 0.9 * points : 3.6 + 0.7 * points
+                      : periodic ? narrow ? 5.4 + 1.1 * points : 4.6 + 0.9 * points
+                      : narrow   ? 4.3 + 0.95 * points : 3.8 + 0.8 * points;
+  return 1.5 + 1.2 * in(blocks, kCUs) < pair;
 }
 
 // Padded points (millions) of an extent box in tiles of tx x ty x tz.
@@ -172,12 +179,12 @@ inline double PaddedMega(long ex, long ey, long ez, int tx, int ty, int tz) {
 // per million padded points against 6 + 1.5: 41x300x300 13 and 15, 33x500x500
 // 31 and 29).  A kernel of many gets (`tiles` false) has no tiles and pays for
 // every lane: its passes have to cover the rows with no more of them.
-inline bool PassesPay(const int *dim, bool periodic, bool tiles) {
+inline bool PassesPay(const int *dim, bool periodic, bool colours, bool tiles) {
   if (dim[0] % 4 == 0) return true;
-  const int wide = PairVX(dim[0], periodic) == 2 ? 128 : 256;
+  const int wide = PairVX(dim, periodic, colours) == 2 ? 128 : 256;
   if (!tiles) return (dim[0] + wide - 1) / wide * wide <= (dim[0] + 63) / 64 * 64;
   if (dim[0] > 64) return true;
-  return TilesBeatPairs(dim, periodic) &&
+  return TilesBeatPairs(dim, periodic, colours) &&
          2.5 * PaddedMega(dim[0], dim[1], dim[2], 16, 16, 8) <
              4.6 + 1.5 * PaddedMega(dim[0], dim[1], dim[2], 64, 1, 1);
 }
@@ -191,12 +198,12 @@ inline bool PassesPay(const int *dim, bool periodic, bool tiles) {
 // from 255^3 on.
 inline bool RedBlackLastAsSweeps(const int *dim, int iterations) {
   if (iterations % 2 == 0 || dim[0] % 4 == 0) return false;
-  const bool narrow = PairVX(dim[0], false) == 2;
+  const bool narrow = PairVX(dim, false, true) == 2;
   const double n = PaddedMega(dim[0], dim[1], dim[2], 1, 1, 1), mb = 4 * n;
   const double sweeps = 2 * (5.5 + 0.75 * n + 0.95 * PaddedMega(dim[0], dim[1],
                                                                  dim[2], 64, 1, 1));
   const double pass =
-      TilesBeatPairs(dim, false)
+      TilesBeatPairs(dim, false, true)
           ? 2 * (1.4 + 2.5 * PaddedMega(dim[0], dim[1], dim[2], 16, 16, 8))
           : 2 * (4.3 + (narrow ? 1.0 : 0.83) *
                            PaddedMega(dim[0], dim[1], dim[2], narrow ? 128 : 256, 8, 1));

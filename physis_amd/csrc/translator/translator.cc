@@ -2506,7 +2506,8 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
     << "static void __PSLaunch2_" << n << "(const struct __PSStencil_" << n
     << " &s, const " << V << " &src, const " << V << " &dst, " << T
     << " *mid, hipStream_t stream) {\n"
-    << "  if (physis_hip::PairVX(s." << I << "->dim[0], " << per << ") == 4)\n    __PSLaunch2V_"
+    << "  if (physis_hip::PairVX(s." << I << "->dim, " << per << ", "
+    << (rb ? "true" : "false") << ") == 4)\n    __PSLaunch2V_"
     << n << "<4>(s, src, dst, mid, stream);\n  else\n    __PSLaunch2V_" << n
     << "<2>(s, src, dst, mid, stream);\n}\n\n";
   // run-time check
@@ -2525,7 +2526,7 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
       << "  for (int d = 0; d < 3; ++d)\n"
          "    if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||\n"
          "        s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;\n"
-      << "  if (!physis_hip::PassesPay(a->dim, false, "
+      << "  if (!physis_hip::PassesPay(a->dim, false, true, "
       << (UsesTiles(k) ? "true" : "false") << ")) return false;\n"
       << "  return physis_hip::WindowsFit({a}, 3) &&\n"
          "         physis_hip::HaveScratch((size_t)a->num_elms * sizeof(" << T
@@ -2550,7 +2551,7 @@ std::string Translator::EmitFusedRunKernel(const KernelInfo &k) {
   for (auto &a : sa)
     o << "  if (__builtin_memcmp(&s0." << a << ", &s1." << a << ", sizeof(s0." << a
       << "))) return false;\n";
-  o << "  if (!physis_hip::PassesPay(a->dim, " << per << ", "
+  o << "  if (!physis_hip::PassesPay(a->dim, " << per << ", false, "
     << (UsesTiles(k) ? "true" : "false") << ")) return false;\n";
   o << "  return physis_hip::WindowsFit({a}, 3);\n}\n\n";
   return o.str();
@@ -2810,7 +2811,8 @@ std::string Translator::SmallExpr(const KernelInfo &k) {
   return k.fuse_domain ? "physis_hip::TilesBeatDomainPairs(s0.dom, s0." + g.name +
                              "->num_elms)"
                        : "physis_hip::TilesBeatPairs(s0." + g.name + "->dim, " +
-                             (g.periodic ? "true" : "false") + ")";
+                             (g.periodic ? "true" : "false") + ", " +
+                             (k.fuse_rb ? "true" : "false") + ")";
 }
 std::string Translator::PassesExpr(const KernelInfo &k) {
   if (!k.rows2d && !UsesTiles(k)) return "iter";

@@ -416,7 +416,7 @@ static void __PSLaunch2V_diffusion7_kernel(const struct __PSStencil_diffusion7_k
 }
 
 static void __PSLaunch2_diffusion7_kernel(const struct __PSStencil_diffusion7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g1->dim[0], false) == 4)
+  if (physis_hip::PairVX(s.g1->dim, false, false) == 4)
     __PSLaunch2V_diffusion7_kernel<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_diffusion7_kernel<2>(s, src, dst, mid, stream);
@@ -441,7 +441,7 @@ static bool __PSFusable2_diffusion7_kernel(const struct __PSStencil_diffusion7_k
   if (__builtin_memcmp(&s0.ct, &s1.ct, sizeof(s0.ct))) return false;
   if (__builtin_memcmp(&s0.cb, &s1.cb, sizeof(s0.cb))) return false;
   if (__builtin_memcmp(&s0.cc, &s1.cc, sizeof(s0.cc))) return false;
-  if (!physis_hip::PassesPay(a->dim, false, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, false, false, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -883,7 +883,7 @@ static void __PSLaunch2V_diffusion7_periodic_kernel(const struct __PSStencil_dif
 }
 
 static void __PSLaunch2_diffusion7_periodic_kernel(const struct __PSStencil_diffusion7_periodic_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g1->dim[0], true) == 4)
+  if (physis_hip::PairVX(s.g1->dim, true, false) == 4)
     __PSLaunch2V_diffusion7_periodic_kernel<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_diffusion7_periodic_kernel<2>(s, src, dst, mid, stream);
@@ -908,7 +908,7 @@ static bool __PSFusable2_diffusion7_periodic_kernel(const struct __PSStencil_dif
   if (__builtin_memcmp(&s0.ct, &s1.ct, sizeof(s0.ct))) return false;
   if (__builtin_memcmp(&s0.cb, &s1.cb, sizeof(s0.cb))) return false;
   if (__builtin_memcmp(&s0.cc, &s1.cc, sizeof(s0.cc))) return false;
-  if (!physis_hip::PassesPay(a->dim, true, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, true, false, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -1006,8 +1006,8 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_diffusion7_kernel s0, 
     const size_t bytes = (size_t)s0.g1->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim, false);
-    const int passes = !physis_hip::TilesBeatPairs(s0.g1->dim, false) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
+    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim, false, false);
+    const int passes = !physis_hip::TilesBeatPairs(s0.g1->dim, false, false) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {
       const __PSGrid3DFloat_dev dst = passes % 2 && j == 0 ? vb
@@ -1054,8 +1054,8 @@ static void __PSStencilRun_1(int iter, struct __PSStencil_diffusion7_periodic_ke
     const size_t bytes = (size_t)s0.g1->num_elms * sizeof(float);
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
-    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim, true);
-    const int passes = !physis_hip::TilesBeatPairs(s0.g1->dim, true) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
+    const bool __small = physis_hip::TilesBeatPairs(s0.g1->dim, true, false);
+    const int passes = !physis_hip::TilesBeatPairs(s0.g1->dim, true, false) ? iter : iter == 2 ? 2 : (iter + 1) / 2;
     __PSGrid3DFloat_dev src = va;
     for (int j = 0; j < passes; ++j) {
       const __PSGrid3DFloat_dev dst = passes % 2 && j == 0 ? vb

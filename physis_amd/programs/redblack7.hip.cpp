@@ -410,7 +410,7 @@ static void __PSLaunch2V_redblack7_kernel(const struct __PSStencil_redblack7_ker
 }
 
 static void __PSLaunch2_redblack7_kernel(const struct __PSStencil_redblack7_kernel &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g->dim[0], false) == 4)
+  if (physis_hip::PairVX(s.g->dim, false, true) == 4)
     __PSLaunch2V_redblack7_kernel<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_redblack7_kernel<2>(s, src, dst, mid, stream);
@@ -425,7 +425,7 @@ static bool __PSFusableRB_redblack7_kernel(const struct __PSStencil_redblack7_ke
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
-  if (!physis_hip::PassesPay(a->dim, false, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, false, true, true)) return false;
   return physis_hip::WindowsFit({a}, 3) &&
          physis_hip::HaveScratch((size_t)a->num_elms * sizeof(float), false);
 }
@@ -523,7 +523,7 @@ static void __PSStencilRun_0(int iter, struct __PSStencil_redblack7_kernel s0) {
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
-    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim, false);
+    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim, false, true);
     // (the last iteration may be left to the colour sweeps below)
     const int last = physis_hip::RedBlackLastAsSweeps(s0.g->dim, iter) ? 1 : 0;
     iter -= last;

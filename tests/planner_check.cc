@@ -2,10 +2,11 @@
 // prints, for each case, the z chunk and window bytes that PlanRunFor picks;
 // "tiles": whether pairs over a domain run in resident tiles
 // (include/physis/hip/tile.h); "fits": whether a pass has a window at all; "one":
-// whether a single sweep runs at one point per lane; "pay": whether passes over
-// a whole grid, and over its interior, beat single sweeps, and whether the last
-// of one red-black iteration runs as colour sweeps.  Built and run by tests/test_planner.py; no
-// device is touched.
+// whether a single sweep runs at one point per lane; "vx": the points per lane of
+// a whole-grid pass, and whether it runs in tiles; "pay": whether passes over a
+// whole grid, and over its interior, beat single sweeps, and whether the last of
+// one red-black iteration runs as colour sweeps.  Built and run by
+// tests/test_planner.py; no device is touched.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -67,6 +68,15 @@ int main(int argc, char **argv) {
                                                  std::atoi(argv[6]) != 0));
     return 0;
   }
+  if (argc == 7 && std::strcmp(argv[1], "vx") == 0) {
+    const int dim[3] = {std::atoi(argv[2]), std::atoi(argv[3]),
+                        std::atoi(argv[4])};
+    const bool periodic = std::atoi(argv[5]) != 0;
+    const bool colours = std::atoi(argv[6]) != 0;
+    std::printf("%d %d\n", physis_hip::PairVX(dim, periodic, colours),
+                physis_hip::TilesBeatPairs(dim, periodic, colours));
+    return 0;
+  }
   if (argc == 6 && std::strcmp(argv[1], "pay") == 0) {
     __PSDomain dom = {};
     int dim[3];
@@ -75,7 +85,7 @@ int main(int argc, char **argv) {
       dom.local_min[d] = 1;
       dom.local_max[d] = dim[d] - 1;
     }
-    std::printf("%d %d %d\n", physis_hip::PassesPay(dim, false, std::atoi(argv[5]) != 0),
+    std::printf("%d %d %d\n", physis_hip::PassesPay(dim, false, false, std::atoi(argv[5]) != 0),
                 physis_hip::DomainPassesPay(dom, dim[0],
                                             (int64_t)dim[0] * dim[1] * dim[2],
                                             std::atoi(argv[5]) != 0),

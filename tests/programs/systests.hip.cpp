@@ -866,7 +866,7 @@ static void __PSLaunch2V_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFl
 }
 
 static void __PSLaunch2_k7p(const struct __PSStencil_k7p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g->dim[0], true) == 4)
+  if (physis_hip::PairVX(s.g->dim, true, false) == 4)
     __PSLaunch2V_k7p<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_k7p<2>(s, src, dst, mid, stream);
@@ -884,7 +884,7 @@ static bool __PSFusable2_k7p(const struct __PSStencil_k7p &s0, const struct __PS
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  if (!physis_hip::PassesPay(a->dim, true, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, true, false, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -1369,7 +1369,7 @@ static void __PSLaunch2V_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFl
 }
 
 static void __PSLaunch2_k7n(const struct __PSStencil_k7n &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g1->dim[0], false) == 4)
+  if (physis_hip::PairVX(s.g1->dim, false, false) == 4)
     __PSLaunch2V_k7n<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_k7n<2>(s, src, dst, mid, stream);
@@ -1387,7 +1387,7 @@ static bool __PSFusable2_k7n(const struct __PSStencil_k7n &s0, const struct __PS
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  if (!physis_hip::PassesPay(a->dim, false, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, false, false, true)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -2771,7 +2771,7 @@ static void __PSLaunch2V_k27p(const struct __PSStencil_k27p &s, const __PSGrid3D
 }
 
 static void __PSLaunch2_k27p(const struct __PSStencil_k27p &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g->dim[0], true) == 4)
+  if (physis_hip::PairVX(s.g->dim, true, false) == 4)
     __PSLaunch2V_k27p<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_k27p<2>(s, src, dst, mid, stream);
@@ -2789,7 +2789,7 @@ static bool __PSFusable2_k27p(const struct __PSStencil_k27p &s0, const struct __
     if (s0.dom.local_min[d] != 0 || s0.dom.local_max[d] != a->dim[d]) return false;
     if (s1.dom.local_min[d] != 0 || s1.dom.local_max[d] != a->dim[d]) return false;
   }
-  if (!physis_hip::PassesPay(a->dim, true, false)) return false;
+  if (!physis_hip::PassesPay(a->dim, true, false, false)) return false;
   return physis_hip::WindowsFit({a}, 3);
 }
 
@@ -3658,7 +3658,7 @@ static void __PSLaunch2V_krb(const struct __PSStencil_krb &s, const __PSGrid3DFl
 }
 
 static void __PSLaunch2_krb(const struct __PSStencil_krb &s, const __PSGrid3DFloat_dev &src, const __PSGrid3DFloat_dev &dst, float *mid, hipStream_t stream) {
-  if (physis_hip::PairVX(s.g->dim[0], false) == 4)
+  if (physis_hip::PairVX(s.g->dim, false, true) == 4)
     __PSLaunch2V_krb<4>(s, src, dst, mid, stream);
   else
     __PSLaunch2V_krb<2>(s, src, dst, mid, stream);
@@ -3673,7 +3673,7 @@ static bool __PSFusableRB_krb(const struct __PSStencil_krb &s0) {
   for (int d = 0; d < 3; ++d)
     if (s0.dom.local_min[d] < 1 || s0.dom.local_max[d] > a->dim[d] - 1 ||
         s0.dom.local_min[d] >= s0.dom.local_max[d]) return false;
-  if (!physis_hip::PassesPay(a->dim, false, true)) return false;
+  if (!physis_hip::PassesPay(a->dim, false, true, true)) return false;
   return physis_hip::WindowsFit({a}, 3) &&
          physis_hip::HaveScratch((size_t)a->num_elms * sizeof(float), false);
 }
@@ -3969,7 +3969,7 @@ static void __PSStencilRun_10(int iter, struct __PSStencil_krb s0) {
     __PSGrid3DFloat_dev vt = va;
     vt.p = (float *)__PSHipScratch(8, bytes);
     __PSGrid3DFloat_dev src = va;
-    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim, false);
+    const bool __small = physis_hip::TilesBeatPairs(s0.g->dim, false, true);
     // (the last iteration may be left to the colour sweeps below)
     const int last = physis_hip::RedBlackLastAsSweeps(s0.g->dim, iter) ? 1 : 0;
     iter -= last;

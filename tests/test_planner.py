@@ -136,3 +136,40 @@ def test_last_red_black_iteration(planner, extents, sweeps):
     r = subprocess.run([planner, "pay", *map(str, extents), "0"], check=True,
                        capture_output=True, text=True)
     assert int(r.stdout.split()[2]) == sweeps
+
+
+# Whole-grid passes at 4 or 2 points per lane, and in tiles: the side measured
+# faster (include/physis/hip/run.h, tile.h).  Grids where the kinds of pass lie
+# within 5 % of each other are left out of the second list: the rule's cost model
+# is no finer than that.
+@pytest.mark.parametrize("extents,periodic,colours,vx", [
+    ((128, 100, 100), 0, 0, 2), ((128, 256, 256), 0, 0, 2),
+    ((384, 60, 60), 0, 0, 4), ((368, 200, 150), 0, 0, 4),
+    ((301, 256, 256), 0, 0, 2), ((384, 384, 384), 0, 0, 2),
+    ((256, 256, 256), 0, 0, 4), ((128, 100, 100), 1, 0, 4),
+    ((100, 128, 128), 1, 0, 2), ((321, 190, 157), 1, 0, 4),
+    ((128, 164, 65), 0, 1, 4), ((100, 128, 128), 0, 1, 2),
+    ((368, 200, 200), 0, 1, 4), ((384, 384, 384), 0, 1, 2)])
+def test_points_per_lane_of_passes(planner, extents, periodic, colours, vx):
+    r = subprocess.run([planner, "vx", *map(str, extents), str(periodic),
+                        str(colours)], check=True, capture_output=True,
+                       text=True)
+    assert int(r.stdout.split()[0]) == vx
+
+
+@pytest.mark.parametrize("extents,periodic,colours,tiles", [
+    ((112, 112, 112), 0, 0, True), ((100, 68, 124), 0, 0, True),
+    ((112, 56, 154), 0, 0, True), ((96, 24, 367), 0, 0, True),
+    ((128, 128, 128), 0, 0, False), ((150, 150, 150), 0, 0, False),
+    ((60, 254, 265), 1, 0, True), ((120, 36, 236), 1, 0, True),
+    ((148, 124, 87), 1, 0, True), ((148, 124, 87), 0, 1, False),
+    ((140, 140, 80), 1, 0, True), ((140, 140, 80), 0, 1, False),
+    ((180, 110, 96), 0, 0, False), ((80, 138, 181), 0, 1, True),
+    ((256, 88, 43), 0, 1, False),
+    ((256, 80, 80), 0, 0, False),
+    ((32, 300, 300), 0, 0, True), ((256, 256, 256), 0, 0, False)])
+def test_tiles_for_whole_grids(planner, extents, periodic, colours, tiles):
+    r = subprocess.run([planner, "vx", *map(str, extents), str(periodic),
+                        str(colours)], check=True, capture_output=True,
+                       text=True)
+    assert int(r.stdout.split()[1]) == tiles
