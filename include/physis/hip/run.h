@@ -223,14 +223,15 @@ inline bool OnePointRows(const __PSDomain &d, bool periodic, bool colour) {
 // 7.6, 100x128x128 7.7 and 7.4, 128x256x256 19.8 and 15.1, 321x190x157 20.9 and
 // 21.4.  Red-black iteration: 128x164x65 11.4 and 11.8, 100x128x128 13.0 and 12.2,
 // 128x256x256 35 and 26; 384x60x60 10.0 and 12.1, 368x200x200 43 and 45,
-// 301x256x256 63 and 64, 384^3 147 and 130.
+// 301x256x256 63 and 64, 375x256x256 65 and 67, 257x218x400 86 and 79,
+// 301x218x400 92 and 82, 384^3 147 and 130.
 inline int PairVX(const int *dim, bool periodic, bool colours) {
   const long wide = (dim[0] + 255) / 256 * 256L, narrow = (dim[0] + 127) / 128 * 128L;
   const double n = (double)dim[0] * dim[1] * dim[2];
   if (narrow * 2 == wide)
     return n >= (periodic || colours ? 1.5e6 : 0.0) ? 2 : 4;
   if (periodic || narrow * 5 >= wide * 4) return 4;
-  return n >= (colours ? 3e7 : 1.6e7) ? 2 : 4;
+  return n >= (colours ? 2e7 : 1.6e7) ? 2 : 4;
 }
 
 // A 3-D grid argument must be live, of the stencil's element type, and small

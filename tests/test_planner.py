@@ -149,7 +149,8 @@ def test_last_red_black_iteration(planner, extents, sweeps):
     ((256, 256, 256), 0, 0, 4), ((128, 100, 100), 1, 0, 4),
     ((100, 128, 128), 1, 0, 2), ((321, 190, 157), 1, 0, 4),
     ((128, 164, 65), 0, 1, 4), ((100, 128, 128), 0, 1, 2),
-    ((368, 200, 200), 0, 1, 4), ((384, 384, 384), 0, 1, 2)])
+    ((368, 200, 200), 0, 1, 4), ((301, 218, 400), 0, 1, 2),
+    ((320, 300, 300), 0, 1, 2), ((384, 384, 384), 0, 1, 2)])
 def test_points_per_lane_of_passes(planner, extents, periodic, colours, vx):
     r = subprocess.run([planner, "vx", *map(str, extents), str(periodic),
                         str(colours)], check=True, capture_output=True,
