@@ -177,13 +177,28 @@ inline double PaddedMega(long ex, long ey, long ez, int tx, int ty, int tz) {
 // 41x700x700 47 and 73, 41x1000x1000 87 and 133; red-black iteration 54x292x284
 // 27 and 30); tiles beat them as long as the sweeps' latency counts (1.4 + 2.5
 // per million padded points against 6 + 1.5: 41x300x300 13 and 15, 33x500x500
-// 31 and 29).  A kernel of many gets (`tiles` false) has no tiles and pays for
-// every lane: its passes have to cover the rows with no more of them.
+// 31 and 29).  Colour sweeps do without the last column and its tile: they also
+// win over large grids whose rows end just past a tile of the pass (us an
+// iteration, sweeps and pass: 129x249x249 34 and 35, 129x422x422 84 and 95,
+// 129x622x623 160 and 193, 257x299x299 80 and 87, 131x617x618 171 and 193,
+// 135x608x609 176 and 181; but 131x247x247 42 and 34, 141x403x404 89 and 79,
+// 257x200x200 43 and 40, 258x440x440 194 and 167, 513x312x312 165 and 141); a lane
+// of a 128-point tile counts 1.2 times.  A kernel of many gets (`tiles` false) has
+// no tiles and pays for every lane: its passes have to cover the rows with no more
+// of them.
 inline bool PassesPay(const int *dim, bool periodic, bool colours, bool tiles) {
   if (dim[0] % 4 == 0) return true;
   const int wide = PairVX(dim, periodic, colours) == 2 ? 128 : 256;
   if (!tiles) return (dim[0] + wide - 1) / wide * wide <= (dim[0] + 63) / 64 * 64;
-  if (dim[0] > 64) return true;
+  if (dim[0] > 64) {
+    const long lanes = (dim[0] + wide - 1) / wide * wide;
+    const long sweep = (dim[0] - 1 + 63) / 64 * 64;
+    const double n = (double)dim[0] * dim[1] * dim[2];
+    return !colours || TilesBeatPairs(dim, periodic, colours) ||
+           !(((wide == 128 ? 1.2 : 1.0) * lanes >= 1.75 * sweep &&
+              n >= (lanes == 256 ? 7.5e6 : 2e7)) ||
+             (lanes >= 1.85 * dim[0] && n >= 2e7));
+  }
   return TilesBeatPairs(dim, periodic, colours) &&
          2.5 * PaddedMega(dim[0], dim[1], dim[2], 16, 16, 8) <
              4.6 + 1.5 * PaddedMega(dim[0], dim[1], dim[2], 64, 1, 1);

@@ -3,10 +3,10 @@
 // "tiles": whether pairs over a domain run in resident tiles
 // (include/physis/hip/tile.h); "fits": whether a pass has a window at all; "one":
 // whether a single sweep runs at one point per lane; "vx": the points per lane of
-// a whole-grid pass, and whether it runs in tiles; "pay": whether passes over a
-// whole grid, and over its interior, beat single sweeps, and whether the last of
-// one red-black iteration runs as colour sweeps.  Built and run by
-// tests/test_planner.py; no device is touched.
+// a whole-grid pass, whether it runs in tiles and whether it beats sweeps; "pay":
+// whether passes over a whole grid, and over its interior, beat single sweeps, and
+// whether the last of one red-black iteration runs as colour sweeps.  Built and
+// run by tests/test_planner.py; no device is touched.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -73,8 +73,9 @@ int main(int argc, char **argv) {
                         std::atoi(argv[4])};
     const bool periodic = std::atoi(argv[5]) != 0;
     const bool colours = std::atoi(argv[6]) != 0;
-    std::printf("%d %d\n", physis_hip::PairVX(dim, periodic, colours),
-                physis_hip::TilesBeatPairs(dim, periodic, colours));
+    std::printf("%d %d %d\n", physis_hip::PairVX(dim, periodic, colours),
+                physis_hip::TilesBeatPairs(dim, periodic, colours),
+                physis_hip::PassesPay(dim, periodic, colours, true));
     return 0;
   }
   if (argc == 6 && std::strcmp(argv[1], "pay") == 0) {

@@ -174,3 +174,20 @@ def test_tiles_for_whole_grids(planner, extents, periodic, colours, tiles):
                         str(colours)], check=True, capture_output=True,
                        text=True)
     assert int(r.stdout.split()[1]) == tiles
+
+
+# Whole-grid red-black maps on rows that end just past a tile of the pass: colour
+# sweeps or passes, as measured.
+@pytest.mark.parametrize("extents,passes", [
+    ((129, 422, 422), False), ((129, 622, 623), False),
+    ((131, 617, 618), False), ((257, 299, 299), False),
+    ((257, 441, 441), False), ((129, 152, 152), True),
+    ((131, 247, 247), True), ((141, 403, 404), True),
+    ((128, 422, 422), True), ((193, 508, 509), True),
+    ((257, 200, 200), True), ((258, 440, 440), True),
+    ((260, 441, 441), True), ((385, 360, 360), True),
+    ((513, 312, 312), True)])
+def test_red_black_passes_just_past_a_tile(planner, extents, passes):
+    r = subprocess.run([planner, "vx", *map(str, extents), "0", "1"], check=True,
+                       capture_output=True, text=True)
+    assert int(r.stdout.split()[2]) == passes
